@@ -28,6 +28,11 @@ ATTN_PROJ = 9216
 CONV_ELEMS = 3 * 8192
 REC_ELEMS = 32 * 128 * 128
 CHUNK_RECORD_BYTES = 115712
+# Rows up to which a block is projected like a decode wave: it streams the same weights, and
+# the wave operators stay on the matrix unit where the block operators evaluate up to 16 rows
+# in the reference's order (12 rows: 28 -> 7 us out-projection, 34 -> 12 us and 27 -> 10 us
+# in-projections).
+WAVE_ROWS = 16
 
 
 def layer_kinds(layers):
@@ -226,7 +231,8 @@ class StubStack:
 
     def _project_in(self, cb, layer, rows, block):
         """normed -> proj: the layer's input projection (a decode wave or a block); with
-        _fused_wave x -> proj through the layer's input norm."""
+        _fused_wave x -> proj through the layer's input norm.  A block of 2..16 rows takes the
+        decode wave's form."""
         gated = layer["kind"] == "G"
         width = GDN_PROJ if gated else ATTN_PROJ
         if "in_q4" not in layer:
@@ -240,11 +246,11 @@ class StubStack:
                 bindings[1 + 3 * index + part] = matrix[part]
         out = 1 + 3 * len(layer["in_q4"])
         bindings[out] = self.proj
-        if block:
+        if block and not 2 <= rows <= WAVE_ROWS:
             cb.encode(self.lib.pipeline(name + "_blk"), bindings, {out + 1: rows},
                       ((width + 3) // 4,), (128,))
         else:
-            # several lanes: the matrix-unit form; one lane: the reference's own order
+            # several rows: the matrix-unit form; one: the reference's own order
             suffix = "_rms_mfma_ms" if fused else "_mfma_ms" if rows >= 2 else "_ms"
             if fused:
                 bindings[out + 3] = layer["input_norm"]
@@ -259,10 +265,10 @@ class StubStack:
             return
         words, scales, biases = layer["out_q4"]
         bindings = {0: self.mixed, 1: words, 2: scales, 3: biases, 4: self.delta}
-        if block:
+        if block and not 2 <= rows <= WAVE_ROWS:
             cb.encode(self.lib.pipeline("outproj_blk"), bindings, {5: rows, 6: 4096},
                       (HIDDEN // 2,), (64,))
-        elif self._fused_wave(layer, rows):
+        elif not block and self._fused_wave(layer, rows):
             # x = bf16(x + bf16(projection)) in place
             cb.encode(self.lib.pipeline("gdn_outproj_residual_mfma_ms"),
                       {**bindings, 4: self.x, 8: self.x}, {5: rows, 6: HIDDEN, 7: 16},
