@@ -662,7 +662,9 @@ uint32_t flash_prefill_splits(uint32_t rows, uint32_t visible, uint32_t compute_
 uint64_t stream_workspace_bytes(uint32_t compute_units) {
     // the shared walk never has more workgroups than compute units; their arrival counts
     // (at most one per two of them) stay under a page
-    return 4096 + static_cast<uint64_t>(compute_units) * kPartialBytes;
+    const uint64_t walks = 4096 + static_cast<uint64_t>(compute_units) * kPartialBytes;
+    const uint64_t projections = q4_workspace_bytes();
+    return walks > projections ? walks : projections;
 }
 
 uint64_t flash_prefill_scratch_bytes(uint32_t rows, uint32_t splits) {

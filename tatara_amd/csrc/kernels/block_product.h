@@ -1,0 +1,350 @@
+// C[m][n] = sum_k X[m][k] W[n][k] on the matrix unit for blocks of rows: both operands 16-bit
+// floats (bf16 or f16) with k contiguous, sums in fp32, and the way a tile of sums leaves is the
+// caller's.  One persistent workgroup of kWavesM x kWavesN waves owns tiles of kTileM x kTileN
+// and walks K in units of 64 columns, two steps of 32 each:
+//   * both operands go from global memory straight into LDS (16 bytes per lane and
+//     transfer, whole 128-byte lines of a row, no registers), a ring of two units.  The
+//     transfers are issued as assembly, so that the only waits are the ones written below
+//     (M0 is used for nothing else in these kernels).  A ring row is one row's 128 bytes of
+//     the unit; 16-byte piece p of row r sits in slot p ^ (r & 7), with which the 16-byte
+//     fragment reads of a wave (sixteen consecutive rows, one piece per quarter wave) were
+//     measured free of bank conflicts.
+//   * a wave multiplies its part of the tile as products of 16 x 16 x 32, W as the left
+//     operand: a lane then holds four consecutive n of one m per product.  The fragments of a
+//     step are read into registers while the step before it is multiplied; one barrier per
+//     unit.
+//   * the first two units of a workgroup's next tile are requested before it converts and
+//     stores the sums of this one.
+// m and n past the end are clamped on the way in; the caller does not store them.
+#pragma once
+
+#include <type_traits>
+
+#include "../tt_internal.h"
+
+namespace tt {
+namespace {
+
+// lane l's 16 bytes at base + offset land at lds_address + 16 l
+__device__ __forceinline__ void block_transfer(const uint8_t* base, uint32_t offset,
+                                               uint32_t lds_address) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(offset), "s"(base)
+                 : "memory");
+}
+
+// two sums to a packed bf16 pair: hardware round to nearest even, then results below the
+// normal range flushed to signed zero
+__device__ __forceinline__ uint32_t block_pack(float a, float b) {
+    typedef __attribute__((ext_vector_type(2))) float Pair;
+    typedef __attribute__((ext_vector_type(2))) __bf16 Rounded;
+    const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector(Pair{a, b}, Rounded));
+    const uint32_t keep = ((pair & 0x00007F80u) ? 0x0000FFFFu : 0x00008000u) |
+                          ((pair & 0x7F800000u) ? 0xFFFF0000u : 0x80000000u);
+    return pair & keep;
+}
+
+// four results as bf16 at columns n .. n + 3 of an output row of `out_dim`; wide: 8-byte aligned
+template <typename Sums>
+__device__ __forceinline__ void block_store(uint16_t* out_row, uint32_t n, uint32_t out_dim,
+                                            bool wide, Sums v) {
+    typedef __attribute__((ext_vector_type(2))) uint32_t Four;
+    const Four four = Four{block_pack(v[0], v[1]), block_pack(v[2], v[3])};
+    if (wide && n + 4 <= out_dim) {
+        *reinterpret_cast<Four*>(out_row + n) = four;
+    } else {
+        for (uint32_t j = 0; j < 4 && n + j < out_dim; ++j) {
+            out_row[n + j] = static_cast<uint16_t>(four[j >> 1] >> (16 * (j & 1)));
+        }
+    }
+}
+
+template <typename Element, uint32_t kTileM_, uint32_t kTileN_, uint32_t kWavesM, uint32_t kWavesN,
+          uint32_t kRing = 2>
+struct BlockProduct {
+    static constexpr uint32_t kTileM = kTileM_, kTileN = kTileN_;
+    static constexpr uint32_t kWaves = kWavesM * kWavesN;
+    static constexpr uint32_t kThreads = 64 * kWaves;
+    static constexpr uint32_t kUnitColumns = 64;
+    static constexpr uint32_t kRowBytes = kUnitColumns * 2;
+    static constexpr uint32_t kXUnitBytes = kTileM * kRowBytes;
+    static constexpr uint32_t kUnitBytes = (kTileM + kTileN) * kRowBytes;
+    static constexpr uint32_t kLdsBytes = kRing * kUnitBytes;
+    static constexpr uint32_t kWaveM = kTileM / kWavesM, kWaveN = kTileN / kWavesN;
+    static constexpr uint32_t kTm = kWaveM / 16, kTn = kWaveN / 16;
+    static constexpr uint32_t kXTransfers = kTileM / 8 / kWaves, kWTransfers = kTileN / 8 / kWaves;
+    static_assert(kLdsBytes <= 160 * 1024, "the ring fits a compute unit");
+    static_assert(kXTransfers * 8 * kWaves == kTileM && kWTransfers * 8 * kWaves == kTileN,
+                  "whole transfers");
+
+    // s_waitcnt until at most `left` transfers are in flight
+    static constexpr uint32_t vmcnt(uint32_t left) {
+        return 0x0F70u | (left & 15u) | ((left >> 4) << 14);
+    }
+    static_assert((kRing - 2) * (kXTransfers + kWTransfers) < 64, "what vmcnt counts");
+
+    typedef __attribute__((ext_vector_type(8))) Element Elements;
+    typedef __attribute__((ext_vector_type(4))) float Sums;
+    struct Fragments {
+        Elements x[kTm], w[kTn];
+    };
+
+    static __device__ __forceinline__ Sums product(Elements w, Elements x, Sums sums) {
+        if constexpr (std::is_same<Element, _Float16>::value) {
+            return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, sums, 0, 0, 0);
+        } else {
+            return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, sums, 0, 0, 0);
+        }
+    }
+
+    // x [rows][in_dim], weights [out_dim][in_dim], in_dim a multiple of 64; 16-byte aligned and
+    // each smaller than 4 GiB.  store(m, n, sums) gets the sums of row m, columns n .. n + 3.
+    template <typename Store>
+    static __device__ __forceinline__ void run(const void* x, const void* weights, uint32_t rows,
+                                               uint32_t in_dim, uint32_t out_dim, Store store) {
+        extern __shared__ __align__(16) uint8_t block_lds[];
+        const uint32_t lane = threadIdx.x & 63;
+        const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const uint32_t i16 = lane & 15, g = lane >> 4;
+        const uint32_t units = in_dim / kUnitColumns;
+        const uint32_t n_tiles = (out_dim + kTileN - 1) / kTileN;
+        const uint32_t m_tiles = (rows + kTileM - 1) / kTileM;
+        const uint32_t tiles = n_tiles * m_tiles;
+        const uint32_t lds_base = static_cast<uint32_t>(
+            reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)block_lds));
+        const uint32_t wave_n = wave % kWavesN, wave_m = wave / kWavesN;
+
+        // staging roles: the x transfers of wave w fill rows 8 kXTransfers w + 8 j .. + 7, the
+        // weight transfers likewise; lane l lands in row + (l >> 3), slot l & 7, so it fetches
+        // piece (l & 7) ^ (l >> 3) of that row
+        const uint8_t* x_base = reinterpret_cast<const uint8_t*>(x);
+        const uint8_t* w_base = reinterpret_cast<const uint8_t*>(weights);
+        const uint32_t piece = ((lane & 7) ^ (lane >> 3)) * 16;
+        const uint32_t x_row = 8 * kXTransfers * wave + (lane >> 3);
+        const uint32_t w_row = 8 * kWTransfers * wave + (lane >> 3);
+        const uint32_t row_bytes = in_dim * 2;
+        uint32_t m_aim = 0, n_aim = 0;   // first row and output of the tile the requests go to
+        // Tiles are numbered along bands of eight tile rows, down a band's columns first, so that
+        // a run of consecutive numbers is a compact patch (32 of them: eight rows x four columns,
+        // twelve operand panels for 32 tiles).
+        auto place = [&](uint32_t tile, uint32_t& m0, uint32_t& n0) {
+            const uint32_t band = tile / (8 * n_tiles);
+            const uint32_t band_rows = min(8u, m_tiles - 8 * band);
+            const uint32_t within = tile - band * 8 * n_tiles;
+            m0 = (8 * band + within % band_rows) * kTileM;
+            n0 = (within / band_rows) * kTileN;
+        };
+        // the lane offsets are worked out per request (a handful of instructions per 64
+        // products) rather than held in registers the products need
+        auto request = [&](uint32_t unit) {
+            const uint32_t to = lds_base + (unit % kRing) * kUnitBytes;
+            const uint8_t* x_unit = x_base + unit * kRowBytes;   // uniform: scalar arithmetic
+            const uint8_t* w_unit = w_base + unit * kRowBytes;
+#pragma unroll
+            for (uint32_t j = 0; j < kXTransfers; ++j) {
+                const uint32_t offset = min(m_aim + x_row + 8 * j, rows - 1) * row_bytes + piece;
+                block_transfer(x_unit, offset, to + (8 * kXTransfers * wave + 8 * j) * kRowBytes);
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kWTransfers; ++j) {
+                const uint32_t offset = min(n_aim + w_row + 8 * j, out_dim - 1) * row_bytes + piece;
+                block_transfer(w_unit, offset,
+                               to + kXUnitBytes + (8 * kWTransfers * wave + 8 * j) * kRowBytes);
+            }
+        };
+
+        // fragment of (row, step of the unit): piece 4 step + g, stored at slot piece ^ (row & 7)
+        const uint32_t frag_row = i16 * kRowBytes;
+        const uint32_t frag_piece[2] = {(g ^ (i16 & 7)) * 16, ((4 + g) ^ (i16 & 7)) * 16};
+        const uint32_t x_frag = kWaveM * wave_m * kRowBytes + frag_row;
+        const uint32_t w_frag = kXUnitBytes + kWaveN * wave_n * kRowBytes + frag_row;
+        Sums acc[kTn][kTm];
+
+        auto read_fragments = [&](uint32_t unit, uint32_t step, Fragments& f)
+                                  __attribute__((always_inline)) {
+            const uint8_t* from = block_lds + (unit % kRing) * kUnitBytes + frag_piece[step];
+#pragma unroll
+            for (uint32_t tile = 0; tile < kTn; ++tile) {
+                f.w[tile] = *reinterpret_cast<const Elements*>(from + w_frag + tile * 16 * kRowBytes);
+            }
+#pragma unroll
+            for (uint32_t tile = 0; tile < kTm; ++tile) {
+                f.x[tile] = *reinterpret_cast<const Elements*>(from + x_frag + tile * 16 * kRowBytes);
+            }
+        };
+        auto multiply = [&](const Fragments& f) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t tm = 0; tm < kTm; ++tm) {
+#pragma unroll
+                for (uint32_t tn = 0; tn < kTn; ++tn) {
+                    acc[tn][tm] = product(f.w[tn], f.x[tm], acc[tn][tm]);
+                }
+            }
+        };
+        // issue order of a slot: a read, then a few products, so that the waves' reads are
+        // spread over the slot instead of queueing at the LDS while the matrix unit waits (left
+        // alone the scheduler sinks each read to the product that needs it, a slot later).  No
+        // branch between the reads and the products: at a join the compiler would wait for the
+        // reads first.
+        auto interleave = [&]() __attribute__((always_inline)) {
+            constexpr uint32_t kReads = kTm + kTn, kBetween = kTm * kTn / kReads;
+#pragma unroll
+            for (uint32_t i = 0; i < kReads; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, kBetween, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, kTm * kTn - kReads * kBetween, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // first step of `unit` (its fragments are in `first`): read the second step's while
+        // multiplying; the unit was published a slot ago, so nothing to wait for
+        auto first_step = [&](uint32_t unit, const Fragments& first, Fragments& second)
+                              __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+            read_fragments(unit, 1, second);
+            multiply(first);
+            interleave();
+        };
+        // second step of `unit`: the next unit (requested a unit ago) has landed - mine, then
+        // everybody's -, and nobody reads the unit before this one any more, so the unit after
+        // the next goes into its place; read the next unit's first fragments while multiplying
+        auto second_step = [&](uint32_t unit, const Fragments& second, Fragments& first_of_next,
+                               auto with_request) __attribute__((always_inline)) {
+            if constexpr (decltype(with_request)::value) {
+                __builtin_amdgcn_s_waitcnt(vmcnt((kRing - 2) * (kXTransfers + kWTransfers)));
+            } else {
+                __builtin_amdgcn_s_waitcnt(vmcnt(0));
+            }
+            __syncthreads();
+            if constexpr (decltype(with_request)::value) request(unit + kRing);
+            __builtin_amdgcn_sched_barrier(0);
+            read_fragments(unit + 1, 0, first_of_next);
+            multiply(second);
+            interleave();
+        };
+        using std::bool_constant;
+
+        // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own:
+        // in a whole round the workgroups of an XCD (b / 8 = 0, 1, ...) take a run of consecutive
+        // tiles together - the operand panels a patch shares are then fetched into one L2 once
+        // instead of into several.  A round that is not filled is dealt in dispatch order, which
+        // spreads its tiles over the XCDs and their compute units.
+        const uint32_t by_xcd = gridDim.x % 8 == 0
+                                    ? (blockIdx.x & 7) * (gridDim.x / 8) + (blockIdx.x >> 3)
+                                    : blockIdx.x;
+        auto of_round = [&](uint32_t first) {
+            return first + (first + gridDim.x <= tiles ? by_xcd : blockIdx.x);
+        };
+        uint32_t round = 0, tile = of_round(0);
+        if (tile >= tiles) return;
+        place(tile, m_aim, n_aim);
+        const uint32_t ahead = min(kRing, units);
+        for (uint32_t unit = 0; unit < ahead; ++unit) request(unit);
+        while (true) {
+#pragma unroll
+            for (uint32_t tn = 0; tn < kTn; ++tn) {
+#pragma unroll
+                for (uint32_t tm = 0; tm < kTm; ++tm) acc[tn][tm] = Sums{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+            // unit 0 has landed (the second unit may be in flight; so may the stores of the tile
+            // before, and reads and writes do not retire in one order: wait for everything)
+            __builtin_amdgcn_s_waitcnt(vmcnt(0));
+            __syncthreads();
+            Fragments a, b;
+            read_fragments(0, 0, a);
+            uint32_t unit = 0;
+            for (; unit + kRing < units; ++unit) {
+                first_step(unit, a, b);
+                second_step(unit, b, a, bool_constant<true>{});
+            }
+            for (; unit + 1 < units; ++unit) {   // nothing left to request
+                first_step(unit, a, b);
+                second_step(unit, b, a, bool_constant<false>{});
+            }
+            first_step(unit, a, b);
+            multiply(b);
+
+            uint32_t m0, n0;
+            place(tile, m0, n0);
+            round += gridDim.x;
+            const uint32_t next_tile = of_round(round);
+            __syncthreads();   // nobody reads the stages any more
+            if (next_tile < tiles) {
+                place(next_tile, m_aim, n_aim);
+                for (uint32_t unit = 0; unit < ahead; ++unit) request(unit);
+            }
+            // the lane holds columns n0 + kWaveN wave_n + 16 tn + 4 g + j of row
+            // m0 + kWaveM wave_m + 16 tm + i16
+#pragma unroll
+            for (uint32_t tm = 0; tm < kTm; ++tm) {
+                const uint32_t m = m0 + kWaveM * wave_m + 16 * tm + i16;
+                if (m >= rows) continue;
+#pragma unroll
+                for (uint32_t tn = 0; tn < kTn; ++tn) {
+                    const uint32_t n = n0 + kWaveN * wave_n + 16 * tn + 4 * g;
+                    if (n < out_dim) store(m, n, acc[tn][tm]);
+                }
+            }
+            if (next_tile >= tiles) break;
+            tile = next_tile;
+        }
+    }
+};
+
+// The tiles a block product is launched with, and what one of them costs on a compute unit.
+// `single` is the time of one tile alone on it, `both`
+// of two side by side, as ns per 64 columns and ns per tile (fitted to products of 33 .. 16384
+// rows with 2048 .. 12352 outputs over K = 2176 and 4352).
+template <typename Element>
+struct BlockTiles {
+    typedef BlockProduct<Element, 256, 256, 2, 4> Large;      // the most products per LDS byte
+    typedef BlockProduct<Element, 128, 128, 2, 4> Even;       // two a compute unit hide each other's waits
+    typedef BlockProduct<Element, 128, 128, 2, 4, 3> Deep;    // one a compute unit, a unit further ahead
+    typedef BlockProduct<Element, 64, 128, 2, 4, 3> Low;
+    typedef BlockProduct<Element, 64, 64, 2, 4, 4> Small;
+};
+enum class BlockTile { Large, Even, Deep, Low, Small };
+
+// The tile with the shortest estimate.  A compute unit takes ceil(tiles / compute_units) tiles,
+// two at a time where two workgroups fit it.
+inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
+                                   uint32_t compute_units) {
+    struct Cost {
+        BlockTile tile;
+        uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
+    };
+    static constexpr Cost kCosts[] = {
+        {BlockTile::Large, 256, 256, 1700, 7000, 3400, 14000},
+        {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
+        {BlockTile::Deep, 128, 128, 570, 2000, 1140, 4000},
+        {BlockTile::Low, 64, 128, 350, 1500, 630, 3000},
+        {BlockTile::Small, 64, 64, 200, 1000, 400, 2000},
+    };
+    const uint64_t units = in_dim / 64;
+    BlockTile best = BlockTile::Large;
+    uint64_t best_time = ~0ull;
+    for (const Cost& c : kCosts) {
+        const uint64_t tiles = static_cast<uint64_t>((rows + c.m - 1) / c.m) * ((out_dim + c.n - 1) / c.n);
+        const uint64_t each = (tiles + compute_units - 1) / compute_units;
+        const uint64_t time = each / 2 * (c.both_unit * units + c.both_tile) +
+                              each % 2 * (c.single_unit * units + c.single_tile);
+        if (time < best_time) {
+            best_time = time;
+            best = c.tile;
+        }
+    }
+    return best;
+}
+// workgroups of a launch: a persistent one per place on the device, or one per tile
+template <typename Product>
+uint32_t block_workgroups(uint32_t rows, uint32_t out_dim, uint32_t compute_units) {
+    const uint32_t per_unit = 160 * 1024 / Product::kLdsBytes;
+    const uint32_t tiles = ((rows + Product::kTileM - 1) / Product::kTileM) *
+                           ((out_dim + Product::kTileN - 1) / Product::kTileN);
+    const uint32_t places = compute_units * (per_unit < 2 ? per_unit : 2);
+    return tiles < places ? tiles : places;
+}
+
+}  // namespace
+}  // namespace tt

@@ -16,11 +16,13 @@
 //    power-of-two pre-scaled inputs against masked nibbles, fused chains, the
 //    adjacent-pairs tree), so every output is the reference's bit pattern.  A half
 //    wave owns an output row; the weights are read once for all input rows.
-//  * block kernel (more rows): the nibbles are exact bf16 integers, so
-//    sum_k x q per 64-column group runs on MFMA with fp32 accumulation and the affine
-//    terms (scale per group and output row, bias against the group sums of x) are
-//    applied in fp32 - the same mathematics in another summation order.
+//  * block product (more rows): both operands are written out once as f16 numbers that
+//    hold them exactly, the affine terms as further columns, and multiplied as one
+//    matrix product with fp32 sums - the same mathematics in another summation order.
+#include <algorithm>
+
 #include "../tt_internal.h"
+#include "block_product.h"
 #include "lane_sums.h"
 #include "rms_row.h"
 
@@ -31,6 +33,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+typedef __attribute__((ext_vector_type(4))) short bf16x4_bits;
 
 constexpr uint32_t kQ4Block = 512;        // columns one pass of a 32-lane row group covers
 constexpr uint32_t kQ4Group = 64;         // columns per {scale, bias}
@@ -69,11 +72,6 @@ struct Q4Projection {
     const uint16_t* norm_weight;           // not null: the input rows go through the RMS norm first
     const uint16_t* residual;              // not null: output = bf16(residual + bf16(projection)),
     uint64_t residual_stride;              //   [rows][residual_stride]; may be the output itself
-    // the block kernel only: how its tiles are dealt to workgroups (see launch_block)
-    uint32_t tiles_n;                      // tiles along the output rows
-    uint32_t whole_tiles;                  // tiles 0 .. whole_tiles - 1 have a workgroup each
-    uint32_t sharers;                      // the others are shared by this many, a slice of K each
-    uint8_t* exchange;                     // arrival counts, then the sharers' partial sums
 };
 
 // The weight matrix that holds output row `n`, with n the same for every lane (matrices have
@@ -236,464 +234,167 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
     return TT_OK;
 }
 
-// ------------------------------------------------------------ block kernel ---
+// ----------------------------------------------------------- block product ---
 //
-// out[m][n] = sum_g scale[n][g] * (sum_{k in g} x[m][k] q[n][k]) + bias[n][g] * xs[m][g],
-// xs[m][g] = sum_{k in g} x[m][k].  A workgroup of eight waves owns 128 output rows (n) x
-// 256 input rows (m) and walks K one group (64 columns) at a time:
-//   * x (three stages), the nibble words (a pair of groups per transfer, two stages) and
-//     the scales and biases (a window of eight groups per transfer, two stages) go from
-//     global memory straight into LDS (no registers), x two groups ahead.  A nibble becomes
-//     the bf16 number 16 + nibble (dropped into mantissa bits 3..6 of 0x4180, three
-//     instructions a pair) and is written to one of two unpacked stages.  Rows are 128 B
-//     without padding; 16-byte piece p of row r sits in slot p ^ (r & 7), which keeps the
-//     16-byte fragment reads of sixteen consecutive rows free of bank conflicts.
-//   * each wave multiplies a 64 x 64 part as 4 x 4 tiles of v_mfma_f32_16x16x32_bf16 with m
-//     along the rows of the result, so a lane holds one n per tile and needs one scale per
-//     tile and group: two MFMAs per tile and group from a zero accumulator, then
-//     acc += scale[n] * partial in fp32.
-//   * xs comes from the same MFMA unit (a ones operand against the x fragments), is split
-//     into bf16 hi + lo and, once every four groups, multiplied by one
-//     v_mfma_f32_16x16x16_bf16 per tile: slots {hi, lo, hi, lo} of four groups against
-//     {bias, bias, -16 scale, -16 scale}, the latter taking the nibble offset back out.
-//   * the eight waves work as two sets of four that alternate between the matrix unit and
-//     everything else of a group, so that the two waves of a SIMD are never in the same
-//     phase (see the schedule before the main loop).
-//   * the result leaves through LDS, so that a row of 64 outputs is stored as 128
-//     contiguous bytes.
-constexpr uint32_t kBlockN = 128;                    // output rows of a workgroup tile
-constexpr uint32_t kBlockM = 256;                    // input rows of a workgroup tile
-constexpr uint32_t kBlockThreads = 512;
-constexpr uint32_t kStages = 3;                      // of what arrives from global memory
-constexpr uint32_t kRowBytes = 128;                  // one group of one row: 64 bf16
-constexpr uint32_t kXStageBytes = kBlockM * kRowBytes;                   // 32768, three of them
-// the nibble words of a pair of groups (an even one and the next): [n][16 words], two of them
-constexpr uint32_t kWordBase = kStages * kXStageBytes;
-constexpr uint32_t kWordPairBytes = kBlockN * 64;
-constexpr uint32_t kQStageBytes = kBlockN * kRowBytes;                   // unpacked: 16384, two of them
-constexpr uint32_t kQBase = kWordBase + 2 * kWordPairBytes;
-constexpr uint32_t kGroupSumBase = kQBase + 2 * kQStageBytes;
-constexpr uint32_t kGroupSumBytes = 2 * kBlockM * 8 * 2;                 // [window of 4 groups][m][4 hi, 4 lo] bf16
-// scales and biases of a window of eight groups, two windows: [window][scales, biases][n]
-// [8 bf16]
-constexpr uint32_t kMetaBase = kGroupSumBase + kGroupSumBytes;
-constexpr uint32_t kMetaKindBytes = kBlockN * 16;
-constexpr uint32_t kMetaWindowBytes = 2 * kMetaKindBytes;
-constexpr uint32_t kBlockLdsBytes = kMetaBase + 2 * kMetaWindowBytes;    // 163840
-constexpr uint32_t kOutRowBytes = 144;               // a wave's 64 results of one m on the way out
-constexpr uint32_t kExchangeCountBytes = 4096;       // arrival counts of the shared tiles (at most 1024)
-constexpr uint64_t kExchangeShareBytes = 512 * 64 * 4;   // a sharer's partial sums: 64 floats a lane
-static_assert(kBlockLdsBytes <= 160 * 1024, "one workgroup per compute unit");
-static_assert(8 * 64 * kOutRowBytes <= kWordBase, "the results leave through the idle x stages");
+// out[m][n] = sum_k x[m][k] (nibble - 8) scale[n][g] + sum_g (bias + 8 scale)[n][g] xs[m][g],
+// xs[m][g] = sum of x over the 64 columns of group g.
+//
+// A scale has 8 significant bits and nibble - 8 (-8 .. 7) three or a power of two, so their
+// product has at most 11: an f16 number, exactly.  So is x, of 8 bits.  Both are brought into
+// f16's range by a power of two per row (an output row's largest of 8 |scale| and |bias| below
+// 2^15, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): what
+// lies so far below the row's largest value that f16 rounds it (2^-26 for x) is off by 2^-34 of
+// that value at most, far less than the fp32 sums resolve.  The affine terms are four further
+// columns a group, {bias, 8 scale, bias, 8 scale} against {hi, hi, lo, lo} of the group sum in
+// two f16 parts.  One pass writes both operands so into the queue's workspace; the product is
+// then a plain one (block_product.h) and the powers of two leave with the result.
+//
+// Why not unpack inside the product: a scale per 64 columns costs a product of its own from a
+// zero accumulator and 64 fused adds a lane for every 32 products, and the unpacking is
+// repeated for every 256 rows.  That kernel reached 28 % of the matrix unit's rate (gdn_project
+// at 16384 / 2048 / 777 / 100 rows: 1178 / 189 / 103 / 38 us, outproj 359 / 65 / 46 / 36 us);
+// this pass is bound by its writes (4.4 bytes per weight byte read).
+constexpr uint32_t kAffineColumns = 4;               // per group
+__host__ __device__ constexpr uint32_t unfolded_columns(uint32_t k_size) {
+    return k_size + k_size / kQ4Group * kAffineColumns;
+}
+typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
 
-typedef __attribute__((ext_vector_type(4))) short bf16x4_bits;
-constexpr float kNibbleOffset = 16.0f;   // nibbles enter the matrix unit as 16 + nibble
+struct Unfold {
+    _Float16* weights;         // [out_rows][unfolded_columns]
+    int32_t* weight_exponents; // [out_rows]: the row's values times 2^-exponent were written
+    _Float16* rows;            // [x_rows][unfolded_columns]
+    int32_t* row_exponents;    // [x_rows]
+    uint32_t weight_rows;      // 0: the weights are there already
+    uint32_t first_row, x_rows;
+};
 
-// eight nibbles of `word` -> the eight bf16 numbers 16 + nibble, low nibble first
-__device__ __forceinline__ u32x4 offset_nibbles(uint32_t word) {
-    // byte i of `even` = 0x80 | nibble 2 i << 3, of `odd` the same for nibble 2 i + 1: the
-    // low byte of the bf16 pattern 0x4180 | nibble << 3
-    const uint32_t even = ((word << 3) & 0x78787878u) | 0x80808080u;
-    const uint32_t odd = ((word >> 1) & 0x78787878u) | 0x80808080u;
-    u32x4 out;
-    out[0] = __builtin_amdgcn_perm(odd, even, 0x0C040C00u) | 0x41004100u;
-    out[1] = __builtin_amdgcn_perm(odd, even, 0x0C050C01u) | 0x41004100u;
-    out[2] = __builtin_amdgcn_perm(odd, even, 0x0C060C02u) | 0x41004100u;
-    out[3] = __builtin_amdgcn_perm(odd, even, 0x0C070C03u) | 0x41004100u;
-    return out;
+// the power of two that brings `largest` (a magnitude) to [2^(below - 1), 2^below)
+__device__ __forceinline__ int32_t shift_below(float largest, int32_t below) {
+    const int32_t field = static_cast<int32_t>(__float_as_uint(largest) >> 23);   // no sign
+    return field == 0 ? (largest == 0.0f ? 0 : below + 125) : below + 126 - field;
 }
 
-__device__ __forceinline__ uint16_t truncate16(float v) {
-    return static_cast<uint16_t>(__float_as_uint(v) >> 16);
-}
-
-// Global memory -> LDS without passing through registers: lane l's 16 bytes at base +
-// offset land at lds_address + 16 l.  Issued as assembly so that the only waits are the
-// ones written below; M0 is used for nothing else in this kernel.
-__device__ __forceinline__ void transfer_to_lds(const uint8_t* base, uint32_t offset,
-                                                uint32_t lds_address) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(offset), "s"(base)
-                 : "memory");
-}
-
-// the same at an address of the lane's own
-__device__ __forceinline__ void transfer_piece_to_lds(const void* address, uint32_t lds_address) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(address)
-                 : "memory");
-}
-
-// the same for 4 bytes per lane at an address of the lane's own: lands at lds_address + 4 l
-__device__ __forceinline__ void transfer_dword_to_lds(const void* address, uint32_t lds_address) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(address)
-                 : "memory");
-}
-
-__global__ __launch_bounds__(kBlockThreads) void q4_block_kernel(Q4Projection p) {
-    extern __shared__ __align__(16) uint8_t lds[];
-    const uint32_t t = threadIdx.x;
-    const uint32_t lane = t & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint32_t i16 = lane & 15, g = lane >> 4;
-    const uint32_t out_rows = p.first_row[p.segments];
-    // tiles in rounds of one per compute unit, n fastest; those of the last, partly filled
-    // round are shared: `sharers` workgroups each take a slice of K (whole windows of eight
-    // groups) and the last to finish adds the others' sums to its own
-    const uint32_t shared = blockIdx.x >= p.whole_tiles;
-    const uint32_t beyond = shared ? blockIdx.x - p.whole_tiles : 0;
-    const uint32_t tile_index = shared ? p.whole_tiles + beyond / p.sharers : blockIdx.x;
-    const uint32_t sharers = shared ? p.sharers : 1;
-    const uint32_t share = shared ? beyond % p.sharers : 0;
-    const uint32_t n0 = (tile_index % p.tiles_n) * kBlockN, m0 = (tile_index / p.tiles_n) * kBlockM;
-    const uint32_t all_groups = p.k_size / kQ4Group;
-    const uint32_t first_group = all_groups / sharers * share;   // a multiple of 8
-    const uint32_t groups = first_group + all_groups / sharers;   // this workgroup's end
-    const uint32_t lds_base = static_cast<uint32_t>(
-        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)lds));
-    // multiply role: the waves form two sets of four, the two waves that share a SIMD in
-    // different sets (waves w and w + 4, as a workgroup's waves are dealt to the SIMDs in
-    // turn); wave (mq, nh) owns m in [64 mq, +64), n in [64 nh, +64) of the tile
-    const uint32_t second_set = wave >> 2;
-    const uint32_t nh = wave & 1, mq = 2 * second_set + ((wave >> 1) & 1);
-
-    // which weight matrix a global output row lives in
-    auto locate = [&](uint32_t n, const uint32_t*& words, const uint16_t*& scales,
-                      const uint16_t*& biases) {
-        uint32_t segment = 0;
-        while (segment + 1 < p.segments && n >= p.first_row[segment + 1]) ++segment;
-        const uint64_t local = n - p.first_row[segment];
-        words = p.words[segment] + local * (p.k_size / 8);
-        scales = p.scales[segment] + local * all_groups;
-        biases = p.biases[segment] + local * all_groups;
-    };
-
-    // ---- staging roles
-    // x: transfer j of wave w fills rows 32 w + 8 j .. + 7; lane l lands in row + (l >> 3),
-    // slot l & 7, so it fetches piece (l & 7) ^ (l >> 3) of that row
-    const uint8_t* x_base = reinterpret_cast<const uint8_t*>(p.input);
-    uint32_t x_offset[4];
+// grid ceil((weight_rows + x_rows) / 4) x 256: a wave per row
+template <uint32_t kBlocks>   // k_size / 512
+__global__ __launch_bounds__(256) void q4_unfold_kernel(Q4Projection p, Unfold u) {
+    constexpr uint32_t kColumns = unfolded_columns(kBlocks * kQ4Block);
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row < u.weight_rows) {
+        const Q4Matrix matrix = matrix_of_row(p, row);
+        const uint64_t local = row - matrix.first_row;
+        const uint32_t* words = matrix.words + local * (kBlocks * 64);
+        const uint16_t* scales = matrix.scales + local * (kBlocks * 8);
+        const uint16_t* biases = matrix.biases + local * (kBlocks * 8);
+        uint32_t packed[kBlocks];
+        float scale[kBlocks], bias[kBlocks];
+        float largest = 0.0f;
 #pragma unroll
-    for (uint32_t j = 0; j < 4; ++j) {
-        const uint32_t row = min(m0 + 32 * wave + 8 * j + (lane >> 3), p.rows - 1);
-        x_offset[j] = static_cast<uint32_t>(row * p.input_stride * 2) + (((lane & 7) ^ (lane >> 3)) * 16);
-    }
-    // words: one transfer of wave w per pair of groups fills rows 16 w .. 16 w + 15 with the
-    // sixteen words of the pair (lane l: piece l & 3 of row l >> 2); the same wave unpacks
-    // them (lane l: words 2 (l & 3), 2 (l & 3) + 1 of a group of row l >> 2), so its own wait
-    // covers them
-    const uint32_t* word_source;
-    {
-        const uint16_t *unused_scales, *unused_bias;
-        locate(min(n0 + 16 * wave + (lane >> 2), out_rows - 1), word_source, unused_scales, unused_bias);
-        word_source += 4 * (lane & 3);
-    }
-    // scales and biases: one 4-byte transfer each per window of eight groups and wave, for a
-    // quarter of the rows of the wave's n half (lane l: groups 2 (l & 3), 2 (l & 3) + 1 of
-    // the window, row l >> 2 of the quarter); the other quarters come from the other three
-    // waves of the half, and two barriers pass between a window's arrival and its first use
-    const uint16_t *scale_source, *bias_source;
-    {
-        const uint32_t* unused_words;
-        locate(min(n0 + 64 * nh + 16 * (wave >> 1) + (lane >> 2), out_rows - 1), unused_words,
-               scale_source, bias_source);
-        scale_source += 2 * (lane & 3);
-        bias_source += 2 * (lane & 3);
-    }
-    const uint32_t q_row = t >> 2, q_quarter = t & 3;
-    const uint32_t q_slot0 = q_row * kRowBytes + (((2 * q_quarter) ^ (q_row & 7)) * 16);
-    const uint32_t q_slot1 = q_row * kRowBytes + (((2 * q_quarter + 1) ^ (q_row & 7)) * 16);
-
-    auto request = [&](uint32_t group) {
-        const uint32_t stage = lds_base + (group % kStages) * kXStageBytes;
-        const uint8_t* x_group = x_base + group * kRowBytes;   // uniform: scalar arithmetic
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            transfer_to_lds(x_group, x_offset[j], stage + (32 * wave + 8 * j) * kRowBytes);
+        for (uint32_t b = 0; b < kBlocks; ++b) {
+            // word `lane` of the block's 64: columns 8 lane .. 8 lane + 7, group lane / 8
+            packed[b] = words[b * 64 + lane];
+            scale[b] = widen(scales[b * 8 + (lane >> 3)]);
+            bias[b] = widen(biases[b * 8 + (lane >> 3)]);
+            largest = fmaxf(largest, fmaxf(8.0f * fabsf(scale[b]), fabsf(bias[b])));
         }
-        if ((group & 1) == 0) {
-            transfer_piece_to_lds(word_source + group * 8,
-                                  lds_base + kWordBase + ((group >> 1) & 1) * kWordPairBytes +
-                                      16 * wave * 64);
-        }
-        if ((group & 7) == 0) {
-            const uint32_t window = lds_base + kMetaBase + ((group >> 3) & 1) * kMetaWindowBytes +
-                                    (64 * nh + 16 * (wave >> 1)) * 16;
-            transfer_dword_to_lds(scale_source + group, window);
-            transfer_dword_to_lds(bias_source + group, window + kMetaKindBytes);
-        }
-    };
-    // the nibble words of `group` that this lane unpacks
-    auto read_words = [&](uint32_t group) {
-        return *reinterpret_cast<const u32x2*>(lds + kWordBase + ((group >> 1) & 1) * kWordPairBytes +
-                                               q_row * 64 + (group & 1) * 32 + q_quarter * 8);
-    };
-    auto commit = [&](uint32_t group, u32x2 words) {
-        uint8_t* stage = lds + kQBase + (group & 1) * kQStageBytes;
-        *reinterpret_cast<u32x4*>(stage + q_slot0) = offset_nibbles(words[0]);
-        *reinterpret_cast<u32x4*>(stage + q_slot1) = offset_nibbles(words[1]);
-    };
-
-    // ---- multiply role: in a 16 x 16 result the lane holds m = 4 g .. 4 g + 3 of column n = i16
-    // fragment of (row, 32-column step): piece 4 step + g, stored at slot piece ^ (row & 7)
-    const uint32_t piece_offset[2] = {((g ^ (i16 & 7)) * 16), (((4 + g) ^ (i16 & 7)) * 16)};
-    const uint32_t x_frag = (64 * mq + i16) * kRowBytes;
-    const uint32_t q_frag = (64 * nh + i16) * kRowBytes;
-    uint16_t* group_sums = reinterpret_cast<uint16_t*>(lds + kGroupSumBase);
-    f32x4 acc[4][4];
 #pragma unroll
-    for (uint32_t tn = 0; tn < 4; ++tn) {
+        for (uint32_t step = 8; step < 64; step *= 2) largest = fmaxf(largest, __shfl_xor(largest, step));
+        const int32_t shift = shift_below(largest, 15);
+        if (lane == 0) u.weight_exponents[row] = -shift;
+        _Float16* out = u.weights + static_cast<uint64_t>(row) * kColumns;
 #pragma unroll
-        for (uint32_t tm = 0; tm < 4; ++tm) acc[tn][tm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    bf16x8 ones;
+        for (uint32_t b = 0; b < kBlocks; ++b) {
+            const _Float16 step = static_cast<_Float16>(ldexpf(scale[b], shift));
+            const f16x2 steps = f16x2{step, step};
+            const f16x2 offset = f16x2{static_cast<_Float16>(1032.0f), static_cast<_Float16>(1032.0f)};
+            u32x4 eight;
 #pragma unroll
-    for (uint32_t e = 0; e < 8; ++e) ones[e] = static_cast<__bf16>(1.0f);
-    const f32x4 zero = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // sum_g (bias[n][g] - 16 scale[n][g]) xs[m][g] over the four groups that start at
-    // `first_group`: one MFMA per tile with the sixteen slots {hi, lo, hi, lo} of the sums
-    // against {bias, bias, -16 scale, -16 scale}
-    bf16x4_bits affine_weights[4], affine_sums[4];
-    auto read_affine_terms = [&](uint32_t first_group) __attribute__((always_inline)) {
-        const uint8_t* meta = lds + kMetaBase + ((first_group >> 3) & 1) * kMetaWindowBytes +
-                              (1 - (g >> 1)) * kMetaKindBytes + (first_group & 4) * 2;
-        // lanes g = 0, 1 carry the biases (which sit after the scales), g = 2, 3 the scales
-        const float factor = (g >> 1) ? -kNibbleOffset : 1.0f;
-#pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
-            const uint32_t row = 64 * nh + 16 * tn + i16;
-            const u32x2 pairs = *reinterpret_cast<const u32x2*>(meta + row * 16);
-            u32x2 bits;
-#pragma unroll
-            for (uint32_t j = 0; j < 2; ++j) {
-                const uint32_t pair = pairs[j];
-                // times 1 or times -16: exact in bf16
-                const float low = factor * __uint_as_float(pair << 16);
-                const float high = factor * __uint_as_float(pair & 0xFFFF0000u);
-                bits[j] = (__float_as_uint(low) >> 16) | (__float_as_uint(high) & 0xFFFF0000u);
+            for (uint32_t i = 0; i < 4; ++i) {
+                // nibbles 2 i and 2 i + 1 as 1024 + nibble
+                const uint32_t pair = 0x64006400u | ((packed[b] >> (8 * i)) & 0xFu) |
+                                      (((packed[b] >> (8 * i + 4)) & 0xFu) << 16);
+                eight[i] = __builtin_bit_cast(uint32_t,
+                                              (__builtin_bit_cast(f16x2, pair) - offset) * steps);
             }
-            affine_weights[tn] = __builtin_bit_cast(bf16x4_bits, bits);
-        }
-        const uint16_t* sums_window = group_sums + ((first_group >> 2) & 1) * (kBlockM * 8);
-#pragma unroll
-        for (uint32_t tm = 0; tm < 4; ++tm) {
-            affine_sums[tm] = *reinterpret_cast<const bf16x4_bits*>(
-                sums_window + (64 * mq + 16 * tm + i16) * 8 + 4 * (g & 1));
-        }
-    };
-    auto add_affine_terms = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (uint32_t tm = 0; tm < 4; ++tm) {
-#pragma unroll
-            for (uint32_t tn = 0; tn < 4; ++tn) {
-                acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                    affine_sums[tm], affine_weights[tn], acc[tn][tm], 0, 0, 0);
+            *reinterpret_cast<u32x4*>(out + b * kQ4Block + lane * 8) = eight;
+            if ((lane & 7) == 0) {
+                const _Float16 first = static_cast<_Float16>(ldexpf(bias[b], shift));
+                const _Float16 second = static_cast<_Float16>(ldexpf(scale[b], shift + 3));
+                *reinterpret_cast<f16x4*>(out + kBlocks * kQ4Block +
+                                          (b * 8 + (lane >> 3)) * kAffineColumns) =
+                    f16x4{first, second, first, second};
             }
         }
-    };
-
-    // The two sets alternate: while one multiplies group g from registers (the matrix
-    // unit), the other does everything else of its group - requests the transfers of two
-    // groups ahead, reads its fragments from LDS, unpacks its share of the next group's
-    // nibbles - and a barrier separates the slots.  The second set runs one slot behind the
-    // first.  In the slot of its `fetch (g)` a wave
-    //   * waits for the transfers it requested in its fetch (g - 1): group g + 1,
-    //   * reads the fragments of group g: x (g) has landed and the nibbles of g are unpacked,
-    //     because every wave waited for its transfers of g and unpacked its share in its
-    //     fetch (g - 1), one or two slots ago,
-    //   * requests group g + 2 into the x stage that both sets read in their fetch (g - 1),
-    //   * unpacks its share of the nibbles of group g + 1 into the unpacked stage that both
-    //     sets read in their fetch (g - 1).
-    // The group sums are exchanged between the two waves of an m quarter, which belong to
-    // the same set; a window of scales and biases arrives two barriers before its first use.
-    bf16x8 xf[4][2], qf[4][2];
-    float scale[4];
-    auto fetch = [&](uint32_t group) __attribute__((always_inline)) {
-        // the transfers this wave requested in its last fetch (group g + 1) have landed
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        u32x2 words;
-        if (group + 1 < groups) words = read_words(group + 1);   // first, to have them first
-        const uint8_t* stage = lds + (group % kStages) * kXStageBytes;
-        const uint8_t* q_stage = lds + kQBase + (group & 1) * kQStageBytes;
+    } else if (row - u.weight_rows < u.x_rows) {
+        const uint32_t at = row - u.weight_rows;
+        const uint16_t* x = p.input + static_cast<uint64_t>(u.first_row + at) * p.input_stride + lane * 8;
+        u32x4 raw[kBlocks];
+        uint32_t largest = 0;   // bf16 magnitudes order as their bits
 #pragma unroll
-        for (uint32_t tile = 0; tile < 4; ++tile) {
+        for (uint32_t b = 0; b < kBlocks; ++b) {
+            raw[b] = *reinterpret_cast<const u32x4*>(x + b * kQ4Block);
 #pragma unroll
-            for (uint32_t step = 0; step < 2; ++step) {
-                xf[tile][step] = *reinterpret_cast<const bf16x8*>(
-                    stage + x_frag + tile * 16 * kRowBytes + piece_offset[step]);
-                qf[tile][step] = *reinterpret_cast<const bf16x8*>(
-                    q_stage + q_frag + tile * 16 * kRowBytes + piece_offset[step]);
+            for (uint32_t i = 0; i < 4; ++i) {
+                largest = max(largest, max(raw[b][i] & 0x7FFFu, (raw[b][i] >> 16) & 0x7FFFu));
             }
         }
-        // everything else the multiply reads from LDS, so that the multiply reads nothing:
-        // the group's scales and, every fourth group, the affine terms of the four before
-        const uint8_t* scale_pairs = lds + kMetaBase + ((group >> 3) & 1) * kMetaWindowBytes +
-                                     ((group >> 1) & 3) * 4;
-        // bytes {0, 1} (even group) or {2, 3} (odd group) of a pair into the upper half, zeros below
-        const uint32_t pick = (group & 1) ? 0x03020C0Cu : 0x01000C0Cu;
 #pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
-            scale[tn] = __uint_as_float(__builtin_amdgcn_perm(
-                0u, *reinterpret_cast<const uint32_t*>(scale_pairs + (64 * nh + 16 * tn + i16) * 16), pick));
+        for (uint32_t step = 1; step < 64; step *= 2) {
+            largest = max(largest, static_cast<uint32_t>(__shfl_xor(static_cast<int>(largest), step)));
         }
-        if ((group & 3) == 0 && group != first_group) read_affine_terms(group - 4);
-        // the transfers overlap the reads above; they go into the x stage that both sets read
-        // in their fetch (g - 1)
-        if (group + 2 < groups) request(group + 2);
-        if (group + 1 < groups) commit(group + 1, words);
-    };
-    auto multiply = [&](uint32_t group) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_setprio(1);
-        // the four groups before this one are complete since this set's last multiply
-        if ((group & 3) == 0 && group != first_group) add_affine_terms();
+        const int32_t shift = shift_below(__uint_as_float(largest << 16), 9);
+        if (lane == 0) u.row_exponents[at] = -shift;
+        _Float16* out = u.rows + static_cast<uint64_t>(at) * kColumns;
 #pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
+        for (uint32_t b = 0; b < kBlocks; ++b) {
+            u32x4 eight;
+            float sum = 0.0f;
 #pragma unroll
-            for (uint32_t tm = 0; tm < 4; ++tm) {
-                f32x4 part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[tm][0], qf[tn][0], zero, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf[tm][1], qf[tn][1], part, 0, 0, 0);
-#pragma unroll
-                for (uint32_t j = 0; j < 4; ++j) acc[tn][tm][j] = fmaf(scale[tn], part[j], acc[tn][tm][j]);
+            for (uint32_t i = 0; i < 4; ++i) {
+                const float low = ldexpf(widen_half(raw[b][i], 0), shift);
+                const float high = ldexpf(widen_half(raw[b][i], 1), shift);
+                sum += low + high;
+                eight[i] = __builtin_bit_cast(
+                    uint32_t, f16x2{static_cast<_Float16>(low), static_cast<_Float16>(high)});
             }
-        }
-        // issue order: the scale FMAs of a tile go into the shadow of the MFMAs two tiles on
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            *reinterpret_cast<u32x4*>(out + b * kQ4Block + lane * 8) = eight;
 #pragma unroll
-        for (uint32_t tile = 0; tile < 14; ++tile) {
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
-        // the FMAs belong to this block: left to itself the compiler sinks all 64 behind the
-        // group sums, where nothing overlaps them
-#pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
-#pragma unroll
-            for (uint32_t tm = 0; tm < 4; ++tm) asm volatile("" : "+v"(acc[tn][tm]));
-        }
-        // group sums of two of this wave's four m tiles (the other n half takes the others):
-        // every row of the result is the sum; lanes g = 0, 2 store hi, lanes g = 1, 3 lo (the
-        // same value to the same place twice, so that no lane has to be switched off)
-        uint16_t* sum_slot = group_sums + ((group >> 2) & 1) * (kBlockM * 8) + (64 * mq + i16) * 8 +
-                             4 * (g & 1) + (group & 3);
-#pragma unroll
-        for (uint32_t tm = 0; tm < 4; ++tm) {
-            if ((tm >> 1) != nh) continue;   // wave-uniform; keeps the fragment index static
-            f32x4 sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, xf[tm][0], zero, 0, 0, 0);
-            sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, xf[tm][1], sum, 0, 0, 0);
-            const float hi = __uint_as_float(__float_as_uint(sum[0]) & 0xFFFF0000u);
-            sum_slot[16 * tm * 8] = truncate16((g & 1) ? sum[0] - hi : hi);
-        }
-        __builtin_amdgcn_s_setprio(0);
-    };
-
-    request(first_group);
-    request(first_group + 1);   // the group count of a share is a multiple of 8
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    commit(first_group, read_words(first_group));
-    __syncthreads();
-    // every wave passes 2 * groups + 1 barriers: the second set one before its first slot,
-    // the first set one after its last
-    if (second_set) __syncthreads();
-    for (uint32_t group = first_group; group < groups; ++group) {
-        fetch(group);
-        __syncthreads();
-        multiply(group);
-        __syncthreads();
-    }
-    if (!second_set) __syncthreads();
-    read_affine_terms(groups - 4);
-    add_affine_terms();
-
-    __syncthreads();   // nobody reads the stages any more (nor the sums, which the tiles do not reach)
-    if (sharers > 1) {
-        // Every sharer but the last to finish leaves its sums - device-scope stores of single
-        // words, which go through to memory whatever an L2 holds, [value][thread] so that a
-        // store instruction writes 256 contiguous bytes - waits for their acknowledgement,
-        // counts itself in and goes; the one whose count comes back sharers - 1 adds the
-        // others' to its own and stores the tile.  The launcher clears the counts.
-        uint32_t* const arrival = reinterpret_cast<uint32_t*>(lds + kBlockLdsBytes - 16);
-        float* const sums = reinterpret_cast<float*>(p.exchange + kExchangeCountBytes) +
-                            static_cast<uint64_t>(beyond / p.sharers) * p.sharers * (kBlockThreads * 64);
-        float* const mine = sums + static_cast<uint64_t>(share) * (kBlockThreads * 64) + t;
-#pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
-#pragma unroll
-            for (uint32_t tm = 0; tm < 4; ++tm) {
-#pragma unroll
-                for (uint32_t j = 0; j < 4; ++j) {
-                    __hip_atomic_store(reinterpret_cast<uint32_t*>(mine + ((tn * 4 + tm) * 4 + j) * kBlockThreads),
-                                       __float_as_uint(acc[tn][tm][j]), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        if (t == 0) {
-            *arrival = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(p.exchange) + beyond / p.sharers, 1u,
-                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        if (*arrival != sharers - 1) return;
-        for (uint32_t other = 0; other < sharers; ++other) {
-            if (other == share) continue;
-            const float* theirs = sums + static_cast<uint64_t>(other) * (kBlockThreads * 64) + t;
-#pragma unroll
-            for (uint32_t tn = 0; tn < 4; ++tn) {
-#pragma unroll
-                for (uint32_t tm = 0; tm < 4; ++tm) {
-#pragma unroll
-                    for (uint32_t j = 0; j < 4; ++j) {
-                        acc[tn][tm][j] += __uint_as_float(__hip_atomic_load(
-                            reinterpret_cast<const uint32_t*>(theirs + ((tn * 4 + tm) * 4 + j) * kBlockThreads),
-                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-                    }
-                }
-            }
-        }
-        __syncthreads();   // the count has been read by every wave before the tiles reach its place
-    }
-    // ---- store: through a tile of the wave's own in LDS ([m][n], rows 16 B apart from a
-    // multiple of 128), read back as 16-byte pieces: 128 contiguous bytes per m
-    uint8_t* tile = lds + wave * 64 * kOutRowBytes;
-#pragma unroll
-    for (uint32_t tm = 0; tm < 4; ++tm) {
-#pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
-#pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
-                *reinterpret_cast<uint16_t*>(tile + (16 * tm + 4 * g + j) * kOutRowBytes +
-                                             (16 * tn + i16) * 2) = store16(acc[tn][tm][j]);
-            }
-        }
-    }
-    const bool wide = ((reinterpret_cast<uintptr_t>(p.output) | (p.output_stride * 2)) & 15) == 0;
-#pragma unroll
-    for (uint32_t piece = lane; piece < 64 * 8; piece += 64) {
-        const uint32_t row = piece >> 3, m = m0 + 64 * mq + row;
-        const uint32_t n = n0 + 64 * nh + 8 * (piece & 7);
-        if (m >= p.rows || n >= out_rows) continue;
-        const u32x4 eight = *reinterpret_cast<const u32x4*>(tile + row * kOutRowBytes + (piece & 7) * 16);
-        uint16_t* out = p.output + static_cast<uint64_t>(m) * p.output_stride + n;
-        if (wide && n + 8 <= out_rows) {
-            *reinterpret_cast<u32x4*>(out) = eight;
-        } else {
-            for (uint32_t e = 0; e < 8 && n + e < out_rows; ++e) {
-                out[e] = static_cast<uint16_t>(eight[e >> 1] >> (16 * (e & 1)));
+            for (uint32_t step = 1; step < 8; step *= 2) sum += __shfl_xor(sum, step);
+            if ((lane & 7) == 0) {
+                const _Float16 high = static_cast<_Float16>(sum);
+                const _Float16 low = static_cast<_Float16>(sum - static_cast<float>(high));
+                *reinterpret_cast<f16x4*>(out + kBlocks * kQ4Block +
+                                          (b * 8 + (lane >> 3)) * kAffineColumns) =
+                    f16x4{high, high, low, low};
             }
         }
     }
 }
 
-// What the block kernel assumes of its operands beyond their sizes: its transfers move
-// 16-byte pieces of x and of the nibble words and 4-byte pairs of scales and biases, and it
-// addresses x with 32-bit byte offsets.
+template <typename Product>
+__global__ __launch_bounds__(Product::kThreads) void q4_product_kernel(Unfold u, uint16_t* output,
+                                                                      uint64_t output_stride,
+                                                                      uint32_t columns,
+                                                                      uint32_t out_rows) {
+    const bool wide = ((reinterpret_cast<uintptr_t>(output) | (output_stride * 2)) & 7) == 0;
+    Product::run(u.rows, u.weights, u.x_rows, columns, out_rows,
+                 [&](uint32_t m, uint32_t n, typename Product::Sums sums) {
+                     typedef __attribute__((ext_vector_type(4))) int32_t Exponents;
+                     const int32_t row_exponent = u.row_exponents[m];
+                     const Exponents exponents = *reinterpret_cast<const Exponents*>(u.weight_exponents + n);
+#pragma unroll
+                     for (uint32_t j = 0; j < 4; ++j) {
+                         sums[j] = ldexpf(sums[j], row_exponent + exponents[j]);
+                     }
+                     block_store(output + static_cast<uint64_t>(u.first_row + m) * output_stride, n,
+                                 out_rows, wide, sums);
+                 });
+}
+
+// What the pass assumes of its operands beyond their sizes: 16-byte pieces of x (and of the
+// nibble words and 4-byte pairs of scales and biases, which every block call has been held to).
 int32_t check_block_operands(const Q4Projection& p) {
     uintptr_t wide = reinterpret_cast<uintptr_t>(p.input), narrow = 0;
     for (uint32_t s = 0; s < p.segments; ++s) {
@@ -709,54 +410,74 @@ int32_t check_block_operands(const Q4Projection& p) {
     return TT_OK;
 }
 
-__global__ void clear_counts_kernel(uint32_t* words, uint32_t count) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) words[i] = 0;
+// The workspace of a block: the unfolded weights of the largest projection and the unfolded
+// rows of 16384 tokens at the hidden width (8192 at the attention width); a longer block goes
+// through in slices of that many rows.
+constexpr uint64_t kUnfoldedWeightBytes =
+    static_cast<uint64_t>(kGdnProjectionRows) * unfolded_columns(kHidden) * 2;
+constexpr uint64_t kUnfoldedRowBytes = 16384ull * unfolded_columns(kHidden) * 2;
+constexpr uint64_t kWeightExponentBytes = (kGdnProjectionRows * 4 + 255) / 256 * 256;
+constexpr uint64_t kRowExponentBytes = 16384ull * 4;
+constexpr uint64_t kUnfoldWorkspaceBytes =
+    kUnfoldedWeightBytes + kUnfoldedRowBytes + kWeightExponentBytes + kRowExponentBytes;
+static_assert(kUnfoldedWeightBytes % 256 == 0 && kUnfoldedRowBytes % 256 == 0, "aligned parts");
+static_assert(static_cast<uint64_t>(kHidden) * unfolded_columns(kGdnValueValues) <=
+                  static_cast<uint64_t>(kGdnProjectionRows) * unfolded_columns(kHidden),
+              "the output projection's weights fit as well");
+
+typedef BlockTiles<_Float16> Q4Tiles;
+template <typename Product>
+void launch_product(const Q4Projection& p, const Unfold& u, uint32_t compute_units, hipStream_t stream) {
+    const uint32_t out_rows = p.first_row[p.segments];
+    hipLaunchKernelGGL(q4_product_kernel<Product>,
+                       dim3(block_workgroups<Product>(u.x_rows, out_rows, compute_units)),
+                       dim3(Product::kThreads), Product::kLdsBytes, stream, u, p.output, p.output_stride,
+                       unfolded_columns(p.k_size), out_rows);
 }
 
-// Tiles go to workgroups in rounds of one per compute unit.  A block of the reference's size
-// leaves the last round partly filled - 2048 rows of the attention in-projection are 576 tiles,
-// two rounds and a quarter on 256 compute units, of the out-projection 128, half a round - and
-// a partly filled round costs a whole one.  Where the queue has a workspace, the tiles of that
-// round are shared: 2, 4 or 8 workgroups (as many as fit the idle compute units and divide
-// the windows of eight groups) take a slice of K each and exchange their sums through it.
-int32_t launch_block(const Q4Projection& projection, hipStream_t stream) {
-    Q4Projection p = projection;
-    const uint32_t out_rows = p.first_row[p.segments];
-    p.tiles_n = (out_rows + kBlockN - 1) / kBlockN;
-    const uint32_t tiles = p.tiles_n * ((p.rows + kBlockM - 1) / kBlockM);
-    p.whole_tiles = tiles;
-    p.sharers = 1;
-    p.exchange = nullptr;
+int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
     const StreamWorkspace workspace = stream_workspace(stream);
-    if (workspace.base != nullptr && workspace.compute_units != 0) {
-        const uint32_t units = workspace.compute_units;
-        const uint32_t last_round = tiles % units;
-        const uint32_t windows = p.k_size / (8 * kQ4Group);
-        uint32_t sharers = 1;
-        for (uint32_t s = 8; s >= 2 && last_round != 0; s >>= 1) {
-            if (last_round * s <= units && windows % s == 0) {
-                sharers = s;
-                break;
-            }
-        }
-        if (sharers > 1 && last_round * 4 <= kExchangeCountBytes &&
-            kExchangeCountBytes + last_round * sharers * kExchangeShareBytes <= workspace.bytes) {
-            p.whole_tiles = tiles - last_round;
-            p.sharers = sharers;
-            p.exchange = workspace.base;
-            hipLaunchKernelGGL(clear_counts_kernel, dim3((last_round + 255) / 256), dim3(256), 0, stream,
-                               reinterpret_cast<uint32_t*>(p.exchange), last_round);
-        }
+    // a queue whose workspace could not be allocated: the rows kernel takes any number of rows
+    if (workspace.base == nullptr || workspace.bytes < kUnfoldWorkspaceBytes ||
+        workspace.compute_units == 0) {
+        return launch_rows(p, stream);
     }
-    const uint32_t workgroups = p.whole_tiles + (tiles - p.whole_tiles) * p.sharers;
-    hipLaunchKernelGGL(q4_block_kernel, dim3(workgroups), dim3(kBlockThreads), kBlockLdsBytes, stream, p);
+    const uint32_t columns = unfolded_columns(p.k_size);
+    const uint32_t out_rows = p.first_row[p.segments];
+    Unfold u{};
+    u.weights = reinterpret_cast<_Float16*>(workspace.base);
+    u.rows = reinterpret_cast<_Float16*>(workspace.base + kUnfoldedWeightBytes);
+    u.weight_exponents =
+        reinterpret_cast<int32_t*>(workspace.base + kUnfoldedWeightBytes + kUnfoldedRowBytes);
+    u.row_exponents = reinterpret_cast<int32_t*>(
+        reinterpret_cast<uint8_t*>(u.weight_exponents) + kWeightExponentBytes);
+    u.weight_rows = out_rows;
+    const uint32_t slice = static_cast<uint32_t>(kUnfoldedRowBytes / 2 / columns) / 256 * 256;
+    for (u.first_row = 0; u.first_row < p.rows; u.first_row += u.x_rows) {
+        u.x_rows = std::min(slice, p.rows - u.first_row);
+        const dim3 grid((u.weight_rows + u.x_rows + 3) / 4);
+        if (p.k_size == 4 * kQ4Block) {
+            hipLaunchKernelGGL(q4_unfold_kernel<4>, grid, dim3(256), 0, stream, p, u);
+        } else {
+            hipLaunchKernelGGL(q4_unfold_kernel<8>, grid, dim3(256), 0, stream, p, u);
+        }
+        u.weight_rows = 0;
+        auto launch = launch_product<Q4Tiles::Large>;
+        switch (choose_block_tile(u.x_rows, columns, out_rows, workspace.compute_units)) {
+        case BlockTile::Large: break;
+        case BlockTile::Even: launch = launch_product<Q4Tiles::Even>; break;
+        case BlockTile::Deep: launch = launch_product<Q4Tiles::Deep>; break;
+        case BlockTile::Low: launch = launch_product<Q4Tiles::Low>; break;
+        case BlockTile::Small: launch = launch_product<Q4Tiles::Small>; break;
+        }
+        launch(p, u, workspace.compute_units, stream);
+    }
     return TT_OK;
 }
 
 // ------------------------------------------------------- decode-wave kernel ---
 //
-// The same mathematics as the block kernel for 2..16 input rows (a decode wave), sized for
+// The same mathematics as the block product for 2..16 input rows (a decode wave), sized for
 // latency: a workgroup owns 16 output rows and all input rows, its waves split K in slices
 // of 512 columns (eight groups each), every operand of a slice is requested before the
 // first is used, and the slices are summed through LDS in a fixed order.  Per group four
@@ -765,6 +486,8 @@ int32_t launch_block(const Q4Projection& projection, hipStream_t stream) {
 // the group sums of x; then acc += scale[n] * products + bias[n] * sums in fp32.  The
 // result has n along its columns, so a lane needs one scale and one bias per group, and
 // reads all eight of a slice with two 16-byte loads.
+
+constexpr float kNibbleOffset = 16.0f;   // nibbles enter the matrix unit as 16 + nibble
 
 // nibbles 0..3 (upper = false) or 4..7 of `word` -> the four bf16 numbers 16 + nibble: a
 // nibble dropped into mantissa bits 3..6 of bf16 16.0 (0x4180), where it counts units.  The
@@ -1177,11 +900,19 @@ int32_t op_outproj_blk(const Bindings& b, const Grid& g, hipStream_t s, bool v) 
 
 }  // namespace
 
+uint64_t q4_workspace_bytes() { return kUnfoldWorkspaceBytes; }
+
 #if !defined(__HIP_DEVICE_COMPILE__)  // host-side table of launchers
 bool prepare_q4_kernels() {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(q4_block_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               kBlockLdsBytes) == hipSuccess &&
+    const auto allow = [](auto product, const void* kernel) {
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   decltype(product)::kLdsBytes) == hipSuccess;
+    };
+    return allow(Q4Tiles::Large{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Large>)) &&
+           allow(Q4Tiles::Even{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Even>)) &&
+           allow(Q4Tiles::Deep{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Deep>)) &&
+           allow(Q4Tiles::Low{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Low>)) &&
+           allow(Q4Tiles::Small{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Small>)) &&
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<4, true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                kRowsStagedBytes) == hipSuccess &&

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "../tt_internal.h"
+#include "block_product.h"
 #include "lane_sums.h"
 #include "rms_row.h"
 
@@ -129,252 +130,16 @@ __global__ __launch_bounds__(256) void dense_bf16_kernel(const uint16_t* input,
     }
 }
 
-// The same for a block of rows, sized for the matrix unit.  One persistent workgroup of
-// eight waves per compute unit; a workgroup owns tiles of 256 rows x 256 outputs (128 flop
-// per operand byte it fetches) and walks K in units of 64 columns, two steps of 32 each:
-//   * both operands go from global memory straight into LDS (16 bytes per lane and
-//     transfer, whole 128-byte lines of a row, no registers), a ring of two units of
-//     64 KiB.  The transfers are issued as assembly, so that the only waits are the ones
-//     written below (M0 is used for nothing else in this kernel).  A ring row is one
-//     row's 128 bytes of the unit; 16-byte piece p of row r sits in slot p ^ (r & 7), with
-//     which the 16-byte fragment reads of a wave (sixteen consecutive rows, one piece per
-//     quarter wave) were measured free of bank conflicts.
-//   * wave (mh, nq) multiplies rows [128 mh, +128) with outputs [64 nq, +64) as 8 x 4 tiles
-//     of v_mfma_f32_16x16x32_bf16 (twelve fragment reads for 32 products), the weights as
-//     the left operand: a lane then holds four consecutive outputs of one row per tile and
-//     stores them as 8 bytes.  The fragments of a step are read into registers while the
-//     step before it is multiplied; one barrier per unit.
-//   * the first two units of a workgroup's next tile are requested before it converts and
-//     stores the sums of this one.
-// Rows and outputs past the end are clamped on the way in and not stored.
-constexpr uint32_t kDenseTileM = 256;
-constexpr uint32_t kDenseTileN = 256;
-constexpr uint32_t kDenseThreads = 512;
-constexpr uint32_t kDenseRing = 2;
-constexpr uint32_t kDenseUnitColumns = 64;
-constexpr uint32_t kDenseRowBytes = kDenseUnitColumns * 2;
-constexpr uint32_t kDenseXUnitBytes = kDenseTileM * kDenseRowBytes;
-constexpr uint32_t kDenseUnitBytes = (kDenseTileM + kDenseTileN) * kDenseRowBytes;
-constexpr uint32_t kDenseLdsBytes = kDenseRing * kDenseUnitBytes;      // 131072
-static_assert(kDenseLdsBytes <= 160 * 1024, "one workgroup per compute unit");
-
-// lane l's 16 bytes at base + offset land at lds_address + 16 l
-__device__ __forceinline__ void dense_transfer(const uint8_t* base, uint32_t offset,
-                                               uint32_t lds_address) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(__builtin_amdgcn_readfirstlane(lds_address)), "v"(offset), "s"(base)
-                 : "memory");
-}
-
-// two sums to a packed bf16 pair: hardware round to nearest even, then results below the
-// normal range flushed to signed zero
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-__device__ __forceinline__ uint32_t dense_pack(float a, float b) {
-    const uint32_t pair = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    const uint32_t keep = ((pair & 0x00007F80u) ? 0x0000FFFFu : 0x00008000u) |
-                          ((pair & 0x7F800000u) ? 0xFFFF0000u : 0x80000000u);
-    return pair & keep;
-}
-
-__global__ __launch_bounds__(kDenseThreads) void dense_block_kernel(const uint16_t* input,
-                                                                   const uint16_t* weights,
-                                                                   uint16_t* output, uint32_t rows,
-                                                                   uint32_t in_dim, uint32_t out_dim) {
-    extern __shared__ __align__(16) uint8_t dense_lds[];
-    const uint32_t t = threadIdx.x;
-    const uint32_t lane = t & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const uint32_t i16 = lane & 15, g = lane >> 4;
-    const uint32_t units = in_dim / kDenseUnitColumns;
-    const uint32_t n_tiles = (out_dim + kDenseTileN - 1) / kDenseTileN;
-    const uint32_t tiles = n_tiles * ((rows + kDenseTileM - 1) / kDenseTileM);
-    const uint32_t lds_base = static_cast<uint32_t>(
-        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)dense_lds));
-    const uint32_t nq = wave & 3, mh = wave >> 2;
-
-    // staging roles: transfers 0..3 of wave w fill x rows 32 w + 8 j .. + 7, transfers 4..7
-    // the weight rows of the same numbers; lane l lands in row + (l >> 3), slot l & 7, so it
-    // fetches piece (l & 7) ^ (l >> 3) of that row
-    const uint8_t* x_base = reinterpret_cast<const uint8_t*>(input);
-    const uint8_t* w_base = reinterpret_cast<const uint8_t*>(weights);
-    const uint32_t piece = ((lane & 7) ^ (lane >> 3)) * 16;
-    const uint32_t staged_row = 32 * wave + (lane >> 3);
-    const uint32_t row_bytes = in_dim * 2;
-    uint32_t m_aim = 0, n_aim = 0;   // first row and output of the tile the requests go to
-    // Tiles are numbered along bands of eight tile rows, down a band's columns first, so that
-    // a run of consecutive numbers is a compact patch (32 of them: eight rows x four columns,
-    // twelve operand panels for 32 tiles).
-    const uint32_t m_tiles = (rows + kDenseTileM - 1) / kDenseTileM;
-    auto place = [&](uint32_t tile, uint32_t& m0, uint32_t& n0) {
-        const uint32_t band = tile / (8 * n_tiles);
-        const uint32_t band_rows = min(8u, m_tiles - 8 * band);
-        const uint32_t within = tile - band * 8 * n_tiles;
-        m0 = (8 * band + within % band_rows) * kDenseTileM;
-        n0 = (within / band_rows) * kDenseTileN;
-    };
-    auto aim = [&](uint32_t tile) { place(tile, m_aim, n_aim); };
-    // the lane offsets are worked out per request (a handful of instructions per 64
-    // products) rather than held in eight registers the products need
-    auto request = [&](uint32_t unit) {
-        const uint32_t place = lds_base + (unit % kDenseRing) * kDenseUnitBytes;
-        const uint8_t* x_unit = x_base + unit * kDenseRowBytes;   // uniform: scalar arithmetic
-        const uint8_t* w_unit = w_base + unit * kDenseRowBytes;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t offset = min(m_aim + staged_row + 8 * j, rows - 1) * row_bytes + piece;
-            dense_transfer(x_unit, offset, place + (32 * wave + 8 * j) * kDenseRowBytes);
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const uint32_t offset = min(n_aim + staged_row + 8 * j, out_dim - 1) * row_bytes + piece;
-            dense_transfer(w_unit, offset,
-                           place + kDenseXUnitBytes + (32 * wave + 8 * j) * kDenseRowBytes);
-        }
-    };
-
-    // fragment of (row, step of the unit): piece 4 step + g, stored at slot piece ^ (row & 7)
-    const uint32_t frag_row = i16 * kDenseRowBytes;
-    const uint32_t frag_piece[2] = {(g ^ (i16 & 7)) * 16, ((4 + g) ^ (i16 & 7)) * 16};
-    const uint32_t x_frag = 128 * mh * kDenseRowBytes + frag_row;
-    const uint32_t w_frag = kDenseXUnitBytes + 64 * nq * kDenseRowBytes + frag_row;
-    f32x4 acc[4][8];   // [tn][tm]
-
-    struct Fragments {
-        bf16x8 x[8], w[4];
-    };
-    auto read_fragments = [&](uint32_t unit, uint32_t step, Fragments& f) __attribute__((always_inline)) {
-        const uint8_t* place = dense_lds + (unit % kDenseRing) * kDenseUnitBytes + frag_piece[step];
-#pragma unroll
-        for (uint32_t tile = 0; tile < 4; ++tile) {
-            f.w[tile] = *reinterpret_cast<const bf16x8*>(place + w_frag + tile * 16 * kDenseRowBytes);
-        }
-#pragma unroll
-        for (uint32_t tile = 0; tile < 8; ++tile) {
-            f.x[tile] = *reinterpret_cast<const bf16x8*>(place + x_frag + tile * 16 * kDenseRowBytes);
-        }
-    };
-    auto multiply = [&](const Fragments& f) __attribute__((always_inline)) {
-#pragma unroll
-        for (uint32_t tm = 0; tm < 8; ++tm) {
-#pragma unroll
-            for (uint32_t tn = 0; tn < 4; ++tn) {
-                acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[tn], f.x[tm], acc[tn][tm],
-                                                                      0, 0, 0);
-            }
-        }
-    };
-    // issue order of a slot: a read, then two products, so that the eight waves' reads are
-    // spread over the slot instead of queueing at the LDS while the matrix unit waits (left
-    // alone the scheduler sinks each read to the product that needs it, a slot later).  No
-    // branch between the reads and the products: at a join the compiler would wait for the
-    // reads first.
-    auto interleave = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (uint32_t i = 0; i < 12; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // first step of `unit` (its fragments are in `first`): read the second step's while
-    // multiplying; the unit was published a slot ago, so nothing to wait for
-    auto first_step = [&](uint32_t unit, const Fragments& first, Fragments& second)
-                          __attribute__((always_inline)) {
-        __builtin_amdgcn_sched_barrier(0);
-        read_fragments(unit, 1, second);
-        multiply(first);
-        interleave();
-    };
-    // second step of `unit`: the next unit (requested a unit ago) has landed - mine, then
-    // everybody's -, and nobody reads the unit before this one any more, so the unit after
-    // the next goes into its place; read the next unit's first fragments while multiplying
-    auto second_step = [&](uint32_t unit, const Fragments& second, Fragments& first_of_next,
-                           auto with_request) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
-        __syncthreads();
-        if constexpr (decltype(with_request)::value) request(unit + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        read_fragments(unit + 1, 0, first_of_next);
-        multiply(second);
-        interleave();
-    };
-    using std::bool_constant;
-
-    // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own:
-    // the workgroups of an XCD (b / 8 = 0, 1, ...) take a run of consecutive tiles together,
-    // the XCDs take the runs in turn - the operand panels a patch shares are then fetched into
-    // one L2 once instead of into several.  (A grid that is no multiple of eight - fewer tiles
-    // than compute units - takes every gridDim.x-th tile.)
-    const bool by_xcd = gridDim.x % 8 == 0;
-    const uint32_t per_xcd = gridDim.x / 8;
-    const uint32_t stride = by_xcd ? 8 * per_xcd : gridDim.x;
-    uint32_t tile = by_xcd ? (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3) : blockIdx.x;
-    if (tile >= tiles) return;
-    aim(tile);
-    request(0);
-    if (units > 1) request(1);
-    while (true) {
-#pragma unroll
-        for (uint32_t tn = 0; tn < 4; ++tn) {
-#pragma unroll
-            for (uint32_t tm = 0; tm < 8; ++tm) acc[tn][tm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-        // unit 0 has landed (the second unit may be in flight; so may the stores of the tile
-        // before, and reads and writes do not retire in one order: wait for everything)
-        __builtin_amdgcn_s_waitcnt(0x0F70);
-        __syncthreads();
-        Fragments a, b;
-        read_fragments(0, 0, a);
-        uint32_t unit = 0;
-        for (; unit + 2 < units; ++unit) {
-            first_step(unit, a, b);
-            second_step(unit, b, a, bool_constant<true>{});
-        }
-        if (units > 1) {   // unit == units - 2
-            first_step(unit, a, b);
-            second_step(unit, b, a, bool_constant<false>{});
-            ++unit;
-        }
-        first_step(unit, a, b);
-        multiply(b);
-
-        uint32_t m0, n0;
-        place(tile, m0, n0);
-        const uint32_t next_tile = tile + stride;
-        __syncthreads();   // nobody reads the stages any more
-        if (next_tile < tiles) {
-            aim(next_tile);
-            request(0);
-            if (units > 1) request(1);
-        }
-        // the lane holds outputs n0 + 64 nq + 16 tn + 4 g + j of row m0 + 128 mh + 16 tm + i16
-        const bool wide = ((reinterpret_cast<uintptr_t>(output) | (out_dim * 2)) & 7) == 0;
-#pragma unroll
-        for (uint32_t tm = 0; tm < 8; ++tm) {
-            const uint32_t row = m0 + 128 * mh + 16 * tm + i16;
-            if (row >= rows) continue;
-            uint16_t* out_row = output + static_cast<uint64_t>(row) * out_dim;
-#pragma unroll
-            for (uint32_t tn = 0; tn < 4; ++tn) {
-                const uint32_t n = n0 + 64 * nq + 16 * tn + 4 * g;
-                if (n >= out_dim) continue;
-                const f32x4 v = acc[tn][tm];
-                const u32x2 four = u32x2{dense_pack(v[0], v[1]), dense_pack(v[2], v[3])};
-                if (wide && n + 4 <= out_dim) {
-                    *reinterpret_cast<u32x2*>(out_row + n) = four;
-                } else {
-                    for (uint32_t j = 0; j < 4 && n + j < out_dim; ++j) {
-                        out_row[n + j] = static_cast<uint16_t>(four[j >> 1] >> (16 * (j & 1)));
-                    }
-                }
-            }
-        }
-        if (next_tile >= tiles) break;
-        tile = next_tile;
-    }
+// The same for a block of rows, sized for the matrix unit (block_product.h).
+template <typename Product>
+__global__ __launch_bounds__(Product::kThreads) void dense_block_kernel(
+    const uint16_t* input, const uint16_t* weights, uint16_t* output, uint32_t rows, uint32_t in_dim,
+    uint32_t out_dim) {
+    const bool wide = ((reinterpret_cast<uintptr_t>(output) | (out_dim * 2)) & 7) == 0;
+    Product::run(input, weights, rows, in_dim, out_dim,
+                 [&](uint32_t m, uint32_t n, typename Product::Sums sums) {
+                     block_store(output + static_cast<uint64_t>(m) * out_dim, n, out_dim, wide, sums);
+                 });
 }
 
 // The same for at most 16 rows (a decode wave), sized for latency: a workgroup owns 16
@@ -534,6 +299,28 @@ bool dense_block_operands_fit(const uint16_t* input, const uint16_t* weights, ui
            static_cast<uint64_t>(out_dim) * in_dim * 2 < (1ull << 32);
 }
 
+template <typename Product>
+void launch_dense_product(const uint16_t* input, const uint16_t* weights, uint16_t* output,
+                          uint32_t rows, uint32_t in_dim, uint32_t out_dim, hipStream_t stream) {
+    hipLaunchKernelGGL(dense_block_kernel<Product>,
+                       dim3(block_workgroups<Product>(rows, out_dim, current_device_compute_units())),
+                       dim3(Product::kThreads), Product::kLdsBytes, stream, input, weights, output, rows,
+                       in_dim, out_dim);
+}
+typedef BlockTiles<__bf16> DenseTiles;
+void launch_dense_block(const uint16_t* input, const uint16_t* weights, uint16_t* output, uint32_t rows,
+                        uint32_t in_dim, uint32_t out_dim, hipStream_t stream) {
+    auto launch = launch_dense_product<DenseTiles::Large>;
+    switch (choose_block_tile(rows, in_dim, out_dim, current_device_compute_units())) {
+    case BlockTile::Large: break;
+    case BlockTile::Even: launch = launch_dense_product<DenseTiles::Even>; break;
+    case BlockTile::Deep: launch = launch_dense_product<DenseTiles::Deep>; break;
+    case BlockTile::Low: launch = launch_dense_product<DenseTiles::Low>; break;
+    case BlockTile::Small: launch = launch_dense_product<DenseTiles::Small>; break;
+    }
+    launch(input, weights, output, rows, in_dim, out_dim, stream);
+}
+
 // dense_bf16: b0 input [rows][in], b1 weights [out][in], b2 output [rows][out], c3 rows,
 // c4 in (multiple of 64), c5 out; grid (ceil(out/64), ceil(rows/16)) x 256.
 int32_t op_dense_bf16(const Bindings& b, const Grid& g, hipStream_t stream, bool validate_only) {
@@ -558,11 +345,7 @@ int32_t op_dense_bf16(const Bindings& b, const Grid& g, hipStream_t stream, bool
         hipLaunchKernelGGL(dense_rows_kernel<8>, dim3((out_dim + 15) / 16), dim3(512), 0, stream, input,
                            weights, output, rows, out_dim);
     } else if (rows > kDenseBlockRowsFrom && dense_block_operands_fit(input, weights, rows, in_dim, out_dim)) {
-        const uint32_t tiles = ((out_dim + kDenseTileN - 1) / kDenseTileN) *
-                               ((rows + kDenseTileM - 1) / kDenseTileM);
-        hipLaunchKernelGGL(dense_block_kernel, dim3(std::min(tiles, current_device_compute_units())),
-                           dim3(kDenseThreads), kDenseLdsBytes, stream, input, weights, output, rows,
-                           in_dim, out_dim);
+        launch_dense_block(input, weights, output, rows, in_dim, out_dim, stream);
     } else {
         hipLaunchKernelGGL(dense_bf16_kernel, dim3((out_dim + 63) / 64, (rows + 15) / 16), dim3(256), 0,
                            stream, input, weights, output, rows, in_dim, out_dim);
@@ -606,9 +389,15 @@ bool prepare_stack_kernels() {
         units > 0) {
         g_compute_units[device] = static_cast<uint32_t>(units);
     }
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(dense_block_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               kDenseLdsBytes) == hipSuccess;
+    const auto allow = [](auto product, const void* kernel) {
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   decltype(product)::kLdsBytes) == hipSuccess;
+    };
+    return allow(DenseTiles::Large{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Large>)) &&
+           allow(DenseTiles::Even{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Even>)) &&
+           allow(DenseTiles::Deep{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Deep>)) &&
+           allow(DenseTiles::Low{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Low>)) &&
+           allow(DenseTiles::Small{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Small>));
 }
 #endif
 

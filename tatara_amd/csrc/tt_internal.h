@@ -94,7 +94,8 @@ hipStream_t queue_stream(const tt_queue* queue);
 uint32_t queue_compute_units(const tt_queue* queue);
 
 // Device memory a queue owns for operators whose reference bindings carry no scratch (the
-// shared key walk of attention_flash_v2_blk on blocks of few rows).  Allocated when the queue
+// shared key walk of attention_flash_v2_blk on blocks of few rows, the operands of a block's
+// 4-bit projection).  Allocated when the queue
 // is created, so never under a stream capture; commands of one queue run in order, so one
 // operator at a time uses it.  base is null for a stream no queue of this library made, or
 // where the allocation failed.
@@ -106,6 +107,8 @@ struct StreamWorkspace {
 StreamWorkspace stream_workspace(hipStream_t stream);
 // the bytes a queue's workspace holds on a device of that many compute units
 uint64_t stream_workspace_bytes(uint32_t compute_units);
+// what a block of the 4-bit projections needs of it
+uint64_t q4_workspace_bytes();
 
 // attention_flash_split_blk: the workgroups that share a position tile's key walk so that a
 // block of `rows` rows whose last row sees `visible` keys fills `compute_units`, and the

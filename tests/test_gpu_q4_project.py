@@ -211,6 +211,61 @@ def test_block_projection_over_several_row_tiles(family, name, rows):
     check_bf16(got[sample], want, f"{name} rows {sample[:4]}..{sample[-1]}", ulps=2)
 
 
+@pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
+                                         (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
+@pytest.mark.parametrize("rows", [17, 63, 65, 129, 511, 8193])
+def test_block_projection_against_64_bit_sums_over_the_whole_range(family, name, rows):
+    """Rows either side of the tile heights a block is launched with, and of the 8192 rows the
+    out-projection takes at a time, over inputs and weights of all magnitudes: rows of 2^-100 to
+    2^100 with a value 2^12 times the others in every 64 columns, a row of zeros, matrices whose
+    groups differ by 2^8 and whose rows by 2^40.  The terms that are summed are exact in fp32 to
+    2^-24 of their group's largest, so an output may differ from the 64-bit sum by half a bf16
+    step (2^-9, doubled to 2^-8 at a binade's lower end) and 2^-20 of the sum of magnitudes."""
+    print(f"[case] {name} rows={rows} whole range", flush=True)
+    B, dev, queue, lib = gpu()
+    rng = np.random.default_rng(rows)
+    k, total = family["k"], sum(family["segments"])
+    x = rng.standard_normal((rows, k), dtype=np.float32)
+    x[:, ::64] *= 4096.0
+    x = ol.f32_to_bf16((x * np.exp2(rng.integers(-100, 60, (rows, 1))).astype(np.float32)).reshape(-1))
+    x = x.reshape(rows, k)
+    x[rows // 2] = 0
+    bindings, host = {0: dev.buffer_from(x.reshape(-1))}, []
+    for index, n in enumerate(family["segments"]):
+        words = rng.integers(0, 2 ** 32, n * k // 8, dtype=np.uint64).astype(np.uint32)
+        scale = rng.uniform(0.5, 1.0, (n, k // 64)) * np.exp2(rng.integers(-8, 1, (n, k // 64)))
+        scale *= np.exp2(rng.integers(-40, 1, (n, 1)))
+        scales = ol.f32_to_bf16(scale.astype(np.float32).reshape(-1))
+        biases = ol.f32_to_bf16((scale * rng.uniform(-8.0, 0.5, scale.shape)).astype(np.float32).reshape(-1))
+        slot = 1 + 3 * index
+        bindings.update({slot: dev.buffer_from(words), slot + 1: dev.buffer_from(scales),
+                         slot + 2: dev.buffer_from(biases)})
+        host.append((words, scales, biases))
+    out = dev.buffer_from(np.full(rows * total, 0x7FC0, np.uint16))      # NaN until written
+    bindings[family["out"]] = out
+    slot = family["out"] + 1
+    constants = {slot: rows, slot + 1: k} if family is OUT else {slot: rows}
+    run(lambda cb: cb.encode(lib.pipeline(name), bindings, constants, (_groups(family), 1, 1),
+                             (family["threads"], 1, 1)))
+    got = ol.bf16_to_f32(out.read(np.uint16)).reshape(rows, total).astype(np.float64)
+    assert np.isfinite(got).all()
+    sample = sorted({0, 15, 16, rows // 2, rows - 2, rows - 1} | {r for r in (63, 64, 127, 128, 8191)
+                                                                  if r < rows})
+    xs = ol.bf16_to_f32(x[sample].reshape(-1)).reshape(len(sample), k).astype(np.float64)
+    first = 0
+    for words, scales, biases in host:
+        n = len(words) * 8 // k
+        nibbles = (words[:, None] >> (4 * np.arange(8, dtype=np.uint32))[None, :]) & 15
+        widened = [np.repeat(ol.bf16_to_f32(v).reshape(n, k // 64), 64, axis=1).astype(np.float64)
+                   for v in (scales, biases)]
+        weights = widened[0] * nibbles.reshape(n, k) + widened[1]
+        want, magnitudes = xs @ weights.T, np.abs(xs) @ np.abs(weights).T
+        error = np.abs(got[sample, first:first + n] - want)
+        bar = np.abs(want) * 2.0 ** -8 + magnitudes * 2.0 ** -20 + 2.0 ** -126
+        assert (error <= bar).all(), np.argwhere(error > bar)[:4]
+        first += n
+
+
 @pytest.mark.parametrize("rows", [2, 4, 13, 16])
 @pytest.mark.parametrize("family", [ATTN, GDN], ids=lambda f: f["name"])
 def test_wave_projection_with_the_norm_in_its_prologue(family, rows):

@@ -338,6 +338,24 @@ def test_dense_bf16_block_kernel(rows, in_dim, out_dim):
     _dense_block_case(rows, in_dim, out_dim, range(rows), 0xB10C + rows)
 
 
+@pytest.mark.parametrize("rows,in_dim,out_dim", [
+    (66, 2048, 515),       # 64 x 64 tiles, two rows into the second
+    (100, 64, 4096),       # fewer units of K than a ring holds
+    (129, 256, 9216),      # one row into a second 64- or 128-row tile, several rounds of them
+    (500, 2048, 9216),     # 128 x 128 tiles, two a compute unit, the last round not filled
+    (2047, 4096, 2048),    # 128 x 128 tiles, one a compute unit
+    (2049, 192, 12352),    # 256 x 256 tiles and a row of one more
+], ids=lambda v: str(v))
+def test_dense_bf16_block_tiles(rows, in_dim, out_dim):
+    """The tiles a block is launched with, at their edges: sampled rows against the checker,
+    every output stored."""
+    print(f"[case] dense_bf16 tiles rows={rows} in={in_dim} out={out_dim}", flush=True)
+    sample = sorted({0, 15, 16, 63, 64, 65, rows // 2, rows - 2, rows - 1} |
+                    {r for r in range(127, rows, 640)} | {r for r in range(128, rows, 640)})
+    got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB111 + rows)
+    assert not np.any((got & 0x7F80) == 0x7F80), "an output was not stored"
+
+
 def test_dense_bf16_block_kernel_at_the_prefill_shape():
     """16384 rows x 2048 -> 9216 (the attention input projection of a 16384-row block): 2304
     tiles on one workgroup per compute unit, nine tiles each.  The checker evaluates every
