@@ -132,6 +132,7 @@ struct PrepareArgs {
     uint32_t rows;
     uint16_t* conv_tape;          // [40][16][3][8192] window after each row, or null
     uint32_t tape_layer;
+    uint32_t rows_per_group;      // block kernel: rows one workgroup walks
 };
 
 constexpr uint32_t kBlockRowsPerGroup = 16;  // block mode: rows one workgroup walks
@@ -214,11 +215,12 @@ __global__ __launch_bounds__(128) void gdn_prepare_kernel(PrepareArgs a) {
 
 // Block form of the prepare step for rows that are consecutive tokens of one lane:
 // a lane owns 8 adjacent channels (16-byte loads and stores), a workgroup of 256
-// lanes 2048 channels, and walks kBlockRowsPerGroup rows with the three earlier taps
-// in registers, so every projection element is read once.  grid.x: 0 q heads, 1 k
-// heads, 2..3 value heads, 4..5 the z gate copy.  Same arithmetic, operation for
-// operation, as gdn_prepare_kernel: a head's 128 squares are summed as 32 runs of
-// four, then the adjacent-pairs tree - a lane holds two runs, 16 lanes a head.
+// lanes 2048 channels, and walks rows_per_group rows with the three earlier taps
+// in registers.  grid 6 ceil(rows / rows_per_group), of each six: 0 q heads, 1 k heads,
+// 2..3 value heads, 4..5 the z gate copy.  Same arithmetic, operation for operation, as
+// gdn_prepare_kernel: a head's 128 squares are summed as 32 runs of four, then the
+// adjacent-pairs tree - a lane holds two runs, 16 lanes a head.
+constexpr uint32_t kPrepareUnitGroups = (kCh + kGdnValueValues) / 8 / 256;
 
 __device__ __forceinline__ float widen_half(uint32_t word, uint32_t j) {
     return __uint_as_float((j & 1) ? (word & 0xFFFF0000u) : (word << 16));
@@ -228,9 +230,9 @@ __device__ __forceinline__ uint32_t narrow_pair(float a, float b) {
 }
 
 __global__ __launch_bounds__(256) void gdn_prepare_block_kernel(PrepareArgs a) {
-    const uint32_t unit = blockIdx.x * 256 + threadIdx.x;  // 8 channels each
-    const uint32_t row_begin = blockIdx.y * kBlockRowsPerGroup;
-    const uint32_t row_end = min(a.rows, row_begin + kBlockRowsPerGroup);
+    const uint32_t unit = blockIdx.x % kPrepareUnitGroups * 256 + threadIdx.x;  // 8 channels each
+    const uint32_t row_begin = blockIdx.x / kPrepareUnitGroups * a.rows_per_group;
+    const uint32_t row_end = min(a.rows, row_begin + a.rows_per_group);
     if (unit >= kCh / 8) {
         const uint32_t index = (unit - kCh / 8) * 8;
         for (uint32_t row = row_begin; row < row_end; ++row) {
@@ -260,9 +262,14 @@ __global__ __launch_bounds__(256) void gdn_prepare_block_kernel(PrepareArgs a) {
     }
     const bool normalised = c < kGdnQkValues;
     const float scale = widen(c < kGdnQkValues / 2 ? kGdnQueryScaleBits : kGdnKeyScaleBits);
-    for (uint32_t row = row_begin; row < row_end; ++row) {
-        const u32x4 t3 = *reinterpret_cast<const u32x4*>(
+    auto newest = [&](uint32_t row) {
+        return *reinterpret_cast<const u32x4*>(
             a.projection + static_cast<uint64_t>(row) * a.projection_stride + c);
+    };
+    u32x4 next = newest(row_begin);
+    for (uint32_t row = row_begin; row < row_end; ++row) {
+        const u32x4 t3 = next;
+        next = newest(min(row + 1, row_end - 1));   // in flight over this row's arithmetic
         float act[8];
 #pragma unroll
         for (uint32_t j = 0; j < 8; j += 2) {
@@ -515,52 +522,49 @@ __global__ __launch_bounds__(128) void gdn_gate_norm_kernel(const uint16_t* y, c
 }
 
 // Block form: a lane owns 8 adjacent channels, 16 lanes a head, a workgroup of 256
-// lanes half a row; grid (2, ceil(rows / rows_per_group)).  Same arithmetic as
+// lanes half a row; grid 2 rows.  Same arithmetic as
 // gdn_gate_norm_kernel (two runs of four squares per lane, then the pair tree).
 __global__ __launch_bounds__(256) void gdn_gate_norm_block_kernel(
-    const uint16_t* y, const uint16_t* z, const uint16_t* weight, uint16_t* out, uint32_t stride,
-    uint32_t rows, uint32_t rows_per_group) {
-    const uint32_t c = (blockIdx.x * 256 + threadIdx.x) * 8;
+    const uint16_t* y, const uint16_t* z, const uint16_t* weight, uint16_t* out, uint32_t stride) {
+    constexpr uint32_t kGroups = kGdnValueValues / 8 / 256;
+    const uint32_t c = (blockIdx.x % kGroups * 256 + threadIdx.x) * 8;
     float w[8];
     {
         const u32x4 bits = *reinterpret_cast<const u32x4*>(weight + (c & (kGD - 1)));
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) w[j] = widen_half(bits[j >> 1], j);
     }
-    const uint32_t row_end = min(rows, (blockIdx.y + 1) * rows_per_group);
-    for (uint32_t row = blockIdx.y * rows_per_group; row < row_end; ++row) {
-        const uint64_t at = static_cast<uint64_t>(row) * stride + c;
-        const u32x4 yb = *reinterpret_cast<const u32x4*>(y + at);
-        const u32x4 zb = *reinterpret_cast<const u32x4*>(z + at);
-        float v[8];
+    const uint64_t at = static_cast<uint64_t>(blockIdx.x / kGroups) * stride + c;
+    const u32x4 yb = *reinterpret_cast<const u32x4*>(y + at);
+    const u32x4 zb = *reinterpret_cast<const u32x4*>(z + at);
+    float v[8];
 #pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) v[j] = widen_half(yb[j >> 1], j);
-        const float run0 = ((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]) + v[3] * v[3];
-        const float run1 = ((v[4] * v[4] + v[5] * v[5]) + v[6] * v[6]) + v[7] * v[7];
-        float total = run0 + run1;
-        total = row_sum(total);
-        const float inverse = 1.0f / sqrtf(total / static_cast<float>(kGD) + kRmsNormEpsilon);
-        u32x4 packed;
+    for (uint32_t j = 0; j < 8; ++j) v[j] = widen_half(yb[j >> 1], j);
+    const float run0 = ((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]) + v[3] * v[3];
+    const float run1 = ((v[4] * v[4] + v[5] * v[5]) + v[6] * v[6]) + v[7] * v[7];
+    float total = run0 + run1;
+    total = row_sum(total);
+    const float inverse = 1.0f / sqrtf(total / static_cast<float>(kGD) + kRmsNormEpsilon);
+    u32x4 packed;
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j += 2) {
-            float r[2];
-            float n0 = v[j] * inverse, n1 = v[j + 1] * inverse;
-            rb_pair(n0, n1);
-            n0 *= w[j];
-            n1 *= w[j + 1];
-            rb_pair(n0, n1);
-            const float normed[2] = {n0, n1};
+    for (uint32_t j = 0; j < 8; j += 2) {
+        float r[2];
+        float n0 = v[j] * inverse, n1 = v[j + 1] * inverse;
+        rb_pair(n0, n1);
+        n0 *= w[j];
+        n1 *= w[j + 1];
+        rb_pair(n0, n1);
+        const float normed[2] = {n0, n1};
 #pragma unroll
-            for (uint32_t e = 0; e < 2; ++e) {
-                const float g = widen_half(zb[j >> 1], e);
-                const float low = 1.0f / (1.0f + expf(fabsf(g)));
-                const float sig = g < 0.0f ? low : 1.0f - low;
-                r[e] = (g * sig) * normed[e];
-            }
-            packed[j >> 1] = rb_pair_bits(r[0], r[1]);
+        for (uint32_t e = 0; e < 2; ++e) {
+            const float g = widen_half(zb[j >> 1], e);
+            const float low = 1.0f / (1.0f + expf(fabsf(g)));
+            const float sig = g < 0.0f ? low : 1.0f - low;
+            r[e] = (g * sig) * normed[e];
         }
-        *reinterpret_cast<u32x4*>(out + at) = packed;
+        packed[j >> 1] = rb_pair_bits(r[0], r[1]);
     }
+    *reinterpret_cast<u32x4*>(out + at) = packed;
 }
 
 // ------------------------------------------------- fused decode step ---------
@@ -1480,12 +1484,27 @@ constexpr uint32_t kScanTiles = 1;
 
 // ---------------------------------------------------------------- launchers --
 
+// Rows a workgroup of the block kernel walks.  A row is a chain of its own (load, two dependent
+// exponentials, a sum over lanes: 1.2 us), so few rows want a workgroup each - 12 / 100 / 300
+// rows take 3.4 / 4.3 / 7.2 us so, 16.2 / 21.5 / 22.0 us sixteen to a workgroup - and many want
+// the three earlier rows read less often: 2048 rows 27.6 / 24.8 / 26.6 us and 16384 rows 245 /
+// 192 / 176 us with 1 / 2 / 4 to a workgroup, 173 us with six, 184 us with sixteen.
+// A window written where the block's earlier taps are read stays with one workgroup as long as
+// sixteen rows allow it.
+uint32_t prepare_rows_per_group(const PrepareArgs& p) {
+    const uintptr_t in = reinterpret_cast<uintptr_t>(p.conv_in), out = reinterpret_cast<uintptr_t>(p.conv_out);
+    constexpr uintptr_t kWindowBytes = 3 * kCh * 2;
+    if (in < out + kWindowBytes && out < in + kWindowBytes) return kBlockRowsPerGroup;
+    return p.rows <= 512 ? 1 : p.rows <= 4096 ? 2 : 6;
+}
+
 int32_t launch_prepare(const PrepareArgs& p, hipStream_t stream) {
     if (p.block_mode) {
-        hipLaunchKernelGGL(gdn_prepare_block_kernel,
-                           dim3((kCh + kGdnValueValues) / 8 / 256,
-                                (p.rows + kBlockRowsPerGroup - 1) / kBlockRowsPerGroup),
-                           dim3(256), 0, stream, p);
+        PrepareArgs block = p;
+        block.rows_per_group = prepare_rows_per_group(p);
+        const uint32_t groups = (p.rows + block.rows_per_group - 1) / block.rows_per_group;
+        hipLaunchKernelGGL(gdn_prepare_block_kernel, dim3(kPrepareUnitGroups * groups), dim3(256), 0, stream,
+                           block);
         return TT_OK;
     }
     hipLaunchKernelGGL(gdn_prepare_kernel, dim3(96, p.rows), dim3(128), 0, stream, p);
@@ -1801,9 +1820,11 @@ int32_t gate_norm_common(Args& a, const Grid& g, uint32_t rows, uint32_t stride,
     a.require(g.gx == 32 && g.gy == rows && g.gz == 1 && g.tx == 128 && g.ty == 1 && g.tz == 1,
               TT_CMD_INVALID_DISPATCH_EXTENT);
     if (a.status != TT_OK || validate_only) return a.status;
-    if (rows > kMaxBatchRows && stride % 8 == 0) {  // blocks: 8 channels per lane, 8 rows per group
-        hipLaunchKernelGGL(gdn_gate_norm_block_kernel, dim3(kGdnValueValues / 8 / 256, (rows + 7) / 8),
-                           dim3(256), 0, stream, y, z, w, out, stride, rows, 8u);
+    // blocks: 8 channels per lane, a row per group (eight rows: 100 rows 9.4 us instead of 3.0,
+    // 2048 rows 15.0 instead of 12.2, 16384 rows 82 instead of 69)
+    if (rows > kMaxBatchRows && stride % 8 == 0) {
+        hipLaunchKernelGGL(gdn_gate_norm_block_kernel, dim3(kGdnValueValues / 8 / 256 * rows), dim3(256), 0,
+                           stream, y, z, w, out, stride);
         return TT_OK;
     }
     hipLaunchKernelGGL(gdn_gate_norm_kernel, dim3(32, rows), dim3(128), 0, stream, y, z, w, out,

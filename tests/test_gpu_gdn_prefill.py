@@ -145,6 +145,29 @@ def test_element_wise_block_kernels_bit_for_bit(rows):
     assert np.array_equal(bufs["gated"].read(np.uint16), ref["gated"])
 
 
+@pytest.mark.parametrize("rows", [512, 513, 4096, 4097])
+def test_element_wise_block_kernels_at_every_rows_per_group(rows):
+    """Either side of the row counts from which a workgroup walks 2 and 6 rows instead of 1,
+    with remainders: the checker's bit patterns as above."""
+    test_element_wise_block_kernels_bit_for_bit(rows)
+
+
+@pytest.mark.parametrize("rows", [2, 12, 16])
+def test_conv_window_written_in_place(rows):
+    """A short block that leaves its conv window in the buffer it read the last one from."""
+    print(f"[case] gdn conv window in place rows={rows}", flush=True)
+    B, dev, queue, lib = gpu()
+    weights = _weights()
+    proj, conv_state, state = _block(rows, 0x5700 + rows)
+    ref = _oracle_block(proj, conv_state, state, weights, rows)
+    bufs = _buffers(dev, proj, conv_state, state, weights, rows)
+    bufs["conv_out"] = bufs["conv_in"]
+    run(lambda cb: _encode_front(cb, lib, bufs, rows))
+    assert np.array_equal(bufs["qk"].read(np.uint16), ref["qk"])
+    assert np.array_equal(bufs["value"].read(np.uint16), ref["value"])
+    assert np.array_equal(bufs["conv_out"].read(np.uint16), ref["conv"])
+
+
 def test_activation_of_every_bf16_value_bit_for_bit():
     """conv + SiLU of all 65536 bf16 bit patterns (the non-finite ones replaced by zero):
     16 rows whose 4096 value channels carry the patterns, taps (0, 0, 0, 1) and an empty
