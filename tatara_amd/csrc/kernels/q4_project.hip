@@ -116,12 +116,22 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
     const uint32_t lane = threadIdx.x & 31;
     const uint32_t row_base = blockIdx.y * p.row_tile;
     const uint32_t tile_rows = min(p.row_tile, p.rows - row_base);
-    for (uint32_t piece = threadIdx.x; kStaged && piece < tile_rows * kPiecesPerRow; piece += 256) {
+    auto slot_of = [&](uint32_t piece) {
         const uint32_t r = piece / kPiecesPerRow, c = piece % kPiecesPerRow;
-        const u32x4 staged = *reinterpret_cast<const u32x4*>(
-            p.input + static_cast<uint64_t>(row_base + r) * p.input_stride + c * 8);
-        const uint32_t slot = (c & ~63u) + ((c & 63u) >> 1) + (c & 1u) * 32;
-        *reinterpret_cast<u32x4*>(rows_lds + (r * kPiecesPerRow + slot) * 16) = staged;
+        return (r * kPiecesPerRow + (c & ~63u) + ((c & 63u) >> 1) + (c & 1u) * 32) * 16;
+    };
+    auto piece_of = [&](uint32_t piece) {
+        return *reinterpret_cast<const u32x4*>(
+            p.input + static_cast<uint64_t>(row_base + piece / kPiecesPerRow) * p.input_stride +
+            piece % kPiecesPerRow * 8);
+    };
+    // the first row's pieces are stored once the weights have been requested as well, so that
+    // the two round trips overlap (a single row, the ordinary case, is all of x)
+    constexpr uint32_t kFirst = kPiecesPerRow / 256;
+    u32x4 first[kFirst];
+    if (kStaged) {
+#pragma unroll
+        for (uint32_t j = 0; j < kFirst; ++j) first[j] = piece_of(threadIdx.x + j * 256);
     }
     // rows past the last one compute on the last row and store nothing
     const uint32_t n = min(blockIdx.x * 8 + (threadIdx.x >> 5), p.first_row[p.segments] - 1);
@@ -141,7 +151,16 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
         scale_bits[b] = scales[b * 8 + (lane >> 2)];
         bias_bits[b] = biases[b * 8 + (lane >> 2)];
     }
-    if (kStaged) __syncthreads();
+    if (kStaged) {
+#pragma unroll
+        for (uint32_t j = 0; j < kFirst; ++j) {
+            *reinterpret_cast<u32x4*>(rows_lds + slot_of(threadIdx.x + j * 256)) = first[j];
+        }
+        for (uint32_t piece = kPiecesPerRow + threadIdx.x; piece < tile_rows * kPiecesPerRow; piece += 256) {
+            *reinterpret_cast<u32x4*>(rows_lds + slot_of(piece)) = piece_of(piece);
+        }
+        __syncthreads();
+    }
     const uint16_t* x0 = p.input + static_cast<uint64_t>(row_base) * p.input_stride + lane * 16;
     float acc[kQ4BatchRowsMax];
 #pragma unroll
@@ -515,7 +534,8 @@ __device__ __forceinline__ bf16x4_bits offset_four(uint32_t word) {
 template <uint32_t kWaves>
 constexpr uint32_t kWaveRowBytes = kWaves * 1024 + 16;
 
-template <uint32_t kWaves, bool kNorm = false, bool kResidual = false>   // kWaves = k_size / 512
+// kWaves = k_size / 512; kRowsMax: the rows this instantiation takes at most
+template <uint32_t kWaves, bool kNorm = false, bool kResidual = false, uint32_t kRowsMax = kQ4BatchRowsMax>
 __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
     // [rows][kWaveRowBytes] of x, then the waves' partial results
     extern __shared__ __align__(16) uint8_t wave_lds[];
@@ -594,23 +614,22 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
             }
         }
     } else {
-        for (uint32_t piece = threadIdx.x; piece < p.rows * kPiecesPerRow; piece += 4 * kThreads) {
-            u32x4 staged[4];
+        // one piece of each row per thread; the weights are requested before the first piece is
+        // stored, so that the two round trips overlap (rows past the last repeat it: no branch
+        // between the requests, where what is in flight would be waited for)
+        static_assert(kPiecesPerRow == kThreads, "a row is one piece per thread");
+        u32x4 raw[kRowsMax];
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
-                const uint32_t at = min(piece + j * kThreads, p.rows * kPiecesPerRow - 1);
-                staged[j] = *reinterpret_cast<const u32x4*>(
-                    p.input + static_cast<uint64_t>(at / kPiecesPerRow) * p.input_stride +
-                    (at % kPiecesPerRow) * 8);
-            }
-#pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
-                const uint32_t at = min(piece + j * kThreads, p.rows * kPiecesPerRow - 1);
-                *reinterpret_cast<u32x4*>(wave_lds + (at / kPiecesPerRow) * kWaveRowBytes<kWaves> +
-                                          (at % kPiecesPerRow) * 16) = staged[j];
-            }
+        for (uint32_t r = 0; r < kRowsMax; ++r) {
+            raw[r] = *reinterpret_cast<const u32x4*>(
+                p.input + static_cast<uint64_t>(min(r, p.rows - 1)) * p.input_stride + threadIdx.x * 8);
         }
         request_weights();
+#pragma unroll
+        for (uint32_t r = 0; r < kRowsMax; ++r) {
+            *reinterpret_cast<u32x4*>(wave_lds + min(r, p.rows - 1) * kWaveRowBytes<kWaves> +
+                                      threadIdx.x * 16) = raw[r];
+        }
     }
     __syncthreads();
 
@@ -667,6 +686,9 @@ constexpr uint32_t wave_lds_bytes(uint32_t rows) {
     return rows * kWaveRowBytes<kWaves> + kWaves * 4 * 64 * 4;
 }
 
+constexpr uint32_t kFewRows = 4;   // of x requested up front by the instantiation for few lanes
+static_assert(wave_lds_bytes<8>(kFewRows) <= 64 * 1024, "needs no larger LDS limit");
+
 int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
     const uint32_t out_rows = p.first_row[p.segments];
     switch (p.k_size / kQ4Block) {
@@ -676,8 +698,9 @@ int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL((q4_wave_kernel<4, true, false>), dim3(out_rows / 16), dim3(256),
                                wave_lds_bytes<4>(p.rows), stream, p);
         } else {
-            hipLaunchKernelGGL((q4_wave_kernel<4>), dim3(out_rows / 16), dim3(256),
-                               wave_lds_bytes<4>(p.rows), stream, p);
+            const auto kernel = p.rows <= kFewRows ? q4_wave_kernel<4, false, false, kFewRows>
+                                                   : q4_wave_kernel<4>;
+            hipLaunchKernelGGL(kernel, dim3(out_rows / 16), dim3(256), wave_lds_bytes<4>(p.rows), stream, p);
         }
         break;
     case 8:
@@ -686,8 +709,9 @@ int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL((q4_wave_kernel<8, false, true>), dim3(out_rows / 16), dim3(512),
                                wave_lds_bytes<8>(p.rows), stream, p);
         } else {
-            hipLaunchKernelGGL((q4_wave_kernel<8>), dim3(out_rows / 16), dim3(512),
-                               wave_lds_bytes<8>(p.rows), stream, p);
+            const auto kernel = p.rows <= kFewRows ? q4_wave_kernel<8, false, false, kFewRows>
+                                                   : q4_wave_kernel<8>;
+            hipLaunchKernelGGL(kernel, dim3(out_rows / 16), dim3(512), wave_lds_bytes<8>(p.rows), stream, p);
         }
         break;
     default: return TT_CMD_INVALID_DISPATCH_EXTENT;
