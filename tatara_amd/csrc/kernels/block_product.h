@@ -75,6 +75,7 @@ struct BlockProduct {
     static constexpr uint32_t kTm = kWaveM / 16, kTn = kWaveN / 16;
     static constexpr uint32_t kXTransfers = kTileM / 8 / kWaves, kWTransfers = kTileN / 8 / kWaves;
     static_assert(kLdsBytes <= 160 * 1024, "the ring fits a compute unit");
+    static constexpr uint32_t kTransfers = kXTransfers + kWTransfers;
     static_assert(kXTransfers * 8 * kWaves == kTileM && kWTransfers * 8 * kWaves == kTileN,
                   "whole transfers");
 
@@ -82,12 +83,16 @@ struct BlockProduct {
     static constexpr uint32_t vmcnt(uint32_t left) {
         return 0x0F70u | (left & 15u) | ((left >> 4) << 14);
     }
-    static_assert((kRing - 2) * (kXTransfers + kWTransfers) < 64, "what vmcnt counts");
+    static_assert((kRing - 2) * kTransfers < 64, "what vmcnt counts");
 
     typedef __attribute__((ext_vector_type(8))) Element Elements;
     typedef __attribute__((ext_vector_type(4))) float Sums;
+    // A step's fragments.  Tall waves keep one set of x fragments, each replaced by the next
+    // step's as soon as its products have been issued (two sets would not fit the registers);
+    // for one or two fragments that would be a wait at the end of every step.
+    static constexpr bool kTwoSetsOfX = kTm <= 2;
     struct Fragments {
-        Elements x[kTm], w[kTn];
+        Elements w[kTn], x[kTwoSetsOfX ? kTm : 1];
     };
 
     static __device__ __forceinline__ Sums product(Elements w, Elements x, Sums sums) {
@@ -124,7 +129,6 @@ struct BlockProduct {
         const uint32_t x_row = 8 * kXTransfers * wave + (lane >> 3);
         const uint32_t w_row = 8 * kWTransfers * wave + (lane >> 3);
         const uint32_t row_bytes = in_dim * 2;
-        uint32_t m_aim = 0, n_aim = 0;   // first row and output of the tile the requests go to
         // Tiles are numbered along bands of eight tile rows, down a band's columns first, so that
         // a run of consecutive numbers is a compact patch (32 of them: eight rows x four columns,
         // twelve operand panels for 32 tiles).
@@ -135,23 +139,33 @@ struct BlockProduct {
             m0 = (8 * band + within % band_rows) * kTileM;
             n0 = (within / band_rows) * kTileN;
         };
-        // the lane offsets are worked out per request (a handful of instructions per 64
-        // products) rather than held in registers the products need
-        auto request = [&](uint32_t unit) {
+        // Transfer `index` of `unit`: of x, then of the weights.  Lane offsets are bytes from the
+        // tile's first row, clamped to the last row that is there (both carry `piece`).
+        const uint32_t x_lane = x_row * row_bytes + piece, w_lane = w_row * row_bytes + piece;
+        uint32_t x_last = 0, w_last = 0;
+        const uint8_t *x_tile = nullptr, *w_tile = nullptr;   // the tile the requests go to
+        auto aim = [&](uint32_t tile) {
+            uint32_t m0, n0;
+            place(tile, m0, n0);
+            x_tile = x_base + static_cast<uint64_t>(m0) * row_bytes;
+            w_tile = w_base + static_cast<uint64_t>(n0) * row_bytes;
+            x_last = (rows - 1 - m0) * row_bytes + piece;
+            w_last = (out_dim - 1 - n0) * row_bytes + piece;
+        };
+        auto request_one = [&](uint32_t unit, uint32_t index) __attribute__((always_inline)) {
             const uint32_t to = lds_base + (unit % kRing) * kUnitBytes;
-            const uint8_t* x_unit = x_base + unit * kRowBytes;   // uniform: scalar arithmetic
-            const uint8_t* w_unit = w_base + unit * kRowBytes;
-#pragma unroll
-            for (uint32_t j = 0; j < kXTransfers; ++j) {
-                const uint32_t offset = min(m_aim + x_row + 8 * j, rows - 1) * row_bytes + piece;
-                block_transfer(x_unit, offset, to + (8 * kXTransfers * wave + 8 * j) * kRowBytes);
-            }
-#pragma unroll
-            for (uint32_t j = 0; j < kWTransfers; ++j) {
-                const uint32_t offset = min(n_aim + w_row + 8 * j, out_dim - 1) * row_bytes + piece;
-                block_transfer(w_unit, offset,
+            if (index < kXTransfers) {
+                block_transfer(x_tile + unit * kRowBytes, min(x_lane + 8 * index * row_bytes, x_last),
+                               to + (8 * kXTransfers * wave + 8 * index) * kRowBytes);
+            } else {
+                const uint32_t j = index - kXTransfers;
+                block_transfer(w_tile + unit * kRowBytes, min(w_lane + 8 * j * row_bytes, w_last),
                                to + kXUnitBytes + (8 * kWTransfers * wave + 8 * j) * kRowBytes);
             }
+        };
+        auto request = [&](uint32_t unit) {
+#pragma unroll
+            for (uint32_t index = 0; index < kTransfers; ++index) request_one(unit, index);
         };
 
         // fragment of (row, step of the unit): piece 4 step + g, stored at slot piece ^ (row & 7)
@@ -161,69 +175,76 @@ struct BlockProduct {
         const uint32_t w_frag = kXUnitBytes + kWaveN * wave_n * kRowBytes + frag_row;
         Sums acc[kTn][kTm];
 
-        auto read_fragments = [&](uint32_t unit, uint32_t step, Fragments& f)
-                                  __attribute__((always_inline)) {
-            const uint8_t* from = block_lds + (unit % kRing) * kUnitBytes + frag_piece[step];
-#pragma unroll
-            for (uint32_t tile = 0; tile < kTn; ++tile) {
-                f.w[tile] = *reinterpret_cast<const Elements*>(from + w_frag + tile * 16 * kRowBytes);
-            }
-#pragma unroll
-            for (uint32_t tile = 0; tile < kTm; ++tile) {
-                f.x[tile] = *reinterpret_cast<const Elements*>(from + x_frag + tile * 16 * kRowBytes);
-            }
+        Elements x_only[kTwoSetsOfX ? 1 : kTm];
+        auto x_of = [&](Fragments& f, uint32_t tm) __attribute__((always_inline)) -> Elements& {
+            return kTwoSetsOfX ? f.x[kTwoSetsOfX ? tm : 0] : x_only[kTwoSetsOfX ? 0 : tm];
         };
-        auto multiply = [&](const Fragments& f) __attribute__((always_inline)) {
+        auto read_weights = [&](uint32_t unit, uint32_t step, uint32_t tn, Fragments& f)
+                                __attribute__((always_inline)) {
+            f.w[tn] = *reinterpret_cast<const Elements*>(block_lds + (unit % kRing) * kUnitBytes +
+                                                         frag_piece[step] + w_frag + tn * 16 * kRowBytes);
+        };
+        auto read_x = [&](uint32_t unit, uint32_t step, uint32_t tm, Fragments& f)
+                          __attribute__((always_inline)) {
+            x_of(f, tm) = *reinterpret_cast<const Elements*>(block_lds + (unit % kRing) * kUnitBytes +
+                                                             frag_piece[step] + x_frag + tm * 16 * kRowBytes);
+        };
+        // One step: multiply, and between the products read the fragments of the step after it
+        // and (requests) send the transfers of a unit off, a few at a time: reads and transfers
+        // that are issued together keep the matrix unit waiting until the last of them has gone
+        // out.  The order is pinned: left alone the scheduler sinks each read to the product
+        // that needs it, a step later.
+        auto multiply = [&](Fragments& now, auto reads, uint32_t unit, uint32_t step, Fragments& next,
+                            auto requests, uint32_t requested) __attribute__((always_inline)) {
+            constexpr bool kRead = decltype(reads)::value, kRequest = decltype(requests)::value;
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (uint32_t tm = 0; tm < kTm; ++tm) {
+                if constexpr (kRead) {
+#pragma unroll
+                    for (uint32_t i = tm * kTn / kTm; i < (tm + 1) * kTn / kTm; ++i) {
+                        read_weights(unit, step, i, next);
+                    }
+                    if (kTwoSetsOfX) {
+                        read_x(unit, step, tm, next);
+                    } else if (tm > 0) {
+                        read_x(unit, step, tm - 1, next);
+                    }
+                }
+                if constexpr (kRequest) {
+#pragma unroll
+                    for (uint32_t i = tm * kTransfers / kTm; i < (tm + 1) * kTransfers / kTm; ++i) {
+                        request_one(requested, i);
+                    }
+                }
 #pragma unroll
                 for (uint32_t tn = 0; tn < kTn; ++tn) {
-                    acc[tn][tm] = product(f.w[tn], f.x[tm], acc[tn][tm]);
+                    acc[tn][tm] = product(now.w[tn], x_of(now, tm), acc[tn][tm]);
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
+            if constexpr (kRead && !kTwoSetsOfX) read_x(unit, step, kTm - 1, next);
         };
-        // issue order of a slot: a read, then a few products, so that the waves' reads are
-        // spread over the slot instead of queueing at the LDS while the matrix unit waits (left
-        // alone the scheduler sinks each read to the product that needs it, a slot later).  No
-        // branch between the reads and the products: at a join the compiler would wait for the
-        // reads first.
-        auto interleave = [&]() __attribute__((always_inline)) {
-            constexpr uint32_t kReads = kTm + kTn, kBetween = kTm * kTn / kReads;
-#pragma unroll
-            for (uint32_t i = 0; i < kReads; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, kBetween, 0);
-            }
-            __builtin_amdgcn_sched_group_barrier(0x008, kTm * kTn - kReads * kBetween, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        };
+        using std::bool_constant;
         // first step of `unit` (its fragments are in `first`): read the second step's while
-        // multiplying; the unit was published a slot ago, so nothing to wait for
-        auto first_step = [&](uint32_t unit, const Fragments& first, Fragments& second)
+        // multiplying; the unit was published a step ago, so nothing to wait for
+        auto first_step = [&](uint32_t unit, Fragments& first, Fragments& second)
                               __attribute__((always_inline)) {
-            __builtin_amdgcn_sched_barrier(0);
-            read_fragments(unit, 1, second);
-            multiply(first);
-            interleave();
+            multiply(first, bool_constant<true>{}, unit, 1, second, bool_constant<false>{}, 0);
         };
-        // second step of `unit`: the next unit (requested a unit ago) has landed - mine, then
-        // everybody's -, and nobody reads the unit before this one any more, so the unit after
-        // the next goes into its place; read the next unit's first fragments while multiplying
-        auto second_step = [&](uint32_t unit, const Fragments& second, Fragments& first_of_next,
+        // second step of `unit`: the next unit has landed - mine, then everybody's -, and nobody
+        // reads this one any more (its last fragments are in `second`), so the unit kRing further
+        // on goes into its place; read the next unit's first fragments while multiplying
+        auto second_step = [&](uint32_t unit, Fragments& second, Fragments& first_of_next,
                                auto with_request) __attribute__((always_inline)) {
             if constexpr (decltype(with_request)::value) {
-                __builtin_amdgcn_s_waitcnt(vmcnt((kRing - 2) * (kXTransfers + kWTransfers)));
+                __builtin_amdgcn_s_waitcnt(vmcnt((kRing - 2) * kTransfers));
             } else {
                 __builtin_amdgcn_s_waitcnt(vmcnt(0));
             }
             __syncthreads();
-            if constexpr (decltype(with_request)::value) request(unit + kRing);
-            __builtin_amdgcn_sched_barrier(0);
-            read_fragments(unit + 1, 0, first_of_next);
-            multiply(second);
-            interleave();
+            multiply(second, bool_constant<true>{}, unit + 1, 0, first_of_next, with_request, unit + kRing);
         };
-        using std::bool_constant;
 
         // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own:
         // in a whole round the workgroups of an XCD (b / 8 = 0, 1, ...) take a run of consecutive
@@ -238,7 +259,7 @@ struct BlockProduct {
         };
         uint32_t round = 0, tile = of_round(0);
         if (tile >= tiles) return;
-        place(tile, m_aim, n_aim);
+        aim(tile);
         const uint32_t ahead = min(kRing, units);
         for (uint32_t unit = 0; unit < ahead; ++unit) request(unit);
         while (true) {
@@ -252,7 +273,10 @@ struct BlockProduct {
             __builtin_amdgcn_s_waitcnt(vmcnt(0));
             __syncthreads();
             Fragments a, b;
-            read_fragments(0, 0, a);
+#pragma unroll
+            for (uint32_t tn = 0; tn < kTn; ++tn) read_weights(0, 0, tn, a);
+#pragma unroll
+            for (uint32_t tm = 0; tm < kTm; ++tm) read_x(0, 0, tm, a);
             uint32_t unit = 0;
             for (; unit + kRing < units; ++unit) {
                 first_step(unit, a, b);
@@ -263,7 +287,7 @@ struct BlockProduct {
                 second_step(unit, b, a, bool_constant<false>{});
             }
             first_step(unit, a, b);
-            multiply(b);
+            multiply(b, bool_constant<false>{}, 0, 0, a, bool_constant<false>{}, 0);
 
             uint32_t m0, n0;
             place(tile, m0, n0);
@@ -271,7 +295,7 @@ struct BlockProduct {
             const uint32_t next_tile = of_round(round);
             __syncthreads();   // nobody reads the stages any more
             if (next_tile < tiles) {
-                place(next_tile, m_aim, n_aim);
+                aim(next_tile);
                 for (uint32_t unit = 0; unit < ahead; ++unit) request(unit);
             }
             // the lane holds columns n0 + kWaveN wave_n + 16 tn + 4 g + j of row
@@ -292,22 +316,12 @@ struct BlockProduct {
     }
 };
 
-// The tiles a block product is launched with, and what one of them costs on a compute unit.
-// `single` is the time of one tile alone on it, `both`
-// of two side by side, as ns per 64 columns and ns per tile (fitted to products of 33 .. 16384
-// rows with 2048 .. 12352 outputs over K = 2176 and 4352).
-template <typename Element>
-struct BlockTiles {
-    typedef BlockProduct<Element, 256, 256, 2, 4> Large;      // the most products per LDS byte
-    typedef BlockProduct<Element, 128, 128, 2, 4> Even;       // two a compute unit hide each other's waits
-    typedef BlockProduct<Element, 128, 128, 2, 4, 3> Deep;    // one a compute unit, a unit further ahead
-    typedef BlockProduct<Element, 64, 128, 2, 4, 3> Low;
-    typedef BlockProduct<Element, 64, 64, 2, 4, 4> Small;
-};
-enum class BlockTile { Large, Even, Deep, Low, Small };
+enum class BlockTile { Large, Even, Deep, Low, Tall, Small, Least };
 
 // The tile with the shortest estimate.  A compute unit takes ceil(tiles / compute_units) tiles,
-// two at a time where two workgroups fit it.
+// two at a time where two workgroups fit it: `single` is the time of one tile alone on it, `both`
+// of two side by side, as ns per 64 columns and ns per tile (fitted to the products below and to
+// others of 33 .. 16384 rows, 2048 .. 12352 outputs and K = 2176 and 4352).
 inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                    uint32_t compute_units) {
     struct Cost {
@@ -315,11 +329,13 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
     };
     static constexpr Cost kCosts[] = {
-        {BlockTile::Large, 256, 256, 1700, 7000, 3400, 14000},
+        {BlockTile::Large, 256, 256, 1580, 8000, 3160, 16000},
         {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
-        {BlockTile::Deep, 128, 128, 570, 2000, 1140, 4000},
-        {BlockTile::Low, 64, 128, 350, 1500, 630, 3000},
+        {BlockTile::Deep, 128, 128, 520, 2000, 1040, 4000},
+        {BlockTile::Low, 64, 128, 330, 1500, 630, 3000},
+        {BlockTile::Tall, 128, 64, 330, 1500, 630, 3000},
         {BlockTile::Small, 64, 64, 200, 1000, 400, 2000},
+        {BlockTile::Least, 32, 64, 155, 1000, 275, 1500},
     };
     const uint64_t units = in_dim / 64;
     BlockTile best = BlockTile::Large;
@@ -336,6 +352,50 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
     }
     return best;
 }
+// The tiles a block product is launched with.  What bounds one is how the products of the two
+// to four waves of a SIMD fill each other's waits (LDS reads take a fifth of the cycles, the
+// matrix unit 58 % of them with eight waves that read, request and multiply in turns); units of
+// 32 columns in a deeper ring, with a barrier each, were 6 to 20 % slower.  Measured, f16 operands:
+//   Large  16384 x 2176 x 12352 / 9216, 8192 x 4352 x 2048: 790 / 563 / 114 us = 1.12 / 1.17 /
+//          1.29 PFLOP/s (eight waves of 128 x 64: 832 / 546 / 110 us; with all transfers of a unit
+//          issued ahead of its products 865 / 573 / 116 us)
+//   Even   2048 x 2176 x 9216: 91 us; Large 106, Deep 97, Low 113
+//   Deep   2048 x 4352 x 2048: 38 us; Even 48, Large 85
+//   Low    777 x 4352 x 2048: 24 us; Deep 30, Even 43
+//   Tall   100 x 2176 x 12352: 13.5 us; Deep 17, Low 19, Small 20
+//   Small  300 x 4352 x 2048: 15 us; Least 20, Low 22, Deep 29
+//   Least  100 x 4352 x 2048: 11 us; Small 14, Low 19, Deep 27
+template <typename Element>
+struct BlockTiles {
+    typedef BlockProduct<Element, 256, 256, 4, 4> Large;      // the most products per byte fetched
+    typedef BlockProduct<Element, 128, 128, 2, 4> Even;       // two a compute unit hide each other's waits
+    typedef BlockProduct<Element, 128, 128, 2, 4, 4> Deep;    // one a compute unit, two units further ahead
+    typedef BlockProduct<Element, 64, 128, 2, 4, 3> Low;
+    typedef BlockProduct<Element, 128, 64, 4, 2, 3> Tall;
+    typedef BlockProduct<Element, 64, 64, 2, 2, 4> Small;
+    typedef BlockProduct<Element, 32, 64, 2, 2, 4> Least;
+
+    // the tile a call takes, as use(product) of a value of its type
+    template <typename Use>
+    static auto choose(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units, Use use) {
+        switch (choose_block_tile(rows, in_dim, out_dim, compute_units)) {
+        case BlockTile::Even: return use(Even{});
+        case BlockTile::Deep: return use(Deep{});
+        case BlockTile::Low: return use(Low{});
+        case BlockTile::Tall: return use(Tall{});
+        case BlockTile::Small: return use(Small{});
+        case BlockTile::Least: return use(Least{});
+        default: return use(Large{});
+        }
+    }
+    // use(product) of every tile, as long as it says true
+    template <typename Use>
+    static bool each(Use use) {
+        return use(Large{}) && use(Even{}) && use(Deep{}) && use(Low{}) && use(Tall{}) && use(Small{}) &&
+               use(Least{});
+    }
+};
+
 // workgroups of a launch: a persistent one per place on the device, or one per tile
 template <typename Product>
 uint32_t block_workgroups(uint32_t rows, uint32_t out_dim, uint32_t compute_units) {

@@ -445,15 +445,6 @@ static_assert(static_cast<uint64_t>(kHidden) * unfolded_columns(kGdnValueValues)
               "the output projection's weights fit as well");
 
 typedef BlockTiles<_Float16> Q4Tiles;
-template <typename Product>
-void launch_product(const Q4Projection& p, const Unfold& u, uint32_t compute_units, hipStream_t stream) {
-    const uint32_t out_rows = p.first_row[p.segments];
-    hipLaunchKernelGGL(q4_product_kernel<Product>,
-                       dim3(block_workgroups<Product>(u.x_rows, out_rows, compute_units)),
-                       dim3(Product::kThreads), Product::kLdsBytes, stream, u, p.output, p.output_stride,
-                       unfolded_columns(p.k_size), out_rows);
-}
-
 int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
     const StreamWorkspace workspace = stream_workspace(stream);
     // a queue whose workspace could not be allocated: the rows kernel takes any number of rows
@@ -481,15 +472,13 @@ int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL(q4_unfold_kernel<8>, grid, dim3(256), 0, stream, p, u);
         }
         u.weight_rows = 0;
-        auto launch = launch_product<Q4Tiles::Large>;
-        switch (choose_block_tile(u.x_rows, columns, out_rows, workspace.compute_units)) {
-        case BlockTile::Large: break;
-        case BlockTile::Even: launch = launch_product<Q4Tiles::Even>; break;
-        case BlockTile::Deep: launch = launch_product<Q4Tiles::Deep>; break;
-        case BlockTile::Low: launch = launch_product<Q4Tiles::Low>; break;
-        case BlockTile::Small: launch = launch_product<Q4Tiles::Small>; break;
-        }
-        launch(p, u, workspace.compute_units, stream);
+        Q4Tiles::choose(u.x_rows, columns, out_rows, workspace.compute_units, [&](auto product) {
+            typedef decltype(product) Product;
+            hipLaunchKernelGGL(q4_product_kernel<Product>,
+                               dim3(block_workgroups<Product>(u.x_rows, out_rows, workspace.compute_units)),
+                               dim3(Product::kThreads), Product::kLdsBytes, stream, u, p.output,
+                               p.output_stride, columns, out_rows);
+        });
     }
     return TT_OK;
 }
@@ -928,15 +917,13 @@ uint64_t q4_workspace_bytes() { return kUnfoldWorkspaceBytes; }
 
 #if !defined(__HIP_DEVICE_COMPILE__)  // host-side table of launchers
 bool prepare_q4_kernels() {
-    const auto allow = [](auto product, const void* kernel) {
-        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   decltype(product)::kLdsBytes) == hipSuccess;
+    const auto allow = [](auto product) {
+        typedef decltype(product) Product;
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(q4_product_kernel<Product>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   Product::kLdsBytes) == hipSuccess;
     };
-    return allow(Q4Tiles::Large{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Large>)) &&
-           allow(Q4Tiles::Even{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Even>)) &&
-           allow(Q4Tiles::Deep{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Deep>)) &&
-           allow(Q4Tiles::Low{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Low>)) &&
-           allow(Q4Tiles::Small{}, reinterpret_cast<const void*>(q4_product_kernel<Q4Tiles::Small>)) &&
+    return Q4Tiles::each(allow) &&
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<4, true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                kRowsStagedBytes) == hipSuccess &&

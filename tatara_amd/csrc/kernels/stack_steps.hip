@@ -299,26 +299,16 @@ bool dense_block_operands_fit(const uint16_t* input, const uint16_t* weights, ui
            static_cast<uint64_t>(out_dim) * in_dim * 2 < (1ull << 32);
 }
 
-template <typename Product>
-void launch_dense_product(const uint16_t* input, const uint16_t* weights, uint16_t* output,
-                          uint32_t rows, uint32_t in_dim, uint32_t out_dim, hipStream_t stream) {
-    hipLaunchKernelGGL(dense_block_kernel<Product>,
-                       dim3(block_workgroups<Product>(rows, out_dim, current_device_compute_units())),
-                       dim3(Product::kThreads), Product::kLdsBytes, stream, input, weights, output, rows,
-                       in_dim, out_dim);
-}
 typedef BlockTiles<__bf16> DenseTiles;
 void launch_dense_block(const uint16_t* input, const uint16_t* weights, uint16_t* output, uint32_t rows,
                         uint32_t in_dim, uint32_t out_dim, hipStream_t stream) {
-    auto launch = launch_dense_product<DenseTiles::Large>;
-    switch (choose_block_tile(rows, in_dim, out_dim, current_device_compute_units())) {
-    case BlockTile::Large: break;
-    case BlockTile::Even: launch = launch_dense_product<DenseTiles::Even>; break;
-    case BlockTile::Deep: launch = launch_dense_product<DenseTiles::Deep>; break;
-    case BlockTile::Low: launch = launch_dense_product<DenseTiles::Low>; break;
-    case BlockTile::Small: launch = launch_dense_product<DenseTiles::Small>; break;
-    }
-    launch(input, weights, output, rows, in_dim, out_dim, stream);
+    const uint32_t units = current_device_compute_units();
+    DenseTiles::choose(rows, in_dim, out_dim, units, [&](auto product) {
+        typedef decltype(product) Product;
+        hipLaunchKernelGGL(dense_block_kernel<Product>, dim3(block_workgroups<Product>(rows, out_dim, units)),
+                           dim3(Product::kThreads), Product::kLdsBytes, stream, input, weights, output, rows,
+                           in_dim, out_dim);
+    });
 }
 
 // dense_bf16: b0 input [rows][in], b1 weights [out][in], b2 output [rows][out], c3 rows,
@@ -389,15 +379,12 @@ bool prepare_stack_kernels() {
         units > 0) {
         g_compute_units[device] = static_cast<uint32_t>(units);
     }
-    const auto allow = [](auto product, const void* kernel) {
-        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   decltype(product)::kLdsBytes) == hipSuccess;
-    };
-    return allow(DenseTiles::Large{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Large>)) &&
-           allow(DenseTiles::Even{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Even>)) &&
-           allow(DenseTiles::Deep{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Deep>)) &&
-           allow(DenseTiles::Low{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Low>)) &&
-           allow(DenseTiles::Small{}, reinterpret_cast<const void*>(dense_block_kernel<DenseTiles::Small>));
+    return DenseTiles::each([](auto product) {
+        typedef decltype(product) Product;
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(dense_block_kernel<Product>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   Product::kLdsBytes) == hipSuccess;
+    });
 }
 #endif
 
