@@ -22,6 +22,7 @@
 // (query, key) pair per head.
 #include "../tt_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace tt {
@@ -88,7 +89,13 @@ struct FlashPrefillArgs {
 // in the register order of its lanes; the last one - told by an arrival count, nobody waits
 // for anybody - adds the others' to its own with the usual reference change and writes the
 // rows.  A walk of fewer than kMinTilesPerSplit key tiles per workgroup is shared by fewer.
+// From kMergeSplitsFrom sharers on, every workgroup leaves its result and a dispatch of many
+// workgroups merges them: the last one alone reads 270 KB per sharer at what one compute unit
+// takes in.  With that, few rows share a walk among more than the kMaxFlashSplits a caller can
+// name (kWideFlashSplits), through the queue's workspace.
 constexpr uint32_t kMaxFlashSplits = 8;
+constexpr uint32_t kWideFlashSplits = 64;
+constexpr uint32_t kMergeSplitsFrom = 3;
 constexpr uint32_t kMinTilesPerSplit = 4;
 constexpr uint32_t kPartialBytes = 512 * 132 * 4;   // per lane 128 values of O, two references, two row-sum shares
 constexpr uint32_t kArrivalBytesPerTile = 4;
@@ -132,6 +139,13 @@ constexpr uint32_t kFlashLdsBytes = kKeyRingBytes + kRing * kValuePairedStageByt
 
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 
+// workgroups that share a walk of that many key tiles
+__device__ __forceinline__ uint32_t flash_sharers(uint32_t splits, uint32_t walk_tiles) {
+    return min(splits, max(walk_tiles / kMinTilesPerSplit, 1u));
+}
+
+// kMerged: the partial results are merged by flash_merge_kernel
+template <bool kMerged>
 __global__ __launch_bounds__(kFlashWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attention_flash_prefill_kernel(FlashPrefillArgs a) {
     constexpr uint32_t NB = 2;
@@ -151,7 +165,7 @@ void attention_flash_prefill_kernel(FlashPrefillArgs a) {
     const uint32_t tile_keys = a.tile_context + min(p0 + kTilePositions, a.rows);  // visible count
     const uint32_t walk_tiles = (tile_keys + kTileKeys - 1) / kTileKeys;
     // this workgroup's share of the walk: key tiles [kb_begin, nkb)
-    const uint32_t sharers = min(a.splits, max(walk_tiles / kMinTilesPerSplit, 1u));
+    const uint32_t sharers = flash_sharers(a.splits, walk_tiles);
     const uint32_t share = blockIdx.z;
     if (share >= sharers) return;
     const uint32_t kb_begin = static_cast<uint32_t>(static_cast<uint64_t>(walk_tiles) * share / sharers);
@@ -474,6 +488,20 @@ void attention_flash_prefill_kernel(FlashPrefillArgs a) {
         // element e of a lane's 132 (O of head b, dim block j, value i at (b*16+j)*4+i, then
         // the two references and the two row-sum shares) lies at [e][thread]
         float* const mine = partials + static_cast<uint64_t>(share) * (kPartialBytes / 4) + threadIdx.x;
+        if constexpr (kMerged) {
+            if (p0 + half * 16 >= a.rows) return;   // no row of this wave is there
+#pragma unroll
+            for (uint32_t b = 0; b < NB; ++b) {
+#pragma unroll
+                for (uint32_t j = 0; j < 16; ++j) {
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) mine[((b * 16 + j) * 4 + i) * 512] = o[b][j][i];
+                }
+                mine[(128 + b) * 512] = m_run[b];
+                mine[(130 + b) * 512] = l_run[b];
+            }
+            return;
+        }
 #pragma unroll
         for (uint32_t b = 0; b < NB; ++b) {
 #pragma unroll
@@ -546,6 +574,79 @@ void attention_flash_prefill_kernel(FlashPrefillArgs a) {
             }
         }
     }
+}
+
+// Merges the partial results of a shared walk.  grid (64 x position tiles, kv heads) x 256: a
+// workgroup takes what one wave of the walk holds of one head and four dim blocks (16 positions
+// x 64 dims) from all sharers, a quarter of them per wave, and writes the rows.  Its time is the
+// chain of one sharer's loads after another, hence few values a lane and many workgroups: 12 rows
+// behind 5003 tokens, walked by 39 workgroups a kv head, 74.5 -> 24.8 us walk and merge (eight,
+// the last merging), 12 rows behind 30000 198 -> 43, 100 behind 8000 97 -> 47, 777 behind 1501
+// (five, merged apart) 72 -> 57.
+__global__ __launch_bounds__(256) void flash_merge_kernel(FlashPrefillArgs a) {
+    __shared__ float sums[4][18][64];
+    const uint32_t part = blockIdx.x & 63, tile = blockIdx.x >> 6, kvh = blockIdx.y;
+    const uint32_t source = part >> 3, b = (part >> 2) & 1, j0 = (part & 3) * 4;
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t p0 = tile * kTilePositions + (source >> 2) * 16;
+    if (p0 >= a.rows) return;
+    const uint32_t tile_keys = a.tile_context + min((tile + 1) * kTilePositions, a.rows);
+    const uint32_t sharers = flash_sharers(a.splits, (tile_keys + kTileKeys - 1) / kTileKeys);
+    if (sharers <= 1) return;   // written by the walk itself
+    const float* partials =
+        reinterpret_cast<const float*>(a.scratch + flash_arrival_bytes(a.rows)) +
+        static_cast<uint64_t>(tile * kAttnKvHeads + kvh) * a.splits * (kPartialBytes / 4) +
+        source * 64 + lane;
+    float reference = -INFINITY;
+    for (uint32_t share = wave; share < sharers; share += 4) {
+        reference = fmaxf(reference,
+                          partials[static_cast<uint64_t>(share) * (kPartialBytes / 4) + (128 + b) * 512]);
+    }
+    float row_sum = 0.0f, o[16];
+#pragma unroll
+    for (uint32_t e = 0; e < 16; ++e) o[e] = 0.0f;
+#pragma unroll 2
+    for (uint32_t share = wave; share < sharers; share += 4) {
+        const float* theirs = partials + static_cast<uint64_t>(share) * (kPartialBytes / 4);
+        const float take = __builtin_amdgcn_exp2f(theirs[(128 + b) * 512] - reference);
+        row_sum += theirs[(130 + b) * 512] * take;
+#pragma unroll
+        for (uint32_t e = 0; e < 16; ++e) o[e] += theirs[((b * 16 + j0) * 4 + e) * 512] * take;
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < 16; ++e) sums[wave][e][lane] = o[e];
+    sums[wave][16][lane] = row_sum;
+    sums[wave][17][lane] = reference;   // -infinity where this wave had no sharer
+    __syncthreads();
+    // wave w finishes dim block j0 + w
+    float common = sums[0][17][lane];
+#pragma unroll
+    for (uint32_t w = 1; w < 4; ++w) common = fmaxf(common, sums[w][17][lane]);
+    float total[4] = {0.0f, 0.0f, 0.0f, 0.0f}, l = 0.0f;
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w) {
+        const float take = __builtin_amdgcn_exp2f(sums[w][17][lane] - common);
+        l += sums[w][16][lane] * take;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) total[i] += sums[w][wave * 4 + i][lane] * take;
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    const uint32_t row = p0 + (lane & 15);
+    if (row >= a.rows) return;
+    const float inv = 1.0f / l;
+    const uint32_t head = kvh * kAttnHeadsPerKv + (source & 3) * 2 + b;
+    const uint64_t at = (static_cast<uint64_t>(row) * kAttnQueryHeads + head) * kD + (j0 + wave) * 16 +
+                        (lane >> 4) * 4;
+    const u32x2 gw = *reinterpret_cast<const u32x2*>(a.gate + at);
+    uint32_t bits[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        const float gate = __uint_as_float((i & 1) ? (gw[i >> 1] & 0xFFFF0000u) : (gw[i >> 1] << 16));
+        const float sig = 1.0f / (1.0f + __expf(-gate));
+        bits[i] = f32_to_bf16_bits((total[i] * inv) * sig);
+    }
+    *reinterpret_cast<u32x2*>(a.out + at) = u32x2{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16)};
 }
 
 // --------------------------------------------------- exact control path ------
@@ -722,26 +823,37 @@ int32_t flash_blk(const Bindings& b, const Grid& g, hipStream_t stream, bool val
         if (f.splits > 1) f.scratch = a.buffer<uint8_t>(9, flash_prefill_scratch_bytes(f.rows, f.splits));
     }
     if (a.status != TT_OK || validate_only) return a.status;
-    if (!shared_walk) {
-        // the reference's bindings carry no scratch: the walk is shared through the queue's
-        // own workspace where the block is too few rows to fill the device
-        const StreamWorkspace workspace = stream_workspace(stream);
-        if (workspace.base != nullptr) {
-            const uint32_t planned = flash_prefill_splits(f.rows, visible, workspace.compute_units);
-            if (planned > 1 && flash_prefill_scratch_bytes(f.rows, planned) <= workspace.bytes) {
-                f.splits = planned;
-                f.scratch = workspace.base;
-            }
+    // The reference's bindings carry no scratch: its walk is shared through the queue's own
+    // workspace where the block is too few rows to fill the device.  So is one that is to be
+    // shared by as many as can be named, among as many as fill the device.
+    const uint32_t tiles = (f.rows + kTilePositions - 1) / kTilePositions;
+    const StreamWorkspace workspace = stream_workspace(stream);
+    if (workspace.base != nullptr && (!shared_walk || f.splits == kMaxFlashSplits)) {
+        uint32_t planned = flash_prefill_splits(f.rows, visible, workspace.compute_units);
+        if (planned == kMaxFlashSplits) {
+            const uint32_t walk_tiles = (visible + kTileKeys - 1) / kTileKeys;
+            planned = std::max(planned, std::min({workspace.compute_units / (tiles * kAttnKvHeads),
+                                                  walk_tiles / kMinTilesPerSplit, kWideFlashSplits}));
+        }
+        if (planned > f.splits && flash_prefill_scratch_bytes(f.rows, planned) <= workspace.bytes) {
+            f.splits = planned;
+            f.scratch = workspace.base;
         }
     }
-    const uint32_t tiles = (f.rows + kTilePositions - 1) / kTilePositions;
+    const dim3 grid(tiles, kAttnKvHeads, f.splits);
+    if (f.splits >= kMergeSplitsFrom) {
+        hipLaunchKernelGGL(attention_flash_prefill_kernel<true>, grid, dim3(kFlashWaves * 64), kFlashLdsBytes,
+                           stream, f);
+        hipLaunchKernelGGL(flash_merge_kernel, dim3(64 * tiles, kAttnKvHeads), dim3(256), 0, stream, f);
+        return TT_OK;
+    }
     if (f.splits > 1) {
         const uint32_t words = tiles * kAttnKvHeads;
         hipLaunchKernelGGL(clear_arrivals_kernel, dim3((words + 255) / 256), dim3(256), 0, stream,
                            reinterpret_cast<uint32_t*>(f.scratch), words);
     }
-    hipLaunchKernelGGL(attention_flash_prefill_kernel, dim3(tiles, kAttnKvHeads, f.splits),
-                       dim3(kFlashWaves * 64), kFlashLdsBytes, stream, f);
+    hipLaunchKernelGGL(attention_flash_prefill_kernel<false>, grid, dim3(kFlashWaves * 64), kFlashLdsBytes,
+                       stream, f);
     return TT_OK;
 }
 
@@ -752,7 +864,7 @@ int32_t op_attention_flash_blk(const Bindings& b, const Grid& g, hipStream_t str
 
 // attention_flash_split_blk (no counterpart in the reference): the bindings, constants and
 // grid of attention_flash_v2_blk, plus b9 scratch and c10 splits (1..8) - the workgroups that
-// share each position tile's key walk.  tt_flash_prefill_splits gives the count that fills
+// share each position tile's key walk (8: or more, see kWideFlashSplits).  tt_flash_prefill_splits gives the count that fills
 // the device for a block of `rows` rows that sees `visible` keys, tt_flash_prefill_scratch_bytes the bytes b9 must hold
 // (none for one split).  Same results as attention_flash_v2_blk up to the order of fp32 sums.
 int32_t op_attention_flash_split_blk(const Bindings& b, const Grid& g, hipStream_t stream,
@@ -819,9 +931,12 @@ int32_t op_attention_combine_blk(const Bindings& b, const Grid& g, hipStream_t s
 
 #if !defined(__HIP_DEVICE_COMPILE__)  // host-side tables of launchers
 bool prepare_prefill_kernels() {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(attention_flash_prefill_kernel),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               kFlashLdsBytes) == hipSuccess;
+    const auto allow = [](const void* kernel) {
+        return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kFlashLdsBytes) ==
+               hipSuccess;
+    };
+    return allow(reinterpret_cast<const void*>(attention_flash_prefill_kernel<false>)) &&
+           allow(reinterpret_cast<const void*>(attention_flash_prefill_kernel<true>));
 }
 
 const KernelDesc kAttentionPrefillKernels[] = {

@@ -199,6 +199,30 @@ def test_shared_walk_with_a_share_in_the_exact_loop():
                   splits=2, select=list(range(0, 320, 7)) + list(range(280, 320)))
 
 
+@pytest.mark.parametrize("rows,base", [(1, 8000), (16, 8000), (17, 6001), (64, 4100), (65, 1023), (12, 1151)])
+def test_walk_shared_by_as_many_as_fill_the_device(rows, base):
+    """attention_flash_v2_blk of few rows plans up to 64 sharers in its queue's workspace and a
+    dispatch of its own merges them: one row, half a position tile and a row more, whole tiles
+    and a row more, walks of a few more key tiles than eight sharers take - against the checker
+    and, replayed, against itself."""
+    print(f"[case] wide shared walk rows {rows} base {base}", flush=True)
+    _prefill_case(rows, base, 8192, 0x5A80 + rows, replays=2)
+
+
+def test_merged_walk_with_a_share_in_the_exact_loop():
+    """As above with the shares merged by a dispatch of its own (three sharers asked, of which
+    the walks of ten key tiles take two)."""
+    print("[case] merged key walk, one share in the exact softmax loop", flush=True)
+    rows = 320
+    proj = ol.gaussian_bf16(0xE8B0, rows * 9216).reshape(rows, 9216)
+    for r in range(288, rows):
+        proj[r, 8192:8448] = proj[rows - 1, 0:256]
+        proj[r, 8448:8704] = proj[rows - 1, 4096:4352]
+    w = np.full(256, 0x4040, np.uint16)                     # 3.0
+    _prefill_case(rows, 0, 512, 0xE8B1, proj=np.ascontiguousarray(proj).reshape(-1), weights=(w, w),
+                  splits=3, select=list(range(0, 320, 7)) + list(range(280, 320)))
+
+
 def test_shared_walk_of_a_2048_row_block_deep_in_a_cache():
     """The shape the operator is for: a 2048-row block behind 6144 cached tokens, as many shares
     as fill the device (two on 256 compute units); sampled rows against the checker, every row
