@@ -211,6 +211,20 @@ int32_t tt_pass_set_bytes(tt_command_buffer* command_buffer, const void* bytes,
 int32_t tt_pass_dispatch(tt_command_buffer* command_buffer, uint64_t groups_x, uint64_t groups_y,
                          uint64_t groups_z, uint64_t threads_x, uint64_t threads_y,
                          uint64_t threads_z);
+/* set_compute_pipeline, the bindings in order and dispatch_threadgroups in one call (no reference
+ * counterpart): a binding with a buffer is set_buffer, one without is set_bytes of the four bytes
+ * of `constant`.  On an error *failed, if given, is 0 for the pipeline, 1 .. count for a binding,
+ * count + 1 for the dispatch; what came before it has taken effect, as with the single calls. */
+typedef struct tt_binding {
+    const tt_buffer* buffer;
+    uint64_t offset_bytes;
+    uint32_t index;
+    uint32_t constant;
+} tt_binding;
+int32_t tt_pass_encode(tt_command_buffer* command_buffer, const tt_pipeline* pipeline,
+                       const tt_binding* bindings, uint32_t count, uint64_t groups_x,
+                       uint64_t groups_y, uint64_t groups_z, uint64_t threads_x,
+                       uint64_t threads_y, uint64_t threads_z, uint32_t* failed);
 /* memory_barrier (commands.h:461): the stream is in-order, so this only
  * validates the pass. */
 int32_t tt_pass_barrier(tt_command_buffer* command_buffer);

@@ -7,6 +7,7 @@ CommandBuffer.set_buffer / set_bytes / dispatch, commit / wait_until_completed
 BackendError; nothing here computes anything."""
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -25,7 +26,7 @@ EXPORTED_SYMBOLS = [
     "tt_library_function_count", "tt_library_function_name", "tt_pipeline_create",
     "tt_pipeline_destroy", "tt_pipeline_name", "tt_command_buffer_create",
     "tt_command_buffer_destroy", "tt_pass_begin", "tt_pass_end", "tt_pass_set_pipeline",
-    "tt_pass_set_buffer", "tt_pass_set_bytes", "tt_pass_dispatch", "tt_pass_barrier",
+    "tt_pass_set_buffer", "tt_pass_set_bytes", "tt_pass_dispatch", "tt_pass_encode", "tt_pass_barrier",
     "tt_blit_copy", "tt_blit_fill", "tt_command_count", "tt_commit", "tt_wait",
     "tt_command_buffer_reset", "tt_command_buffer_compile", "tt_command_buffer_set_profiling",
     "tt_command_name", "tt_command_gpu_ms", "tt_attention_decode_lanes_static",
@@ -92,6 +93,7 @@ def lib():
         "tt_pass_set_pipeline": (i32, [vp, vp]),
         "tt_pass_set_buffer": (i32, [vp, vp, u64, u32]),
         "tt_pass_set_bytes": (i32, [vp, vp, u32, u32]),
+        "tt_pass_encode": (i32, [vp, vp, C.c_char_p, u32] + [u64] * 6 + [C.POINTER(u32)]),
         "tt_pass_dispatch": (i32, [vp, u64, u64, u64, u64, u64, u64]),
         "tt_pass_barrier": (i32, [vp]),
         "tt_blit_copy": (i32, [vp, vp, u64, vp, u64, u64]),
@@ -368,6 +370,23 @@ class CommandBuffer:
     def encode(self, pipeline, buffers, constants, groups, threads):
         """set_pipeline + bindings + dispatch; buffers {index: Buffer | (Buffer, offset)},
         constants {index: uint32}."""
+        # one call into the library for the whole command: a prefill block of eight layers is
+        # about 600 bindings, and a call each took longer than a short block takes on the GPU
+        flat, refs = [], [pipeline]
+        for index, b in buffers.items():
+            buffer, offset = b if isinstance(b, tuple) else (b, 0)
+            flat += (buffer.handle.value or 0 if buffer.handle else 0, int(offset), int(index), 0)
+            refs.append(buffer)
+        plain = 0 not in flat[::4]   # a released buffer is set_buffer's error
+        for index, c in constants.items():
+            plain = plain and isinstance(c, (int, np.integer))   # set_bytes takes bytes as well
+            flat += (0, 0, int(index), int(c) if plain else 0)
+        try:
+            packed = struct.pack("QQII" * (len(flat) // 4), *flat) if plain else None
+        except struct.error:   # out of range: as the single calls see it
+            packed = None
+        if packed is not None:
+            return self._encode(pipeline, packed, flat, refs, groups, threads)
         self.set_pipeline(pipeline)
         for index, b in buffers.items():
             if isinstance(b, tuple):
@@ -377,6 +396,19 @@ class CommandBuffer:
         for index, c in constants.items():
             self.set_bytes(c, index)
         self.dispatch(groups, threads)
+
+    def _encode(self, pipeline, packed, flat, refs, groups, threads):
+        count = len(flat) // 4
+        failed = C.c_uint32()
+        status = lib().tt_pass_encode(self.handle, pipeline.handle, packed, count, *map(int, groups),
+                                      *(1,) * (3 - len(groups)), *map(int, threads),
+                                      *(1,) * (3 - len(threads)), C.byref(failed))
+        self._refs += refs
+        if status:
+            at = failed.value
+            where = ("set_compute_pipeline" if at == 0 else "dispatch_threadgroups" if at > count else
+                     f"set_{'buffer' if flat[4 * at - 4] else 'bytes'}[{flat[4 * at - 2]}]")
+            raise BackendError(status, where)
 
     def copy_buffer(self, source, source_offset, destination, destination_offset, length):
         _check(lib().tt_blit_copy(self.handle, source.handle, source_offset, destination.handle,

@@ -714,6 +714,25 @@ int32_t tt_pass_dispatch(tt_command_buffer* cb, uint64_t gx, uint64_t gy, uint64
     return TT_OK;
 }
 
+int32_t tt_pass_encode(tt_command_buffer* cb, const tt_pipeline* pipeline, const tt_binding* bindings,
+                       uint32_t count, uint64_t gx, uint64_t gy, uint64_t gz, uint64_t tx, uint64_t ty,
+                       uint64_t tz, uint32_t* failed) {
+    uint32_t at = 0;
+    int32_t status = tt_pass_set_pipeline(cb, pipeline);
+    if (status == TT_OK && bindings == nullptr && count != 0) status = TT_CMD_INVALID_BUFFER;
+    while (status == TT_OK && at < count) {
+        const tt_binding& b = bindings[at++];
+        status = b.buffer != nullptr ? tt_pass_set_buffer(cb, b.buffer, b.offset_bytes, b.index)
+                                     : tt_pass_set_bytes(cb, &b.constant, 4, b.index);
+    }
+    if (status == TT_OK) {
+        at = count + 1;
+        status = tt_pass_dispatch(cb, gx, gy, gz, tx, ty, tz);
+    }
+    if (status != TT_OK && failed != nullptr) *failed = at;
+    return status;
+}
+
 int32_t tt_pass_barrier(tt_command_buffer* cb) {
     if (cb == nullptr || !cb->pass_open) return TT_CMD_INVALID_COMPUTE_PASS;
     return TT_OK;
