@@ -433,6 +433,7 @@ struct FlashArgs {
     uint32_t row_limit;         // rows the q / gate / out / table operands hold
     uint32_t interleave;        // 1: a row's workgroups take its 32-key blocks in turn
     uint32_t compact;           // 1: the splits that hold keys lead the dispatch order
+    uint32_t balanced;          // 1: see flash_decode_kernel's kBalanced
     uint32_t rotate;            // != 0: a workgroup starts (its place x rotate) blocks into its range
     // rope form (flash_decode_kernel<true>): q is null, the query heads come from the
     // projection rows and are normed and rotated by the workgroup itself
@@ -479,9 +480,48 @@ __device__ __forceinline__ void key_block_transfers(const uint8_t* from, uint8_t
     (key_row_transfer<kI>(from, stage), ...);
 }
 
+// Keys per workgroup by what the rows hold instead of by what their caches could: the finest
+// multiple of 32, at least kFinestPart, with which the rows' splits fit `slots`, the splits the
+// records have room for (`part`, which fits whatever the rows hold, where no candidate does).
+// One wave; lane r hands in the keys of row r (0: none), every lane gets the answer: lane i tries
+// (1 + i / 32) times the quotient of all keys and all slots.  Counts are of 32-key blocks, below
+// 2^18, where the fp32 quotient is off by less than half a step of 1 / divisor.
+constexpr uint32_t kFinestPart = 128;
+constexpr uint32_t kBalancedCapacity = 1u << 23;
+__device__ __forceinline__ uint32_t balanced_part(uint32_t keys, uint32_t rows, uint32_t slots, uint32_t part) {
+    const uint32_t blocks = (keys + kBlockKeys - 1) / kBlockKeys;
+    uint32_t all = 0;
+    for (uint32_t r = 0; r < rows; ++r) all += static_cast<uint32_t>(__builtin_amdgcn_readlane(blocks, r));
+    const uint32_t least = max(kFinestPart / kBlockKeys, (all + slots - 1) / slots);
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t tried = least + least * lane / 32;
+    const float inverse = 1.0f / static_cast<float>(tried);
+    uint32_t splits = 0;
+    for (uint32_t r = 0; r < rows; ++r) {
+        const uint32_t of_row = static_cast<uint32_t>(__builtin_amdgcn_readlane(blocks, r));
+        splits += static_cast<uint32_t>((static_cast<float>(of_row + tried - 1) + 0.5f) * inverse);
+    }
+    const uint64_t fit = __ballot(splits <= slots);
+    if (fit == 0) return part;
+    return min(part, static_cast<uint32_t>(__builtin_amdgcn_readlane(tried, __builtin_ctzll(fit))) * kBlockKeys);
+}
+// the sum over lanes 0 .. l of a value that lanes 0 .. 15 hold
+__device__ __forceinline__ uint32_t sum_through(uint32_t mine) {
+    uint32_t through = mine;
+    through += __builtin_amdgcn_update_dpp(0, through, 0x111, 0xF, 0xF, true);   // row_shr:1
+    through += __builtin_amdgcn_update_dpp(0, through, 0x112, 0xF, 0xF, true);
+    through += __builtin_amdgcn_update_dpp(0, through, 0x114, 0xF, 0xF, true);
+    through += __builtin_amdgcn_update_dpp(0, through, 0x118, 0xF, 0xF, true);
+    return through;
+}
+
 // kFinal: one workgroup sees every key of its (row, kv head) and writes the gated bf16
 // output itself instead of a split record.
-template <bool kRope, bool kFinal = false>
+// kBalanced (with the compact order and a state table): the keys per workgroup follow from what
+// the rows hold (balanced_part), so that a deep row among shallow ones, or shallow rows in deep
+// caches, still spread over the device; row r's records are then those behind the records of the
+// rows before it, sixteen heads a split.
+template <bool kRope, bool kFinal = false, bool kBalanced = false>
 __global__ __launch_bounds__(kWaves * 64, 2) void flash_decode_kernel(FlashArgs a) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     // (rope form) the rotation's inverse frequency of pair lane & 31
@@ -516,6 +556,8 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_decode_kernel(FlashArgs 
     uint32_t row = blockIdx.z;
     uint64_t kv_offset = 0;
     uint32_t context = a.context;
+    uint32_t planned_part = a.part;
+    [[maybe_unused]] uint32_t first_record = 0;
     if (a.compact) {
         // The grid covers the capacity of every row, but only ceil(keys / part) splits of a row
         // hold keys.  Taken by grid position, the empty ones lie between the others in the
@@ -526,22 +568,24 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_decode_kernel(FlashArgs 
         // workgroup.  (Launched with a state table, without a row list, never in final mode.)
         const uint32_t l = threadIdx.x & 63;
         const u32x2 entry = *reinterpret_cast<const u32x2*>(a.table + min(l, gridDim.z - 1) * 4);
-        uint32_t mine = 0;
+        uint32_t row_keys = 0;
         if (l < gridDim.z && entry[1] < a.capacity) {
-            const uint32_t keys = kRope ? entry[1] : entry[1] + 1;
-            if (!(a.long_rows_only && keys <= a.single_partition)) mine = (keys + a.part - 1) / a.part;
+            row_keys = kRope ? entry[1] : entry[1] + 1;
+            if (a.long_rows_only && row_keys <= a.single_partition) row_keys = 0;
         }
-        uint32_t through = mine;   // splits of rows 0 .. l
-        through += __builtin_amdgcn_update_dpp(0, through, 0x111, 0xF, 0xF, true);   // row_shr:1
-        through += __builtin_amdgcn_update_dpp(0, through, 0x112, 0xF, 0xF, true);
-        through += __builtin_amdgcn_update_dpp(0, through, 0x114, 0xF, 0xF, true);
-        through += __builtin_amdgcn_update_dpp(0, through, 0x118, 0xF, 0xF, true);
+        if constexpr (kBalanced) {
+            planned_part = balanced_part(row_keys, gridDim.z, a.record_splits * gridDim.z, a.part);
+        }
+        const uint32_t mine = (row_keys + planned_part - 1) / planned_part;
+        const uint32_t through = sum_through(mine);   // splits of rows 0 .. l
         const uint32_t linear = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
         const uint64_t passed = __ballot(l < kMaxBatchRows && kAttnKvHeads * through <= linear);
         row = __builtin_popcountll(passed);
         if (row >= gridDim.z) return;
         const uint32_t row_splits = __builtin_amdgcn_readlane(mine, row);
-        const uint32_t place = linear - kAttnKvHeads * (__builtin_amdgcn_readlane(through, row) - row_splits);
+        const uint32_t before = __builtin_amdgcn_readlane(through, row) - row_splits;
+        const uint32_t place = linear - kAttnKvHeads * before;
+        first_record = before;
         kvh = place >= row_splits ? 1u : 0u;   // two kv heads
         split = place - kvh * row_splits;
         // (the builtin returns int: without the cast an offset past 2^31 elements would be
@@ -561,7 +605,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_decode_kernel(FlashArgs 
     if (context >= a.capacity) return;  // a bad table row must not read outside the cache
     const uint32_t n = kRope ? context : context + 1;
     if (a.long_rows_only && n <= a.single_partition) return;
-    const uint32_t part = kFinal ? n : a.part;
+    const uint32_t part = kFinal ? n : planned_part;
     if (split * part >= n) return;
     // The workgroup's blocks of 32 keys: block b of its own is block first_block + b *
     // block_stride of the row.  Contiguous: the keys [split * part, + part).  Interleaved: the
@@ -857,11 +901,12 @@ __global__ __launch_bounds__(kWaves * 64, 2) void flash_decode_kernel(FlashArgs 
             denom = fmaf(scale[w], lsum[w], denom);
         }
         const uint32_t head = kvh * kAttnHeadsPerKv + h;
-        float* record = kFinal
-                            ? nullptr
-                            : a.partials + static_cast<uint64_t>(row) * a.partial_row_floats +
-                                  (static_cast<uint64_t>(head) * a.record_splits + split) *
-                                      kAttnRecordFloats;
+        const uint64_t record_index =
+            kBalanced ? static_cast<uint64_t>(first_record + split) * kAttnQueryHeads + head
+                      : static_cast<uint64_t>(head) * a.record_splits + split;
+        float* record = kFinal ? nullptr
+                               : a.partials + (kBalanced ? 0 : row * a.partial_row_floats) +
+                                     record_index * kAttnRecordFloats;
 #pragma unroll
         for (uint32_t c = 0; c < 4; ++c) {
             const uint32_t d = lane + 64 * c;
@@ -1050,6 +1095,7 @@ struct FinishArgs {
     uint32_t part;
     uint32_t record_splits;
     uint32_t parts_hint;          // records per head the caller expects the deepest row to have
+    uint32_t balanced;            // 1: the records lie as a balanced walk leaves them
     uint64_t partial_row_floats;
 };
 
@@ -1059,20 +1105,20 @@ struct MergedParts {
 
 // Numerators of up to kParts records requested at once by the thread that owns the
 // dimension; their maxima and sums go through LDS (one thread per record).  `held` = how
-// many records the buffer holds from `base` on (requests beyond it repeat the last one);
+// many records the buffer holds from `base` on, `stride` floats apart (requests beyond it repeat the last one);
 // which of them count is decided in reduce_parts, so nothing here waits for the state
 // table.  The caller places a barrier between request_parts and reduce_parts.
 template <uint32_t kParts>
-__device__ __forceinline__ void request_parts(const float* base, uint32_t held, uint32_t d,
+__device__ __forceinline__ void request_parts(const float* base, uint32_t stride, uint32_t held, uint32_t d,
                                               float (&numerator)[kParts], float* part_max,
                                               float* part_sum) {
     const uint32_t last = held - 1;
 #pragma unroll
     for (uint32_t p = 0; p < kParts; ++p) {
-        numerator[p] = base[static_cast<uint64_t>(min(p, last)) * kAttnRecordFloats + d];
+        numerator[p] = base[static_cast<uint64_t>(min(p, last)) * stride + d];
     }
     if (d < kParts) {
-        const float* rec = base + static_cast<uint64_t>(min(d, last)) * kAttnRecordFloats;
+        const float* rec = base + static_cast<uint64_t>(min(d, last)) * stride;
         part_max[d] = rec[kD];
         part_sum[d] = rec[kD + 1];
     }
@@ -1109,7 +1155,7 @@ __device__ __forceinline__ MergedParts reduce_parts(const float (&numerator)[kPa
 // One (row, head) by one workgroup.  Every load - the state table entry, the projection
 // row's four slices, the two norm weights and the first kParts records - is requested
 // before the first is used: the kernel is one trip to memory deep.
-template <uint32_t kParts>
+template <uint32_t kParts, bool kBalanced>
 __device__ __forceinline__ void finish_row_head(const FinishArgs& a, uint32_t head, uint32_t row,
                                                 uint32_t d) {
     __shared__ __attribute__((aligned(16))) float part_max[kParts];
@@ -1119,6 +1165,14 @@ __device__ __forceinline__ void finish_row_head(const FinishArgs& a, uint32_t he
     const uint16_t* proj = a.projection + static_cast<uint64_t>(row) * a.projection_stride;
     const float* base = a.partials + static_cast<uint64_t>(row) * a.partial_row_floats +
                         static_cast<uint64_t>(head) * a.record_splits * kAttnRecordFloats;
+    constexpr uint32_t kStride = (kBalanced ? kAttnQueryHeads : 1) * kAttnRecordFloats;
+    const uint32_t rows = gridDim.y;
+    // (balanced) every row's entry: the plan of the walk is worked out again from them, while
+    // the other loads are in flight
+    u32x2 entries = {0, 0};
+    if constexpr (kBalanced) {
+        entries = *reinterpret_cast<const u32x2*>(a.table + min(d & 63, rows - 1) * 4);
+    }
     const u32x2 entry = *reinterpret_cast<const u32x2*>(a.table + row * 4);
     const float inverse_frequency = rope_inverse_frequency(d & (kAttnRopePairs - 1));
     const uint16_t xq = proj[head * 2 * kD + d];
@@ -1128,14 +1182,28 @@ __device__ __forceinline__ void finish_row_head(const FinishArgs& a, uint32_t he
     const uint16_t wq = a.q_weight[d];
     const uint16_t wk = a.k_weight[d];
     float numerator[kParts];
-    request_parts<kParts>(base, min(kParts, a.record_splits), d, numerator, part_max, part_sum);
+    uint32_t part = a.part;
+    uint32_t held = a.record_splits;
+    if constexpr (kBalanced) {
+        const uint32_t l = d & 63, slots = a.record_splits * rows;
+        const uint32_t keys = l < rows && entries[1] < a.capacity ? entries[1] : 0;
+        part = balanced_part(keys, rows, slots, a.part);
+        const uint32_t mine = (keys + part - 1) / part;
+        const uint32_t through = sum_through(mine);
+        held = max(static_cast<uint32_t>(__builtin_amdgcn_readlane(mine, row)), 1u);
+        const uint32_t first = min(static_cast<uint32_t>(__builtin_amdgcn_readlane(through, row) -
+                                                         __builtin_amdgcn_readlane(mine, row)),
+                                   slots - 1);
+        base = a.partials + (static_cast<uint64_t>(first) * kAttnQueryHeads + head) * kAttnRecordFloats;
+    }
+    request_parts<kParts>(base, kStride, min(kParts, held), d, numerator, part_max, part_sum);
 
     const uint64_t kv_offset = entry[0];
     const uint32_t context = entry[1];
     // a row the table places outside its cache has no records and no slot to append to
     if (context >= a.capacity) return;
-    const uint32_t nparts = (context + a.part - 1) / a.part;
-    if (nparts > a.record_splits) return;
+    const uint32_t nparts = (context + part - 1) / part;
+    if (!kBalanced && nparts > a.record_splits) return;
     float c = 1.0f, sn = 0.0f;
     if (d < 2 * kAttnRopePairs) {
         const RopeAngle angle = rope_angle_of(context, inverse_frequency);
@@ -1177,7 +1245,7 @@ __device__ __forceinline__ void finish_row_head(const FinishArgs& a, uint32_t he
         // caller's hint, or more than 128 records): the rest in batches, merged as they come
         for (uint32_t p0 = kParts; p0 < nparts; p0 += kParts) {
             const uint32_t count = min(kParts, nparts - p0);
-            request_parts<kParts>(base + static_cast<uint64_t>(p0) * kAttnRecordFloats, count, d,
+            request_parts<kParts>(base + static_cast<uint64_t>(p0) * kStride, kStride, count, d,
                                   numerator, part_max, part_sum);
             __syncthreads();
             const MergedParts next = reduce_parts<kParts>(numerator, count, part_max, part_sum);
@@ -1214,9 +1282,13 @@ __global__ __launch_bounds__(256) void attention_finish_kernel(FinishArgs a) {
     const uint32_t row = blockIdx.y;
     const uint32_t d = threadIdx.x;
     const uint32_t expected = min(a.parts_hint == 0 ? a.record_splits : a.parts_hint, a.record_splits);
-    if (expected <= 32) return finish_row_head<32>(a, head, row, d);
-    if (expected <= 64) return finish_row_head<64>(a, head, row, d);
-    return finish_row_head<128>(a, head, row, d);
+    if (a.balanced) {
+        if (a.parts_hint <= 32) return finish_row_head<32, true>(a, head, row, d);
+        return finish_row_head<64, true>(a, head, row, d);
+    }
+    if (expected <= 32) return finish_row_head<32, false>(a, head, row, d);
+    if (expected <= 64) return finish_row_head<64, false>(a, head, row, d);
+    return finish_row_head<128, false>(a, head, row, d);
 }
 
 // ---------------------------------------- separate score / value stages ------
@@ -1420,7 +1492,10 @@ int32_t op_attn_qk_rope_blk(const Bindings& b, const Grid& g, hipStream_t stream
 namespace {
 
 int32_t launch_flash(const FlashArgs& f, uint32_t splits, uint32_t rows, hipStream_t stream) {
-    if (f.projection != nullptr) {
+    if (f.projection != nullptr && f.balanced) {
+        hipLaunchKernelGGL((flash_decode_kernel<true, false, true>), dim3(splits, kAttnKvHeads, rows),
+                           dim3(kWaves * 64), kWaves * kWaveLdsBytes, stream, f);
+    } else if (f.projection != nullptr) {
         hipLaunchKernelGGL(flash_decode_kernel<true>, dim3(splits, kAttnKvHeads, rows), dim3(kWaves * 64),
                            kWaves * kWaveLdsBytes, stream, f);
     } else if (f.final_mode) {
@@ -1622,7 +1697,9 @@ int32_t op_attention_combine_ms(const Bindings& b, const Grid& g, hipStream_t st
 // b5 state_table, b6 split records [rows][16][max_splits][258] fp32, b7 out slab
 // [rows][query stride], c8 capacity, c9 projection stride, c10 query stride, c11 part (keys
 // per workgroup, multiple of 32), c12 max_splits, c13 bit 1 interleave, bit 2 compact, bits
-// 3..7 rotate (as c9 of attention_decode_split_ms), c14 records per head the deepest row is
+// 3..7 rotate (as c9 of attention_decode_split_ms), bit 8 balanced (the same in both
+// dispatches: keys per workgroup by what the rows hold, at most c11; the records' order inside
+// b6 is then the walk's own), c14 records per head the deepest row is
 // expected to have (0: as many as the buffer holds; a hint that sizes the finishing
 // dispatch's first batch of requests, any value gives the same result).
 struct TokenLayer {
@@ -1645,6 +1722,10 @@ TokenLayer token_layer_args(Args& a, uint32_t rows) {
     f.interleave = (flags >> 1) & 1;
     f.compact = (flags >> 2) & 1;
     f.rotate = (flags >> 3) & 31;
+    // (a cache of more positions is beyond what balanced_part counts: both dispatches then do
+    // without)
+    f.balanced = n.balanced = ((flags >> 8) & 1) && f.capacity <= kBalancedCapacity;
+    if (f.balanced) f.compact = 1;
     a.require(rows >= 1 && rows <= kMaxBatchRows, TT_CMD_INVALID_DISPATCH_EXTENT);
     a.require(f.capacity != 0 && f.projection_stride >= kAttnProjectionRows &&
                   f.projection_stride % 4 == 0 && n.query_stride >= kAttnQueryValues &&
@@ -1775,6 +1856,9 @@ bool prepare_current_device() {
                             hipFuncAttributeMaxDynamicSharedMemorySize,
                             kWaves * kWaveLdsBytes) != hipSuccess ||
         hipFuncSetAttribute(reinterpret_cast<const void*>(flash_decode_kernel<false, true>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            kWaves * kWaveLdsBytes) != hipSuccess ||
+        hipFuncSetAttribute(reinterpret_cast<const void*>(flash_decode_kernel<true, false, true>),
                             hipFuncAttributeMaxDynamicSharedMemorySize,
                             kWaves * kWaveLdsBytes) != hipSuccess ||
         hipFuncSetAttribute(reinterpret_cast<const void*>(flash_decode_kernel<true>),

@@ -307,6 +307,20 @@ class StubStack:
         # (bits 3..7: contiguous ranges are walked from a rotated starting block)
         return (2 if rows <= 2 else 8) | (4 if grid > live and grid > self.groups else 0)
 
+    def _token_flags(self, rows):
+        """c13 and c14 of the token form.  Where the lanes leave half of the workgroups without
+        keys or more - shallow lanes in deep caches, deep lanes among shallow ones - the split
+        follows what they hold (bit 8: a wave of 16 lanes of 150 .. 12000 keys in caches of
+        16384 399 -> 359 us, of 4 lanes of 700 .. 6001 in 32768 272 -> 248).  Full lanes keep
+        the fixed split: it names a workgroup's row before the state table has arrived."""
+        contexts = self.context[:rows]
+        deepest = max(contexts)
+        live = split_workgroups([max(c, 1) for c in contexts], self.split_keys)
+        finest = choose_split_keys([max(c, 1) for c in contexts], 2 * rows * self.max_splits)
+        if live > rows * self.max_splits or finest >= self.split_keys:
+            return self._split_flags(rows), -(-deepest // self.split_keys)
+        return self._split_flags(rows) | 256, -(-deepest // finest)
+
     # ---- one token for every lane ----
     def record_token_wave(self, cb, with_head=True):
         """Records one decode step of all lanes; the lanes' inputs are rows of self.x.
@@ -324,10 +338,9 @@ class StubStack:
             elif self.attention_form == "token":
                 bind = {0: self.proj, 1: layer["q_norm"], 2: layer["k_norm"], 3: layer["keys"],
                         4: layer["values"], 5: layer["table"], 6: self.partials, 7: self.mixed}
-                deepest = max(self.context[:rows])
+                flags, records = self._token_flags(rows)
                 const = {8: self.capacity, 9: ATTN_PROJ, 10: 4096, 11: self.split_keys,
-                         12: self.max_splits, 13: self._split_flags(rows),
-                         14: -(-deepest // self.split_keys)}
+                         12: self.max_splits, 13: flags, 14: records}
                 cb.encode(P("attention_decode_token_ms"), bind, const, (self.max_splits, 2, rows),
                           (256,))
                 cb.barrier()

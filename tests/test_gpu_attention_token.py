@@ -168,3 +168,24 @@ def test_token_finish_hint_is_only_a_hint(hint):
     per head here, past the largest batch of 128."""
     print(f"[case] token layer, finish hint {hint}", flush=True)
     token_batch([5000, 31, 2100, 0], 5024, [(32, flags(rotate=1))], 0x7117, parts_hint=hint)
+
+
+@pytest.mark.parametrize("contexts,cap,part", [
+    ([2000, 1499, 700, 100, 255, 256, 0], 2048, 256),      # ragged, an empty cache among them
+    ([3000], 4096, 2048),                                  # one lane: two records' room, one finer split
+    ([5, 3900, 0, 0], 4096, 1024),                         # one deep lane takes the others' room
+    ([4095] * 3, 4096, 512),                               # full caches: no finer split fits
+    ([1, 129, 128, 127, 33, 32, 31, 0, 640, 97, 96, 64, 300, 900, 1023, 1000], 1024, 1024),
+    ([9000, 20, 4000], 9024, 288),                         # more records than one batch takes
+], ids=["ragged", "one", "deep-one", "full", "sixteen", "many"])
+def test_token_split_by_what_the_lanes_hold(contexts, cap, part):
+    """Bit 8 of c13: the keys per workgroup follow from the contexts, the records lie row after
+    row; the same layer, held to the checker and to replays."""
+    print(f"[case] token layer, balanced, {len(contexts)} lanes, part {part}", flush=True)
+    token_batch(contexts, cap, [(part, 256), (part, 256 | flags(rotate=1))], 0x8A1A + len(contexts), replays=2)
+
+
+@pytest.mark.parametrize("hint", [0, 1, 40, 200])
+def test_token_balanced_finish_hint_is_only_a_hint(hint):
+    print(f"[case] token layer, balanced, finish hint {hint}", flush=True)
+    token_batch([10000, 31, 0, 0], 10016, [(320, 256)], 0x8A71, parts_hint=hint)
