@@ -316,7 +316,7 @@ struct BlockProduct {
     }
 };
 
-enum class BlockTile { Large, Even, Deep, Low, Tall, Small, Least };
+enum class BlockTile { Large, Even, Deep, Tall, Small, Least };
 
 // The tile with the shortest estimate.  A compute unit takes ceil(tiles / compute_units) tiles,
 // two at a time where two workgroups fit it: `single` is the time of one tile alone on it, `both`
@@ -332,7 +332,6 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         {BlockTile::Large, 256, 256, 1580, 8000, 3160, 16000},
         {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
         {BlockTile::Deep, 128, 128, 520, 2000, 1040, 4000},
-        {BlockTile::Low, 64, 128, 330, 1500, 630, 3000},
         {BlockTile::Tall, 128, 64, 330, 1500, 630, 3000},
         {BlockTile::Small, 64, 64, 200, 1000, 400, 2000},
         {BlockTile::Least, 32, 64, 155, 1000, 275, 1500},
@@ -359,18 +358,17 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
 //   Large  16384 x 2176 x 12352 / 9216, 8192 x 4352 x 2048: 790 / 563 / 114 us = 1.12 / 1.17 /
 //          1.29 PFLOP/s (eight waves of 128 x 64: 832 / 546 / 110 us; with all transfers of a unit
 //          issued ahead of its products 865 / 573 / 116 us)
-//   Even   2048 x 2176 x 9216: 91 us; Large 106, Deep 97, Low 113
+//   Even   2048 x 2176 x 9216: 91 us; Large 106, Deep 97, Tall 106
 //   Deep   2048 x 4352 x 2048: 38 us; Even 48, Large 85
-//   Low    777 x 4352 x 2048: 24 us; Deep 30, Even 43
-//   Tall   100 x 2176 x 12352: 13.5 us; Deep 17, Low 19, Small 20
-//   Small  300 x 4352 x 2048: 15 us; Least 20, Low 22, Deep 29
-//   Least  100 x 4352 x 2048: 11 us; Small 14, Low 19, Deep 27
+//   Tall   100 x 2176 x 12352: 13.5 us; Deep 17, Small 20 (as 64 x 128, 19)
+//          777 x 4352 x 2048: 24 us; Deep 30, Even 43
+//   Small  300 x 4352 x 2048: 15 us; Least 20, Tall 22, Deep 29
+//   Least  100 x 4352 x 2048: 11 us; Small 14, Tall 19, Deep 27
 template <typename Element>
 struct BlockTiles {
     typedef BlockProduct<Element, 256, 256, 4, 4> Large;      // the most products per byte fetched
     typedef BlockProduct<Element, 128, 128, 2, 4> Even;       // two a compute unit hide each other's waits
     typedef BlockProduct<Element, 128, 128, 2, 4, 4> Deep;    // one a compute unit, two units further ahead
-    typedef BlockProduct<Element, 64, 128, 2, 4, 3> Low;
     typedef BlockProduct<Element, 128, 64, 4, 2, 3> Tall;
     typedef BlockProduct<Element, 64, 64, 2, 2, 4> Small;
     typedef BlockProduct<Element, 32, 64, 2, 2, 4> Least;
@@ -381,7 +379,6 @@ struct BlockTiles {
         switch (choose_block_tile(rows, in_dim, out_dim, compute_units)) {
         case BlockTile::Even: return use(Even{});
         case BlockTile::Deep: return use(Deep{});
-        case BlockTile::Low: return use(Low{});
         case BlockTile::Tall: return use(Tall{});
         case BlockTile::Small: return use(Small{});
         case BlockTile::Least: return use(Least{});
@@ -391,8 +388,7 @@ struct BlockTiles {
     // use(product) of every tile, as long as it says true
     template <typename Use>
     static bool each(Use use) {
-        return use(Large{}) && use(Even{}) && use(Deep{}) && use(Low{}) && use(Tall{}) && use(Small{}) &&
-               use(Least{});
+        return use(Large{}) && use(Even{}) && use(Deep{}) && use(Tall{}) && use(Small{}) && use(Least{});
     }
 };
 
