@@ -1916,12 +1916,18 @@ int32_t op_gdn_chunk_scan(const Bindings& b, const Grid& g, hipStream_t stream,
 // of a group (118 MB) stay in the 256 MB last-level cache between the two stages.
 constexpr uint32_t kChunkGroupRows = 2048;
 
+// Up to this many rows the token loop is the shorter chain (and the reference's own order): both
+// dispatches of a chunk take 21 us whatever it holds, the loop 8.3 us for 12 rows, 16.4 for 32,
+// 22.4 for 48.  (Requesting a step's operands a step ahead made the loop slower, 9.0 us for 12.)
+constexpr uint32_t kTokenLoopRows = 40;
+
 // gdn_chunk_recurrence_blk (no reference counterpart: the chunked evaluation of
 // gdn_recurrence_gates_blk, prefill_step.cpp:1988-2040, in one dispatch): b0 qk
 // [rows][4096], b1 value [rows][4096], b2 decay [rows][32], b3 beta [rows][32],
 // b4 scratch (chunk records of min(rows, 2048) rows), b5 state_in, b6 y [rows][4096],
 // b7 state_out, c8 rows; grid (8, 32) x 256.  Walks the block in groups of 2048
-// rows, stage 1 then stage 2 per group; state_in and state_out may be the same plane.
+// rows, stage 1 then stage 2 per group, or, up to kTokenLoopRows, token by token; state_in and
+// state_out may be the same plane.
 int32_t op_gdn_chunk_recurrence(const Bindings& b, const Grid& g, hipStream_t stream,
                                 bool validate_only) {
     Args a(b);
@@ -1939,6 +1945,20 @@ int32_t op_gdn_chunk_recurrence(const Bindings& b, const Grid& g, hipStream_t st
     uint16_t* y = a.buffer<uint16_t>(6, row_bytes);
     float* state_out = a.buffer<float>(7, kGdnStateFloats * 4ull);
     if (a.status != TT_OK || validate_only) return a.status;
+    if (rows <= kTokenLoopRows) {
+        RecurrenceArgs r{};
+        r.qk = qk;
+        r.value = value;
+        r.decay = decay;
+        r.beta = beta;
+        r.state_in = state_in;
+        r.state_out = state_out;
+        r.y = y;
+        r.qk_stride = kGdnQkValues;
+        r.value_stride = r.y_stride = kGdnValueValues;
+        r.steps = rows;
+        return launch_recurrence(r, 1, stream);
+    }
     for (uint32_t start = 0; start < rows; start += kChunkGroupRows) {
         const uint32_t count = min(kChunkGroupRows, rows - start);
         ChunkPrepareArgs p{};

@@ -317,6 +317,13 @@ def test_chunked_recurrence_matches_token_loop(rows):
     check_bf16(bufs["gated"].read(np.uint16), ref["gated"], "chunked gated", ulps=4)
 
 
+@pytest.mark.parametrize("rows", [2, 12, 39, 40, 41])
+def test_chunked_recurrence_either_side_of_the_token_loop(rows):
+    """Short blocks, which gdn_chunk_recurrence_blk walks token by token (the checker's order) up
+    to 40 rows and as a chunk from 41 on."""
+    test_chunked_recurrence_matches_token_loop(rows)
+
+
 def test_chunked_recurrence_with_harsh_gates():
     """Gates far from the seeded tests' mild ones: exp(A_log) from 0.4 to 16 and a wide a row,
     so that decays run from 1 down to exp(-100) and underflow inside a chunk, betas from 0 to 1.
