@@ -287,9 +287,10 @@ uint32_t current_device_compute_units() {
     return g_compute_units[device] != 0 ? g_compute_units[device] : 256;
 }
 
-// Blocks of more rows than this take the LDS-staged kernel (below it a 256-row tile is
-// mostly padding).
-constexpr uint32_t kDenseBlockRowsFrom = 64;
+// Blocks of more rows than this take the LDS-staged kernel, whose smallest tile has 32 rows (the
+// kernel straight from memory walks K one load after the other: 17 / 33 / 64 rows of 2048 -> 12352
+// 26 / 40 / 60 us against 11 / 11 / 12, 4096 -> 2048 30 against 11).
+constexpr uint32_t kDenseBlockRowsFrom = 16;
 // What the block kernel assumes beyond the sizes: 16-byte pieces of both operands and
 // 32-bit byte offsets into them.
 bool dense_block_operands_fit(const uint16_t* input, const uint16_t* weights, uint32_t rows,
