@@ -603,21 +603,41 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
             }
         }
     } else {
-        // one piece of each row per thread; the weights are requested before the first piece is
-        // stored, so that the two round trips overlap (rows past the last repeat it: no branch
-        // between the requests, where what is in flight would be waited for)
+        // One piece of each row per thread.  Over 2048 columns the weights are requested before the
+        // first piece is stored, so that the two round trips overlap (rows past the last repeat it:
+        // no branch between the requests, where what is in flight would be waited for): gdn_project
+        // of 4 / 8 / 12 / 16 rows 8.24 / 8.92 / 10.16 / 12.04 -> 8.14 / 8.70 / 9.37 / 10.66 us.  Over
+        // 4096, half a workgroup to a compute unit, the weights first cost 0.1 .. 0.2 us of 6 .. 7.
         static_assert(kPiecesPerRow == kThreads, "a row is one piece per thread");
-        u32x4 raw[kRowsMax];
+        if constexpr (kWaves == 4) {
+            u32x4 raw[kRowsMax];
 #pragma unroll
-        for (uint32_t r = 0; r < kRowsMax; ++r) {
-            raw[r] = *reinterpret_cast<const u32x4*>(
-                p.input + static_cast<uint64_t>(min(r, p.rows - 1)) * p.input_stride + threadIdx.x * 8);
-        }
-        request_weights();
+            for (uint32_t r = 0; r < kRowsMax; ++r) {
+                raw[r] = *reinterpret_cast<const u32x4*>(
+                    p.input + static_cast<uint64_t>(min(r, p.rows - 1)) * p.input_stride + threadIdx.x * 8);
+            }
+            request_weights();
 #pragma unroll
-        for (uint32_t r = 0; r < kRowsMax; ++r) {
-            *reinterpret_cast<u32x4*>(wave_lds + min(r, p.rows - 1) * kWaveRowBytes<kWaves> +
-                                      threadIdx.x * 16) = raw[r];
+            for (uint32_t r = 0; r < kRowsMax; ++r) {
+                *reinterpret_cast<u32x4*>(wave_lds + min(r, p.rows - 1) * kWaveRowBytes<kWaves> +
+                                          threadIdx.x * 16) = raw[r];
+            }
+        } else {
+            for (uint32_t first = 0; first < p.rows; first += 4) {
+                u32x4 staged[4];
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    staged[j] = *reinterpret_cast<const u32x4*>(
+                        p.input + static_cast<uint64_t>(min(first + j, p.rows - 1)) * p.input_stride +
+                        threadIdx.x * 8);
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    *reinterpret_cast<u32x4*>(wave_lds + min(first + j, p.rows - 1) * kWaveRowBytes<kWaves> +
+                                              threadIdx.x * 16) = staged[j];
+                }
+            }
+            request_weights();
         }
     }
     __syncthreads();
@@ -675,8 +695,13 @@ constexpr uint32_t wave_lds_bytes(uint32_t rows) {
     return rows * kWaveRowBytes<kWaves> + kWaves * 4 * 64 * 4;
 }
 
-constexpr uint32_t kFewRows = 4;   // of x requested up front by the instantiation for few lanes
-static_assert(wave_lds_bytes<8>(kFewRows) <= 64 * 1024, "needs no larger LDS limit");
+// The instantiation for 2048 columns that requests the fewest rows of x, repeats included.
+auto wave_kernel_for(uint32_t rows) {
+    return rows <= 4    ? q4_wave_kernel<4, false, false, 4>
+           : rows <= 8  ? q4_wave_kernel<4, false, false, 8>
+           : rows <= 12 ? q4_wave_kernel<4, false, false, 12>
+                        : q4_wave_kernel<4, false, false, 16>;
+}
 
 int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
     const uint32_t out_rows = p.first_row[p.segments];
@@ -687,9 +712,8 @@ int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL((q4_wave_kernel<4, true, false>), dim3(out_rows / 16), dim3(256),
                                wave_lds_bytes<4>(p.rows), stream, p);
         } else {
-            const auto kernel = p.rows <= kFewRows ? q4_wave_kernel<4, false, false, kFewRows>
-                                                   : q4_wave_kernel<4>;
-            hipLaunchKernelGGL(kernel, dim3(out_rows / 16), dim3(256), wave_lds_bytes<4>(p.rows), stream, p);
+            hipLaunchKernelGGL(wave_kernel_for(p.rows), dim3(out_rows / 16), dim3(256),
+                               wave_lds_bytes<4>(p.rows), stream, p);
         }
         break;
     case 8:
@@ -698,9 +722,8 @@ int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL((q4_wave_kernel<8, false, true>), dim3(out_rows / 16), dim3(512),
                                wave_lds_bytes<8>(p.rows), stream, p);
         } else {
-            const auto kernel = p.rows <= kFewRows ? q4_wave_kernel<8, false, false, kFewRows>
-                                                   : q4_wave_kernel<8>;
-            hipLaunchKernelGGL(kernel, dim3(out_rows / 16), dim3(512), wave_lds_bytes<8>(p.rows), stream, p);
+            hipLaunchKernelGGL((q4_wave_kernel<8>), dim3(out_rows / 16), dim3(512),
+                               wave_lds_bytes<8>(p.rows), stream, p);
         }
         break;
     default: return TT_CMD_INVALID_DISPATCH_EXTENT;
@@ -923,6 +946,10 @@ bool prepare_q4_kernels() {
                                    hipFuncAttributeMaxDynamicSharedMemorySize,
                                    Product::kLdsBytes) == hipSuccess;
     };
+    const auto allow_wave = [](void (*kernel)(Q4Projection), uint32_t bytes) {
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
+    };
     return Q4Tiles::each(allow) &&
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<4, true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -930,12 +957,11 @@ bool prepare_q4_kernels() {
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<8, true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                kRowsStagedBytes) == hipSuccess &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(q4_wave_kernel<4>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               wave_lds_bytes<4>(kQ4BatchRowsMax)) == hipSuccess &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(q4_wave_kernel<8>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               wave_lds_bytes<8>(kQ4BatchRowsMax)) == hipSuccess &&
+           allow_wave(wave_kernel_for(4), wave_lds_bytes<4>(4)) &&
+           allow_wave(wave_kernel_for(8), wave_lds_bytes<4>(8)) &&
+           allow_wave(wave_kernel_for(12), wave_lds_bytes<4>(12)) &&
+           allow_wave(wave_kernel_for(16), wave_lds_bytes<4>(16)) &&
+           allow_wave(q4_wave_kernel<8>, wave_lds_bytes<8>(16)) &&
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_wave_kernel<4, true, false>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                wave_lds_bytes<4>(kQ4BatchRowsMax)) == hipSuccess &&

@@ -317,7 +317,8 @@ class StubStack:
         deepest = max(contexts)
         live = split_workgroups([max(c, 1) for c in contexts], self.split_keys)
         finest = choose_split_keys([max(c, 1) for c in contexts], 2 * rows * self.max_splits)
-        if live > rows * self.max_splits or finest >= self.split_keys:
+        # (the plan costs both dispatches together about 2.5 us, 256 keys of a walk about 5)
+        if live > rows * self.max_splits or min(deepest, self.split_keys) - finest < 256:
             return self._split_flags(rows), -(-deepest // self.split_keys)
         return self._split_flags(rows) | 256, -(-deepest // finest)
 
