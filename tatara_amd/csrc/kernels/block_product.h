@@ -3,7 +3,7 @@
 // caller's.  One persistent workgroup of kWavesM x kWavesN waves owns tiles of kTileM x kTileN
 // and walks K in units of 64 columns, two steps of 32 each:
 //   * both operands go from global memory straight into LDS (16 bytes per lane and
-//     transfer, whole 128-byte lines of a row, no registers), a ring of two units.  The
+//     transfer, whole 128-byte lines of a row, no registers), a ring of kRing units.  The
 //     transfers are issued as assembly, so that the only waits are the ones written below
 //     (M0 is used for nothing else in these kernels).  A ring row is one row's 128 bytes of
 //     the unit; 16-byte piece p of row r sits in slot p ^ (r & 7), with which the 16-byte
@@ -13,7 +13,7 @@
 //     operand: a lane then holds four consecutive n of one m per product.  The fragments of a
 //     step are read into registers while the step before it is multiplied; one barrier per
 //     unit.
-//   * the first two units of a workgroup's next tile are requested before it converts and
+//   * the first units of a workgroup's next tile are requested before it converts and
 //     stores the sums of this one.
 // m and n past the end are clamped on the way in; the caller does not store them.
 #pragma once
