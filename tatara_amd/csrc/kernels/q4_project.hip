@@ -20,6 +20,7 @@
 //    hold them exactly, the affine terms as further columns, and multiplied as one
 //    matrix product with fp32 sums - the same mathematics in another summation order.
 #include <algorithm>
+#include <type_traits>
 
 #include "../tt_internal.h"
 #include "block_product.h"
@@ -72,6 +73,7 @@ struct Q4Projection {
     const uint16_t* norm_weight;           // not null: the input rows go through the RMS norm first
     const uint16_t* residual;              // not null: output = bf16(residual + bf16(projection)),
     uint64_t residual_stride;              //   [rows][residual_stride]; may be the output itself
+    bool centred;                          // a block's rows: the exact small nibbles (centred_eight)
 };
 
 // The weight matrix that holds output row `n`, with n the same for every lane (matrices have
@@ -518,13 +520,33 @@ __device__ __forceinline__ bf16x4_bits offset_four(uint32_t word) {
     return __builtin_bit_cast(bf16x4_bits, out);
 }
 
+// The eight nibbles of `word` less 8, as bf16, for a block of 2..16 rows.  A block used to be
+// evaluated in the reference's own order, and its fp32 sums may be no further from the exact ones
+// than there: the nibbles stay small (16 + nibble makes the partial sums three times as large), and
+// the groups of a slice, whose products come from the matrix unit in fp32, are added up in 64 bits.
+// Rms left where the exact result is zero (rows of N(0, 1), scales 0.5 .. 0.9) over 2048 / 4096
+// columns: reference's order 6.5e-6 / 11.6e-6, this 4.1e-6 / 5.8e-6, a decode wave's form 22.5e-6 /
+// 31.9e-6.
+// Time against the decode wave's form, 12 rows: gdn_project 9.0 -> 9.2 us, outproj 6.3 -> 6.6 us.
+__device__ __forceinline__ bf16x8 centred_eight(uint32_t word) {
+    const uint32_t twos = word ^ 0x88888888u;   // nibble - 8 as four bits of two's complement
+    bf16x8 out;
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        out[i] = static_cast<__bf16>(static_cast<float>(static_cast<int32_t>(twos << (28 - 4 * i)) >> 28));
+    }
+    return out;
+}
+
 // bytes between the x rows staged in LDS: 16 more than a row, so that the sixteen lanes of
 // a fragment read (one row each, the same columns) fall on different banks
 template <uint32_t kWaves>
 constexpr uint32_t kWaveRowBytes = kWaves * 1024 + 16;
 
-// kWaves = k_size / 512; kRowsMax: the rows this instantiation takes at most
-template <uint32_t kWaves, bool kNorm = false, bool kResidual = false, uint32_t kRowsMax = kQ4BatchRowsMax>
+// kWaves = k_size / 512; kRowsMax: the rows this instantiation takes at most; kCentred: a block's
+// rows, see centred_eight
+template <uint32_t kWaves, bool kNorm = false, bool kResidual = false, uint32_t kRowsMax = kQ4BatchRowsMax,
+          bool kCentred = false>
 __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
     // [rows][kWaveRowBytes] of x, then the waves' partial results
     extern __shared__ __align__(16) uint8_t wave_lds[];
@@ -647,11 +669,29 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
     const bf16x4_bits ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
     const f32x4 zero = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 acc = zero;
+    [[maybe_unused]] double wide[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (uint32_t group = 0; group < 8; ++group) {
         const u32x4 x_low = *reinterpret_cast<const u32x4*>(x_row + group * (kQ4Group * 2));
         const u32x4 x_high = *reinterpret_cast<const u32x4*>(x_row + group * (kQ4Group * 2) + 16);
         f32x4 products = zero, sums = zero;
+        if constexpr (kCentred) {
+            bf16x8 eight_ones;
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) eight_ones[j] = static_cast<__bf16>(1.0f);
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j) {
+                const bf16x8 xf = __builtin_bit_cast(bf16x8, j == 0 ? x_low : x_high);
+                products = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, centred_eight(q[group][j]), products,
+                                                                   0, 0, 0);
+                sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, eight_ones, sums, 0, 0, 0);
+            }
+            const float scale = widen_half(scale_bits[group >> 1], group & 1);
+            const float bias = fmaf(8.0f, scale, widen_half(bias_bits[group >> 1], group & 1));
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) wide[i] += fmaf(scale, products[i], bias * sums[i]);
+            continue;
+        }
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j) {
             const u32x4 half = j < 2 ? x_low : x_high;
@@ -669,14 +709,17 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
         for (uint32_t i = 0; i < 4; ++i) acc[i] = fmaf(bias, sums[i], fmaf(scale, products[i], acc[i]));
     }
 #pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) partial[(wave * 4 + i) * 64 + lane] = acc[i];
+    for (uint32_t i = 0; i < 4; ++i) {
+        partial[(wave * 4 + i) * 64 + lane] = kCentred ? static_cast<float>(wide[i]) : acc[i];
+    }
     __syncthreads();
     if (wave != 0) return;
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
-        float total = partial[i * 64 + lane];
+        std::conditional_t<kCentred, double, float> sum = partial[i * 64 + lane];
 #pragma unroll
-        for (uint32_t w = 1; w < kWaves; ++w) total += partial[(w * 4 + i) * 64 + lane];
+        for (uint32_t w = 1; w < kWaves; ++w) sum += partial[(w * 4 + i) * 64 + lane];
+        const float total = static_cast<float>(sum);
         const uint32_t m = 4 * g + i;   // the result has the input rows along its rows
         if (m < p.rows) {
             uint16_t result = store16(total);
@@ -696,11 +739,12 @@ constexpr uint32_t wave_lds_bytes(uint32_t rows) {
 }
 
 // The instantiation for 2048 columns that requests the fewest rows of x, repeats included.
+template <bool kCentred>
 auto wave_kernel_for(uint32_t rows) {
-    return rows <= 4    ? q4_wave_kernel<4, false, false, 4>
-           : rows <= 8  ? q4_wave_kernel<4, false, false, 8>
-           : rows <= 12 ? q4_wave_kernel<4, false, false, 12>
-                        : q4_wave_kernel<4, false, false, 16>;
+    return rows <= 4    ? q4_wave_kernel<4, false, false, 4, kCentred>
+           : rows <= 8  ? q4_wave_kernel<4, false, false, 8, kCentred>
+           : rows <= 12 ? q4_wave_kernel<4, false, false, 12, kCentred>
+                        : q4_wave_kernel<4, false, false, 16, kCentred>;
 }
 
 int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
@@ -712,8 +756,8 @@ int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL((q4_wave_kernel<4, true, false>), dim3(out_rows / 16), dim3(256),
                                wave_lds_bytes<4>(p.rows), stream, p);
         } else {
-            hipLaunchKernelGGL(wave_kernel_for(p.rows), dim3(out_rows / 16), dim3(256),
-                               wave_lds_bytes<4>(p.rows), stream, p);
+            hipLaunchKernelGGL(p.centred ? wave_kernel_for<true>(p.rows) : wave_kernel_for<false>(p.rows),
+                               dim3(out_rows / 16), dim3(256), wave_lds_bytes<4>(p.rows), stream, p);
         }
         break;
     case 8:
@@ -722,8 +766,8 @@ int32_t launch_wave(const Q4Projection& p, hipStream_t stream) {
             hipLaunchKernelGGL((q4_wave_kernel<8, false, true>), dim3(out_rows / 16), dim3(512),
                                wave_lds_bytes<8>(p.rows), stream, p);
         } else {
-            hipLaunchKernelGGL((q4_wave_kernel<8>), dim3(out_rows / 16), dim3(512),
-                               wave_lds_bytes<8>(p.rows), stream, p);
+            hipLaunchKernelGGL((p.centred ? q4_wave_kernel<8, false, false, 16, true> : q4_wave_kernel<8>),
+                               dim3(out_rows / 16), dim3(512), wave_lds_bytes<8>(p.rows), stream, p);
         }
         break;
     default: return TT_CMD_INVALID_DISPATCH_EXTENT;
@@ -849,20 +893,22 @@ int32_t project_tiled(const Bindings& b, const Grid& g, hipStream_t stream, bool
 }
 
 // a block of consecutive tokens: c[out+1] rows, then the input width where the
-// operator takes one; grid (groups) x threads
+// operator takes one; grid (groups) x threads.  wave_kernel: at most 16 rows, on q4_wave_kernel
 int32_t project_block(const Bindings& b, const Grid& g, hipStream_t stream, bool validate_only,
-                      const Family& f, bool variable_width) {
+                      const Family& f, bool variable_width, bool wave_kernel = false) {
     Args a(b);
     Q4Projection p{};
     p.rows = a.constant(f.out_slot + 1);
     const uint32_t k_size = variable_width ? a.constant(f.out_slot + 2) : f.k_size;
     // the two input widths of the model: hidden (2048) and the attention / value width (4096)
-    a.require(p.rows >= 1 && (k_size == kHidden || k_size == kGdnValueValues),
+    a.require(p.rows >= 1 && (k_size == kHidden || k_size == kGdnValueValues) &&
+                  (!wave_kernel || p.rows <= kMaxBatchRows),
               TT_CMD_INVALID_DISPATCH_EXTENT);
     if (a.status != TT_OK) return a.status;
     p.row_tile = kQ4BatchRowsMax;
     p.output_stride = f.out_rows();
-    return finish(a, g, stream, validate_only, f, p, k_size, 1);
+    p.centred = wave_kernel;
+    return finish(a, g, stream, validate_only, f, p, k_size, 1, wave_kernel);
 }
 
 // attn_project: b0 input[2048], b1-3 query+gate (8192 rows), b4-6 key (512), b7-9 value
@@ -933,6 +979,19 @@ int32_t op_gdn_outproj_residual_mfma_ms(const Bindings& b, const Grid& g, hipStr
 int32_t op_outproj_blk(const Bindings& b, const Grid& g, hipStream_t s, bool v) {
     return project_block(b, g, s, v, kOutProject, true);
 }
+// attn_project_mfma_blk, gdn_project_mfma_blk, outproj_mfma_blk (no reference counterpart): the
+// bindings and grids of the _blk forms for at most 16 rows, evaluated on the matrix unit with fp32
+// sums no further from the exact ones than the reference's order (centred_eight); the _blk forms
+// themselves keep that order, and its bits, up to 16 rows.
+int32_t op_attn_project_mfma_blk(const Bindings& b, const Grid& g, hipStream_t s, bool v) {
+    return project_block(b, g, s, v, kAttnProject, false, true);
+}
+int32_t op_gdn_project_mfma_blk(const Bindings& b, const Grid& g, hipStream_t s, bool v) {
+    return project_block(b, g, s, v, kGdnProject, false, true);
+}
+int32_t op_outproj_mfma_blk(const Bindings& b, const Grid& g, hipStream_t s, bool v) {
+    return project_block(b, g, s, v, kOutProject, true, true);
+}
 
 }  // namespace
 
@@ -950,6 +1009,10 @@ bool prepare_q4_kernels() {
         return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess;
     };
+    const auto allow_rows = [&](uint32_t rows) {
+        return allow_wave(wave_kernel_for<false>(rows), wave_lds_bytes<4>(rows)) &&
+               allow_wave(wave_kernel_for<true>(rows), wave_lds_bytes<4>(rows));
+    };
     return Q4Tiles::each(allow) &&
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<4, true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -957,11 +1020,9 @@ bool prepare_q4_kernels() {
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<8, true>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                kRowsStagedBytes) == hipSuccess &&
-           allow_wave(wave_kernel_for(4), wave_lds_bytes<4>(4)) &&
-           allow_wave(wave_kernel_for(8), wave_lds_bytes<4>(8)) &&
-           allow_wave(wave_kernel_for(12), wave_lds_bytes<4>(12)) &&
-           allow_wave(wave_kernel_for(16), wave_lds_bytes<4>(16)) &&
+           allow_rows(4) && allow_rows(8) && allow_rows(12) && allow_rows(16) &&
            allow_wave(q4_wave_kernel<8>, wave_lds_bytes<8>(16)) &&
+           allow_wave(q4_wave_kernel<8, false, false, 16, true>, wave_lds_bytes<8>(16)) &&
            hipFuncSetAttribute(reinterpret_cast<const void*>(q4_wave_kernel<4, true, false>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                wave_lds_bytes<4>(kQ4BatchRowsMax)) == hipSuccess &&
@@ -989,6 +1050,9 @@ const KernelDesc kQ4ProjectKernels[] = {
     {"attn_project_rms_mfma_ms", op_attn_project_rms_mfma_ms},
     {"gdn_project_rms_mfma_ms", op_gdn_project_rms_mfma_ms},
     {"gdn_outproj_residual_mfma_ms", op_gdn_outproj_residual_mfma_ms},
+    {"attn_project_mfma_blk", op_attn_project_mfma_blk},
+    {"gdn_project_mfma_blk", op_gdn_project_mfma_blk},
+    {"outproj_mfma_blk", op_outproj_mfma_blk},
 };
 const uint32_t kQ4ProjectKernelCount = sizeof(kQ4ProjectKernels) / sizeof(kQ4ProjectKernels[0]);
 #endif

@@ -28,10 +28,11 @@ ATTN_PROJ = 9216
 CONV_ELEMS = 3 * 8192
 REC_ELEMS = 32 * 128 * 128
 CHUNK_RECORD_BYTES = 115712
-# Rows up to which a block is projected like a decode wave: it streams the same weights, and
-# the wave operators stay on the matrix unit where the block operators evaluate up to 16 rows
-# in the reference's order (12 rows: 28 -> 7 us out-projection, 34 -> 12 us and 27 -> 10 us
-# in-projections).
+# Rows up to which a block is projected by the _mfma_blk operators: they stream the weights
+# through the matrix unit, as a decode wave does, where the _blk operators evaluate up to 16
+# rows in the reference's order on the vector unit (12 rows: out-projection 23.7 -> 6.6 us,
+# in-projections 32.5 -> 9.2 and 26.8 -> 7.7 us).  Their fp32 sums are no further from the exact
+# ones than that order's.
 WAVE_ROWS = 16
 
 
@@ -231,8 +232,7 @@ class StubStack:
 
     def _project_in(self, cb, layer, rows, block):
         """normed -> proj: the layer's input projection (a decode wave or a block); with
-        _fused_wave x -> proj through the layer's input norm.  A block of 2..16 rows takes the
-        decode wave's form."""
+        _fused_wave x -> proj through the layer's input norm."""
         gated = layer["kind"] == "G"
         width = GDN_PROJ if gated else ATTN_PROJ
         if "in_q4" not in layer:
@@ -246,8 +246,9 @@ class StubStack:
                 bindings[1 + 3 * index + part] = matrix[part]
         out = 1 + 3 * len(layer["in_q4"])
         bindings[out] = self.proj
-        if block and not 2 <= rows <= WAVE_ROWS:
-            cb.encode(self.lib.pipeline(name + "_blk"), bindings, {out + 1: rows},
+        if block:
+            suffix = "_mfma_blk" if 2 <= rows <= WAVE_ROWS else "_blk"
+            cb.encode(self.lib.pipeline(name + suffix), bindings, {out + 1: rows},
                       ((width + 3) // 4,), (128,))
         else:
             # several rows: the matrix-unit form; one: the reference's own order
@@ -265,10 +266,10 @@ class StubStack:
             return
         words, scales, biases = layer["out_q4"]
         bindings = {0: self.mixed, 1: words, 2: scales, 3: biases, 4: self.delta}
-        if block and not 2 <= rows <= WAVE_ROWS:
-            cb.encode(self.lib.pipeline("outproj_blk"), bindings, {5: rows, 6: 4096},
-                      (HIDDEN // 2,), (64,))
-        elif not block and self._fused_wave(layer, rows):
+        if block:
+            name = "outproj_mfma_blk" if 2 <= rows <= WAVE_ROWS else "outproj_blk"
+            cb.encode(self.lib.pipeline(name), bindings, {5: rows, 6: 4096}, (HIDDEN // 2,), (64,))
+        elif self._fused_wave(layer, rows):
             # x = bf16(x + bf16(projection)) in place
             cb.encode(self.lib.pipeline("gdn_outproj_residual_mfma_ms"),
                       {**bindings, 4: self.x, 8: self.x}, {5: rows, 6: HIDDEN, 7: 16},
