@@ -329,7 +329,7 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
     };
     static constexpr Cost kCosts[] = {
-        {BlockTile::Large, 256, 256, 1580, 8000, 3160, 16000},
+        {BlockTile::Large, 256, 256, 1520, 7500, 3040, 15000},
         {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
         {BlockTile::Deep, 128, 128, 520, 2000, 1040, 4000},
         {BlockTile::Tall, 128, 64, 330, 1500, 630, 3000},
@@ -342,8 +342,13 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
     for (const Cost& c : kCosts) {
         const uint64_t tiles = static_cast<uint64_t>((rows + c.m - 1) / c.m) * ((out_dim + c.n - 1) / c.n);
         const uint64_t each = (tiles + compute_units - 1) / compute_units;
-        const uint64_t time = each / 2 * (c.both_unit * units + c.both_tile) +
-                              each % 2 * (c.single_unit * units + c.single_tile);
+        uint64_t time = each / 2 * (c.both_unit * units + c.both_tile) +
+                        each % 2 * (c.single_unit * units + c.single_tile);
+        // (compute units that the last round leaves idle make the others faster, up to a quarter:
+        // 2048 x 4096 x 2048, 64 tiles, 77 us, 6500 x 4096 x 2048, 208 tiles, 94, 8192, 256 tiles, 105)
+        if (c.tile == BlockTile::Large) {
+            time -= (c.single_unit * units + c.single_tile) * (each * compute_units - tiles) / (4 * compute_units);
+        }
         if (time < best_time) {
             best_time = time;
             best = c.tile;
@@ -355,18 +360,19 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
 // to four waves of a SIMD fill each other's waits (LDS reads take a fifth of the cycles, the
 // matrix unit 58 % of them with eight waves that read, request and multiply in turns); units of
 // 32 columns in a deeper ring, with a barrier each, were 6 to 20 % slower.  Measured, f16 operands:
-//   Large  16384 x 2176 x 12352 / 9216, 8192 x 4352 x 2048: 790 / 563 / 114 us = 1.12 / 1.17 /
-//          1.29 PFLOP/s (eight waves of 128 x 64: 832 / 546 / 110 us; with all transfers of a unit
-//          issued ahead of its products 865 / 573 / 116 us)
-//   Even   2048 x 2176 x 9216: 91 us; Large 106, Deep 97, Tall 106
-//   Deep   2048 x 4352 x 2048: 38 us; Even 48, Large 85
+//   Large  16384 x 2176 x 12352 / 9216, 8192 x 4352 x 2048: 763 / 553 / 110 us = 1.15 / 1.19 /
+//          1.33 PFLOP/s.  Eight waves of 128 x 64: sixteen of 64 x 64 read a third more and were 2
+//          to 5 % slower at every size (785 / 575 / 114; bf16 operands, 16384 x 2048 x 12352 /
+//          9216 and 16384 x 4096 x 2048: 697 / 502 / 197 against 729 / 529 / 204)
+//   Even   2048 x 2176 x 9216: 92 us; Large 103, Deep 97, Tall 106
+//   Deep   2048 x 4352 x 2048: 38 us; Even 48, Large 81
 //   Tall   100 x 2176 x 12352: 13.5 us; Deep 17, Small 20 (as 64 x 128, 19)
 //          777 x 4352 x 2048: 24 us; Deep 30, Even 43
 //   Small  300 x 4352 x 2048: 15 us; Least 20, Tall 22, Deep 29
 //   Least  100 x 4352 x 2048: 11 us; Small 14, Tall 19, Deep 27
 template <typename Element>
 struct BlockTiles {
-    typedef BlockProduct<Element, 256, 256, 4, 4> Large;      // the most products per byte fetched
+    typedef BlockProduct<Element, 256, 256, 2, 4> Large;      // the most products per byte fetched
     typedef BlockProduct<Element, 128, 128, 2, 4> Even;       // two a compute unit hide each other's waits
     typedef BlockProduct<Element, 128, 128, 2, 4, 4> Deep;    // one a compute unit, two units further ahead
     typedef BlockProduct<Element, 128, 64, 4, 2, 3> Tall;
