@@ -32,7 +32,7 @@ EXPORTED_SYMBOLS = [
     "tt_command_name", "tt_command_gpu_ms", "tt_attention_decode_lanes_static",
     "tt_event_create", "tt_event_destroy", "tt_encode_signal_event", "tt_encode_wait_for_event",
     "tt_split_workgroups", "tt_choose_split_keys",
-    "tt_flash_prefill_splits", "tt_flash_prefill_scratch_bytes",
+    "tt_flash_prefill_splits", "tt_flash_prefill_scratch_bytes", "tt_block_product_tile",
 ]
 
 
@@ -109,6 +109,7 @@ def lib():
         "tt_split_workgroups": (u32, [C.POINTER(u32), u32, u32]),
         "tt_choose_split_keys": (u32, [C.POINTER(u32), u32, u32]),
         "tt_flash_prefill_splits": (u32, [u32, u32, u32]),
+        "tt_block_product_tile": (u32, [u32] * 4),
         "tt_flash_prefill_scratch_bytes": (u64, [u32, u32]),
         "tt_event_create": (i32, [vp, pvp]), "tt_event_destroy": (None, [vp]),
         "tt_encode_signal_event": (i32, [vp, vp, u64]),
@@ -490,6 +491,15 @@ def choose_split_keys(visible_keys, compute_units=256):
     """Keys per split-K workgroup for a token wave (tt_choose_split_keys)."""
     array, count = _u32_array(visible_keys)
     return int(lib().tt_choose_split_keys(array, count, int(compute_units)))
+
+
+BLOCK_TILES = ("256x256", "128x128", "128x128-deep", "128x64", "64x64", "32x64")
+
+
+def block_product_tile(rows, in_dim, out_dim, compute_units=256):
+    """The tile (a name of BLOCK_TILES, rows x outputs) that a block product of that size is
+    multiplied with (tt_block_product_tile)."""
+    return BLOCK_TILES[lib().tt_block_product_tile(int(rows), int(in_dim), int(out_dim), int(compute_units))]
 
 
 def flash_prefill_splits(rows, visible_keys, compute_units=256):

@@ -182,10 +182,9 @@ def test_block_projection(family, name, rows):
                                          (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
 @pytest.mark.parametrize("rows", [256, 257, 700, 2048, 16384])
 def test_block_projection_over_several_row_tiles(family, name, rows):
-    """Blocks that span more than one 256-row tile of the block kernel, up to the 16384 rows
-    the benchmark times, among them the reference's 2048-row block, whose last, partly filled
-    round of tiles is shared between workgroups (as that of most sizes here is): every output
-    row is produced, and a sample of rows - the first and last of the block, the rows either
+    """Blocks that span more than one tile of rows, up to the 16384 rows the benchmark times,
+    among them the reference's 2048-row block, whose last round of tiles is partly filled (as that
+    of most sizes here is): every output row is produced, and a sample of rows - the first and last of the block, the rows either
     side of each tile boundary sampled, a few inside - is held to the checker."""
     print(f"[case] {name} rows={rows} (sampled rows)", flush=True)
     B, dev, queue, lib = gpu()

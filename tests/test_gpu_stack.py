@@ -13,6 +13,7 @@ import pytest
 
 import oracle_lib as ol
 from gpu_util import gpu, run
+from test_host_rules import DENSE_TILE_CASES
 
 pytestmark = pytest.mark.gpu
 o = ol.oracle
@@ -332,25 +333,21 @@ def _dense_block_case(rows, in_dim, out_dim, sample_rows, seed):
     (640, 192, 1024),      # six steps: one round of the steady loop
 ], ids=["65x64x70", "257x2048x300", "300x4096x2048", "1000x2048x515", "513x128x256", "640x192x1024"])
 def test_dense_bf16_block_kernel(rows, in_dim, out_dim):
-    """Blocks of more than 64 rows take the LDS-staged 256 x 256 kernel: every row against the
-    checker, partial tiles either way, every length of the K walk's lead-in and lead-out."""
+    """Blocks of more than 16 rows take an LDS-staged product: every row against the checker,
+    partial tiles either way (these sizes take the 32 x 64 and 64 x 64 tiles), every length of
+    the K walk's lead-in and lead-out."""
     print(f"[case] dense_bf16 block rows={rows} in={in_dim} out={out_dim}", flush=True)
     _dense_block_case(rows, in_dim, out_dim, range(rows), 0xB10C + rows)
 
 
-@pytest.mark.parametrize("rows,in_dim,out_dim", [
-    (66, 2048, 515),       # 64 x 64 tiles, two rows into the second
-    (100, 64, 4096),       # fewer units of K than a ring holds
-    (129, 256, 9216),      # one row into a second 64- or 128-row tile, several rounds of them
-    (500, 2048, 9216),     # 128 x 128 tiles, two a compute unit, the last round not filled
-    (2047, 4096, 2048),    # 128 x 128 tiles, one a compute unit
-    (2049, 192, 12352),    # 256 x 256 tiles and a row of one more
-], ids=lambda v: str(v))
-def test_dense_bf16_block_tiles(rows, in_dim, out_dim):
+@pytest.mark.parametrize("tile,rows,in_dim,out_dim", DENSE_TILE_CASES, ids=lambda v: str(v))
+def test_dense_bf16_block_tiles(tile, rows, in_dim, out_dim):
     """The tiles a block is launched with, at their edges: sampled rows against the checker,
     every output stored."""
-    print(f"[case] dense_bf16 tiles rows={rows} in={in_dim} out={out_dim}", flush=True)
-    sample = sorted({0, 15, 16, 63, 64, 65, rows // 2, rows - 2, rows - 1} |
+    print(f"[case] dense_bf16 tile {tile} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    B, dev, queue, lib = gpu()
+    assert B.block_product_tile(rows, in_dim, out_dim, dev.compute_units) == tile
+    sample = sorted({r for r in (0, 15, 16, 31, 32, 63, 64, 65, rows // 2, rows - 2, rows - 1) if r < rows} |
                     {r for r in range(127, rows, 640)} | {r for r in range(128, rows, 640)})
     got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB111 + rows)
     assert not np.any((got & 0x7F80) == 0x7F80), "an output was not stored"
@@ -358,7 +355,7 @@ def test_dense_bf16_block_tiles(rows, in_dim, out_dim):
 
 def test_dense_bf16_block_kernel_at_the_prefill_shape():
     """16384 rows x 2048 -> 9216 (the attention input projection of a 16384-row block): 2304
-    tiles on one workgroup per compute unit, nine tiles each.  The checker evaluates every
+    256 x 256 tiles on one workgroup per compute unit, nine tiles each.  The checker evaluates every
     251st row (66 rows, each at another position inside its tile) and the last rows."""
     rows, in_dim, out_dim = 16384, 2048, 9216
     print(f"[case] dense_bf16 block rows={rows} in={in_dim} out={out_dim}, sampled rows", flush=True)

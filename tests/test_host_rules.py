@@ -59,3 +59,48 @@ def test_flash_prefill_sharing_plan(rows, units, splits, scratch):
     assert B.flash_prefill_splits(rows, 481, units) == splits
     assert B.flash_prefill_scratch_bytes(rows, splits) == scratch
     assert B.flash_prefill_scratch_bytes(rows, 1) == 0
+
+
+# (tile, rows, in_dim, out_dim) of the dense_bf16 blocks that tests/test_gpu_stack.py runs: every tile
+# with fewer units of 64 columns than its ring holds, as many and more, at remainders of rows and
+# outputs and at output rows that are not 8-byte aligned.
+DENSE_TILE_CASES = [(tile, rows, in_dim, out_dim) for tile, rows, out_dim in [
+    ("256x256", 2049, 6141), ("128x128", 641, 6141), ("128x128-deep", 129, 12350), ("128x64", 65, 12350),
+    ("64x64", 33, 9213), ("32x64", 17, 61)] for in_dim in (64, 128, 192, 256)] + [
+    ("256x256", 1025, 2048, 12349), ("256x256", 2049, 192, 12352), ("256x256", 5000, 4096, 2046),
+    ("128x128", 500, 2048, 9213), ("128x128", 500, 2048, 9216), ("128x128-deep", 2047, 4096, 2045),
+    ("128x64", 777, 4096, 2046), ("128x64", 100, 2048, 12352), ("64x64", 129, 256, 9216),
+    ("64x64", 129, 2048, 9213), ("32x64", 66, 2048, 515), ("32x64", 100, 64, 4096)]
+
+
+@pytest.mark.parametrize("tile,rows,in_dim,out_dim", DENSE_TILE_CASES, ids=lambda v: str(v))
+def test_block_tile_of_the_cases(tile, rows, in_dim, out_dim):
+    """The rule still gives the cases the tiles they are there for: a change of its figures that
+    left a tile without a case fails here."""
+    from tatara_amd import backend as B
+    assert B.block_product_tile(rows, in_dim, out_dim, 256) == tile
+
+
+def test_every_block_tile_has_cases():
+    from tatara_amd import backend as B
+    assert {case[0] for case in DENSE_TILE_CASES} == set(B.BLOCK_TILES)
+    # the 4-bit blocks of tests/test_gpu_q4_project.py: their operands are 17/16 of the input wide, and
+    # the out-projection takes 8192 rows at a time
+    taken = {B.block_product_tile(min(rows, limit), k * 17 // 16, n, 256)
+             for k, n, limit in ((2048, 9216, 16384), (2048, 12352, 16384), (4096, 2048, 8192))
+             for rows in (17, 37, 63, 65, 129, 130, 511, 8193)}
+    assert taken == set(B.BLOCK_TILES)
+
+
+@pytest.mark.parametrize("rows,in_dim,out_dim,tile", [
+    (16384, 2048, 9216, "256x256"), (16384, 2048, 12352, "256x256"), (8192, 4096, 2048, "256x256"),
+    (5500, 4096, 2048, "256x256"),      # 176 tiles: idle compute units make the others faster
+    (4096, 2048, 9216, "128x128"), (2048, 2048, 9216, "128x128"), (2048, 4096, 2048, "128x128-deep"),
+    (100, 2048, 12352, "128x64"), (300, 4096, 2048, "64x64"), (100, 4096, 2048, "32x64")])
+def test_block_tile_where_it_was_measured(rows, in_dim, out_dim, tile):
+    """The fastest tile at sizes where all of them were timed on 256 compute units; and a tile for
+    any number of compute units."""
+    from tatara_amd import backend as B
+    assert B.block_product_tile(rows, in_dim, out_dim, 256) == tile
+    for units in (0, 1, 64, 304):
+        assert B.block_product_tile(rows, in_dim, out_dim, units) in B.BLOCK_TILES
