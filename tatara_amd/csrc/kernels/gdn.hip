@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void gdn_prepare_block_kernel(PrepareArgs a) {
             act[j + 1] = conv[1] * gate1;
             rb_pair(act[j], act[j + 1]);
         }
-        if (row == a.rows - 1) {
+        if (row == a.rows - 1 && a.conv_out != nullptr) {
             *reinterpret_cast<u32x4*>(a.conv_out + c) = t1;
             *reinterpret_cast<u32x4*>(a.conv_out + kCh + c) = t2;
             *reinterpret_cast<u32x4*>(a.conv_out + 2 * kCh + c) = t3;
@@ -329,6 +329,24 @@ __global__ __launch_bounds__(256) void gdn_prepare_block_kernel(PrepareArgs a) {
         t2 = t3;
     }
 }
+
+// The window a block leaves where it overlaps the window it starts from: by one workgroup of 1024,
+// behind the block's dispatch, every value read before the first is written.
+__global__ __launch_bounds__(1024) void gdn_window_kernel(PrepareArgs a) {
+    u32x4 kept[3];
+    const uint32_t c = threadIdx.x * 8;
+#pragma unroll
+    for (uint32_t tap = 0; tap < 3; ++tap) {
+        const uint32_t index = a.rows + tap;   // of the three state rows and the block's
+        kept[tap] = index < 3 ? *reinterpret_cast<const u32x4*>(a.conv_in + index * kCh + c)
+                              : *reinterpret_cast<const u32x4*>(
+                                    a.projection + static_cast<uint64_t>(index - 3) * a.projection_stride + c);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t tap = 0; tap < 3; ++tap) *reinterpret_cast<u32x4*>(a.conv_out + tap * kCh + c) = kept[tap];
+}
+static_assert(kCh == 1024 * 8, "a thread's eight channels");
 
 // ------------------------------------------------------------- recurrence ----
 
@@ -1489,22 +1507,21 @@ constexpr uint32_t kScanTiles = 1;
 // rows take 3.4 / 4.3 / 7.2 us so, 16.2 / 21.5 / 22.0 us sixteen to a workgroup - and many want
 // the three earlier rows read less often: 2048 rows 27.6 / 24.8 / 26.6 us and 16384 rows 245 /
 // 192 / 176 us with 1 / 2 / 4 to a workgroup, 173 us with six, 184 us with sixteen.
-// A window written where the block's earlier taps are read stays with one workgroup as long as
-// sixteen rows allow it.
-uint32_t prepare_rows_per_group(const PrepareArgs& p) {
-    const uintptr_t in = reinterpret_cast<uintptr_t>(p.conv_in), out = reinterpret_cast<uintptr_t>(p.conv_out);
-    constexpr uintptr_t kWindowBytes = 3 * kCh * 2;
-    if (in < out + kWindowBytes && out < in + kWindowBytes) return kBlockRowsPerGroup;
-    return p.rows <= 512 ? 1 : p.rows <= 4096 ? 2 : 6;
-}
+uint32_t prepare_rows_per_group(uint32_t rows) { return rows <= 512 ? 1 : rows <= 4096 ? 2 : 6; }
 
 int32_t launch_prepare(const PrepareArgs& p, hipStream_t stream) {
     if (p.block_mode) {
         PrepareArgs block = p;
-        block.rows_per_group = prepare_rows_per_group(p);
+        block.rows_per_group = prepare_rows_per_group(p.rows);
+        // The workgroups of the first rows read the window that the last row's would write.
+        const uintptr_t in = reinterpret_cast<uintptr_t>(p.conv_in), out = reinterpret_cast<uintptr_t>(p.conv_out);
+        constexpr uintptr_t kWindowBytes = 3 * kCh * 2;
+        const bool in_place = in < out + kWindowBytes && out < in + kWindowBytes;
+        if (in_place) block.conv_out = nullptr;
         const uint32_t groups = (p.rows + block.rows_per_group - 1) / block.rows_per_group;
         hipLaunchKernelGGL(gdn_prepare_block_kernel, dim3(kPrepareUnitGroups * groups), dim3(256), 0, stream,
                            block);
+        if (in_place) hipLaunchKernelGGL(gdn_window_kernel, dim3(1), dim3(1024), 0, stream, p);
         return TT_OK;
     }
     hipLaunchKernelGGL(gdn_prepare_kernel, dim3(96, p.rows), dim3(128), 0, stream, p);

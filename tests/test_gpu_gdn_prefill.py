@@ -152,20 +152,25 @@ def test_element_wise_block_kernels_at_every_rows_per_group(rows):
     test_element_wise_block_kernels_bit_for_bit(rows)
 
 
-@pytest.mark.parametrize("rows", [2, 12, 16])
-def test_conv_window_written_in_place(rows):
-    """A short block that leaves its conv window in the buffer it read the last one from."""
-    print(f"[case] gdn conv window in place rows={rows}", flush=True)
+@pytest.mark.parametrize("shift", [0, 8192, -2048], ids=["same", "a-row-on", "overlapping"])
+@pytest.mark.parametrize("rows", [1, 2, 3, 12, 16, 17, 100, 600])
+def test_conv_window_written_in_place(rows, shift):
+    """A block that leaves its conv window in the buffer it read the last one from, in the same
+    place or so that the two overlap by some channels."""
+    print(f"[case] gdn conv window in place rows={rows} shift={shift}", flush=True)
     B, dev, queue, lib = gpu()
     weights = _weights()
     proj, conv_state, state = _block(rows, 0x5700 + rows)
     ref = _oracle_block(proj, conv_state, state, weights, rows)
     bufs = _buffers(dev, proj, conv_state, state, weights, rows)
-    bufs["conv_out"] = bufs["conv_in"]
+    pool = np.full(5 * 8192, 0x7FC0, np.uint16)
+    pool[8192:4 * 8192] = conv_state
+    pool = dev.buffer_from(pool)
+    bufs["conv_in"], bufs["conv_out"] = (pool, 8192 * 2), (pool, (8192 + shift) * 2)
     run(lambda cb: _encode_front(cb, lib, bufs, rows))
     assert np.array_equal(bufs["qk"].read(np.uint16), ref["qk"])
     assert np.array_equal(bufs["value"].read(np.uint16), ref["value"])
-    assert np.array_equal(bufs["conv_out"].read(np.uint16), ref["conv"])
+    assert np.array_equal(pool.read(np.uint16)[8192 + shift:4 * 8192 + shift], ref["conv"])
 
 
 def test_activation_of_every_bf16_value_bit_for_bit():
