@@ -143,7 +143,9 @@ uint32_t tt_device_compute_units(const tt_device* device);
  * operators whose reference bindings carry no scratch - attention_flash_v2_blk /
  * attention_streaming_blk share the key walks of a block of few rows through it,
  * attn_project_blk / gdn_project_blk / outproj_blk lay their operands out in it; a queue whose
- * workspace could not be allocated works without, its blocks more slowly. */
+ * workspace could not be allocated works without, its blocks more slowly.
+ * One thread records a command buffer; several may commit theirs to one queue: a commit's commands
+ * go onto the stream together, so that no other commit's use the workspace in between. */
 int32_t tt_queue_create(tt_device* device, tt_queue** out);
 void tt_queue_destroy(tt_queue* queue);
 /* The HIP stream (hipStream_t) behind a queue, for event timing by the caller. */

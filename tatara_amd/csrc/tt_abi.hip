@@ -30,6 +30,9 @@ struct tt_queue {
     hipStream_t stream = nullptr;
     uint8_t* workspace = nullptr;   // see tt::StreamWorkspace
     uint64_t workspace_bytes = 0;
+    // held while a command buffer's commands go onto the stream: an operator may be several
+    // launches with the workspace between them, which another thread's must not come between
+    std::mutex submission;
 };
 
 struct tt_buffer {
@@ -891,6 +894,7 @@ int32_t tt_commit(tt_command_buffer* cb) {
     hipStream_t stream = cb->queue->stream;
     cb->submit_error = hipSuccess;
     cb->marks_valid = false;
+    std::lock_guard<std::mutex> submission(cb->queue->submission);
     (void)hipEventRecord(cb->begin, stream);
     if (cb->graph_exec != nullptr) {
         cb->submit_error = hipGraphLaunch(cb->graph_exec, stream);
@@ -915,6 +919,8 @@ int32_t tt_command_buffer_compile(tt_command_buffer* cb) {
     if (cb->committed) (void)hipEventSynchronize(cb->end);
     drop_graph(cb);
     hipStream_t stream = cb->queue->stream;
+    // (a commit by another thread would be captured as well)
+    std::lock_guard<std::mutex> submission(cb->queue->submission);
     if (hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed) != hipSuccess) {
         (void)hipGetLastError();
         return TT_CMD_COMMAND_BUFFER_CREATION_FAILED;

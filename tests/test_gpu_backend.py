@@ -164,3 +164,59 @@ def test_event_encoding_errors():
     assert e.value.status == 19
     cb2.commit().wait()
     cb.commit().wait()                         # now the value has been signalled
+
+
+def test_threads_that_commit_to_one_queue_do_not_meet_in_its_workspace():
+    """Four threads, each with command buffers of its own of one queue and 4-bit blocks of its own
+    size: a block's operands lie in the queue's workspace between two launches, which no other
+    thread's may come between.  Every result is the one the block has alone."""
+    import threading
+    import oracle_lib as ol
+    B, dev, _, lib = gpu()
+    queue = dev.create_queue()
+    rng = np.random.default_rng(0x7EAD)
+    pipeline = lib.pipeline("outproj_blk")
+    jobs = []
+    for rows in (17, 40, 100, 300):
+        words = rng.integers(0, 2 ** 32, 2048 * 512, dtype=np.uint64).astype(np.uint32)
+        scales = ol.f32_to_bf16(rng.uniform(0.002, 0.01, 2048 * 64).astype(np.float32))
+        biases = ol.f32_to_bf16(rng.uniform(-0.05, 0.02, 2048 * 64).astype(np.float32))
+        x = ol.gaussian_bf16(rows, rows * 4096)
+        jobs.append((rows, [dev.buffer_from(v) for v in (x, words, scales, biases)]))
+
+    def block(job, out):
+        cb = queue.create_command_buffer()
+        cb.begin_compute_pass()
+        cb.encode(pipeline, {**dict(enumerate(job[1])), 4: out}, {5: job[0], 6: 4096}, (1024,), (64,))
+        cb.end_compute_pass()
+        return cb
+
+    alone = []
+    for job in jobs:
+        out = dev.create_buffer(job[0] * 4096)
+        block(job, out).commit().wait()
+        alone.append(out.read(np.uint16))
+    outs = [[dev.create_buffer(job[0] * 4096) for _ in range(25)] for job in jobs]
+    errors = []
+    start = threading.Barrier(len(jobs))
+
+    def work(index):
+        try:
+            buffers = [block(jobs[index], out) for out in outs[index]]
+            start.wait()
+            for cb in buffers:
+                cb.commit()
+            for cb in buffers:
+                cb.wait()
+        except Exception as e:   # shown by the test, not by the thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for index, want in enumerate(alone):
+        for out in outs[index]:
+            assert np.array_equal(out.read(np.uint16), want), f"rows {jobs[index][0]}"
