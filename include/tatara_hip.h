@@ -142,11 +142,13 @@ uint32_t tt_device_compute_units(const tt_device* device);
  * workspace in device memory (125 MB, or 270,336 bytes per compute unit where that is more) for
  * operators whose reference bindings carry no scratch - attention_flash_v2_blk /
  * attention_streaming_blk share the key walks of a block of few rows through it,
- * attn_project_blk / gdn_project_blk / outproj_blk lay their operands out in it; a queue whose
- * workspace could not be allocated works without, its blocks more slowly.
+ * attn_project_blk / gdn_project_blk / outproj_blk lay their operands out in it.  Where device
+ * memory is short the queue takes less, or none, and its blocks take longer.
  * One thread records a command buffer; several may commit theirs to one queue: a commit's commands
  * go onto the stream together, so that no other commit's use the workspace in between. */
 int32_t tt_queue_create(tt_device* device, tt_queue** out);
+/* The same with at most that many bytes of workspace (0: none), for a host with many queues. */
+int32_t tt_queue_create_with_workspace(tt_device* device, uint64_t workspace_bytes, tt_queue** out);
 void tt_queue_destroy(tt_queue* queue);
 /* The HIP stream (hipStream_t) behind a queue, for event timing by the caller. */
 void* tt_queue_native_stream(tt_queue* queue);

@@ -18,7 +18,8 @@ LIBRARY_PATH = os.environ.get("TATARA_HIP_LIBRARY") or os.path.join(_HERE, "lib"
 
 EXPORTED_SYMBOLS = [
     "tt_abi_version", "tt_status_name", "tt_device_create", "tt_device_destroy",
-    "tt_device_name", "tt_device_compute_units", "tt_queue_create", "tt_queue_destroy",
+    "tt_device_name", "tt_device_compute_units", "tt_queue_create",
+    "tt_queue_create_with_workspace", "tt_queue_destroy",
     "tt_queue_native_stream", "tt_buffer_create", "tt_pool_create", "tt_buffer_window",
     "tt_buffer_wrap", "tt_buffer_destroy", "tt_buffer_size", "tt_buffer_contents",
     "tt_buffer_device_pointer", "tt_buffer_did_modify", "tt_buffer_synchronize",
@@ -70,6 +71,7 @@ def lib():
         "tt_status_name": (C.c_char_p, [i32]),
         "tt_device_create": (i32, [pvp]), "tt_device_destroy": (None, [vp]),
         "tt_device_name": (C.c_char_p, [vp]), "tt_device_compute_units": (u32, [vp]),
+        "tt_queue_create_with_workspace": (i32, [vp, u64, pvp]),
         "tt_queue_create": (i32, [vp, pvp]), "tt_queue_destroy": (None, [vp]),
         "tt_queue_native_stream": (vp, [vp]),
         "tt_buffer_create": (i32, [vp, u64, pvp]),
@@ -149,8 +151,10 @@ class Device:
         self.name = lib().tt_device_name(h).decode()
         self.compute_units = lib().tt_device_compute_units(h)
 
-    def create_queue(self):
-        return CommandQueue(self)
+    def create_queue(self, workspace_bytes=None):
+        """workspace_bytes: the most device memory the queue keeps for its operators (None: all they
+        can use, 0: none)."""
+        return CommandQueue(self, workspace_bytes)
 
     def create_buffer(self, size_bytes):
         h = C.c_void_p()
@@ -200,9 +204,11 @@ class Event:
 
 
 class CommandQueue:
-    def __init__(self, device):
+    def __init__(self, device, workspace_bytes=None):
         h = C.c_void_p()
-        _check(lib().tt_queue_create(device.handle, C.byref(h)), "create_command_queue")
+        status = (lib().tt_queue_create(device.handle, C.byref(h)) if workspace_bytes is None else
+                  lib().tt_queue_create_with_workspace(device.handle, int(workspace_bytes), C.byref(h)))
+        _check(status, "create_command_queue")
         self.handle, self.device = h, device
 
     @property

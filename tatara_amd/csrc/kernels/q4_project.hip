@@ -288,6 +288,7 @@ struct Unfold {
     _Float16* rows;            // [x_rows][unfolded_columns]
     int32_t* row_exponents;    // [x_rows]
     uint32_t weight_rows;      // 0: the weights are there already
+    uint32_t first_weight;     // the output row that row 0 of `weights` is
     uint32_t first_row, x_rows;
 };
 
@@ -304,8 +305,8 @@ __global__ __launch_bounds__(256) void q4_unfold_kernel(Q4Projection p, Unfold u
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (row < u.weight_rows) {
-        const Q4Matrix matrix = matrix_of_row(p, row);
-        const uint64_t local = row - matrix.first_row;
+        const Q4Matrix matrix = matrix_of_row(p, u.first_weight + row);
+        const uint64_t local = u.first_weight + row - matrix.first_row;
         const uint32_t* words = matrix.words + local * (kBlocks * 64);
         const uint16_t* scales = matrix.scales + local * (kBlocks * 8);
         const uint16_t* biases = matrix.biases + local * (kBlocks * 8);
@@ -433,7 +434,8 @@ int32_t check_block_operands(const Q4Projection& p) {
 
 // The workspace of a block: the unfolded weights of the largest projection and the unfolded
 // rows of 16384 tokens at the hidden width (8192 at the attention width); a longer block goes
-// through in slices of that many rows.
+// through in slices of that many rows.  In a smaller workspace (device memory was short when the
+// queue was made) the weights go through in slices as well, half of it for either.
 constexpr uint64_t kUnfoldedWeightBytes =
     static_cast<uint64_t>(kGdnProjectionRows) * unfolded_columns(kHidden) * 2;
 constexpr uint64_t kUnfoldedRowBytes = 16384ull * unfolded_columns(kHidden) * 2;
@@ -449,38 +451,50 @@ static_assert(static_cast<uint64_t>(kHidden) * unfolded_columns(kGdnValueValues)
 typedef BlockTiles<_Float16> Q4Tiles;
 int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
     const StreamWorkspace workspace = stream_workspace(stream);
-    // a queue whose workspace could not be allocated: the rows kernel takes any number of rows
-    if (workspace.base == nullptr || workspace.bytes < kUnfoldWorkspaceBytes ||
-        workspace.compute_units == 0) {
-        return launch_rows(p, stream);
-    }
     const uint32_t columns = unfolded_columns(p.k_size);
     const uint32_t out_rows = p.first_row[p.segments];
+    const bool whole = workspace.bytes >= kUnfoldWorkspaceBytes;
+    constexpr uint64_t kExponentBytes = kWeightExponentBytes + kRowExponentBytes;
+    const uint64_t unfolded_bytes = whole ? kUnfoldedWeightBytes + kUnfoldedRowBytes
+                                          : (std::max(workspace.bytes, kExponentBytes) - kExponentBytes) / 512 * 512;
+    const uint64_t weight_bytes = whole ? kUnfoldedWeightBytes : unfolded_bytes / 2;
+    // whole tiles of either operand, as many as there are exponents for
+    const auto slice_of = [&](uint64_t bytes, uint32_t most) {
+        return static_cast<uint32_t>(std::min<uint64_t>(bytes / 2 / columns / 256 * 256, most));
+    };
+    const uint32_t weight_slice = whole ? out_rows : slice_of(weight_bytes, kGdnProjectionRows);
+    const uint32_t slice = slice_of(unfolded_bytes - weight_bytes, 16384);
+    // a queue (almost) without workspace: the rows kernel takes any number of rows
+    if (workspace.base == nullptr || workspace.compute_units == 0 || weight_slice == 0 || slice == 0) {
+        return launch_rows(p, stream);
+    }
     Unfold u{};
     u.weights = reinterpret_cast<_Float16*>(workspace.base);
-    u.rows = reinterpret_cast<_Float16*>(workspace.base + kUnfoldedWeightBytes);
-    u.weight_exponents =
-        reinterpret_cast<int32_t*>(workspace.base + kUnfoldedWeightBytes + kUnfoldedRowBytes);
+    u.rows = reinterpret_cast<_Float16*>(workspace.base + weight_bytes);
+    u.weight_exponents = reinterpret_cast<int32_t*>(workspace.base + unfolded_bytes);
     u.row_exponents = reinterpret_cast<int32_t*>(
         reinterpret_cast<uint8_t*>(u.weight_exponents) + kWeightExponentBytes);
-    u.weight_rows = out_rows;
-    const uint32_t slice = static_cast<uint32_t>(kUnfoldedRowBytes / 2 / columns) / 256 * 256;
-    for (u.first_row = 0; u.first_row < p.rows; u.first_row += u.x_rows) {
-        u.x_rows = std::min(slice, p.rows - u.first_row);
-        const dim3 grid((u.weight_rows + u.x_rows + 3) / 4);
-        if (p.k_size == 4 * kQ4Block) {
-            hipLaunchKernelGGL(q4_unfold_kernel<4>, grid, dim3(256), 0, stream, p, u);
-        } else {
-            hipLaunchKernelGGL(q4_unfold_kernel<8>, grid, dim3(256), 0, stream, p, u);
+    for (; u.first_weight < out_rows; u.first_weight += weight_slice) {
+        const uint32_t columns_out = std::min(weight_slice, out_rows - u.first_weight);
+        u.weight_rows = columns_out;
+        for (u.first_row = 0; u.first_row < p.rows; u.first_row += u.x_rows) {
+            u.x_rows = std::min(slice, p.rows - u.first_row);
+            const dim3 grid((u.weight_rows + u.x_rows + 3) / 4);
+            if (p.k_size == 4 * kQ4Block) {
+                hipLaunchKernelGGL(q4_unfold_kernel<4>, grid, dim3(256), 0, stream, p, u);
+            } else {
+                hipLaunchKernelGGL(q4_unfold_kernel<8>, grid, dim3(256), 0, stream, p, u);
+            }
+            u.weight_rows = 0;
+            Q4Tiles::choose(u.x_rows, columns, columns_out, workspace.compute_units, [&](auto product) {
+                typedef decltype(product) Product;
+                hipLaunchKernelGGL(
+                    q4_product_kernel<Product>,
+                    dim3(block_workgroups<Product>(u.x_rows, columns_out, workspace.compute_units)),
+                    dim3(Product::kThreads), Product::kLdsBytes, stream, u, p.output + u.first_weight,
+                    p.output_stride, columns, columns_out);
+            });
         }
-        u.weight_rows = 0;
-        Q4Tiles::choose(u.x_rows, columns, out_rows, workspace.compute_units, [&](auto product) {
-            typedef decltype(product) Product;
-            hipLaunchKernelGGL(q4_product_kernel<Product>,
-                               dim3(block_workgroups<Product>(u.x_rows, out_rows, workspace.compute_units)),
-                               dim3(Product::kThreads), Product::kLdsBytes, stream, u, p.output,
-                               p.output_stride, columns, out_rows);
-        });
     }
     return TT_OK;
 }

@@ -332,7 +332,15 @@ uint32_t tt_device_compute_units(const tt_device* device) {
     return device != nullptr ? device->compute_units : 0;
 }
 
+// Half the workspace is asked for again and again down to this, where device memory is short.
+constexpr uint64_t kLeastWorkspaceBytes = 8ull << 20;
+
 int32_t tt_queue_create(tt_device* device, tt_queue** out) {
+    return tt_queue_create_with_workspace(
+        device, device != nullptr ? tt::stream_workspace_bytes(device->compute_units) : 0, out);
+}
+
+int32_t tt_queue_create_with_workspace(tt_device* device, uint64_t workspace_bytes, tt_queue** out) {
     if (out == nullptr) return TT_RES_INVALID_DEVICE;
     *out = nullptr;
     if (device == nullptr) return TT_RES_INVALID_DEVICE;
@@ -352,17 +360,20 @@ int32_t tt_queue_create(tt_device* device, tt_queue** out) {
     // of the static scratch): done here so that an entry point that launches directly on
     // the queue never has to do it inside a stream capture.  A failure shows at that call.
     (void)tt::prepare_decode_kernels();
-    // The queue's workspace.  Doing without it is not an error: the operators that would
+    // The queue's workspace.  Doing with less or without is not an error: the operators that would
     // use it run as they do on a foreign stream.
-    const uint64_t bytes = tt::stream_workspace_bytes(device->compute_units);
     void* workspace = nullptr;
-    if (bytes != 0 && hipMalloc(&workspace, bytes) == hipSuccess) {
+    uint64_t bytes = workspace_bytes;
+    while (bytes != 0 && hipMalloc(&workspace, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        workspace = nullptr;
+        bytes = bytes / 2 >= kLeastWorkspaceBytes ? bytes / 2 : 0;
+    }
+    if (workspace != nullptr) {
         queue->workspace = static_cast<uint8_t*>(workspace);
         queue->workspace_bytes = bytes;
         std::lock_guard<std::mutex> lock(tt::g_workspace_mutex);
         tt::g_workspaces[stream] = tt::StreamWorkspace{queue->workspace, bytes, device->compute_units};
-    } else {
-        (void)hipGetLastError();
     }
     *out = queue;
     return TT_OK;

@@ -265,6 +265,42 @@ def test_block_projection_against_64_bit_sums_over_the_whole_range(family, name,
         first += n
 
 
+@pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
+                                         (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
+@pytest.mark.parametrize("rows", [17, 300, 1500])
+def test_block_projection_in_queues_of_less_workspace(family, name, rows):
+    """A queue that could not have its whole workspace takes the operands through in slices of output
+    rows and of input rows (8 MiB: 768 outputs and rows at a time at the hidden width, 256 at
+    the attention width): the same sums, bit for bit.  One without workspace evaluates the rows in
+    the reference's order: the checker's bits."""
+    B, dev, _, lib = gpu()
+    host, bindings = _family(dev, family, 0xA800)
+    k, total = family["k"], sum(family["segments"])
+    x = ol.gaussian_bf16(0xA900 + rows, rows * k, 0.0, 1.0)
+    bindings[0] = dev.buffer_from(x)
+    slot = family["out"] + 1
+    constants = {slot: rows, slot + 1: k} if family is OUT else {slot: rows}
+    got = {}
+    for workspace in (None, 60 << 20, 20 << 20, 8 << 20, 1 << 20, 0):
+        print(f"[case] {name} rows={rows} workspace={workspace}", flush=True)
+        queue = dev.create_queue(workspace)
+        out = dev.buffer_from(np.full(rows * total, 0x7FC0, np.uint16))
+        cb = queue.create_command_buffer()
+        cb.begin_compute_pass()
+        cb.encode(lib.pipeline(name), {**bindings, family["out"]: out}, constants, (_groups(family), 1, 1),
+                  (family["threads"], 1, 1))
+        cb.end_compute_pass()
+        ms = cb.commit().wait()
+        got[workspace] = out.read(np.uint16).reshape(rows, total)
+        print(f"[time] {ms * 1e3:.1f} us", flush=True)
+    for workspace in (60 << 20, 20 << 20, 8 << 20):
+        assert np.array_equal(got[workspace], got[None]), workspace
+    assert np.array_equal(got[0], got[1 << 20])
+    sample = sorted({0, 15, 16, rows // 2, rows - 1})
+    want = _expected(family, host, np.ascontiguousarray(x.reshape(rows, k)[sample]).reshape(-1), len(sample))
+    assert np.array_equal(got[0][sample].reshape(-1), want)
+
+
 def _cancelling_matrix(rng, rows, k):
     """Matrices whose second half of K undoes the first: columns k / 2 on hold, permuted, 16 minus the
     nibbles (1 .. 15) of the first, one scale to a row, biases of -7.5 scales and then -8.5 (scales of
