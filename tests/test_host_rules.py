@@ -95,6 +95,9 @@ def test_every_block_tile_has_cases():
 @pytest.mark.parametrize("rows,in_dim,out_dim,tile", [
     (16384, 2048, 9216, "256x256"), (16384, 2048, 12352, "256x256"), (8192, 4096, 2048, "256x256"),
     (5500, 4096, 2048, "256x256"),      # 176 tiles: idle compute units make the others faster
+    (4050, 2048, 12352, "128x128"), (5450, 2176, 9216, "128x128"),   # just over three rounds of 256 x 256
+    (3000, 2176, 12352, "256x256"), (10300, 4096, 2048, "128x128"),
+    (4102, 4096, 2048, "256x256"),
     (4096, 2048, 9216, "128x128"), (2048, 2048, 9216, "128x128"), (2048, 4096, 2048, "128x128-deep"),
     (100, 2048, 12352, "128x64"), (300, 4096, 2048, "64x64"), (100, 4096, 2048, "32x64")])
 def test_block_tile_where_it_was_measured(rows, in_dim, out_dim, tile):
