@@ -313,7 +313,9 @@ class StubStack:
         keys or more - shallow lanes in deep caches, deep lanes among shallow ones - the split
         follows what they hold (bit 8: a wave of 16 lanes of 150 .. 12000 keys in caches of
         16384 399 -> 359 us, of 4 lanes of 700 .. 6001 in 32768 272 -> 248).  Full lanes keep
-        the fixed split: it names a workgroup's row before the state table has arrived."""
+        the fixed split: it names a workgroup's row before the state table has arrived.  (With bit
+        8 the order of a lane's fp32 sums follows from all lanes of the wave: beside other lanes
+        its result may differ in the last place, no further from the exact one.)"""
         contexts = self.context[:rows]
         deepest = max(contexts)
         live = split_workgroups([max(c, 1) for c in contexts], self.split_keys)
