@@ -835,7 +835,9 @@ int32_t flash_blk(const Bindings& b, const Grid& g, hipStream_t stream, bool val
             planned = std::max(planned, std::min({workspace.compute_units / (tiles * kAttnKvHeads),
                                                   walk_tiles / kMinTilesPerSplit, kWideFlashSplits}));
         }
-        if (planned > f.splits && flash_prefill_scratch_bytes(f.rows, planned) <= workspace.bytes) {
+        // (a queue may have less workspace than the plan wants)
+        while (planned > f.splits && flash_prefill_scratch_bytes(f.rows, planned) > workspace.bytes) --planned;
+        if (planned > f.splits) {
             f.splits = planned;
             f.scratch = workspace.base;
         }
@@ -864,9 +866,9 @@ int32_t op_attention_flash_blk(const Bindings& b, const Grid& g, hipStream_t str
 
 // attention_flash_split_blk (no counterpart in the reference): the bindings, constants and
 // grid of attention_flash_v2_blk, plus b9 scratch and c10 splits (1..8) - the workgroups that
-// share each position tile's key walk (8: or more, see kWideFlashSplits).  tt_flash_prefill_splits gives the count that fills
-// the device for a block of `rows` rows that sees `visible` keys, tt_flash_prefill_scratch_bytes the bytes b9 must hold
-// (none for one split).  Same results as attention_flash_v2_blk up to the order of fp32 sums.
+// share each position tile's key walk (8: or more, see kWideFlashSplits, b9 then left alone).
+// tt_flash_prefill_splits gives the count that fills the device for a block of `rows` rows that sees
+// `visible` keys, tt_flash_prefill_scratch_bytes the bytes b9 must hold (none for one split).  Same results as attention_flash_v2_blk up to the order of fp32 sums.
 int32_t op_attention_flash_split_blk(const Bindings& b, const Grid& g, hipStream_t stream,
                                      bool validate_only) {
     return flash_blk(b, g, stream, validate_only, true);

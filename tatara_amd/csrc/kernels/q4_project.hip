@@ -263,11 +263,11 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
 // A scale has 8 significant bits and nibble - 8 (-8 .. 7) three or a power of two, so their
 // product has at most 11: an f16 number, exactly.  So is x, of 8 bits.  Both are brought into
 // f16's range by a power of two per row (an output row's largest of 8 |scale| and |bias| below
-// 2^15, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): what
-// lies so far below the row's largest value that f16 rounds it (2^-26 for x) is off by 2^-34 of
-// that value at most, far less than the fp32 sums resolve.  The affine terms are four further
-// columns a group, {bias, 8 scale, bias, 8 scale} against {hi, hi, lo, lo} of the group sum in
-// two f16 parts.  One pass writes both operands so into the queue's workspace; the product is
+// 2^15, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): an x that
+// lies so far below the row's largest that f16 rounds it is off by 2^-33 of that one at most, a
+// weight by 2^-39.  The affine terms are four further columns a group, {bias, 8 scale, bias,
+// 8 scale} against {hi, hi, lo, lo} of the group sum in two f16 parts, 2^-23 of the sum at most
+// from it: the largest of these roundings, about one of the fp32 sums' own.  One pass writes both operands so into the queue's workspace; the product is
 // then a plain one (block_product.h) and the powers of two leave with the result.
 //
 // Why not unpack inside the product: a scale per 64 columns costs a product of its own from a

@@ -209,6 +209,31 @@ def test_walk_shared_by_as_many_as_fill_the_device(rows, base):
     _prefill_case(rows, base, 8192, 0x5A80 + rows, replays=2)
 
 
+@pytest.mark.parametrize("rows,base", [(12, 5003), (65, 4100)])
+def test_walk_shared_by_as_many_as_the_workspace_holds(rows, base):
+    """The same in queues of less workspace: as many sharers as it holds (12 rows in 4 MiB: seven a
+    kv head), one workgroup a tile without any; the results differ as two plans do."""
+    B, dev, _, lib = gpu()
+    cap = 8192
+    b_q, b_g = (dev.buffer_from(ol.gaussian_bf16(0x5B00 + i, rows * 4096)) for i in range(2))
+    b_k, b_v = (dev.buffer_from(ol.gaussian_bf16(0x5B10 + i, 2 * cap * 256)) for i in range(2))
+    got = {}
+    for workspace in (None, 20 << 20, 4 << 20, 0):
+        print(f"[case] wide shared walk rows {rows} base {base} workspace {workspace}", flush=True)
+        queue = dev.create_queue(workspace)
+        out = dev.buffer_from(np.full(rows * 4096, 0x7FC0, np.uint16))
+        cb = queue.create_command_buffer()
+        cb.begin_compute_pass()
+        cb.encode(lib.pipeline("attention_flash_v2_blk"), {0: b_q, 1: b_k, 2: b_v, 3: b_g, 4: out},
+                  {5: base + rows, 6: cap, 7: rows, 8: base}, (16, (rows + 15) // 16), (256,))
+        cb.end_compute_pass()
+        cb.commit().wait()
+        got[workspace] = out.read(np.uint16)
+        check_bf16(got[workspace], got[None], f"rows {rows} workspace {workspace}", max_abs=8e-3, mean_abs=2e-4,
+                   ulps=2)
+    assert not np.array_equal(got[0], got[None]), "both ran one workgroup a tile"
+
+
 def test_merged_walk_with_a_share_in_the_exact_loop():
     """As above with the shares merged by a dispatch of its own (three sharers asked, of which
     the walks of ten key tiles take two)."""
