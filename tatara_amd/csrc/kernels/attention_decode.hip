@@ -1701,8 +1701,8 @@ int32_t op_attention_combine_ms(const Bindings& b, const Grid& g, hipStream_t st
 // 3..7 rotate (as c9 of attention_decode_split_ms), bit 8 balanced (the same in both
 // dispatches: keys per workgroup by what the rows hold, at most c11; the records' order inside
 // b6 is then the walk's own, and the order of a row's fp32 sums follows from the keys of all rows
-// of the dispatch, so that a row's result may differ in the last place beside other rows), c14 records per head the deepest row is
-// expected to have (0: as many as the buffer holds; a hint that sizes the finishing
+// of the dispatch, so that a row's result may differ in the last place beside other rows), c14
+// records per head the deepest row is expected to have (0: as many as the buffer holds; a hint that sizes the finishing
 // dispatch's first batch of requests, any value gives the same result).
 struct TokenLayer {
     FlashArgs walk;

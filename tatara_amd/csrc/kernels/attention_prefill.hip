@@ -868,7 +868,8 @@ int32_t op_attention_flash_blk(const Bindings& b, const Grid& g, hipStream_t str
 // grid of attention_flash_v2_blk, plus b9 scratch and c10 splits (1..8) - the workgroups that
 // share each position tile's key walk (8: or more, see kWideFlashSplits, b9 then left alone).
 // tt_flash_prefill_splits gives the count that fills the device for a block of `rows` rows that sees
-// `visible` keys, tt_flash_prefill_scratch_bytes the bytes b9 must hold (none for one split).  Same results as attention_flash_v2_blk up to the order of fp32 sums.
+// `visible` keys, tt_flash_prefill_scratch_bytes the bytes b9 must hold (none for one split).  Same
+// results as attention_flash_v2_blk up to the order of fp32 sums.
 int32_t op_attention_flash_split_blk(const Bindings& b, const Grid& g, hipStream_t stream,
                                      bool validate_only) {
     return flash_blk(b, g, stream, validate_only, true);

@@ -267,8 +267,9 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
 // lies so far below the row's largest that f16 rounds it is off by 2^-33 of that one at most, a
 // weight by 2^-39.  The affine terms are four further columns a group, {bias, 8 scale, bias,
 // 8 scale} against {hi, hi, lo, lo} of the group sum in two f16 parts, 2^-23 of the sum at most
-// from it: the largest of these roundings, about one of the fp32 sums' own.  One pass writes both operands so into the queue's workspace; the product is
-// then a plain one (block_product.h) and the powers of two leave with the result.
+// from it: the largest of these roundings, about one of the fp32 sums' own.  One pass writes both
+// operands so into the queue's workspace; the product is then a plain one (block_product.h) and the
+// powers of two leave with the result.
 //
 // Why not unpack inside the product: a scale per 64 columns costs a product of its own from a
 // zero accumulator and 64 fused adds a lane for every 32 products, and the unpacking is

@@ -203,7 +203,7 @@ def test_token_lane_beside_shallow_and_deep_neighbours():
     the wave.  One lane of 4000 keys alone, beside shallow and beside deep lanes, against attention in
     64 bits: the bf16 result is half a step off at most (2^-8 of itself at a binade's lower end), a
     probability enters the products as two bf16 parts (2^-17 of it is dropped), and where the device's
-    cosine puts a query element one bf16 step from the checker's, a score moves by about 2^-8 / 16, so
+    cosine puts a query element one bf16 step from the oracle's, a score moves by about 2^-8 / 16, so
     an output stays within 2^-8 of itself and 2^-11 of the weighted magnitudes; and the error is no
     larger than with the split fixed by the capacity."""
     cap, context, seed = 4096, 4000, 0x8A55

@@ -272,7 +272,7 @@ def test_block_projection_in_queues_of_less_workspace(family, name, rows):
     """A queue that could not have its whole workspace takes the operands through in slices of output
     rows and of input rows (8 MiB: 768 outputs and rows at a time at the hidden width, 256 at
     the attention width): the same sums, bit for bit.  One without workspace evaluates the rows in
-    the reference's order: the checker's bits."""
+    the reference's order: the oracle's bits."""
     B, dev, _, lib = gpu()
     host, bindings = _family(dev, family, 0xA800)
     k, total = family["k"], sum(family["segments"])

@@ -333,7 +333,7 @@ def _dense_block_case(rows, in_dim, out_dim, sample_rows, seed):
     (640, 192, 1024),      # six steps: one round of the steady loop
 ], ids=["65x64x70", "257x2048x300", "300x4096x2048", "1000x2048x515", "513x128x256", "640x192x1024"])
 def test_dense_bf16_block_kernel(rows, in_dim, out_dim):
-    """Blocks of more than 16 rows take an LDS-staged product: every row against the checker,
+    """Blocks of more than 16 rows take an LDS-staged product: every row against the oracle,
     partial tiles either way (these sizes take the 32 x 64 and 64 x 64 tiles), every length of
     the K walk's lead-in and lead-out."""
     print(f"[case] dense_bf16 block rows={rows} in={in_dim} out={out_dim}", flush=True)
