@@ -329,7 +329,7 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
     };
     static constexpr Cost kCosts[] = {
-        {BlockTile::Large, 256, 256, 1530, 7500, 3060, 15000},
+        {BlockTile::Large, 256, 256, 1480, 9000, 2960, 18000},
         {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
         {BlockTile::Deep, 128, 128, 520, 2000, 1040, 4000},
         {BlockTile::Tall, 128, 64, 330, 1500, 630, 3000},
@@ -347,9 +347,9 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         // Compute units that the last round leaves idle make the others faster (they share the
         // power and the L2): one round of 256 x 256 tiles over K = 4096 takes 77 / 94 / 105 us with 64 /
         // 208 / 256 of them, two over K = 2048 104 with 392, three 159 with 576.  Fitted, the share of
-        // the last round that is saved is the idle share by 1 / (rounds + 2), or by a third for a 128 x
-        // 128 tile left over behind pairs.
-        const uint64_t idle = (c.single_unit * units + c.single_tile) * (each * compute_units - tiles) / compute_units;
+        // the last round's walk that is saved is the idle share by 1 / (rounds + 2), or by a third for
+        // a 128 x 128 tile left over behind pairs.
+        const uint64_t idle = c.single_unit * units * (each * compute_units - tiles) / compute_units;
         if (c.tile == BlockTile::Large) time -= idle / (each + 2);
         if (c.tile == BlockTile::Even && each > 1 && each % 2 == 1) time -= idle / 3;
         if (time < best_time) {
