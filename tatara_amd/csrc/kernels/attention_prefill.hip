@@ -827,11 +827,11 @@ int32_t flash_blk(const Bindings& b, const Grid& g, hipStream_t stream, bool val
     // workspace where the block is too few rows to fill the device.  So is one that is to be
     // shared by as many as can be named, among as many as fill the device.
     const uint32_t tiles = (f.rows + kTilePositions - 1) / kTilePositions;
+    const uint32_t walk_tiles = (visible + kTileKeys - 1) / kTileKeys;
     const StreamWorkspace workspace = stream_workspace(stream);
     if (workspace.base != nullptr && (!shared_walk || f.splits == kMaxFlashSplits)) {
         uint32_t planned = flash_prefill_splits(f.rows, visible, workspace.compute_units);
         if (planned == kMaxFlashSplits) {
-            const uint32_t walk_tiles = (visible + kTileKeys - 1) / kTileKeys;
             planned = std::max(planned, std::min({workspace.compute_units / (tiles * kAttnKvHeads),
                                                   walk_tiles / kMinTilesPerSplit, kWideFlashSplits}));
         }
@@ -842,6 +842,8 @@ int32_t flash_blk(const Bindings& b, const Grid& g, hipStream_t stream, bool val
             f.scratch = workspace.base;
         }
     }
+    // where even the longest walk is too short to be shared there is nothing to clear or to merge
+    if (walk_tiles < 2 * kMinTilesPerSplit) f.splits = 1;
     const dim3 grid(tiles, kAttnKvHeads, f.splits);
     if (f.splits >= kMergeSplitsFrom) {
         hipLaunchKernelGGL(attention_flash_prefill_kernel<true>, grid, dim3(kFlashWaves * 64), kFlashLdsBytes,

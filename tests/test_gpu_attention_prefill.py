@@ -209,6 +209,15 @@ def test_walk_shared_by_as_many_as_fill_the_device(rows, base):
     _prefill_case(rows, base, 8192, 0x5A80 + rows, replays=2)
 
 
+@pytest.mark.parametrize("rows,base", [(1, 0), (17, 20), (3, 252), (4, 252), (64, 192)])
+def test_sharers_of_walks_too_short_to_share(rows, base):
+    """Eight sharers asked, where a walk of eight key tiles (256 keys, the last two cases past and
+    at it) is the first that two take: shorter ones are walked by one workgroup, and the scratch
+    stays as it is."""
+    print(f"[case] sharers of a short walk, rows {rows} base {base}", flush=True)
+    _prefill_case(rows, base, 512, 0x5C00 + rows, splits=8, replays=2)
+
+
 @pytest.mark.parametrize("rows,base", [(12, 5003), (65, 4100)])
 def test_walk_shared_by_as_many_as_the_workspace_holds(rows, base):
     """The same in queues of less workspace: as many sharers as it holds (12 rows in 4 MiB: seven a
