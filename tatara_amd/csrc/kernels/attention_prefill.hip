@@ -89,9 +89,9 @@ struct FlashPrefillArgs {
 // in the register order of its lanes; the last one - told by an arrival count, nobody waits
 // for anybody - adds the others' to its own with the usual reference change and writes the
 // rows.  A walk of fewer than kMinTilesPerSplit key tiles per workgroup is shared by fewer.
-// From kMergeSplitsFrom sharers on, every workgroup leaves its result and a dispatch of many
-// workgroups merges them: the last one alone reads 270 KB per sharer at what one compute unit
-// takes in.  With that, few rows share a walk among more than the kMaxFlashSplits a caller can
+// From kMergeSplitsFrom sharers on, where tiles are few, every workgroup leaves its result and a
+// dispatch of many workgroups merges them: the last one alone reads 270 KB per sharer at what one
+// compute unit takes in.  With that, few rows share a walk among more than the kMaxFlashSplits a caller can
 // name (kWideFlashSplits), through the queue's workspace.
 constexpr uint32_t kMaxFlashSplits = 8;
 constexpr uint32_t kWideFlashSplits = 64;
@@ -845,7 +845,12 @@ int32_t flash_blk(const Bindings& b, const Grid& g, hipStream_t stream, bool val
     // where even the longest walk is too short to be shared there is nothing to clear or to merge
     if (walk_tiles < 2 * kMinTilesPerSplit) f.splits = 1;
     const dim3 grid(tiles, kAttnKvHeads, f.splits);
-    if (f.splits >= kMergeSplitsFrom) {
+    // With so many position tiles that three workgroups each are more than the device, the last of
+    // a tile merges while others walk, and a dispatch behind them all is the slower form: 2048 rows
+    // behind 3000 tokens by three 172 against 179 us, 3008 from nothing 123 / 135, 4096 184 / 215; 1536
+    // rows are level (149 / 150), 1024 by five 120 / 111.
+    const uint32_t units = workspace.compute_units != 0 ? workspace.compute_units : 256;
+    if (f.splits >= kMergeSplitsFrom && tiles * kAttnKvHeads * kMergeSplitsFrom <= units + units / 8) {
         hipLaunchKernelGGL(attention_flash_prefill_kernel<true>, grid, dim3(kFlashWaves * 64), kFlashLdsBytes,
                            stream, f);
         hipLaunchKernelGGL(flash_merge_kernel, dim3(64 * tiles, kAttnKvHeads), dim3(256), 0, stream, f);

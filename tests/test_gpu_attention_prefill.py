@@ -209,6 +209,15 @@ def test_walk_shared_by_as_many_as_fill_the_device(rows, base):
     _prefill_case(rows, base, 8192, 0x5A80 + rows, replays=2)
 
 
+@pytest.mark.parametrize("rows,splits", [(1536, 3), (1537, 3), (1537, 8), (3008, 4)])
+def test_shared_walks_merged_apart_up_to_as_many_tiles_as_fill_the_device(rows, splits):
+    """48 position tiles (on 256 compute units) are the most whose shares a dispatch of its own merges;
+    of more, the last sharer does."""
+    print(f"[case] shared walk rows {rows} splits {splits}", flush=True)
+    sample = sorted(set(range(0, rows, 97)) | {31, 32, rows - 2, rows - 1})
+    _prefill_case(rows, 700, 4096, 0x5D00 + rows, select=sample, splits=splits, replays=2)
+
+
 @pytest.mark.parametrize("rows,base", [(1, 0), (17, 20), (3, 252), (4, 252), (64, 192)])
 def test_sharers_of_walks_too_short_to_share(rows, base):
     """Eight sharers asked, where a walk of eight key tiles (256 keys, the last two cases past and
