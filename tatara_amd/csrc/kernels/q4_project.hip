@@ -111,7 +111,8 @@ __device__ __forceinline__ Q4Matrix matrix_of_row(const Q4Projection& p, uint32_
 // half wave read 512 contiguous bytes twice.  Where the tiles of the workgroups that share
 // a compute unit do not fit its LDS (kStaged = false) x is read from global memory: there
 // the workgroups per compute unit matter more than the x traffic.
-template <uint32_t kBlocks, bool kStaged>
+// kEarly: the weights are requested before the first row's pieces are stored (see launch_rows).
+template <uint32_t kBlocks, bool kStaged, bool kEarly = kStaged>
 __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
     extern __shared__ __align__(16) uint8_t rows_lds[];   // [tile rows][kBlocks][1024]
     constexpr uint32_t kPiecesPerRow = kBlocks * 64;
@@ -131,9 +132,13 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
     // the two round trips overlap (a single row, the ordinary case, is all of x)
     constexpr uint32_t kFirst = kPiecesPerRow / 256;
     u32x4 first[kFirst];
-    if (kStaged) {
+    if constexpr (kEarly) {
 #pragma unroll
         for (uint32_t j = 0; j < kFirst; ++j) first[j] = piece_of(threadIdx.x + j * 256);
+    } else if constexpr (kStaged) {
+        for (uint32_t piece = threadIdx.x; piece < tile_rows * kPiecesPerRow; piece += 256) {
+            *reinterpret_cast<u32x4*>(rows_lds + slot_of(piece)) = piece_of(piece);
+        }
     }
     // rows past the last one compute on the last row and store nothing
     const uint32_t n = min(blockIdx.x * 8 + (threadIdx.x >> 5), p.first_row[p.segments] - 1);
@@ -153,7 +158,7 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
         scale_bits[b] = scales[b * 8 + (lane >> 2)];
         bias_bits[b] = biases[b * 8 + (lane >> 2)];
     }
-    if (kStaged) {
+    if constexpr (kEarly) {
 #pragma unroll
         for (uint32_t j = 0; j < kFirst; ++j) {
             *reinterpret_cast<u32x4*>(rows_lds + slot_of(threadIdx.x + j * 256)) = first[j];
@@ -161,8 +166,8 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
         for (uint32_t piece = kPiecesPerRow + threadIdx.x; piece < tile_rows * kPiecesPerRow; piece += 256) {
             *reinterpret_cast<u32x4*>(rows_lds + slot_of(piece)) = piece_of(piece);
         }
-        __syncthreads();
     }
+    if (kStaged) __syncthreads();
     const uint16_t* x0 = p.input + static_cast<uint64_t>(row_base) * p.input_stride + lane * 16;
     float acc[kQ4BatchRowsMax];
 #pragma unroll
@@ -235,16 +240,23 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
         return tile_rows * row_bytes * resident <= kRowsStagedBytes;
     };
     switch (p.k_size / kQ4Block) {
-    // LDS: the tile's x rows where they fit kRowsStagedBytes
+    // LDS: the tile's x rows where they fit kRowsStagedBytes.  Requesting the weights before the
+    // first row is stored hides a round trip from a single row, which is all of x (gdn_project
+    // 7.2 -> 7.1 us, outproj 6.0 -> 5.8, and up to 13 rows of it by 2 to 4 %); the in-projections
+    // of 2 .. 5 rows were 1 to 2 % slower so, 16 rows of outproj 3 %.
     case 4:
-        if (staged(4096)) {
+        if (staged(4096) && tile_rows > 1) {
+            hipLaunchKernelGGL((q4_rows_kernel<4, true, false>), grid, dim3(256), tile_rows * 4096, stream, p);
+        } else if (staged(4096)) {
             hipLaunchKernelGGL((q4_rows_kernel<4, true>), grid, dim3(256), tile_rows * 4096, stream, p);
         } else {
             hipLaunchKernelGGL((q4_rows_kernel<4, false>), grid, dim3(256), 0, stream, p);
         }
         break;
     case 8:
-        if (staged(8192)) {
+        if (staged(8192) && tile_rows > 13) {
+            hipLaunchKernelGGL((q4_rows_kernel<8, true, false>), grid, dim3(256), tile_rows * 8192, stream, p);
+        } else if (staged(8192)) {
             hipLaunchKernelGGL((q4_rows_kernel<8, true>), grid, dim3(256), tile_rows * 8192, stream, p);
         } else {
             hipLaunchKernelGGL((q4_rows_kernel<8, false>), grid, dim3(256), 0, stream, p);
@@ -1029,12 +1041,10 @@ bool prepare_q4_kernels() {
                allow_wave(wave_kernel_for<true>(rows), wave_lds_bytes<4>(rows));
     };
     return Q4Tiles::each(allow) &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<4, true>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               kRowsStagedBytes) == hipSuccess &&
-           hipFuncSetAttribute(reinterpret_cast<const void*>(q4_rows_kernel<8, true>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               kRowsStagedBytes) == hipSuccess &&
+           allow_wave(q4_rows_kernel<4, true>, kRowsStagedBytes) &&
+           allow_wave(q4_rows_kernel<4, true, false>, kRowsStagedBytes) &&
+           allow_wave(q4_rows_kernel<8, true>, kRowsStagedBytes) &&
+           allow_wave(q4_rows_kernel<8, true, false>, kRowsStagedBytes) &&
            allow_rows(4) && allow_rows(8) && allow_rows(12) && allow_rows(16) &&
            allow_wave(q4_wave_kernel<8>, wave_lds_bytes<8>(16)) &&
            allow_wave(q4_wave_kernel<8, false, false, 16, true>, wave_lds_bytes<8>(16)) &&
