@@ -329,7 +329,7 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
     };
     static constexpr Cost kCosts[] = {
-        {BlockTile::Large, 256, 256, 1480, 9000, 2960, 18000},
+        {BlockTile::Large, 256, 256, 1480, 8800, 2960, 17600},
         {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
         {BlockTile::Deep, 128, 128, 520, 2000, 1040, 4000},
         {BlockTile::Tall, 128, 64, 330, 1500, 630, 3000},
