@@ -116,6 +116,16 @@ __device__ __forceinline__ void head_gates(uint16_t a_bits, uint16_t b_bits, uin
     beta = sigmoid_bf16(widen(b_bits));
 }
 
+__device__ __forceinline__ void write_gates(const uint16_t* projection, const uint16_t* a_log,
+                                            const uint16_t* dt_bias, float* decay, float* beta,
+                                            uint32_t row, uint32_t h) {
+    const uint16_t* proj = projection + static_cast<uint64_t>(row) * kGdnProjectionRows;
+    float d, b;
+    head_gates(proj[kGdnARowOffset + h], proj[kGdnBRowOffset + h], a_log[h], dt_bias[h], d, b);
+    decay[row * kGdnValueHeads + h] = d;
+    beta[row * kGdnValueHeads + h] = b;
+}
+
 // ------------------------------------------------------------ prepare/conv ---
 
 struct PrepareArgs {
@@ -133,6 +143,11 @@ struct PrepareArgs {
     uint16_t* conv_tape;          // [40][16][3][8192] window after each row, or null
     uint32_t tape_layer;
     uint32_t rows_per_group;      // block kernel: rows one workgroup walks
+    // gdn_conv_gates_blk: the rows' gates instead of the copy of z (decay null: the copy)
+    const uint16_t* a_log;
+    const uint16_t* dt_bias;
+    float* decay;                 // [rows][32]
+    float* beta;
 };
 
 constexpr uint32_t kBlockRowsPerGroup = 16;  // block mode: rows one workgroup walks
@@ -220,7 +235,16 @@ __global__ __launch_bounds__(128) void gdn_prepare_kernel(PrepareArgs a) {
 // 2..3 value heads, 4..5 the z gate copy.  Same arithmetic, operation for operation, as
 // gdn_prepare_kernel: a head's 128 squares are summed as 32 runs of four, then the
 // adjacent-pairs tree - a lane holds two runs, 16 lanes a head.
+//
+// kGates: no copy of z (the gate-norm that follows reads it where the projection left it: a third
+// of this kernel's traffic and its one part without arithmetic), and the rows' decay and beta by
+// ceil(rows / 8) workgroups in front of the others, a row's 32 heads to half a wave, instead of
+// by a dispatch of their own.  gdn_conv_blk + gdn_gates_blk
+// 3.4 + 2.4 / 4.2 + 2.5 / 13.3 + 2.5 / 24.6 + 2.6 / 172 + 4.3 us for 12 / 100 / 777 / 2048 / 16384
+// rows, this 3.3 / 4.3 / 12.5 / 24.0 / 167 (the copy cost little: the arithmetic of the rest bounds it).
 constexpr uint32_t kPrepareUnitGroups = (kCh + kGdnValueValues) / 8 / 256;
+constexpr uint32_t kConvUnitGroups = kCh / 8 / 256;
+constexpr uint32_t kGateRowsPerGroup = 256 / kGdnValueHeads;
 
 __device__ __forceinline__ float widen_half(uint32_t word, uint32_t j) {
     return __uint_as_float((j & 1) ? (word & 0xFFFF0000u) : (word << 16));
@@ -229,11 +253,24 @@ __device__ __forceinline__ uint32_t narrow_pair(float a, float b) {
     return static_cast<uint32_t>(narrow(a)) | (static_cast<uint32_t>(narrow(b)) << 16);
 }
 
+template <bool kGates>
 __global__ __launch_bounds__(256) void gdn_prepare_block_kernel(PrepareArgs a) {
-    const uint32_t unit = blockIdx.x % kPrepareUnitGroups * 256 + threadIdx.x;  // 8 channels each
-    const uint32_t row_begin = blockIdx.x / kPrepareUnitGroups * a.rows_per_group;
+    constexpr uint32_t kUnitGroups = kGates ? kConvUnitGroups : kPrepareUnitGroups;
+    uint32_t block = blockIdx.x;
+    if constexpr (kGates) {
+        const uint32_t gate_groups = (a.rows + kGateRowsPerGroup - 1) / kGateRowsPerGroup;
+        if (block < gate_groups) {
+            const uint32_t h = threadIdx.x % kGdnValueHeads;
+            const uint32_t row = block * kGateRowsPerGroup + threadIdx.x / kGdnValueHeads;
+            if (row < a.rows) write_gates(a.projection, a.a_log, a.dt_bias, a.decay, a.beta, row, h);
+            return;
+        }
+        block -= gate_groups;
+    }
+    const uint32_t unit = block % kUnitGroups * 256 + threadIdx.x;  // 8 channels each
+    const uint32_t row_begin = block / kUnitGroups * a.rows_per_group;
     const uint32_t row_end = min(a.rows, row_begin + a.rows_per_group);
-    if (unit >= kCh / 8) {
+    if (!kGates && unit >= kCh / 8) {
         const uint32_t index = (unit - kCh / 8) * 8;
         for (uint32_t row = row_begin; row < row_end; ++row) {
             *reinterpret_cast<u32x4*>(a.z + static_cast<uint64_t>(row) * a.z_stride + index) =
@@ -494,11 +531,7 @@ __global__ void gdn_gates_kernel(const uint16_t* projection, const uint16_t* a_l
     const uint32_t h = threadIdx.x;
     const uint32_t step = blockIdx.x * blockDim.y + threadIdx.y;
     if (h >= kGdnValueHeads || step >= steps) return;
-    const uint16_t* proj = projection + static_cast<uint64_t>(step) * kGdnProjectionRows;
-    float d, b;
-    head_gates(proj[kGdnARowOffset + h], proj[kGdnBRowOffset + h], a_log[h], dt_bias[h], d, b);
-    decay[step * kGdnValueHeads + h] = d;
-    beta[step * kGdnValueHeads + h] = b;
+    write_gates(projection, a_log, dt_bias, decay, beta, step, h);
 }
 
 // --------------------------------------------------------------- gate norm ---
@@ -508,8 +541,8 @@ __global__ void gdn_gates_kernel(const uint16_t* projection, const uint16_t* a_l
 // the end (gdn.metal:174-207).
 __global__ __launch_bounds__(128) void gdn_gate_norm_kernel(const uint16_t* y, const uint16_t* z,
                                                             const uint16_t* weight, uint16_t* out,
-                                                            uint32_t stride, uint32_t rows,
-                                                            uint32_t rows_per_group) {
+                                                            uint32_t stride, uint32_t z_stride,
+                                                            uint32_t rows, uint32_t rows_per_group) {
     __shared__ float partial[2];
     const uint32_t head = blockIdx.x;
     const uint32_t lane = threadIdx.x;
@@ -532,7 +565,7 @@ __global__ __launch_bounds__(128) void gdn_gate_norm_kernel(const uint16_t* y, c
         const float inverse =
             1.0f / sqrtf((partial[0] + partial[1]) / static_cast<float>(kGD) + kRmsNormEpsilon);
         const float normed = rb(w * rb(v * inverse));
-        const float g = widen(z[at]);
+        const float g = widen(z[static_cast<uint64_t>(row) * z_stride + head * kGD + lane]);
         const float low = 1.0f / (1.0f + expf(fabsf(g)));
         const float sig = g < 0.0f ? low : 1.0f - low;
         out[at] = narrow((g * sig) * normed);
@@ -543,7 +576,8 @@ __global__ __launch_bounds__(128) void gdn_gate_norm_kernel(const uint16_t* y, c
 // lanes half a row; grid 2 rows.  Same arithmetic as
 // gdn_gate_norm_kernel (two runs of four squares per lane, then the pair tree).
 __global__ __launch_bounds__(256) void gdn_gate_norm_block_kernel(
-    const uint16_t* y, const uint16_t* z, const uint16_t* weight, uint16_t* out, uint32_t stride) {
+    const uint16_t* y, const uint16_t* z, const uint16_t* weight, uint16_t* out, uint32_t stride,
+    uint32_t z_stride) {
     constexpr uint32_t kGroups = kGdnValueValues / 8 / 256;
     const uint32_t c = (blockIdx.x % kGroups * 256 + threadIdx.x) * 8;
     float w[8];
@@ -554,7 +588,8 @@ __global__ __launch_bounds__(256) void gdn_gate_norm_block_kernel(
     }
     const uint64_t at = static_cast<uint64_t>(blockIdx.x / kGroups) * stride + c;
     const u32x4 yb = *reinterpret_cast<const u32x4*>(y + at);
-    const u32x4 zb = *reinterpret_cast<const u32x4*>(z + at);
+    const u32x4 zb = *reinterpret_cast<const u32x4*>(
+        z + static_cast<uint64_t>(blockIdx.x / kGroups) * z_stride + c);
     float v[8];
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) v[j] = widen_half(yb[j >> 1], j);
@@ -1519,8 +1554,14 @@ int32_t launch_prepare(const PrepareArgs& p, hipStream_t stream) {
         const bool in_place = in < out + kWindowBytes && out < in + kWindowBytes;
         if (in_place) block.conv_out = nullptr;
         const uint32_t groups = (p.rows + block.rows_per_group - 1) / block.rows_per_group;
-        hipLaunchKernelGGL(gdn_prepare_block_kernel, dim3(kPrepareUnitGroups * groups), dim3(256), 0, stream,
-                           block);
+        if (p.decay != nullptr) {
+            const uint32_t gate_groups = (p.rows + kGateRowsPerGroup - 1) / kGateRowsPerGroup;
+            hipLaunchKernelGGL(gdn_prepare_block_kernel<true>, dim3(kConvUnitGroups * groups + gate_groups),
+                               dim3(256), 0, stream, block);
+        } else {
+            hipLaunchKernelGGL(gdn_prepare_block_kernel<false>, dim3(kPrepareUnitGroups * groups), dim3(256), 0,
+                               stream, block);
+        }
         if (in_place) hipLaunchKernelGGL(gdn_window_kernel, dim3(1), dim3(1024), 0, stream, p);
         return TT_OK;
     }
@@ -1621,6 +1662,37 @@ int32_t op_gdn_conv_blk(const Bindings& b, const Grid& g, hipStream_t stream, bo
 int32_t op_gdn_conv_tape_blk(const Bindings& b, const Grid& g, hipStream_t stream,
                              bool validate_only) {
     return conv_blk_common(b, g, stream, validate_only, true);
+}
+
+// gdn_conv_gates_blk (no reference counterpart: gdn_conv_blk without its copy of z, and
+// gdn_gates_blk, in one dispatch): b0 projection[rows][12352], b1 conv_in, b2 conv_w, b3
+// qk[rows][4096], b4 value, b5 a_log, b6 dt_bias, b7 decay[rows][32], b8 beta[rows][32], b9
+// conv_out, c10 rows; grid (64, rows) x 128.
+int32_t op_gdn_conv_gates_blk(const Bindings& b, const Grid& g, hipStream_t stream,
+                              bool validate_only) {
+    Args a(b);
+    PrepareArgs p{};
+    p.rows = a.constant(10);
+    a.require(p.rows >= 1 && g.gx == 64 && g.gy == p.rows && g.gz == 1 && g.tx == 128 &&
+                  g.ty == 1 && g.tz == 1,
+              TT_CMD_INVALID_DISPATCH_EXTENT);
+    const uint64_t rows = p.rows;
+    p.projection = a.buffer<const uint16_t>(0, rows * kGdnProjectionRows * 2);
+    p.conv_in = a.buffer<const uint16_t>(1, 3 * kCh * 2);
+    p.conv_weights = a.buffer<const uint16_t>(2, 4 * kCh * 2);
+    p.qk = a.buffer<uint16_t>(3, rows * kGdnQkValues * 2);
+    p.value = a.buffer<uint16_t>(4, rows * kGdnValueValues * 2);
+    p.a_log = a.buffer<const uint16_t>(5, kGdnValueHeads * 2);
+    p.dt_bias = a.buffer<const uint16_t>(6, kGdnValueHeads * 2);
+    p.decay = a.buffer<float>(7, rows * kGdnValueHeads * 4);
+    p.beta = a.buffer<float>(8, rows * kGdnValueHeads * 4);
+    p.conv_out = a.buffer<uint16_t>(9, 3 * kCh * 2);
+    p.projection_stride = kGdnProjectionRows;
+    p.qk_stride = kGdnQkValues;
+    p.value_stride = kGdnValueValues;
+    p.block_mode = 1;
+    if (a.status != TT_OK || validate_only) return a.status;
+    return launch_prepare(p, stream);
 }
 
 int32_t launch_recurrence(const RecurrenceArgs& r, uint32_t rows, hipStream_t stream) {
@@ -1827,25 +1899,30 @@ int32_t op_gdn_tape_replay_blk(const Bindings& b, const Grid& g, hipStream_t str
     return TT_OK;
 }
 
-int32_t gate_norm_common(Args& a, const Grid& g, uint32_t rows, uint32_t stride,
-                         hipStream_t stream, bool validate_only) {
-    const uint64_t bytes = (static_cast<uint64_t>(rows - 1) * stride + kGdnValueValues) * 2;
+// `z_column`: z is that column of rows of `z_stride` (the projection's)
+int32_t gate_norm_common(Args& a, const Grid& g, uint32_t rows, uint32_t stride, uint32_t z_stride,
+                         uint32_t z_column, hipStream_t stream, bool validate_only) {
+    const auto extent = [&](uint32_t row_stride, uint32_t columns) {
+        return (static_cast<uint64_t>(rows - 1) * row_stride + columns) * 2;
+    };
+    const uint64_t bytes = extent(stride, kGdnValueValues);
     const uint16_t* y = a.buffer<const uint16_t>(0, bytes);
-    const uint16_t* z = a.buffer<const uint16_t>(1, bytes);
+    const uint16_t* z = a.buffer<const uint16_t>(1, extent(z_stride, z_column + kGdnValueValues));
     const uint16_t* w = a.buffer<const uint16_t>(2, kGD * 2);
     uint16_t* out = a.buffer<uint16_t>(3, bytes);
     a.require(g.gx == 32 && g.gy == rows && g.gz == 1 && g.tx == 128 && g.ty == 1 && g.tz == 1,
               TT_CMD_INVALID_DISPATCH_EXTENT);
     if (a.status != TT_OK || validate_only) return a.status;
+    z += z_column;
     // blocks: 8 channels per lane, a row per group (eight rows: 100 rows 9.4 us instead of 3.0,
     // 2048 rows 15.0 instead of 12.2, 16384 rows 82 instead of 69)
     if (rows > kMaxBatchRows && stride % 8 == 0) {
         hipLaunchKernelGGL(gdn_gate_norm_block_kernel, dim3(kGdnValueValues / 8 / 256 * rows), dim3(256), 0,
-                           stream, y, z, w, out, stride);
+                           stream, y, z, w, out, stride, z_stride);
         return TT_OK;
     }
     hipLaunchKernelGGL(gdn_gate_norm_kernel, dim3(32, rows), dim3(128), 0, stream, y, z, w, out,
-                       stride, rows, 1u);
+                       stride, z_stride, rows, 1u);
     return TT_OK;
 }
 
@@ -1853,7 +1930,7 @@ int32_t gate_norm_common(Args& a, const Grid& g, uint32_t rows, uint32_t stride,
 int32_t op_gdn_gate_norm(const Bindings& b, const Grid& g, hipStream_t stream,
                          bool validate_only) {
     Args a(b);
-    return gate_norm_common(a, g, 1, kGdnValueValues, stream, validate_only);
+    return gate_norm_common(a, g, 1, kGdnValueValues, kGdnValueValues, 0, stream, validate_only);
 }
 // gdn_gate_norm_ms: + c4 value stride; grid (32, rows) x 128 (decode_step.cpp:1184-1190)
 int32_t op_gdn_gate_norm_ms(const Bindings& b, const Grid& g, hipStream_t stream,
@@ -1864,17 +1941,27 @@ int32_t op_gdn_gate_norm_ms(const Bindings& b, const Grid& g, hipStream_t stream
     a.require(stride >= kGdnValueValues && rows >= 1 && rows <= kMaxBatchRows,
               TT_CMD_INVALID_DISPATCH_EXTENT);
     if (a.status != TT_OK) return a.status;
-    return gate_norm_common(a, g, rows, stride, stream, validate_only);
+    return gate_norm_common(a, g, rows, stride, stride, 0, stream, validate_only);
 }
-// gdn_gate_norm_blk: rows from the grid; grid (32, rows) x 128 (prefill_step.cpp:2040-2050)
-int32_t op_gdn_gate_norm_blk(const Bindings& b, const Grid& g, hipStream_t stream,
-                             bool validate_only) {
+int32_t gate_norm_block(const Bindings& b, const Grid& g, hipStream_t stream, bool validate_only,
+                        uint32_t z_stride, uint32_t z_column) {
     Args a(b);
     const uint32_t rows = static_cast<uint32_t>(g.gy);
     a.require(rows >= 1 && g.gy <= 0x7fffffffull / kGdnValueValues,
               TT_CMD_INVALID_DISPATCH_EXTENT);
     if (a.status != TT_OK) return a.status;
-    return gate_norm_common(a, g, rows, kGdnValueValues, stream, validate_only);
+    return gate_norm_common(a, g, rows, kGdnValueValues, z_stride, z_column, stream, validate_only);
+}
+// gdn_gate_norm_blk: rows from the grid; grid (32, rows) x 128 (prefill_step.cpp:2040-2050)
+int32_t op_gdn_gate_norm_blk(const Bindings& b, const Grid& g, hipStream_t stream,
+                             bool validate_only) {
+    return gate_norm_block(b, g, stream, validate_only, kGdnValueValues, 0);
+}
+// gdn_gate_norm_proj_blk (no reference counterpart): gdn_gate_norm_blk with b1 the projection
+// [rows][12352], whose z columns are read in place
+int32_t op_gdn_gate_norm_proj_blk(const Bindings& b, const Grid& g, hipStream_t stream,
+                                  bool validate_only) {
+    return gate_norm_block(b, g, stream, validate_only, kGdnProjectionRows, kCh);
 }
 
 
@@ -2015,9 +2102,11 @@ const uint32_t kGdnDecodeKernelCount = sizeof(kGdnDecodeKernels) / sizeof(kGdnDe
 const KernelDesc kGdnPrefillKernels[] = {
     {"gdn_conv_blk", op_gdn_conv_blk},
     {"gdn_gates_blk", op_gdn_gates_blk},
+    {"gdn_conv_gates_blk", op_gdn_conv_gates_blk},
     {"gdn_recurrence_gates_blk", op_gdn_recurrence_gates_blk},
     {"gdn_recurrence_blk", op_gdn_recurrence_blk},
     {"gdn_gate_norm_blk", op_gdn_gate_norm_blk},
+    {"gdn_gate_norm_proj_blk", op_gdn_gate_norm_proj_blk},
     {"gdn_conv_tape_blk", op_gdn_conv_tape_blk},
     {"gdn_recurrence_gates_tape_blk", op_gdn_recurrence_gates_tape_blk},
     {"gdn_tape_replay_blk", op_gdn_tape_replay_blk},

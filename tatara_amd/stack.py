@@ -164,7 +164,7 @@ class StubStack:
         self.proj = mk(rows * GDN_PROJ * 2)
         self.mixed = mk(rows * 4096 * 2)
         self.delta = mk(rows * HIDDEN * 2)
-        self.qk, self.v, self.z, self.y = (mk(rows * 8192) for _ in range(4))
+        self.qk, self.v, self.y = (mk(rows * 8192) for _ in range(3))
         self.q, self.gate = mk(rows * 8192), mk(rows * 8192)
         self.decay, self.beta = mk(rows * 128), mk(rows * 128)
         self.partials = mk(lanes * 16 * self.max_splits * 258 * 4)
@@ -402,12 +402,11 @@ class StubStack:
                 conv_out = (layer["conv"], plane_out * CONV_ELEMS * 2)
                 rec_in = (layer["rec"], plane_in * REC_ELEMS * 4)
                 rec_out = (layer["rec"], plane_out * REC_ELEMS * 4)
-                cb.encode(P("gdn_conv_blk"),
+                # conv and gates in one dispatch, z read from the projection by the gate-norm
+                cb.encode(P("gdn_conv_gates_blk"),
                           {0: self.proj, 1: conv_in, 2: layer["conv_w"], 3: self.qk, 4: self.v,
-                           5: self.z, 6: conv_out}, {7: rows}, (96, rows), (128,))
-                cb.encode(P("gdn_gates_blk"),
-                          {0: self.proj, 1: layer["a_log"], 2: layer["dt_bias"], 3: self.decay,
-                           4: self.beta}, {5: rows}, (1, (rows + 3) // 4, 1), (32, 4, 1))
+                           5: layer["a_log"], 6: layer["dt_bias"], 7: self.decay, 8: self.beta,
+                           9: conv_out}, {10: rows}, (64, rows), (128,))
                 cb.barrier()
                 if chunked:
                     cb.encode(P("gdn_chunk_recurrence_blk"),
@@ -418,8 +417,8 @@ class StubStack:
                               {0: self.qk, 1: self.v, 2: self.decay, 3: layer["a_log"], 4: self.beta,
                                5: rec_in, 6: self.y, 7: rec_out}, {8: rows}, (1, 32, 32), (32, 4, 1))
                 cb.barrier()
-                cb.encode(P("gdn_gate_norm_blk"), {0: self.y, 1: self.z, 2: layer["norm_w"], 3: self.mixed},
-                          {}, (32, rows), (128,))
+                cb.encode(P("gdn_gate_norm_proj_blk"),
+                          {0: self.y, 1: self.proj, 2: layer["norm_w"], 3: self.mixed}, {}, (32, rows), (128,))
             else:
                 keys = (layer["keys"], lane * stripe_bytes)
                 values = (layer["values"], lane * stripe_bytes)

@@ -152,6 +152,41 @@ def test_element_wise_block_kernels_at_every_rows_per_group(rows):
     test_element_wise_block_kernels_bit_for_bit(rows)
 
 
+@pytest.mark.parametrize("in_place", [False, True], ids=["apart", "in-place"])
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 17, 513, 4097])
+def test_conv_with_gates_and_gate_norm_from_the_projection(rows, in_place):
+    """gdn_conv_gates_blk and gdn_gate_norm_proj_blk either side of the 8 rows a workgroup gates,
+    of the 16 from which the gate-norm is vectorised and at 1, 2 and 6 rows a workgroup: the
+    checker's bit patterns, and gdn_gates_blk's decay and beta bit for bit."""
+    print(f"[case] gdn conv with gates rows={rows} in place={in_place}", flush=True)
+    B, dev, queue, lib = gpu()
+    weights = _weights()
+    proj, conv_state, state = _block(rows, 0x5900 + rows)
+    ref = _oracle_block(proj, conv_state, state, weights, rows)
+    bufs = _buffers(dev, proj, conv_state, state, weights, rows)
+    run(lambda cb: _encode_front(cb, lib, bufs, rows))
+    decay, beta = bufs["decay"].read(np.float32), bufs["beta"].read(np.float32)
+    bufs["y"] = dev.buffer_from(ref["y"])
+    for name, size in (("qk", 8192), ("value", 8192), ("decay", 128), ("beta", 128)):
+        bufs[name] = dev.create_buffer(rows * size)
+    conv_out = bufs["conv_in"] if in_place else dev.create_buffer(3 * 8192 * 2)
+
+    def rec(cb):
+        cb.encode(lib.pipeline("gdn_conv_gates_blk"),
+                  {0: bufs["proj"], 1: bufs["conv_in"], 2: bufs["conv_w"], 3: bufs["qk"],
+                   4: bufs["value"], 5: bufs["a_log"], 6: bufs["dt_bias"], 7: bufs["decay"],
+                   8: bufs["beta"], 9: conv_out}, {10: rows}, (64, rows, 1), (128, 1, 1))
+        cb.encode(lib.pipeline("gdn_gate_norm_proj_blk"),
+                  {0: bufs["y"], 1: bufs["proj"], 2: bufs["norm_w"], 3: bufs["gated"]}, {},
+                  (32, rows, 1), (128, 1, 1))
+    run(rec)
+    for name in ("qk", "value", "gated"):
+        assert np.array_equal(bufs[name].read(np.uint16), ref[name]), name
+    assert np.array_equal(conv_out.read(np.uint16), ref["conv"])
+    assert np.array_equal(bufs["decay"].read(np.float32), decay)
+    assert np.array_equal(bufs["beta"].read(np.float32), beta)
+
+
 @pytest.mark.parametrize("shift", [0, 8192, -2048], ids=["same", "a-row-on", "overlapping"])
 @pytest.mark.parametrize("rows", [1, 2, 3, 12, 16, 17, 100, 600])
 def test_conv_window_written_in_place(rows, shift):
