@@ -34,6 +34,9 @@ __device__ __forceinline__ void block_transfer(const uint8_t* base, uint32_t off
                  : "memory");
 }
 
+// s_waitcnt until at most `left` (< 64) transfers are in flight
+constexpr uint32_t block_vmcnt(uint32_t left) { return 0x0F70u | (left & 15u) | ((left >> 4) << 14); }
+
 // two sums to a packed bf16 pair: hardware round to nearest even, then results below the
 // normal range flushed to signed zero
 __device__ __forceinline__ uint32_t block_pack(float a, float b) {
@@ -79,10 +82,7 @@ struct BlockProduct {
     static_assert(kXTransfers * 8 * kWaves == kTileM && kWTransfers * 8 * kWaves == kTileN,
                   "whole transfers");
 
-    // s_waitcnt until at most `left` transfers are in flight
-    static constexpr uint32_t vmcnt(uint32_t left) {
-        return 0x0F70u | (left & 15u) | ((left >> 4) << 14);
-    }
+    static constexpr uint32_t vmcnt(uint32_t left) { return block_vmcnt(left); }
     static_assert((kRing - 2) * kTransfers < 64, "what vmcnt counts");
 
     typedef __attribute__((ext_vector_type(8))) Element Elements;
@@ -322,8 +322,12 @@ enum class BlockTile { Large, Even, Deep, Tall, Small, Least };
 // two at a time where two workgroups fit it: `single` is the time of one tile alone on it, `both`
 // of two side by side, as ns per 64 columns and ns per tile (fitted to the products below and to
 // others of 33 .. 16384 rows, 2048 .. 12352 outputs and K = 2176 and 4352).
-inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
-                                   uint32_t compute_units) {
+struct BlockChoice {
+    BlockTile tile;
+    uint64_t ns;
+};
+inline BlockChoice choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
+                                     uint32_t compute_units) {
     struct Cost {
         BlockTile tile;
         uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
@@ -337,8 +341,7 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         {BlockTile::Least, 32, 64, 155, 1000, 275, 1500},
     };
     const uint64_t units = in_dim / 64;
-    BlockTile best = BlockTile::Large;
-    uint64_t best_time = ~0ull;
+    BlockChoice best{BlockTile::Large, ~0ull};
     for (const Cost& c : kCosts) {
         const uint64_t tiles = static_cast<uint64_t>((rows + c.m - 1) / c.m) * ((out_dim + c.n - 1) / c.n);
         const uint64_t each = (tiles + compute_units - 1) / compute_units;
@@ -352,10 +355,7 @@ inline BlockTile choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_
         const uint64_t idle = c.single_unit * units * (each * compute_units - tiles) / compute_units;
         if (c.tile == BlockTile::Large) time -= idle / (each + 2);
         if (c.tile == BlockTile::Even && each > 1 && each % 2 == 1) time -= idle / 3;
-        if (time < best_time) {
-            best_time = time;
-            best = c.tile;
-        }
+        if (time < best.ns) best = BlockChoice{c.tile, time};
     }
     return best;
 }
@@ -385,7 +385,7 @@ struct BlockTiles {
     // the tile a call takes, as use(product) of a value of its type
     template <typename Use>
     static auto choose(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units, Use use) {
-        switch (choose_block_tile(rows, in_dim, out_dim, compute_units)) {
+        switch (choose_block_tile(rows, in_dim, out_dim, compute_units).tile) {
         case BlockTile::Even: return use(Even{});
         case BlockTile::Deep: return use(Deep{});
         case BlockTile::Tall: return use(Tall{});

@@ -275,9 +275,9 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
 // A scale has 8 significant bits and nibble - 8 (-8 .. 7) three or a power of two, so their
 // product has at most 11: an f16 number, exactly.  So is x, of 8 bits.  Both are brought into
 // f16's range by a power of two per row (an output row's largest of 8 |scale| and |bias| below
-// 2^15, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): an x that
+// 2^14, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): an x that
 // lies so far below the row's largest that f16 rounds it is off by 2^-33 of that one at most, a
-// weight by 2^-39.  The affine terms are four further columns a group, {bias, 8 scale, bias,
+// weight by 2^-38.  The affine terms are four further columns a group, {bias, 8 scale, bias,
 // 8 scale} against {hi, hi, lo, lo} of the group sum in two f16 parts, 2^-23 of the sum at most
 // from it: the largest of these roundings, about one of the fp32 sums' own.  One pass writes both
 // operands so into the queue's workspace; the product is then a plain one (block_product.h) and the
@@ -303,12 +303,40 @@ struct Unfold {
     uint32_t weight_rows;      // 0: the weights are there already
     uint32_t first_weight;     // the output row that row 0 of `weights` is
     uint32_t first_row, x_rows;
+    bool short_rows;           // the rows' pieces in q4_short_kernel's order (unfolded_piece)
 };
 
 // the power of two that brings `largest` (a magnitude) to [2^(below - 1), 2^below)
 __device__ __forceinline__ int32_t shift_below(float largest, int32_t below) {
     const int32_t field = static_cast<int32_t>(__float_as_uint(largest) >> 23);   // no sign
     return field == 0 ? (largest == 0.0f ? 0 : below + 125) : below + 126 - field;
+}
+
+// The columns of an unfolded row stand in an order of their own, the same in both operands (a
+// product does not ask for one).  Of eight columns, in pairs: 0 and 4, 1 and 5, 2 and 6, 3 and 7 -
+// a word's nibbles come apart so with one shift and one mask a pair.  For q4_short_kernel the rows
+// of x also have the pieces of eight columns of every four units in the order 0, 4, 8 .., 1, 5,
+// 9 ..: a unit then takes one word of every 16 bytes of a weight row, so that it can load whole 16
+// bytes.  (Written in that order for the block product as well, both operands took 1 to
+// 2 us longer at 2048 rows: a store's lanes no longer fall together.)
+template <uint32_t kBlocks>
+__device__ __forceinline__ uint32_t unfolded_piece(uint32_t piece) {
+    constexpr uint32_t kSpan = kBlocks == 4 ? 64 : 128;   // pieces
+    const uint32_t within = piece % kSpan;
+    return piece - within + within % 4 * (kSpan / 4) + within / 4;
+}
+// Nibbles i and i + 4 of `word`, less 8, times the steps, exactly: a nibble in bits 6 .. 9 of
+// f16 16.0 counts units, and both (16 + nibble) step and 24 step (of 10 bits) are what the fused
+// multiply-add says they are.  A shift, a mask and an add for two weights.
+__device__ __forceinline__ f16x2 unfold_offset(f16x2 steps) {
+    return steps * f16x2{static_cast<_Float16>(-24.0f), static_cast<_Float16>(-24.0f)};
+}
+__device__ __forceinline__ uint32_t unfold_pair(uint32_t word, uint32_t i, f16x2 steps, f16x2 offset) {
+    const uint32_t there = i == 0 ? word << 6 : i == 1 ? word << 2 : i == 2 ? word >> 2 : word >> 6;
+    uint32_t sixteens = 0x4C004C00u;
+    asm("" : "+v"(sixteens));   // kept in a register: one v_and_or_b32 instead of two instructions
+    const uint32_t pair = (there & 0x03C003C0u) | sixteens;
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, pair), steps, offset));
 }
 
 // grid ceil((weight_rows + x_rows) / 4) x 256: a wave per row
@@ -336,22 +364,18 @@ __global__ __launch_bounds__(256) void q4_unfold_kernel(Q4Projection p, Unfold u
         }
 #pragma unroll
         for (uint32_t step = 8; step < 64; step *= 2) largest = fmaxf(largest, __shfl_xor(largest, step));
-        const int32_t shift = shift_below(largest, 15);
+        const int32_t shift = shift_below(largest, 14);
         if (lane == 0) u.weight_exponents[row] = -shift;
         _Float16* out = u.weights + static_cast<uint64_t>(row) * kColumns;
 #pragma unroll
         for (uint32_t b = 0; b < kBlocks; ++b) {
             const _Float16 step = static_cast<_Float16>(ldexpf(scale[b], shift));
             const f16x2 steps = f16x2{step, step};
-            const f16x2 offset = f16x2{static_cast<_Float16>(1032.0f), static_cast<_Float16>(1032.0f)};
+            const f16x2 offset = unfold_offset(steps);
             u32x4 eight;
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
-                // nibbles 2 i and 2 i + 1 as 1024 + nibble
-                const uint32_t pair = 0x64006400u | ((packed[b] >> (8 * i)) & 0xFu) |
-                                      (((packed[b] >> (8 * i + 4)) & 0xFu) << 16);
-                eight[i] = __builtin_bit_cast(uint32_t,
-                                              (__builtin_bit_cast(f16x2, pair) - offset) * steps);
+                eight[i] = unfold_pair(packed[b], i, steps, offset);
             }
             *reinterpret_cast<u32x4*>(out + b * kQ4Block + lane * 8) = eight;
             if ((lane & 7) == 0) {
@@ -384,17 +408,22 @@ __global__ __launch_bounds__(256) void q4_unfold_kernel(Q4Projection p, Unfold u
         _Float16* out = u.rows + static_cast<uint64_t>(at) * kColumns;
 #pragma unroll
         for (uint32_t b = 0; b < kBlocks; ++b) {
-            u32x4 eight;
+            float value[8];
             float sum = 0.0f;
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
-                const float low = ldexpf(widen_half(raw[b][i], 0), shift);
-                const float high = ldexpf(widen_half(raw[b][i], 1), shift);
-                sum += low + high;
-                eight[i] = __builtin_bit_cast(
-                    uint32_t, f16x2{static_cast<_Float16>(low), static_cast<_Float16>(high)});
+                value[2 * i] = ldexpf(widen_half(raw[b][i], 0), shift);
+                value[2 * i + 1] = ldexpf(widen_half(raw[b][i], 1), shift);
+                sum += value[2 * i] + value[2 * i + 1];
             }
-            *reinterpret_cast<u32x4*>(out + b * kQ4Block + lane * 8) = eight;
+            u32x4 eight;
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                eight[i] = __builtin_bit_cast(uint32_t, f16x2{static_cast<_Float16>(value[i]),
+                                                              static_cast<_Float16>(value[i + 4])});
+            }
+            const uint32_t piece = b * 64 + lane;
+            *reinterpret_cast<u32x4*>(out + (u.short_rows ? unfolded_piece<kBlocks>(piece) : piece) * 8) = eight;
 #pragma unroll
             for (uint32_t step = 1; step < 8; step *= 2) sum += __shfl_xor(sum, step);
             if ((lane & 7) == 0) {
@@ -426,6 +455,259 @@ __global__ __launch_bounds__(Product::kThreads) void q4_product_kernel(Unfold u,
                      block_store(output + static_cast<uint64_t>(u.first_row + m) * output_stride, n,
                                  out_rows, wide, sums);
                  });
+}
+
+// ------------------------------------------------------------ short blocks ---
+//
+// The same product for blocks of few rows, with the weights unpacked where they are multiplied:
+// only the rows of x are unfolded.  A workgroup of eight waves owns 32 kNWaves outputs and 16 kTm
+// rows and walks the columns in units of 32 for each of its 8 / kNWaves waves along them; a wave multiplies 32
+// outputs with all the rows over its 32 columns of every unit (as many partial sums an output, added
+// up at the end), which lets every fragment of x feed two products and every unpacked fragment of
+// weights kTm.  A lane's operand of one product is the eight nibbles of one word, and a lane's words of
+// four units are 16 bytes of a weight row (unfolded_piece): everything a workgroup needs of the
+// weights is requested at its start.  x comes through LDS as in block_product.h, a ring of units.
+// Over 2048 columns two waves share the columns' work (as many workgroups as compute units, nearly);
+// the 2048 outputs over 4096 columns are cut finer, and take half as many units.
+template <uint32_t kTm_, uint32_t kBlocks_>   // kBlocks: k_size / 512
+struct ShortProduct {
+    static constexpr uint32_t kTm = kTm_, kBlocks = kBlocks_;
+    static constexpr uint32_t kNWaves = kBlocks == 4 ? 2 : 1, kKWaves = 8 / kNWaves;
+    static constexpr uint32_t kTileM = 16 * kTm, kTileN = 32 * kNWaves;
+    static constexpr uint32_t kThreads = 512;
+    static constexpr uint32_t kUnitColumns = 32 * kKWaves, kRowBytes = 2 * kUnitColumns;
+    static constexpr uint32_t kUnitBytes = kTileM * kRowBytes;
+    static constexpr uint32_t kRing = kBlocks == 4 || kTm == 2 ? 4 : kTm == 4 ? 4 : kTm == 6 ? 3 : 2;
+    static constexpr uint32_t kExponentBytes = kTileN * 4;
+    static constexpr uint32_t kLdsBytes = kRing * kUnitBytes + kExponentBytes;
+    static constexpr uint32_t kTransfers = kUnitBytes / 1024 / 8;   // of a wave and unit
+    static_assert(kTm % 2 == 0 && kLdsBytes <= 160 * 1024);
+    // the partial sums of all eight waves take the ring's place
+    static_assert(8 * kTm * 2 * 1024 <= kRing * kUnitBytes);
+    // waves to a SIMD: 128 registers each, for a second workgroup, where that costs no spills
+    static constexpr uint32_t kWavesPerSimd = kTm <= 4 ? 4 : 2;
+};
+
+typedef u32x4 u32x4_pairs __attribute__((aligned(4)));   // scales and biases: see check_block_operands
+
+// grid (out_rows / kTileN, ceil(x_rows / kTileM))
+template <typename Product>
+__global__ __launch_bounds__(512, Product::kWavesPerSimd) void q4_short_kernel(Q4Projection p, Unfold u) {
+    constexpr uint32_t kTm = Product::kTm, kBlocks = Product::kBlocks;
+    constexpr uint32_t kGroups = kBlocks * 8;
+    constexpr uint32_t kUnitColumns = Product::kUnitColumns;
+    constexpr uint32_t kAffineUnits = kGroups * kAffineColumns / kUnitColumns;
+    constexpr uint32_t kSpans = kBlocks * kQ4Block / kUnitColumns / 4;   // of four units, 16 bytes a lane
+    static_assert(kAffineUnits == 1 && kSpans == 4);
+    constexpr uint32_t kUnits = kSpans * 4 + kAffineUnits;
+    constexpr uint32_t kRowBytes = unfolded_columns(kBlocks * kQ4Block) * 2;
+    constexpr uint32_t kTransfers = Product::kTransfers;
+    constexpr uint32_t kRing = Product::kRing;
+    constexpr uint32_t kPieces = kUnitColumns / 8;   // of a unit's row
+    typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+    extern __shared__ __align__(16) uint8_t short_lds[];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t i16 = lane & 15, g = lane >> 4;
+    const uint32_t nw = wave % Product::kNWaves, kh = wave / Product::kNWaves;
+    const uint32_t first_out = blockIdx.x * Product::kTileN;
+    const uint32_t m0 = blockIdx.y * Product::kTileM;
+    const uint32_t lds_base = static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)short_lds));
+
+    // In a row of the ring, one row's unit, the 16-byte piece c sits in slot c ^ (row & 15), so
+    // that the sixteen rows of a fragment read fall on different banks.
+    const uint8_t* x = reinterpret_cast<const uint8_t*>(u.rows);
+    uint32_t x_offset[kTransfers];
+#pragma unroll
+    for (uint32_t t = 0; t < kTransfers; ++t) {
+        const uint32_t row = (wave * kTransfers + t) * (64 / kPieces) + lane / kPieces;
+        x_offset[t] = min(m0 + row, u.x_rows - 1) * kRowBytes + (lane % kPieces ^ (row & 15)) * 16;
+    }
+    const auto request = [&](uint32_t unit) __attribute__((always_inline)) {
+        // the affine columns first: their operand is not kept
+        const uint32_t column = unit < kAffineUnits ? kBlocks * kQ4Block : (unit - kAffineUnits) * kUnitColumns;
+#pragma unroll
+        for (uint32_t t = 0; t < kTransfers; ++t) {
+            block_transfer(x + column * 2, x_offset[t],
+                           lds_base + unit % kRing * Product::kUnitBytes +
+                               (wave * kTransfers + t) * 1024);
+        }
+    };
+
+    // Scales and biases: of all the row's groups for its exponent (a quarter by each g), those of the
+    // affine operand.
+    u32x4 words[2][kSpans];
+    u32x4 scale_bits[2][kBlocks / 4], bias_bits[2][kBlocks / 4];
+    uint32_t affine_scale[2], affine_bias[2];
+    const uint32_t* word_rows[2];
+#pragma unroll
+    for (uint32_t tn = 0; tn < 2; ++tn) {
+        const uint32_t n = first_out + nw * 32 + tn * 16;   // every matrix has a multiple of 16 rows
+        const Q4Matrix matrix = matrix_of_row(p, n);
+        const uint64_t local = n + i16 - matrix.first_row;
+        word_rows[tn] = matrix.words + local * (kBlocks * 64) + (4 * kh + g) * 4;
+        const uint16_t* scales = matrix.scales + local * kGroups;
+        const uint16_t* biases = matrix.biases + local * kGroups;
+#pragma unroll
+        for (uint32_t i = 0; i < kBlocks / 4; ++i) {
+            scale_bits[tn][i] = *reinterpret_cast<const u32x4_pairs*>(scales + g * (kGroups / 4) + i * 8);
+            bias_bits[tn][i] = *reinterpret_cast<const u32x4_pairs*>(biases + g * (kGroups / 4) + i * 8);
+        }
+        affine_scale[tn] = *reinterpret_cast<const uint32_t*>(scales + kh * 8 + g * 2);
+        affine_bias[tn] = *reinterpret_cast<const uint32_t*>(biases + kh * 8 + g * 2);
+    }
+#pragma unroll
+    for (uint32_t unit = 0; unit < kRing - 1; ++unit) request(unit);
+#pragma unroll
+    for (uint32_t span = 0; span < kSpans; ++span) {
+#pragma unroll
+        for (uint32_t tn = 0; tn < 2; ++tn) {
+            words[tn][span] = *reinterpret_cast<const u32x4*>(word_rows[tn] + span * (kUnitColumns / 2));
+        }
+    }
+
+    int32_t shift[2];
+#pragma unroll
+    for (uint32_t tn = 0; tn < 2; ++tn) {
+        float largest = 0.0f;
+#pragma unroll
+        for (uint32_t i = 0; i < kBlocks; ++i) {
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j) {
+                largest = fmaxf(largest, 8.0f * fabsf(widen_half(scale_bits[tn][i >> 2][i & 3], j)));
+                largest = fmaxf(largest, fabsf(widen_half(bias_bits[tn][i >> 2][i & 3], j)));
+            }
+        }
+        largest = fmaxf(largest, __shfl_xor(largest, 16));
+        largest = fmaxf(largest, __shfl_xor(largest, 32));
+        shift[tn] = shift_below(largest, 14);
+        if (kh == 0 && g == 0) {
+            *reinterpret_cast<int32_t*>(short_lds + kRing * Product::kUnitBytes +
+                                        (nw * 32 + tn * 16 + i16) * 4) = -shift[tn];
+        }
+    }
+    // the step of span s: of its groups the one of number 2 kh + (g >> 1), all held by lane group s
+    f16x2 steps[2][kSpans], offsets[2][kSpans];
+#pragma unroll
+    for (uint32_t tn = 0; tn < 2; ++tn) {
+        const u32x4 held = scale_bits[tn][kBlocks == 4 ? 0 : kh >> 2];
+        const uint32_t at = kh & 3;
+        const uint32_t mine = at == 0 ? held[0] : at == 1 ? held[1] : at == 2 ? held[2] : held[3];
+#pragma unroll
+        for (uint32_t span = 0; span < kSpans; ++span) {
+            const uint32_t pair =
+                static_cast<uint32_t>(__shfl(static_cast<int>(mine), span * 16 + i16));
+            const _Float16 step = static_cast<_Float16>(ldexpf(widen_half(pair, g >> 1), shift[tn]));
+            steps[tn][span] = f16x2{step, step};
+            offsets[tn][span] = unfold_offset(steps[tn][span]);
+        }
+    }
+
+    f32x4 acc[2][kTm];
+#pragma unroll
+    for (uint32_t tn = 0; tn < 2; ++tn) {
+#pragma unroll
+        for (uint32_t tm = 0; tm < kTm; ++tm) acc[tn][tm] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const uint32_t fragment = i16 * Product::kRowBytes + ((4 * kh + g) ^ i16) * 16;
+    const auto step = [&](uint32_t unit, const f16x8 (&w)[2]) __attribute__((always_inline)) {
+        const uint8_t* at = short_lds + unit % kRing * Product::kUnitBytes + fragment;
+#pragma unroll
+        for (uint32_t tm = 0; tm < kTm; ++tm) {
+            const f16x8 rows = *reinterpret_cast<const f16x8*>(at + tm * 16 * Product::kRowBytes);
+#pragma unroll
+            for (uint32_t tn = 0; tn < 2; ++tn) {
+                acc[tn][tm] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[tn], rows, acc[tn][tm], 0, 0, 0);
+            }
+        }
+    };
+    // Unit `unit` has landed, mine, then everybody's, and nobody reads the one before it: the unit
+    // after the last requested takes its place.  (At most kRing - 2 units were requested after
+    // `unit`; whatever else is in flight only makes the wait longer.)
+    const auto arrive = [&](uint32_t unit) __attribute__((always_inline)) {
+        if (unit + kRing - 1 <= kUnits) {
+            __builtin_amdgcn_s_waitcnt(block_vmcnt((kRing - 2) * kTransfers));
+        } else {
+            __builtin_amdgcn_s_waitcnt(block_vmcnt(0));
+        }
+        __syncthreads();
+        if (unit + kRing - 1 < kUnits) request(unit + kRing - 1);
+    };
+    const auto affine = [&](f16x8 (&w)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t tn = 0; tn < 2; ++tn) {
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j) {
+                const _Float16 first =
+                    static_cast<_Float16>(ldexpf(widen_half(affine_bias[tn], j), shift[tn]));
+                const _Float16 second =
+                    static_cast<_Float16>(ldexpf(widen_half(affine_scale[tn], j), shift[tn] + 3));
+                w[tn][4 * j] = w[tn][4 * j + 2] = first;
+                w[tn][4 * j + 1] = w[tn][4 * j + 3] = second;
+            }
+        }
+    };
+    // the operand of a unit: affine columns, or a word of the span it is of
+    const auto unpack = [&](uint32_t unit, f16x8 (&w)[2]) __attribute__((always_inline)) {
+        if (unit < kAffineUnits) {
+            affine(w);
+            return;
+        }
+        const uint32_t span = (unit - kAffineUnits) / 4, j = (unit - kAffineUnits) % 4;
+#pragma unroll
+        for (uint32_t tn = 0; tn < 2; ++tn) {
+            u32x4 eight;
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                eight[i] = unfold_pair(words[tn][span][j], i, steps[tn][span], offsets[tn][span]);
+            }
+            w[tn] = __builtin_bit_cast(f16x8, eight);
+        }
+    };
+    f16x8 w[2][2];
+    unpack(0, w[0]);
+#pragma unroll
+    for (uint32_t unit = 0; unit < kUnits; ++unit) {
+        arrive(unit);
+        if (unit + 1 < kUnits) unpack(unit + 1, w[(unit + 1) & 1]);   // beside the products
+        step(unit, w[unit & 1]);
+    }
+
+    // the partial sums of every output, in the ring's place: [kh][nw][tm][tn][lane]
+    __syncthreads();
+    f32x4* partial = reinterpret_cast<f32x4*>(short_lds) + lane;
+    const auto place = [&](uint32_t part, uint32_t tm, uint32_t tn) {
+        return (((part * Product::kNWaves + nw) * kTm + tm) * 2 + tn) * 64;
+    };
+#pragma unroll
+    for (uint32_t tm = 0; tm < kTm; ++tm) {
+#pragma unroll
+        for (uint32_t tn = 0; tn < 2; ++tn) partial[place(kh, tm, tn)] = acc[tn][tm];
+    }
+    __syncthreads();
+    const bool wide = ((reinterpret_cast<uintptr_t>(p.output) | (p.output_stride * 2)) & 7) == 0;
+    const uint32_t out_rows = p.first_row[p.segments];
+    // of the 2 kTm fragments of its outputs a wave finishes every kKWaves-th
+#pragma unroll
+    for (uint32_t f = 0; f < 2 * kTm; f += Product::kKWaves) {
+        if (f + kh >= 2 * kTm) break;
+        const uint32_t tm = (f + kh) >> 1, tn = (f + kh) & 1;
+        f32x4 sums = partial[place(0, tm, tn)];
+#pragma unroll
+        for (uint32_t part = 1; part < Product::kKWaves; ++part) sums += partial[place(part, tm, tn)];
+        const uint32_t m = m0 + tm * 16 + i16;
+        if (m >= u.x_rows) continue;
+        typedef __attribute__((ext_vector_type(4))) int32_t Exponents;
+        const uint32_t column = nw * 32 + tn * 16 + g * 4;
+        const Exponents exponents = *reinterpret_cast<const Exponents*>(
+            short_lds + kRing * Product::kUnitBytes + column * 4);
+        const int32_t row_exponent = u.row_exponents[m];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) sums[j] = ldexpf(sums[j], row_exponent + exponents[j]);
+        block_store(p.output + static_cast<uint64_t>(u.first_row + m) * p.output_stride, first_out + column,
+                    out_rows, wide, sums);
+    }
 }
 
 // What the pass assumes of its operands beyond their sizes: 16-byte pieces of x (and of the
@@ -461,6 +743,59 @@ static_assert(static_cast<uint64_t>(kHidden) * unfolded_columns(kGdnValueValues)
                   static_cast<uint64_t>(kGdnProjectionRows) * unfolded_columns(kHidden),
               "the output projection's weights fit as well");
 
+// The row tile of a short block with the shortest estimate, and that estimate: ns of a launch, a
+// fixed part and one per workgroup of a compute unit, fitted to 17 .. 777 rows.  gdn_project_blk /
+// attn_project_blk / outproj_blk with unfolding, before (weights written out, block product) and now:
+// 17 rows 24.4 / 26.4 / 25.3 -> 12.7 / 12.6 / 14.7 us, 100 rows 28.1 / 30.6 / 26.7 -> 20 / 19.5 / 15.4,
+// 256 rows 36.4 / 35.3 / 26.6 -> 35.8 / 29.3 / 20.3, 300 rows 51.8 / 37.1 / 28.6 -> 37 / 29.6 / 25.2; from
+// about 400 rows on (outproj 350) the weights written out once are as fast or faster.  What bounds it: at 100
+// rows of gdn_project the x rows' unfolding and two launches 5.5 us, the weights' arrival 3, the products
+// and the barrier of each unit 7 (4 of them on the matrix unit), the partial sums 2.
+struct ShortChoice {
+    uint32_t tm;
+    uint64_t ns;
+};
+inline ShortChoice choose_short_tile(uint32_t rows, uint32_t k_size, uint32_t out_rows, uint32_t compute_units) {
+    struct Cost {
+        uint32_t tm, fixed[2], each[2];   // over 2048 and 4096 columns
+    };
+    static constexpr Cost kCosts[] = {
+        {2, {3200, 1500}, {5200, 8500}},
+        {4, {3500, 0}, {7000, 13500}},
+        {6, {500, 0}, {12600, 18000}},
+        {8, {1800, 0}, {14200, 23000}},
+    };
+    const uint32_t deep = k_size > kHidden ? 1 : 0;
+    ShortChoice best{0, ~0ull};
+    for (const Cost& c : kCosts) {
+        const uint64_t groups = static_cast<uint64_t>((rows + 16 * c.tm - 1) / (16 * c.tm)) * (out_rows / (deep ? 32 : 64));
+        const uint64_t ns = c.fixed[deep] + (groups + compute_units - 1) / compute_units * c.each[deep];
+        if (ns < best.ns) best = ShortChoice{c.tm, ns};
+    }
+    return best;
+}
+// use(product) of a short block's tile
+template <uint32_t kBlocks, typename Use>
+void short_product(uint32_t tm, Use use) {
+    switch (tm) {
+    case 2: use(ShortProduct<2, kBlocks>{}); break;
+    case 4: use(ShortProduct<4, kBlocks>{}); break;
+    case 6: use(ShortProduct<6, kBlocks>{}); break;
+    default: use(ShortProduct<8, kBlocks>{}); break;
+    }
+}
+template <uint32_t kBlocks>
+void launch_short(const Q4Projection& p, const Unfold& u, uint32_t tm, hipStream_t stream) {
+    hipLaunchKernelGGL(q4_unfold_kernel<kBlocks>, dim3((u.x_rows + 3) / 4), dim3(256), 0, stream, p, u);
+    short_product<kBlocks>(tm, [&](auto product) {
+        typedef decltype(product) Product;
+        hipLaunchKernelGGL(q4_short_kernel<Product>,
+                           dim3(p.first_row[p.segments] / Product::kTileN,
+                                (u.x_rows + Product::kTileM - 1) / Product::kTileM),
+                           dim3(Product::kThreads), Product::kLdsBytes, stream, p, u);
+    });
+}
+
 typedef BlockTiles<_Float16> Q4Tiles;
 int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
     const StreamWorkspace workspace = stream_workspace(stream);
@@ -487,6 +822,21 @@ int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
     u.weight_exponents = reinterpret_cast<int32_t*>(workspace.base + unfolded_bytes);
     u.row_exponents = reinterpret_cast<int32_t*>(
         reinterpret_cast<uint8_t*>(u.weight_exponents) + kWeightExponentBytes);
+    // what writing the weights out takes, 5 bytes a ns, is spared where each row tile unpacks its own
+    const ShortChoice brief = choose_short_tile(p.rows, p.k_size, out_rows, workspace.compute_units);
+    if (brief.ns < choose_block_tile(p.rows, columns, out_rows, workspace.compute_units).ns +
+                       static_cast<uint64_t>(out_rows) * columns * 2 / 5000) {
+        u.short_rows = true;
+        for (; u.first_row < p.rows; u.first_row += u.x_rows) {
+            u.x_rows = std::min(slice, p.rows - u.first_row);
+            if (p.k_size == 4 * kQ4Block) {
+                launch_short<4>(p, u, brief.tm, stream);
+            } else {
+                launch_short<8>(p, u, brief.tm, stream);
+            }
+        }
+        return TT_OK;
+    }
     for (; u.first_weight < out_rows; u.first_weight += weight_slice) {
         const uint32_t columns_out = std::min(weight_slice, out_rows - u.first_weight);
         u.weight_rows = columns_out;
@@ -1040,7 +1390,19 @@ bool prepare_q4_kernels() {
         return allow_wave(wave_kernel_for<false>(rows), wave_lds_bytes<4>(rows)) &&
                allow_wave(wave_kernel_for<true>(rows), wave_lds_bytes<4>(rows));
     };
-    return Q4Tiles::each(allow) &&
+    bool short_allowed = true;
+    const auto allow_short = [&](auto product) {
+        typedef decltype(product) Product;
+        short_allowed = short_allowed &&
+                        hipFuncSetAttribute(reinterpret_cast<const void*>(q4_short_kernel<Product>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            Product::kLdsBytes) == hipSuccess;
+    };
+    for (const uint32_t tm : {2u, 4u, 6u, 8u}) {
+        short_product<4>(tm, allow_short);
+        short_product<8>(tm, allow_short);
+    }
+    return short_allowed && Q4Tiles::each(allow) &&
            allow_wave(q4_rows_kernel<4, true>, kRowsStagedBytes) &&
            allow_wave(q4_rows_kernel<4, true, false>, kRowsStagedBytes) &&
            allow_wave(q4_rows_kernel<8, true>, kRowsStagedBytes) &&

@@ -267,6 +267,15 @@ def test_block_projection_against_64_bit_sums_over_the_whole_range(family, name,
 
 @pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
                                          (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
+@pytest.mark.parametrize("rows", [32, 33, 64, 66, 96, 97, 128, 130, 200, 385, 420])
+def test_block_projection_with_the_weights_unpacked_in_the_product(family, name, rows):
+    """Either side of the row tiles of 32, 64, 96 and 128 that short blocks are multiplied in, one
+    and several of them, against the 64-bit sums and with the bound above."""
+    test_block_projection_against_64_bit_sums_over_the_whole_range(family, name, rows)
+
+
+@pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
+                                         (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
 @pytest.mark.parametrize("rows", [17, 300, 1500])
 def test_block_projection_in_queues_of_less_workspace(family, name, rows):
     """A queue that could not have its whole workspace takes the operands through in slices of output
