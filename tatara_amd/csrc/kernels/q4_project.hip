@@ -112,7 +112,11 @@ __device__ __forceinline__ Q4Matrix matrix_of_row(const Q4Projection& p, uint32_
 // a compute unit do not fit its LDS (kStaged = false) x is read from global memory: there
 // the workgroups per compute unit matter more than the x traffic.
 // kEarly: the weights are requested before the first row's pieces are stored (see launch_rows).
-template <uint32_t kBlocks, bool kStaged, bool kEarly = kStaged>
+// kRowsMax: input rows of a tile this instantiation takes at most.  A single row has one of its own:
+// in sixteen rows' code its instructions lie a row's apart, and a kernel of a few us waits for each
+// fresh cache line of them (gdn_project / attn_project / gdn_outproj of one row 8.0 / 7.0 / 6.4 ->
+// 6.8 / 5.9 / 4.5 us; 31 and 57 KB of code -> 3 and 5).
+template <uint32_t kBlocks, bool kStaged, bool kEarly = kStaged, uint32_t kRowsMax = kQ4BatchRowsMax>
 __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
     extern __shared__ __align__(16) uint8_t rows_lds[];   // [tile rows][kBlocks][1024]
     constexpr uint32_t kPiecesPerRow = kBlocks * 64;
@@ -163,15 +167,16 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
         for (uint32_t j = 0; j < kFirst; ++j) {
             *reinterpret_cast<u32x4*>(rows_lds + slot_of(threadIdx.x + j * 256)) = first[j];
         }
-        for (uint32_t piece = kPiecesPerRow + threadIdx.x; piece < tile_rows * kPiecesPerRow; piece += 256) {
+        for (uint32_t piece = kPiecesPerRow + threadIdx.x; kRowsMax > 1 && piece < tile_rows * kPiecesPerRow;
+             piece += 256) {
             *reinterpret_cast<u32x4*>(rows_lds + slot_of(piece)) = piece_of(piece);
         }
     }
     if (kStaged) __syncthreads();
     const uint16_t* x0 = p.input + static_cast<uint64_t>(row_base) * p.input_stride + lane * 16;
-    float acc[kQ4BatchRowsMax];
+    float acc[kRowsMax];
 #pragma unroll
-    for (uint32_t r = 0; r < kQ4BatchRowsMax; ++r) acc[r] = 0.0f;
+    for (uint32_t r = 0; r < kRowsMax; ++r) acc[r] = 0.0f;
 #pragma unroll
     for (uint32_t b = 0; b < kBlocks; ++b) {
         float wq[16];   // masked, never shifted
@@ -187,8 +192,8 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
         const float bias = widen(bias_bits[b]);
         const uint8_t* xk = rows_lds + b * 1024 + lane * 16;
 #pragma unroll
-        for (uint32_t r = 0; r < kQ4BatchRowsMax; ++r) {
-            if (r < tile_rows) {
+        for (uint32_t r = 0; r < kRowsMax; ++r) {
+            if (kRowsMax == 1 || r < tile_rows) {
                 u32x4 lo, hi;
                 if (kStaged) {
                     lo = *reinterpret_cast<const u32x4*>(xk + r * (kPiecesPerRow * 16));
@@ -217,8 +222,8 @@ __global__ __launch_bounds__(256) void q4_rows_kernel(Q4Projection p) {
         }
     }
 #pragma unroll
-    for (uint32_t r = 0; r < kQ4BatchRowsMax; ++r) {
-        if (r < tile_rows) {
+    for (uint32_t r = 0; r < kRowsMax; ++r) {
+        if (kRowsMax == 1 || r < tile_rows) {
             const float total = half_wave_sum(acc[r]);
             if (lane == 0 && stores) {
                 p.output[static_cast<uint64_t>(row_base + r) * p.output_stride + n] = store16(total);
@@ -248,7 +253,7 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
         if (staged(4096) && tile_rows > 1) {
             hipLaunchKernelGGL((q4_rows_kernel<4, true, false>), grid, dim3(256), tile_rows * 4096, stream, p);
         } else if (staged(4096)) {
-            hipLaunchKernelGGL((q4_rows_kernel<4, true>), grid, dim3(256), tile_rows * 4096, stream, p);
+            hipLaunchKernelGGL((q4_rows_kernel<4, true, true, 1>), grid, dim3(256), tile_rows * 4096, stream, p);
         } else {
             hipLaunchKernelGGL((q4_rows_kernel<4, false>), grid, dim3(256), 0, stream, p);
         }
@@ -256,6 +261,8 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
     case 8:
         if (staged(8192) && tile_rows > 13) {
             hipLaunchKernelGGL((q4_rows_kernel<8, true, false>), grid, dim3(256), tile_rows * 8192, stream, p);
+        } else if (staged(8192) && tile_rows == 1) {
+            hipLaunchKernelGGL((q4_rows_kernel<8, true, true, 1>), grid, dim3(256), 8192, stream, p);
         } else if (staged(8192)) {
             hipLaunchKernelGGL((q4_rows_kernel<8, true>), grid, dim3(256), tile_rows * 8192, stream, p);
         } else {
@@ -1403,7 +1410,6 @@ bool prepare_q4_kernels() {
         short_product<8>(tm, allow_short);
     }
     return short_allowed && Q4Tiles::each(allow) &&
-           allow_wave(q4_rows_kernel<4, true>, kRowsStagedBytes) &&
            allow_wave(q4_rows_kernel<4, true, false>, kRowsStagedBytes) &&
            allow_wave(q4_rows_kernel<8, true>, kRowsStagedBytes) &&
            allow_wave(q4_rows_kernel<8, true, false>, kRowsStagedBytes) &&
