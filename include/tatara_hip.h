@@ -343,13 +343,18 @@ uint32_t tt_choose_split_keys(const uint32_t* visible_keys, uint32_t rows, uint3
 uint32_t tt_flash_prefill_splits(uint32_t rows, uint32_t visible_keys, uint32_t compute_units);
 uint64_t tt_flash_prefill_scratch_bytes(uint32_t rows, uint32_t splits);
 
-/* The tile with which dense_bf16 (and the 4-bit blocks, in_dim then being the columns of their
- * unfolded operands, 17/16 of the input width) multiplies a block of more than 16 rows on that
+/* The tile, of six, with which dense_bf16 (and the 4-bit blocks, in_dim then being the columns of
+ * their unfolded operands, 17/16 of the input width) multiplies a block of more than 16 rows on that
  * many compute units: 0 256 x 256, 1 128 x 128 (two workgroups a compute unit), 2 128 x 128
- * (one), 3 128 x 64, 4 64 x 64, 5 32 x 64 rows x outputs.  For tests and measurements; the results
- * do not depend on it. */
+ * (one), 3 128 x 64, 4 64 x 64, 5 32 x 64 rows x outputs.  From 1024 columns on another shape takes
+ * its place where it fills the rounds of the compute units better: tt_block_product_shape gives the
+ * one that is launched, its rows in the upper 16 bits and its outputs in the lower.  (4-bit blocks of
+ * up to about 400 rows are not multiplied by these tiles at all.)  For tests and measurements; the
+ * results do not depend on it. */
 uint32_t tt_block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                uint32_t compute_units);
+uint32_t tt_block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
+                                uint32_t compute_units);
 
 #ifdef __cplusplus
 }

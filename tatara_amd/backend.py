@@ -34,6 +34,7 @@ EXPORTED_SYMBOLS = [
     "tt_event_create", "tt_event_destroy", "tt_encode_signal_event", "tt_encode_wait_for_event",
     "tt_split_workgroups", "tt_choose_split_keys",
     "tt_flash_prefill_splits", "tt_flash_prefill_scratch_bytes", "tt_block_product_tile",
+    "tt_block_product_shape",
 ]
 
 
@@ -112,6 +113,7 @@ def lib():
         "tt_choose_split_keys": (u32, [C.POINTER(u32), u32, u32]),
         "tt_flash_prefill_splits": (u32, [u32, u32, u32]),
         "tt_block_product_tile": (u32, [u32] * 4),
+        "tt_block_product_shape": (u32, [u32] * 4),
         "tt_flash_prefill_scratch_bytes": (u64, [u32, u32]),
         "tt_event_create": (i32, [vp, pvp]), "tt_event_destroy": (None, [vp]),
         "tt_encode_signal_event": (i32, [vp, vp, u64]),
@@ -503,9 +505,15 @@ BLOCK_TILES = ("256x256", "128x128", "128x128-deep", "128x64", "64x64", "32x64")
 
 
 def block_product_tile(rows, in_dim, out_dim, compute_units=256):
-    """The tile (a name of BLOCK_TILES, rows x outputs) that a block product of that size is
-    multiplied with (tt_block_product_tile)."""
+    """The tile of the six of BLOCK_TILES (rows x outputs) that a block product of that size is
+    multiplied with, unless a refined shape takes its place (tt_block_product_tile)."""
     return BLOCK_TILES[lib().tt_block_product_tile(int(rows), int(in_dim), int(out_dim), int(compute_units))]
+
+
+def block_product_shape(rows, in_dim, out_dim, compute_units=256):
+    """(rows, outputs) of the tile that is launched (tt_block_product_shape)."""
+    shape = lib().tt_block_product_shape(int(rows), int(in_dim), int(out_dim), int(compute_units))
+    return shape >> 16, shape & 0xFFFF
 
 
 def flash_prefill_splits(rows, visible_keys, compute_units=256):

@@ -76,11 +76,16 @@ struct BlockProduct {
     static constexpr uint32_t kLdsBytes = kRing * kUnitBytes;
     static constexpr uint32_t kWaveM = kTileM / kWavesM, kWaveN = kTileN / kWavesN;
     static constexpr uint32_t kTm = kWaveM / 16, kTn = kWaveN / 16;
-    static constexpr uint32_t kXTransfers = kTileM / 8 / kWaves, kWTransfers = kTileN / 8 / kWaves;
     static_assert(kLdsBytes <= 160 * 1024, "the ring fits a compute unit");
-    static constexpr uint32_t kTransfers = kXTransfers + kWTransfers;
-    static_assert(kXTransfers * 8 * kWaves == kTileM && kWTransfers * 8 * kWaves == kTileN,
-                  "whole transfers");
+    // A unit is kTileM + kTileN rows in transfers of eight.  Where both operands' divide among the
+    // waves, a wave has its share of either, known when this is compiled (the 256 x 256 tile took 2 %
+    // longer without that); other tiles deal them in runs of both, and what is over repeats the last.
+    static constexpr uint32_t kXTransfers = kTileM / 8, kAllTransfers = (kTileM + kTileN) / 8;
+    static constexpr bool kEvenShares = kXTransfers % kWaves == 0 && kAllTransfers % kWaves == 0;
+    static constexpr uint32_t kTransfers = (kAllTransfers + kWaves - 1) / kWaves;   // of a wave
+    static_assert(kXTransfers * 8 == kTileM && kAllTransfers * 8 == kTileM + kTileN &&
+                      kTm * 16 * kWavesM == kTileM && kTn * 16 * kWavesN == kTileN,
+                  "whole transfers and fragments");
 
     static constexpr uint32_t vmcnt(uint32_t left) { return block_vmcnt(left); }
     static_assert((kRing - 2) * kTransfers < 64, "what vmcnt counts");
@@ -120,14 +125,12 @@ struct BlockProduct {
             reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)block_lds));
         const uint32_t wave_n = wave % kWavesN, wave_m = wave / kWavesN;
 
-        // staging roles: the x transfers of wave w fill rows 8 kXTransfers w + 8 j .. + 7, the
-        // weight transfers likewise; lane l lands in row + (l >> 3), slot l & 7, so it fetches
-        // piece (l & 7) ^ (l >> 3) of that row
+        // staging roles: transfer t fills rows 8 t .. 8 t + 7, those of x and then those of the
+        // weights; lane l lands in row + (l >> 3), slot l & 7, so it fetches piece (l & 7) ^ (l >> 3)
+        // of that row
         const uint8_t* x_base = reinterpret_cast<const uint8_t*>(x);
         const uint8_t* w_base = reinterpret_cast<const uint8_t*>(weights);
         const uint32_t piece = ((lane & 7) ^ (lane >> 3)) * 16;
-        const uint32_t x_row = 8 * kXTransfers * wave + (lane >> 3);
-        const uint32_t w_row = 8 * kWTransfers * wave + (lane >> 3);
         const uint32_t row_bytes = in_dim * 2;
         // Tiles are numbered along bands of eight tile rows, down a band's columns first, so that
         // a run of consecutive numbers is a compact patch (32 of them: eight rows x four columns,
@@ -139,9 +142,12 @@ struct BlockProduct {
             m0 = (8 * band + within % band_rows) * kTileM;
             n0 = (within / band_rows) * kTileN;
         };
-        // Transfer `index` of `unit`: of x, then of the weights.  Lane offsets are bytes from the
-        // tile's first row, clamped to the last row that is there (both carry `piece`).
-        const uint32_t x_lane = x_row * row_bytes + piece, w_lane = w_row * row_bytes + piece;
+        // This wave's transfer `index` of `unit`.  Lane offsets are bytes from the tile's first row
+        // of its operand, clamped to the last row that is there (both carry `piece`).
+        constexpr uint32_t kXShare = kEvenShares ? kXTransfers / kWaves : 0, kWShare = kTransfers - kXShare;
+        const uint32_t lane_offset = (lane >> 3) * row_bytes + piece;
+        const uint32_t x_lane = lane_offset + 8 * kXShare * wave * row_bytes;
+        const uint32_t w_lane = lane_offset + 8 * kWShare * wave * row_bytes;
         uint32_t x_last = 0, w_last = 0;
         const uint8_t *x_tile = nullptr, *w_tile = nullptr;   // the tile the requests go to
         auto aim = [&](uint32_t tile) {
@@ -154,13 +160,19 @@ struct BlockProduct {
         };
         auto request_one = [&](uint32_t unit, uint32_t index) __attribute__((always_inline)) {
             const uint32_t to = lds_base + (unit % kRing) * kUnitBytes;
-            if (index < kXTransfers) {
+            if constexpr (!kEvenShares) {
+                const uint32_t t = min(kTransfers * wave + index, kAllTransfers - 1);
+                const bool of_x = t < kXTransfers;
+                const uint32_t first = (of_x ? t : t - kXTransfers) * 8 * row_bytes;
+                block_transfer((of_x ? x_tile : w_tile) + unit * kRowBytes,
+                               min(lane_offset + first, of_x ? x_last : w_last), to + t * 8 * kRowBytes);
+            } else if (index < kXShare) {
                 block_transfer(x_tile + unit * kRowBytes, min(x_lane + 8 * index * row_bytes, x_last),
-                               to + (8 * kXTransfers * wave + 8 * index) * kRowBytes);
+                               to + (8 * kXShare * wave + 8 * index) * kRowBytes);
             } else {
-                const uint32_t j = index - kXTransfers;
+                const uint32_t j = index - kXShare;
                 block_transfer(w_tile + unit * kRowBytes, min(w_lane + 8 * j * row_bytes, w_last),
-                               to + kXUnitBytes + (8 * kWTransfers * wave + 8 * j) * kRowBytes);
+                               to + kXUnitBytes + (8 * kWShare * wave + 8 * j) * kRowBytes);
             }
         };
         auto request = [&](uint32_t unit) {
@@ -246,16 +258,17 @@ struct BlockProduct {
             multiply(second, bool_constant<true>{}, unit + 1, 0, first_of_next, with_request, unit + kRing);
         };
 
-        // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own:
-        // in a whole round the workgroups of an XCD (b / 8 = 0, 1, ...) take a run of consecutive
-        // tiles together - the operand panels a patch shares are then fetched into one L2 once
-        // instead of into several.  A round that is not filled is dealt in dispatch order, which
-        // spreads its tiles over the XCDs and their compute units.
-        const uint32_t by_xcd = gridDim.x % 8 == 0
-                                    ? (blockIdx.x & 7) * (gridDim.x / 8) + (blockIdx.x >> 3)
-                                    : blockIdx.x;
+        // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own: of
+        // a round's tiles, filled or not, the workgroups of an XCD (b / 8 = 0, 1, ...) take a run of
+        // consecutive ones - the operand panels a patch shares are then fetched into one L2 once
+        // instead of into several.  (Only for whole rounds of a multiple of eight workgroups, and
+        // otherwise in dispatch order: 777 x 2048 x 12352, one round of 245 tiles, 49 us instead of 39.5, and
+        // 1000 x 2048 x 9216 53 instead of 40; 300 x 2048 x 12352, 256 and 35 tiles, 33 instead of 26.)
+        const uint32_t xcd = blockIdx.x & 7;
         auto of_round = [&](uint32_t first) {
-            return first + (first + gridDim.x <= tiles ? by_xcd : blockIdx.x);
+            const uint32_t count = min(gridDim.x, tiles - min(first, tiles));
+            const uint32_t share = count / 8, more = count % 8, at = blockIdx.x >> 3;
+            return at < share + (xcd < more ? 1 : 0) ? first + xcd * share + min(xcd, more) + at : tiles;
         };
         uint32_t round = 0, tile = of_round(0);
         if (tile >= tiles) return;
@@ -316,23 +329,41 @@ struct BlockProduct {
     }
 };
 
-enum class BlockTile { Large, Even, Deep, Tall, Small, Least };
+enum class BlockTile { Large, Even, Deep, Tall, Small, Least, Wide, Seven, Five };
+
+struct BlockCost {
+    BlockTile tile;
+    uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
+};
+struct BlockChoice {
+    BlockTile tile;
+    uint32_t m, n;
+    uint64_t ns;
+};
 
 // The tile with the shortest estimate.  A compute unit takes ceil(tiles / compute_units) tiles,
 // two at a time where two workgroups fit it: `single` is the time of one tile alone on it, `both`
 // of two side by side, as ns per 64 columns and ns per tile (fitted to the products below and to
 // others of 33 .. 16384 rows, 2048 .. 12352 outputs and K = 2176 and 4352).
-struct BlockChoice {
-    BlockTile tile;
-    uint64_t ns;
-};
+inline uint64_t block_ns(const BlockCost& c, uint32_t rows, uint32_t in_dim, uint32_t out_dim,
+                         uint32_t compute_units) {
+    const uint64_t units = in_dim / 64;
+    const uint64_t tiles = static_cast<uint64_t>((rows + c.m - 1) / c.m) * ((out_dim + c.n - 1) / c.n);
+    const uint64_t each = (tiles + compute_units - 1) / compute_units;
+    const uint64_t time = each / 2 * (c.both_unit * units + c.both_tile) +
+                          each % 2 * (c.single_unit * units + c.single_tile);
+    // Compute units that the last round leaves idle make the others faster (they share the
+    // power and the L2): one round of 256 x 256 tiles over K = 4096 takes 77 / 94 / 105 us with 64 /
+    // 208 / 256 of them, two over K = 2048 104 with 392, three 159 with 576.  Fitted, the share of
+    // the last round's walk that is saved is the idle share by 1 / (rounds + 2), or by a third for
+    // a 128 x 128 tile left over behind pairs.
+    const uint64_t idle = c.single_unit * units * (each * compute_units - tiles) / compute_units;
+    if (c.n >= 256) return time - idle / (each + 2);
+    return c.tile == BlockTile::Even && each > 1 && each % 2 == 1 ? time - idle / 3 : time;
+}
 inline BlockChoice choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                      uint32_t compute_units) {
-    struct Cost {
-        BlockTile tile;
-        uint32_t m, n, single_unit, single_tile, both_unit, both_tile;
-    };
-    static constexpr Cost kCosts[] = {
+    static constexpr BlockCost kCosts[] = {
         {BlockTile::Large, 256, 256, 1480, 8800, 2960, 17600},
         {BlockTile::Even, 128, 128, 600, 2000, 920, 4000},
         {BlockTile::Deep, 128, 128, 520, 2000, 1040, 4000},
@@ -340,24 +371,37 @@ inline BlockChoice choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t ou
         {BlockTile::Small, 64, 64, 200, 1000, 400, 2000},
         {BlockTile::Least, 32, 64, 155, 1000, 275, 1500},
     };
-    const uint64_t units = in_dim / 64;
-    BlockChoice best{BlockTile::Large, ~0ull};
-    for (const Cost& c : kCosts) {
-        const uint64_t tiles = static_cast<uint64_t>((rows + c.m - 1) / c.m) * ((out_dim + c.n - 1) / c.n);
-        const uint64_t each = (tiles + compute_units - 1) / compute_units;
-        uint64_t time = each / 2 * (c.both_unit * units + c.both_tile) +
-                        each % 2 * (c.single_unit * units + c.single_tile);
-        // Compute units that the last round leaves idle make the others faster (they share the
-        // power and the L2): one round of 256 x 256 tiles over K = 4096 takes 77 / 94 / 105 us with 64 /
-        // 208 / 256 of them, two over K = 2048 104 with 392, three 159 with 576.  Fitted, the share of
-        // the last round's walk that is saved is the idle share by 1 / (rounds + 2), or by a third for
-        // a 128 x 128 tile left over behind pairs.
-        const uint64_t idle = c.single_unit * units * (each * compute_units - tiles) / compute_units;
-        if (c.tile == BlockTile::Large) time -= idle / (each + 2);
-        if (c.tile == BlockTile::Even && each > 1 && each % 2 == 1) time -= idle / 3;
-        if (time < best.ns) best = BlockChoice{c.tile, time};
+    BlockChoice best{BlockTile::Large, 0, 0, ~0ull};
+    for (const BlockCost& c : kCosts) {
+        const uint64_t ns = block_ns(c, rows, in_dim, out_dim, compute_units);
+        if (ns < best.ns) best = BlockChoice{c.tile, c.m, c.n, ns};
     }
     return best;
+}
+// Where 256 x 256 leaves a round short (or 128 x 128 takes its place for that) another height or a
+// wider tile may fill the rounds better.  Taken where its estimate is 3 % shorter, which is what
+// the estimates are good for, and from 1024 columns on: they were fitted to 2048 and more.
+inline BlockChoice refine_block_tile(BlockChoice choice, uint32_t rows, uint32_t in_dim, uint32_t out_dim,
+                                     uint32_t compute_units) {
+    static constexpr BlockCost kCosts[] = {
+        {BlockTile::Wide, 256, 288, 1800, 10500, 3600, 21000},
+        {BlockTile::Seven, 224, 256, 1370, 8000, 2740, 16000},
+        {BlockTile::Five, 160, 256, 1130, 5000, 2260, 10000},
+    };
+    if (in_dim < 1024) return choice;
+    uint64_t bar = choice.ns - choice.ns * 3 / 100;
+    for (const BlockCost& c : kCosts) {
+        const uint64_t ns = block_ns(c, rows, in_dim, out_dim, compute_units);
+        if (ns < bar) {
+            choice = BlockChoice{c.tile, c.m, c.n, ns};
+            bar = ns;
+        }
+    }
+    return choice;
+}
+inline BlockChoice block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
+    return refine_block_tile(choose_block_tile(rows, in_dim, out_dim, compute_units), rows, in_dim, out_dim,
+                             compute_units);
 }
 // The tiles a block product is launched with.  What bounds one is how the products of the two
 // to four waves of a SIMD fill each other's waits, and the power (Large, 8192 x 4352 x 2048: matrix unit
@@ -367,7 +411,10 @@ inline BlockChoice choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t ou
 //          1.33 PFLOP/s.  Eight waves of 128 x 64: sixteen of 64 x 64 read a third more and were 2
 //          to 5 % slower at every size (785 / 575 / 114; bf16 operands, 16384 x 2048 x 12352 /
 //          9216 and 16384 x 4096 x 2048: 697 / 502 / 197 against 729 / 529 / 204)
-//   Even   2048 x 2176 x 9216: 92 us; Large 103, Deep 97, Tall 106
+//   Wide   2048 x 2176 x 9216, one round of 256 tiles: 71 us; Even 91, Large 112; 8192 rows 290, Large 313
+//   Seven  2048 x 2176 x 12352: 109 us; Large 112, Wide 127; 3000 x 2176 x 9216 112, Large 119, Even 125
+//   Five   777 x 2048 x 12352, one round of 245 tiles: 39.5 us; 4096 x 2176 x 12352 217, Large 243
+//   Even   300 x 2048 x 12352: 26 us; Tall 33
 //   Deep   2048 x 4352 x 2048: 38 us; Even 48, Large 81
 //   Tall   100 x 2176 x 12352: 13.5 us; Deep 17, Small 20 (as 64 x 128, 19)
 //          777 x 4352 x 2048: 24 us; Deep 30, Even 43
@@ -381,23 +428,31 @@ struct BlockTiles {
     typedef BlockProduct<Element, 128, 64, 4, 2, 3> Tall;
     typedef BlockProduct<Element, 64, 64, 2, 2, 4> Small;
     typedef BlockProduct<Element, 32, 64, 2, 2, 4> Least;
+    // where 256 x 256 leaves a round short: other heights and a wider one
+    typedef BlockProduct<Element, 256, 288, 4, 2> Wide;
+    typedef BlockProduct<Element, 224, 256, 2, 4> Seven;
+    typedef BlockProduct<Element, 160, 256, 2, 4, 3> Five;
 
     // the tile a call takes, as use(product) of a value of its type
     template <typename Use>
     static auto choose(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units, Use use) {
-        switch (choose_block_tile(rows, in_dim, out_dim, compute_units).tile) {
+        switch (block_tile(rows, in_dim, out_dim, compute_units).tile) {
         case BlockTile::Even: return use(Even{});
         case BlockTile::Deep: return use(Deep{});
         case BlockTile::Tall: return use(Tall{});
         case BlockTile::Small: return use(Small{});
         case BlockTile::Least: return use(Least{});
+        case BlockTile::Wide: return use(Wide{});
+        case BlockTile::Seven: return use(Seven{});
+        case BlockTile::Five: return use(Five{});
         default: return use(Large{});
         }
     }
     // use(product) of every tile, as long as it says true
     template <typename Use>
     static bool each(Use use) {
-        return use(Large{}) && use(Even{}) && use(Deep{}) && use(Tall{}) && use(Small{}) && use(Least{});
+        return use(Large{}) && use(Even{}) && use(Deep{}) && use(Tall{}) && use(Small{}) && use(Least{}) &&
+               use(Wide{}) && use(Seven{}) && use(Five{});
     }
 };
 

@@ -366,6 +366,10 @@ int32_t op_add_bf16(const Bindings& b, const Grid& g, hipStream_t stream, bool v
 uint32_t block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
     return static_cast<uint32_t>(choose_block_tile(rows, in_dim, out_dim, std::max(compute_units, 1u)).tile);
 }
+uint32_t block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
+    const BlockChoice choice = block_tile(rows, in_dim, out_dim, std::max(compute_units, 1u));
+    return choice.m << 16 | choice.n;
+}
 
 #if !defined(__HIP_DEVICE_COMPILE__)  // host-side table of launchers
 const KernelDesc kStackStepKernels[] = {

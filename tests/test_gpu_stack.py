@@ -13,7 +13,7 @@ import pytest
 
 import oracle_lib as ol
 from gpu_util import gpu, run
-from test_host_rules import DENSE_TILE_CASES
+from test_host_rules import DENSE_TILE_CASES, REFINED_TILE_CASES
 
 pytestmark = pytest.mark.gpu
 o = ol.oracle
@@ -350,6 +350,20 @@ def test_dense_bf16_block_tiles(tile, rows, in_dim, out_dim):
     sample = sorted({r for r in (0, 15, 16, 31, 32, 63, 64, 65, rows // 2, rows - 2, rows - 1) if r < rows} |
                     {r for r in range(127, rows, 640)} | {r for r in range(128, rows, 640)})
     got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB111 + rows)
+    assert not np.any((got & 0x7F80) == 0x7F80), "an output was not stored"
+
+
+@pytest.mark.parametrize("shape,rows,in_dim,out_dim", REFINED_TILE_CASES, ids=lambda v: str(v))
+def test_dense_bf16_refined_tiles(shape, rows, in_dim, out_dim):
+    """The tiles that fill the rounds better, at their edges: sampled rows against the checker,
+    every output stored."""
+    print(f"[case] dense_bf16 tile {shape} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    B, dev, queue, lib = gpu()
+    assert B.block_product_shape(rows, in_dim, out_dim, dev.compute_units) == shape
+    height = shape[0]
+    sample = sorted({0, 15, 16, rows // 2, rows - 2, rows - 1} | set(range(height - 1, rows, 2 * height)) |
+                    set(range(height, rows, 2 * height)))
+    got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB222 + rows)
     assert not np.any((got & 0x7F80) == 0x7F80), "an output was not stored"
 
 

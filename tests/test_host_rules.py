@@ -108,3 +108,29 @@ def test_block_tile_where_it_was_measured(rows, in_dim, out_dim, tile):
     assert B.block_product_tile(rows, in_dim, out_dim, 256) == tile
     for units in (0, 1, 64, 304):
         assert B.block_product_tile(rows, in_dim, out_dim, units) in B.BLOCK_TILES
+
+
+# (shape, rows, in_dim, out_dim) of the dense_bf16 blocks that tests/test_gpu_stack.py runs on the tiles
+# that fill the rounds better: one and two rounds, remainders of rows and outputs, an odd number of
+# units, output rows that are not 8-byte aligned.
+REFINED_TILE_CASES = [
+    ((256, 288), 2048, 2048, 9216), ((256, 288), 2047, 1088, 9213),
+    ((224, 256), 1000, 1024, 12349), ((224, 256), 2049, 2048, 12352), ((224, 256), 3000, 2048, 9214),
+    ((160, 256), 777, 1088, 12350), ((160, 256), 790, 2048, 11000), ((160, 256), 1590, 1024, 12352)]
+
+
+@pytest.mark.parametrize("shape,rows,in_dim,out_dim", REFINED_TILE_CASES, ids=lambda v: str(v))
+def test_refined_shape_of_the_cases(shape, rows, in_dim, out_dim):
+    from tatara_amd import backend as B
+    assert B.block_product_shape(rows, in_dim, out_dim, 256) == shape
+    for units in (0, 1, 64, 304):
+        assert B.block_product_shape(rows, in_dim, out_dim, units)[0] in (32, 64, 128, 160, 224, 256)
+
+
+@pytest.mark.parametrize("rows,in_dim,out_dim,shape", [
+    (16384, 2048, 12352, (256, 256)), (100, 2048, 12352, (128, 64)), (2048, 4096, 2048, (128, 128)),
+    (640, 960, 12352, (128, 128)),       # under 1024 columns the six tiles only
+])
+def test_shape_is_the_basic_tile_where_no_other_fills_better(rows, in_dim, out_dim, shape):
+    from tatara_amd import backend as B
+    assert B.block_product_shape(rows, in_dim, out_dim, 256) == shape
