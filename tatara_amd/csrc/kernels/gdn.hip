@@ -820,45 +820,53 @@ __global__ __launch_bounds__(kThreads) void gdn_decode_fused_kernel(FusedDecodeA
 // The reference walks a block token by token (prefill_gdn.metal:204-281).  The
 // same recurrence is evaluated here 64 tokens at a time so that its products run
 // on MFMA.  With g_t the product of the decays up to token t inside a chunk,
-// L[t][s] = beta_t (g_t/g_s)(k_t.k_s) for s < t and A[t][s] = (g_t/g_s)(q_t.k_s)
-// for s <= t, the per-token deltas u_t of the delta rule satisfy
-//     (I + L) U = beta o (V - (g o K) S0^T)
-// so with Wk = (I+L)^-1 (beta o g o K) and Wv = (I+L)^-1 (beta o V):
-//     U  = Wv - Wk S0^T
-//     Y  = (g o Q) S0^T + A U
-//     S' = g_C S0 + U^T ((g_C/g) o K)
-// Stage 1 (parallel over chunks and heads) builds Wk, Wv, g o Q, (g_C/g) o K and
-// A for every chunk: the k.k and q.k Gram tiles on MFMA, the unit-triangular
-// solve by forward substitution in fp32 (one right-hand-side column per thread).
-// Stage 2 walks the chunks in order, one workgroup per (value head, 32-wide
-// slice of the value dimension), with the fp32 state slice held in MFMA
-// accumulators and every product on v_mfma_f32_16x16x32_bf16.
+// L[t][s] = beta_t (g_t/g_s)(k_t.k_s) for s < t, A[t][s] = (g_t/g_s)(q_t.k_s) for s <= t and
+// T = (I + L)^-1, the per-token deltas u_t of the delta rule satisfy
+//     (I + L) U = beta o (V - (g o K) S0^T) = R,   U = T R
+// so that a chunk is, from the state S0 it starts with,
+//     R  = beta o (V - g o (K S0^T))
+//     Y  = g o (Q S0^T) + (A T) R
+//     S'^T = g_C S0^T + (K^T ((g_C/g) o T)) R
+// Stage 1 (parallel over chunks and heads) builds A T and K^T ((g_C/g) o T): the k.k and q.k Gram
+// tiles, the unit-triangular inverse and the two products on MFMA.  Stage 2 walks the chunks
+// in order, one workgroup per (value head, 16-wide slice of the value dimension), with the fp32
+// state slice held in MFMA accumulators and every product on v_mfma_f32_16x16x32_bf16.
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 constexpr uint32_t kChunk = 64;
 // per (chunk, head) record, byte offsets.  Everything that feeds the recurrent
 // state or the output keeps fp32-grade precision: bf16 MFMA operands that are
-// not exact already are stored as hi/lo pairs, Wv in fp32 (it is only added).
+// not exact already are stored as hi/lo pairs.
 // Operands are stored in the order stage 2 consumes them: one 1 KiB fragment per
 // wave-level load (64 lanes x 16 B, lane = 16 g + m), so every load instruction
 // of stage 2 reads whole cache lines.
-//   token-by-key operands (Wk hi, Wk lo, Q): fragment (token tile w, key step kk),
-//     lane (m, g) = token 16w+m, keys 32kk+8g..+7
-//   K^T: fragment (key tile 2w+mt, token step k2), lane = key 16(2w+mt)+m, tokens 32k2+8g..+7
-//   A hi/lo: fragment (token tile w, token step k2), lane = token 16w+m, tokens 32k2+8g..+7
-//   Wv (fp32): fragment (value slice of 16, token tile w), lane = value 16 slice+m, tokens 16w+4g..+3
-constexpr uint32_t kRecWkHi = 0;
-constexpr uint32_t kRecWkLo = 16384;
-constexpr uint32_t kRecQ = 32768;
-constexpr uint32_t kRecKt = 49152;
-constexpr uint32_t kRecAqkHi = 65536;
-constexpr uint32_t kRecAqkLo = 73728;
-constexpr uint32_t kRecWv = 81920;
-constexpr uint32_t kRecRatio = 114688;                  // f32  [64]: g_C / g_t
-constexpr uint32_t kRecGam = 114944;                    // f32  [64]: g_t
-constexpr uint32_t kRecGamma = 115200;                  // f32: g_C
+//   K^T ((g_C/g) o T) hi/lo: fragment (key tile, token step k2), lane = key 16 tile + m
+//   A T hi/lo: fragment (token tile w, token step k2), lane = token 16w+m (k2 = 1 of tiles 0 and 1
+//     is zero and neither written nor read)
+// and of a lane's eight tokens the first four are 32k2+4g..+3, the others 32k2+16+4g..+3: the rows a
+// lane holds of two result tiles, so that results are stored as operands without changing lanes.
+constexpr uint32_t kRecKtHi = 0;
+constexpr uint32_t kRecKtLo = 16384;
+constexpr uint32_t kRecAtHi = 32768;
+constexpr uint32_t kRecAtLo = 40960;
+constexpr uint32_t kRecGam = 49152;                     // f32  [64]: g_t
+constexpr uint32_t kRecBeta = 49408;                    // f32  [64]: beta_t
+constexpr uint32_t kRecGamma = 49664;                   // f32: g_C
+constexpr uint32_t kRecV = 49920;   // bf16: (value slice of 16, token tile w), lane = value 16 slice+m, tokens 16w+4g..+3
+constexpr uint32_t kRecordBytes = kRecV + kChunk * kGD * 2;
+// behind a chunk's 32 records, per key head: its keys and queries, the same fragments of both value
+// heads: (token tile w, key step kk), lane (m, g) = token 16w+m, keys 32kk+8g..+7.  (Read where they
+// are, rows 8 KiB apart all came from one or two of an L2's channels, and from memory: the scan took half
+// as long again.)
+constexpr uint32_t kKeyRecK = 0;
+constexpr uint32_t kKeyRecQ = 16384;
+constexpr uint32_t kKeyRecBytes = 32768;
+constexpr uint32_t kChunkKeys = kGdnValueHeads * kRecordBytes;
+constexpr uint32_t kChunkRecords = kChunkKeys + kGdnKeyHeads * kKeyRecBytes;
+// what a caller binds, per chunk and head
 constexpr uint32_t kRecBytes = 115712;
+static_assert(kRecordBytes % 256 == 0 && kChunkRecords <= kGdnValueHeads * kRecBytes);
 
 struct ChunkPrepareArgs {
     const uint16_t* qk;      // [rows][4096]
@@ -907,73 +915,54 @@ __device__ __forceinline__ void split8(const float* x, bf16x8& hi, bf16x8& lo) {
     lo = __builtin_bit_cast(bf16x8, u32x4{l[0], l[1], l[2], l[3]});
 }
 
-// A wave's 16 x 16 MFMA result tile (this lane: rows 4g+i of column m) as bf16 hi/lo
-// pairs into fragment order: through a per-wave LDS tile so that every lane ends
-// up with eight consecutive columns of one row and stores 16 bytes; lanes 0..31
-// write the hi fragment piece, lanes 32..63 the lo piece, 512 contiguous bytes each.
-// `piece` is the byte offset of the tile's 512-byte run inside a fragment array.
-__device__ __forceinline__ void store_tile_hi_lo(uint16_t (*tile)[16][24], const f32x4 acc,
-                                                 uint32_t lane, uint8_t* hi_base, uint8_t* lo_base,
-                                                 uint32_t piece) {
-    const uint32_t m = lane & 15;
-    const uint32_t g = lane >> 4;
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-        const uint16_t hi = narrow(acc[i]);
-        tile[0][g * 4 + i][m] = hi;
-        tile[1][g * 4 + i][m] = narrow(acc[i] - widen(hi));
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const uint32_t half = lane >> 5;
-    const uint32_t row = lane & 15;
-    const uint32_t group = (lane >> 4) & 1;  // which run of eight columns
-    const u32x4 v = *reinterpret_cast<const u32x4*>(&tile[half][row][group * 8]);
-    *reinterpret_cast<u32x4*>((half ? lo_base : hi_base) + piece + (group * 16 + row) * 16) = v;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // Stage 1, grid (chunks, 32) x 256: decay products, Gram tiles on MFMA, the
 // inverse T of the unit lower-triangular I + L (diagonal 16x16 blocks by forward
-// substitution in registers, the rest by block recursion, all fp32), then
-// [Wk | Wv] = T (beta o [g o K | V]) on MFMA with hi/lo operands.
-__global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs a) {
+// substitution in registers, the rest by block recursion, all fp32), then A T and
+// K^T ((g_C/g) o T) on MFMA, both as their transposes: a lane then holds runs of the tokens that
+// stage 2 contracts over, and stores them as they are.
+//
+// 2048 rows (1024 workgroups, four to a compute unit): 25 us.  Formerly [Wk | Wv] = T (beta o [g o K | V]), A, K and Q were stored, 115,712
+// bytes a record through staging tiles in LDS: 41 us, 16 us for the two chunks of 100 rows (now 9).
+// Precision: a pair of bf16 parts is good for 2^-17.  (g_C/g) o T goes into its product in three parts,
+// so that the state sees two such roundings a chunk, of this product and of R, as it did before (of
+// T and of the deltas): state against 64 bits, 1000 rows, 3.6e-6 -> 3.4e-6 (with two parts and without the
+// product of the low parts in stage 2 4.8e-6).
+__global__ __launch_bounds__(256, 4) void gdn_chunk_prepare_kernel(ChunkPrepareArgs a) {
     constexpr uint32_t kLd = 68;  // fp32 row stride: 16-byte aligned, bank-skewed
-    constexpr uint32_t kTileLd = 136;  // bf16 row stride of the key and value tiles
-    constexpr uint32_t kStripLd = 72;  // 64 rows + pad: 16-byte reads of 16 columns spread over the banks
+    constexpr uint32_t kTileLd = 136;  // bf16 row stride of the key tile
+    constexpr uint32_t kStripLd = 68;  // 64 rows + pad: 8-byte reads of 16 columns spread over the banks
+    // L, then T
     __shared__ __attribute__((aligned(16))) float lower[kChunk][kLd];
     // inverses of the four 16x16 diagonal blocks of I + L: tdiag[16 b + r][c]
     __shared__ __attribute__((aligned(16))) float tdiag[kChunk][20];
-    // per wave: a 16-column strip of the solution as bf16 hi/lo, [half][column][row]
-    // (rows 0..47 the finished block rows, 48..63 the right-hand side being solved),
-    // rows contiguous so that a lane reads its 8 contraction slots with 16 bytes; the
-    // same memory stages the 16x16 result tiles on their way to the record
-    __shared__ __attribute__((aligned(16))) uint16_t strip[4][2][16][kStripLd];
     __shared__ __attribute__((aligned(16))) float log_g[kChunk];
-    __shared__ __attribute__((aligned(16))) float scale_k[kChunk];  // beta_t g_t
     __shared__ __attribute__((aligned(16))) float scale_v[kChunk];  // beta_t
-    // the head's keys and values of the chunk, row-major [token][128], rows padded to
-    // 272 bytes so that 16-byte operand reads of 16 rows spread over the banks
+    __shared__ __attribute__((aligned(16))) float ratio_g[kChunk];  // g_C / g_t
+    // the head's keys of the chunk, row-major [token][128], rows padded to
+    // 272 bytes so that 16-byte operand reads of 16 rows spread over the banks; then its values; then,
+    // per wave, a 16-column strip of the solution as bf16 hi/lo, [half][column][row] (rows 0..47
+    // the finished block rows, 48..63 the right-hand side being solved), rows contiguous.  (Each
+    // with memory of its own, three workgroups fit a compute unit instead of four.)
     __shared__ __attribute__((aligned(16))) uint16_t ktile[kChunk][kTileLd];
-    __shared__ __attribute__((aligned(16))) uint16_t vtile[kChunk][kTileLd];
+    uint16_t (*strip)[2][16][kStripLd] = reinterpret_cast<uint16_t (*)[2][16][kStripLd]>(&ktile[0][0]);
+    static_assert(4 * 2 * 16 * kStripLd <= kChunk * kTileLd);
     const uint32_t chunk = blockIdx.x;
     const uint32_t h = blockIdx.y;
     const uint32_t kh = h >> 1;
     const uint32_t tid = threadIdx.x;
-    const uint32_t wave = tid >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lane = tid & 63;
     const uint32_t m = lane & 15;
     const uint32_t g = lane >> 4;
     const uint32_t t0 = chunk * kChunk;
     const uint32_t valid = min(kChunk, a.rows - t0);
-    uint8_t* rec = a.scratch + (static_cast<uint64_t>(chunk) * kGdnValueHeads + h) * kRecBytes;
+    uint8_t* records = a.scratch + static_cast<uint64_t>(chunk) * kChunkRecords;
+    uint8_t* rec = records + h * kRecordBytes;
+    uint8_t* key_rec = records + kChunkKeys + kh * kKeyRecBytes;
 
-    // Keys and values of the chunk into LDS with 16-byte loads: 16 lanes per row, 16
-    // rows per pass; rows past the block repeat the last one (their scales are zero).
+    // Keys of the chunk into LDS with 16-byte loads: 16 lanes per row, 16
+    // rows per pass; rows past the block repeat the last one (their betas are zero).
     // The wave's query rows (token rows 16w .. 16w+15) are requested with them.
-    const bool is_k = wave < 2;
     bf16x8 aq[4];
     {
         const uint16_t* qrow = a.qk + static_cast<uint64_t>(t0 + min(wave * 16 + m, valid - 1)) * kGdnQkValues +
@@ -981,10 +970,11 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
 #pragma unroll
         for (uint32_t kk = 0; kk < 4; ++kk) aq[kk] = operand(qrow + kk * 32 + g * 8);
     }
+    u32x4 vv[4];
     {
         const uint16_t* ksrc = a.qk + static_cast<uint64_t>(t0) * kGdnQkValues + kGdnKOffset + kh * kGD;
         const uint16_t* vsrc = a.value + static_cast<uint64_t>(t0) * kGdnValueValues + h * kGD;
-        u32x4 kv[4], vv[4];
+        u32x4 kv[4];
 #pragma unroll
         for (uint32_t pass = 0; pass < 4; ++pass) {
             const uint32_t r = min(pass * 16 + (tid >> 4), valid - 1);
@@ -996,7 +986,6 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
 #pragma unroll
         for (uint32_t pass = 0; pass < 4; ++pass) {
             *reinterpret_cast<u32x4*>(&ktile[pass * 16 + (tid >> 4)][(tid & 15) * 8]) = kv[pass];
-            *reinterpret_cast<u32x4*>(&vtile[pass * 16 + (tid >> 4)][(tid & 15) * 8]) = vv[pass];
         }
     }
 
@@ -1013,50 +1002,90 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
             if (lane >= off) lg += up;
         }
         log_g[tid] = lg;
-        scale_k[tid] = b * __expf(lg);
         scale_v[tid] = b;
         const float log_gc = __shfl(lg, kChunk - 1, 64);
-        reinterpret_cast<float*>(rec + kRecRatio)[tid] = __expf(log_gc - lg);
+        ratio_g[tid] = __expf(log_gc - lg);
         reinterpret_cast<float*>(rec + kRecGam)[tid] = __expf(lg);
+        reinterpret_cast<float*>(rec + kRecBeta)[tid] = b;
         if (tid == kChunk - 1) *reinterpret_cast<float*>(rec + kRecGamma) = __expf(lg);
     }
     __syncthreads();
 
+    // Wave w: rows 16w .. 16w+15 of L, and columns 16w .. 16w+15 of A^T as they are contracted
+    // with T (a lane's rows s of column t = 16w + m), both up to the diagonal.
+    bf16x8 at_hi[2], at_lo[2];
     {
-        // wave w owns token rows 16w..16w+15 against all 64 columns
         bf16x8 ak[4];
 #pragma unroll
         for (uint32_t kk = 0; kk < 4; ++kk) {
             ak[kk] = operand(&ktile[wave * 16 + m][kk * 32 + g * 8]);
-            *reinterpret_cast<u32x4*>(rec + kRecQ + ((wave * 4 + kk) * 64 + lane) * 16) =
-                __builtin_bit_cast(u32x4, aq[kk]);
+            if ((h & 1) == 0) {
+                const uint32_t at = ((wave * 4 + kk) * 64 + lane) * 16;
+                *reinterpret_cast<u32x4*>(key_rec + kKeyRecK + at) = __builtin_bit_cast(u32x4, ak[kk]);
+                *reinterpret_cast<u32x4*>(key_rec + kKeyRecQ + at) = __builtin_bit_cast(u32x4, aq[kk]);
+            }
         }
+        const uint32_t t_col = wave * 16 + m;
+        const float log_col = log_g[t_col];
+        const f32x4 log_rows = *reinterpret_cast<const f32x4*>(&log_g[wave * 16 + g * 4]);
+        const f32x4 beta_rows = *reinterpret_cast<const f32x4*>(&scale_v[wave * 16 + g * 4]);
 #pragma unroll
-        for (uint32_t nt = 0; nt < 4; ++nt) {
-            f32x4 kkacc = {0.0f, 0.0f, 0.0f, 0.0f};
-            f32x4 qkacc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (uint32_t ks = 0; ks < 2; ++ks) {
+            float transposed[8];
 #pragma unroll
-            for (uint32_t kk = 0; kk < 4; ++kk) {
-                const bf16x8 bk = operand(&ktile[nt * 16 + m][kk * 32 + g * 8]);
-                kkacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ak[kk], bk, kkacc, 0, 0, 0);
-                qkacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aq[kk], bk, qkacc, 0, 0, 0);
+            for (uint32_t half = 0; half < 2; ++half) {
+                const uint32_t nt = 2 * ks + half;
+                f32x4 kkacc = {0.0f, 0.0f, 0.0f, 0.0f};
+                f32x4 kqacc = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (nt <= wave) {
+#pragma unroll
+                    for (uint32_t kk = 0; kk < 4; ++kk) {
+                        const bf16x8 bk = operand(&ktile[nt * 16 + m][kk * 32 + g * 8]);
+                        kkacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ak[kk], bk, kkacc, 0, 0, 0);
+                        kqacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bk, aq[kk], kqacc, 0, 0, 0);
+                    }
+                    const uint32_t s_col = nt * 16 + m;
+                    const float log_s = log_g[s_col];
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        const uint32_t t = wave * 16 + g * 4 + i;
+                        lower[t][s_col] = (s_col < t && t < valid)
+                                              ? beta_rows[i] * __expf(log_rows[i] - log_s) * kkacc[i] : 0.0f;
+                    }
+                    const f32x4 log_s_rows = *reinterpret_cast<const f32x4*>(&log_g[nt * 16 + g * 4]);
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        const uint32_t s = nt * 16 + g * 4 + i;
+                        transposed[half * 4 + i] =
+                            (s <= t_col && t_col < valid) ? __expf(log_col - log_s_rows[i]) * kqacc[i] : 0.0f;
+                    }
+                } else {
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) transposed[half * 4 + i] = 0.0f;
+                }
             }
-            const uint32_t s = nt * 16 + m;
-            f32x4 aqk;
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) {
-                const uint32_t t = wave * 16 + g * 4 + i;
-                const float ratio = s <= t ? __expf(log_g[t] - log_g[s]) : 0.0f;
-                lower[t][s] = (s < t && t < valid) ? scale_v[t] * ratio * kkacc[i] : 0.0f;
-                aqk[i] = (s <= t && t < valid) ? ratio * qkacc[i] : 0.0f;
-            }
-            // fragment (token tile `wave`, token step nt >> 1), column groups 2(nt&1), +1
-            store_tile_hi_lo(reinterpret_cast<uint16_t (*)[16][24]>(&strip[wave][0][0][0]), aqk, lane, rec + kRecAqkHi, rec + kRecAqkLo,
-                             ((wave * 2 + (nt >> 1)) * 64 + (nt & 1) * 32) * 16);
+            split8(transposed, at_hi[ks], at_lo[ks]);
         }
     }
     __syncthreads();
 
+    // the keys as right operands, [key tile][ks]: column 16 (2 wave + tile) + m, its eight tokens
+    bf16x8 keys[2][2];
+#pragma unroll
+    for (uint32_t tile = 0; tile < 2; ++tile) {
+#pragma unroll
+        for (uint32_t ks = 0; ks < 2; ++ks) {
+            // transposing reads: 16 lanes hand in 4 token rows x 16 columns, lane m receives
+            // column m of the 4 rows
+            const uint16_t* from = &ktile[ks * 32 + g * 4 + (m >> 2)][(2 * wave + tile) * 16 + (m & 3) * 4];
+            const s16x4 first = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(from));
+            const s16x4 second = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (__attribute__((address_space(3))) s16x4*)(from + 16 * kTileLd));
+            const u32x2 low = __builtin_bit_cast(u32x2, first), high = __builtin_bit_cast(u32x2, second);
+            keys[tile][ks] = __builtin_bit_cast(bf16x8, u32x4{low[0], low[1], high[0], high[1]});
+        }
+    }
     // diagonal blocks: thread (block b, column c) solves (I + L_bb) x = e_c
     if (tid < kChunk) {
         const uint32_t b = tid >> 4;
@@ -1073,12 +1102,11 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
         for (uint32_t r = 0; r < 16; ++r) tdiag[b * 16 + r][c] = x[r];
     }
     __syncthreads();
-    // [Wk | Wv] = (I + L)^-1 B with B = beta o [g o K | V], solved by block forward
-    // substitution, every wave for its own 64 columns (waves 0,1 the keys, 2,3 the
-    // values): W_i = T_ii (B_i - sum_{j<i} L_ij W_j) with the diagonal inverses T_ii.
-    // All products on MFMA with hi/lo operand pairs; a finished block row goes, as
-    // bf16 hi/lo, into the wave's strip in LDS, from where it is read back as the
-    // right operand of the next products (rows contiguous: one 16-byte read per lane).
+    // every wave has read its keys: the values take their place, to be read by columns
+#pragma unroll
+    for (uint32_t pass = 0; pass < 4; ++pass) {
+        *reinterpret_cast<u32x4*>(&ktile[pass * 16 + (tid >> 4)][(tid & 15) * 8]) = vv[pass];
+    }
     uint16_t (*hi_strip)[kStripLd] = strip[wave][0];
     uint16_t (*lo_strip)[kStripLd] = strip[wave][1];
     // left operands, the same for every column: lane (row m, slot group g).  K = 16
@@ -1121,8 +1149,11 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
     // slot groups 0 and 1 are live (K = 16)
     const auto get = [&](uint32_t row0, bool narrow_k, bf16x8& hi, bf16x8& lo) {
         const uint32_t row = row0 + (narrow_k ? (g & 1) : g) * 8;
-        u32x4 h = *reinterpret_cast<const u32x4*>(&hi_strip[m][row]);
-        u32x4 l = *reinterpret_cast<const u32x4*>(&lo_strip[m][row]);
+        const u32x2 h0 = *reinterpret_cast<const u32x2*>(&hi_strip[m][row]);
+        const u32x2 h1 = *reinterpret_cast<const u32x2*>(&hi_strip[m][row + 4]);
+        const u32x2 l0 = *reinterpret_cast<const u32x2*>(&lo_strip[m][row]);
+        const u32x2 l1 = *reinterpret_cast<const u32x2*>(&lo_strip[m][row + 4]);
+        u32x4 h = u32x4{h0[0], h0[1], h1[0], h1[1]}, l = u32x4{l0[0], l0[1], l1[0], l1[1]};
         if (narrow_k && g >= 2) {
             h = u32x4{0u, 0u, 0u, 0u};
             l = u32x4{0u, 0u, 0u, 0u};
@@ -1133,6 +1164,13 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     // every wave holds its left operands: `lower` and `tdiag` are free from here on
     __syncthreads();
+#pragma unroll
+    for (uint32_t slice = 0; slice < kGD / 16; ++slice) {
+        const uint16_t* from = &ktile[wave * 16 + g * 4 + (m >> 2)][slice * 16 + (m & 3) * 4];
+        const s16x4 column = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(from));
+        *reinterpret_cast<u32x2*>(rec + kRecV + ((slice * 4 + wave) * 64 + lane) * 8) = __builtin_bit_cast(u32x2, column);
+    }
+    __syncthreads();   // the strips take the values' place
 
     // Block column `wave` of T = (I + L)^-1 by block forward substitution on the
     // identity: X_i = T_ii (E_i - sum_{j<i} L_ij X_j).  All products on MFMA with hi/lo
@@ -1180,77 +1218,68 @@ __global__ __launch_bounds__(256) void gdn_chunk_prepare_kernel(ChunkPrepareArgs
     }
     __syncthreads();
 
-    // [Wk | Wv] = T (beta o [g o K | V]) = (T o scale) [K | V]: the scales go into the
-    // columns of T (fp32, then hi/lo), which leaves the exact bf16 keys and values as the
-    // other operand - two products per step and no chain between them.  Every wave takes
-    // its own 64 columns (waves 0,1 the keys, 2,3 the values).  Block (mt, ks) of T,
-    // token rows 16 mt .., token columns 32 ks ..; T is lower triangular: ks <= mt / 2.
-    const uint16_t (*source)[kTileLd] = is_k ? ktile : vtile;
-    const float* scale = is_k ? scale_k : scale_v;
-    bf16x8 ts_hi[4][2], ts_lo[4][2];
+    // Columns of T as left operands, T^T[s][r]: lane (s = 16 st + m, its eight r of step ks), by
+    // themselves for A T and times g_C/g_r for the keys.  T is lower triangular: r >= s.  The products
+    // are transposes: a lane's results are rows s = 16 st + 4 g + i of one column (token or key).
+    f32x4 at_sums[4], kt_sums[2][4];
 #pragma unroll
-    for (uint32_t mt = 0; mt < 4; ++mt) {
+    for (uint32_t st = 0; st < 4; ++st) at_sums[st] = kt_sums[0][st] = kt_sums[1][st] = zero;
 #pragma unroll
-        for (uint32_t ks = 0; ks < 2; ++ks) {
-            if (2 * ks > mt) continue;
+    for (uint32_t ks = 0; ks < 2; ++ks) {
+        const f32x4 ratio_low = *reinterpret_cast<const f32x4*>(&ratio_g[32 * ks + 4 * g]);
+        const f32x4 ratio_high = *reinterpret_cast<const f32x4*>(&ratio_g[32 * ks + 16 + 4 * g]);
+#pragma unroll
+        for (uint32_t st = 0; st < 4; ++st) {
+            if (st >= 2 && ks == 0) continue;
             float x[8];
 #pragma unroll
-            for (uint32_t e = 0; e < 8; ++e) {
-                x[e] = lower[16 * mt + m][32 * ks + 8 * g + e] * scale[32 * ks + 8 * g + e];
+            for (uint32_t e = 0; e < 4; ++e) {
+                x[e] = lower[32 * ks + 4 * g + e][16 * st + m];
+                x[4 + e] = lower[32 * ks + 16 + 4 * g + e][16 * st + m];
             }
-            split8(x, ts_hi[mt][ks], ts_lo[mt][ks]);
-        }
-    }
-    for (uint32_t ct = 0; ct < 4; ++ct) {
-        const uint32_t col0 = (wave & 1) * 64 + ct * 16;
-        // the exact rows, token-contiguous: lane = column col0 + m, tokens 32 ks + 8 g .. +7,
-        // by transposing reads (16 lanes hand in 4 token rows x 16 columns, lane m
-        // receives column m of the 4 rows)
-        bf16x8 rows8[2];
-#pragma unroll
-        for (uint32_t ks = 0; ks < 2; ++ks) {
-            const uint16_t* at = &source[ks * 32 + g * 8 + (m >> 2)][col0 + (m & 3) * 4];
-            const s16x4 first = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(at));
-            const s16x4 second = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) s16x4*)(at + 4 * kTileLd));
-            uint32_t bits[8];
+            bf16x8 hi, lo;
+            if (st <= wave && 2 * ks <= wave) {   // A T up to the diagonal
+                split8(x, hi, lo);
+                at_sums[st] = product(hi, lo, at_hi[ks], at_lo[ks], at_sums[st]);
+            }
 #pragma unroll
             for (uint32_t e = 0; e < 4; ++e) {
-                bits[e] = ks * 32 + g * 8 + e < valid ? static_cast<uint16_t>(first[e]) : 0u;
-                bits[4 + e] = ks * 32 + g * 8 + 4 + e < valid ? static_cast<uint16_t>(second[e]) : 0u;
+                x[e] *= ratio_low[e];
+                x[4 + e] *= ratio_high[e];
             }
-            const u32x4 packed = u32x4{bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16),
-                                       bits[4] | (bits[5] << 16), bits[6] | (bits[7] << 16)};
-            rows8[ks] = __builtin_bit_cast(bf16x8, packed);
-            if (is_k) {
-                // fragment (key tile, token step ks) of the record
-                *reinterpret_cast<u32x4*>(rec + kRecKt + (((col0 >> 4) * 2 + ks) * 64 + lane) * 16) = packed;
+            split8(x, hi, lo);
+            bf16x8 rest;   // to 2^-25: stage 2 works with this product's roundings as with R's own
+#pragma unroll
+            for (uint32_t e = 0; e < 8; ++e) {
+                rest[e] = static_cast<__bf16>(x[e] - static_cast<float>(hi[e]) - static_cast<float>(lo[e]));
+            }
+#pragma unroll
+            for (uint32_t tile = 0; tile < 2; ++tile) {
+                kt_sums[tile][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rest, keys[tile][ks], kt_sums[tile][st], 0, 0, 0);
+                kt_sums[tile][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, keys[tile][ks], kt_sums[tile][st], 0, 0, 0);
+                kt_sums[tile][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, keys[tile][ks], kt_sums[tile][st], 0, 0, 0);
             }
         }
-        f32x4 w[4];
+    }
+    // two result tiles are one fragment of stage 2
+    const auto store_fragment = [&](const f32x4 first, const f32x4 second, uint8_t* hi_at, uint8_t* lo_at) {
+        u32x2 hi0, lo0, hi1, lo1;
+        split4(first, hi0, lo0);
+        split4(second, hi1, lo1);
+        *reinterpret_cast<u32x4*>(hi_at) = u32x4{hi0[0], hi0[1], hi1[0], hi1[1]};
+        *reinterpret_cast<u32x4*>(lo_at) = u32x4{lo0[0], lo0[1], lo1[0], lo1[1]};
+    };
 #pragma unroll
-        for (uint32_t mt = 0; mt < 4; ++mt) {
-            f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ts_lo[mt][0], rows8[0], zero, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ts_hi[mt][0], rows8[0], acc, 0, 0, 0);
-            if (mt >= 2) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ts_lo[mt][1], rows8[1], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ts_hi[mt][1], rows8[1], acc, 0, 0, 0);
-            }
-            w[mt] = acc;
+    for (uint32_t k2 = 0; k2 < 2; ++k2) {
+        if (2 * k2 <= wave) {
+            const uint32_t at = ((wave * 2 + k2) * 64 + lane) * 16;
+            store_fragment(at_sums[2 * k2], at_sums[2 * k2 + 1], rec + kRecAtHi + at, rec + kRecAtLo + at);
         }
-        // lane holds tokens 16mt+4g+i of column col0 + m
 #pragma unroll
-        for (uint32_t mt = 0; mt < 4; ++mt) {
-            if (is_k) {
-                // fragment (token tile mt, key step col0 >> 5), column groups (col0 & 31) >> 3, +1
-                store_tile_hi_lo(reinterpret_cast<uint16_t (*)[16][24]>(&strip[wave][0][0][0]), w[mt],
-                                 lane, rec + kRecWkHi, rec + kRecWkLo,
-                                 ((mt * 4 + (col0 >> 5)) * 64 + ((col0 & 31) >> 3) * 16) * 16);
-            } else {
-                *reinterpret_cast<f32x4*>(rec + kRecWv +
-                                          ((((col0 + m) >> 4) * 4 + mt) * 64 + g * 16 + m) * 16) = w[mt];
-            }
+        for (uint32_t tile = 0; tile < 2; ++tile) {
+            const uint32_t at = (((2 * wave + tile) * 2 + k2) * 64 + lane) * 16;
+            store_fragment(kt_sums[tile][2 * k2], kt_sums[tile][2 * k2 + 1], rec + kRecKtHi + at,
+                           rec + kRecKtLo + at);
         }
     }
 }
@@ -1263,91 +1292,45 @@ struct ChunkScanArgs {
     uint32_t rows;
 };
 
-// One chunk's operands of one wave, loaded a chunk ahead of their use.  The state
+// One chunk's operands of one wave, loaded two chunks ahead of their use.  The state
 // waves carry the recurrence, the output waves everything that only leaves it.
-template <uint32_t NT>
 struct StateOperands {
-    bf16x8 wk_hi[4], wk_lo[4], kt[2][2];
-    f32x4 wv[NT];
-    f32x4 ratio;
+    bf16x8 k[4], kt_hi[2][2], kt_lo[2][2];
+    u32x2 v;
+    f32x4 gam, beta;
     float gamma_c;
 };
 struct OutputOperands {
-    bf16x8 q[4], aq_hi[2], aq_lo[2];
+    bf16x8 q[4], at_hi[2], at_lo[2];
     f32x4 gam;
 };
 
-__device__ __forceinline__ const uint8_t* chunk_record(const ChunkScanArgs& a, uint32_t chunk,
-                                                       uint32_t h) {
-    return a.scratch + (static_cast<uint64_t>(chunk) * kGdnValueHeads + h) * kRecBytes;
-}
 __device__ __forceinline__ u32x4 record_fragment(const uint8_t* rec, uint32_t base, uint32_t index,
                                                  uint32_t lane) {
     return *reinterpret_cast<const u32x4*>(rec + base + (index * 64 + lane) * 16);
 }
 
-template <uint32_t NT>
-__device__ __forceinline__ StateOperands<NT> load_state_operands(const uint8_t* rec, uint32_t slice,
-                                                                 uint32_t w, uint32_t lane) {
-    StateOperands<NT> o;
-    const uint32_t g = lane >> 4;
-#pragma unroll
-    for (uint32_t kk = 0; kk < 4; ++kk) {
-        o.wk_hi[kk] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecWkHi, w * 4 + kk, lane));
-        o.wk_lo[kk] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecWkLo, w * 4 + kk, lane));
-    }
-#pragma unroll
-    for (uint32_t k2 = 0; k2 < 2; ++k2) {
-#pragma unroll
-        for (uint32_t mt = 0; mt < 2; ++mt) {
-            o.kt[mt][k2] =
-                __builtin_bit_cast(bf16x8, record_fragment(rec, kRecKt, (w * 2 + mt) * 2 + k2, lane));
-        }
-    }
-#pragma unroll
-    for (uint32_t nt = 0; nt < NT; ++nt) {
-        o.wv[nt] = __builtin_bit_cast(f32x4, record_fragment(rec, kRecWv, (slice * NT + nt) * 4 + w, lane));
-    }
-    o.ratio = *reinterpret_cast<const f32x4*>(rec + kRecRatio + (w * 16 + g * 4) * 4);
-    o.gamma_c = *reinterpret_cast<const float*>(rec + kRecGamma);
-    return o;
-}
-
-__device__ __forceinline__ OutputOperands load_output_operands(const uint8_t* rec, uint32_t w,
-                                                               uint32_t lane) {
-    OutputOperands o;
-    const uint32_t g = lane >> 4;
-#pragma unroll
-    for (uint32_t kk = 0; kk < 4; ++kk) {
-        o.q[kk] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecQ, w * 4 + kk, lane));
-    }
-#pragma unroll
-    for (uint32_t k2 = 0; k2 < 2; ++k2) {
-        o.aq_hi[k2] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecAqkHi, w * 2 + k2, lane));
-        o.aq_lo[k2] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecAqkLo, w * 2 + k2, lane));
-    }
-    o.gam = *reinterpret_cast<const f32x4*>(rec + kRecGam + (w * 16 + g * 4) * 4);
-    return o;
-}
-
 // Stage 2.  grid (8, 32) x 512: a workgroup owns a 16-wide slice of the value
 // dimension of one head and walks the chunks in order.  Waves 0..3 (state waves)
-// carry the recurrence: wave w owns token rows 16w..16w+15 of U and key columns
+// carry the recurrence: wave w owns token rows 16w..16w+15 of R and key columns
 // 32w..32w+31 of the state slice, whose fp32 master copy lives in its MFMA
 // accumulators for the whole block.  Waves 4..7 (output waves) compute what only
-// leaves the recurrence - Y = g o (Q S^T) + A U of token rows 16w..16w+15 - from the
-// state and U copies in LDS, so that their loads, products and stores stay off the
+// leaves the recurrence - Y = g o (Q S^T) + (A T) R of token rows 16w..16w+15 - from the
+// state and R copies in LDS, so that their loads, products and stores stay off the
 // chain from one chunk's state to the next.  Two barriers per chunk order the two
 // LDS copies between all eight waves.
-template <uint32_t NT>
+//
+// 2048 rows: 42 us as before, a chain of 32 steps of 1.3 us.  Without the output waves it is 31 us (their loads
+// 6 of the 15, their stores 3), without P still 46, with all records in the L2 44: no one of loads,
+// LDS and products bounds a step, they add up along it.  Tried: the state waves at a higher wave
+// priority and y stored four columns a lane, gates through LDS - no change.
 __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {
-    constexpr uint32_t DV = 16 * NT;
+    constexpr uint32_t DV = 16;
     __shared__ __attribute__((aligned(16))) uint16_t s_hi[DV][136];  // bf16 S slice [dv][dk+pad]
     __shared__ __attribute__((aligned(16))) uint16_t s_lo[DV][136];  // S - s_hi
-    __shared__ __attribute__((aligned(16))) uint16_t u_hi[DV][72];   // U^T [dv][token+pad]
-    __shared__ __attribute__((aligned(16))) uint16_t u_lo[DV][72];
-    __shared__ __attribute__((aligned(16))) uint16_t d_hi[DV][72];   // ((g_C/g) o U)^T
-    __shared__ __attribute__((aligned(16))) uint16_t d_lo[DV][72];
+    // R^T [dv][token+pad], the tokens in the order the operands have them
+    __shared__ __attribute__((aligned(16))) uint16_t r_hi[DV][72];
+    __shared__ __attribute__((aligned(16))) uint16_t r_lo[DV][72];
     // Workgroups are dealt round-robin over the 8 XCDs, each with its own L2, in
     // linear order (x fastest): blockIdx.x names the XCD.  All slices of a head
     // read the same chunk records, so a head's slices stay on one XCD.
@@ -1355,6 +1338,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {
     const uint32_t local = blockIdx.y;
     const uint32_t slice = local % kSlicesPerHead;
     const uint32_t h = blockIdx.x * (kGdnValueHeads / 8) + local / kSlicesPerHead;
+    const uint32_t kh = h >> 1;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t w = wave & 3;
     const bool state_wave = wave < 4;
@@ -1362,92 +1346,120 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {
     const uint32_t m = lane & 15;
     const uint32_t g = lane >> 4;
     const uint32_t chunks = (a.rows + kChunk - 1) / kChunk;
+    const uint32_t last = chunks - 1;
     const uint32_t at = w * 16 + g * 4;  // this lane's token rows of a chunk
+    const uint32_t at_slot = 32 * (w >> 1) + 8 * g + 4 * (w & 1);   // where they stand in r_hi, r_lo
+    const auto records_of = [&](uint32_t chunk) {
+        return a.scratch + static_cast<uint64_t>(chunk) * kChunkRecords;
+    };
 
     if (state_wave) {
         // State slice transposed, [dk tile][dv]: this lane holds key rows
         // 32w+16mt+4g+i of value column m, four consecutive keys of one state row.
-        f32x4 sacc[2][NT];
+        f32x4 sacc[2];
 #pragma unroll
         for (uint32_t mt = 0; mt < 2; ++mt) {
-#pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-                const uint32_t j = nt * 16 + m;
-                const uint32_t dk = w * 32 + mt * 16 + g * 4;
-                const f32x4 v = *reinterpret_cast<const f32x4*>(
-                    a.state_in + (static_cast<uint64_t>(h) * kGD + slice * DV + j) * kGD + dk);
-                sacc[mt][nt] = v;
-                u32x2 hi, lo;
-                split4(v, hi, lo);
-                *reinterpret_cast<u32x2*>(&s_hi[j][dk]) = hi;
-                *reinterpret_cast<u32x2*>(&s_lo[j][dk]) = lo;
-            }
+            const uint32_t dk = w * 32 + mt * 16 + g * 4;
+            const f32x4 v = *reinterpret_cast<const f32x4*>(
+                a.state_in + (static_cast<uint64_t>(h) * kGD + slice * DV + m) * kGD + dk);
+            sacc[mt] = v;
+            u32x2 hi, lo;
+            split4(v, hi, lo);
+            *reinterpret_cast<u32x2*>(&s_hi[m][dk]) = hi;
+            *reinterpret_cast<u32x2*>(&s_lo[m][dk]) = lo;
         }
-        const uint32_t last = chunks - 1;
-        const auto fetch = [&](uint32_t chunk) {
-            return load_state_operands<NT>(chunk_record(a, min(chunk, last), h), slice, w, lane);
+        const auto fetch = [&](uint32_t ahead) {
+            const uint32_t chunk = min(ahead, last);
+            const uint8_t* records = records_of(chunk);
+            const uint8_t* rec = records + h * kRecordBytes;
+            const uint8_t* key_rec = records + kChunkKeys + kh * kKeyRecBytes;
+            StateOperands o;
+#pragma unroll
+            for (uint32_t kk = 0; kk < 4; ++kk) {
+                o.k[kk] = __builtin_bit_cast(bf16x8, record_fragment(key_rec, kKeyRecK, w * 4 + kk, lane));
+            }
+            o.v = *reinterpret_cast<const u32x2*>(rec + kRecV + ((slice * 4 + w) * 64 + lane) * 8);
+#pragma unroll
+            for (uint32_t k2 = 0; k2 < 2; ++k2) {
+#pragma unroll
+                for (uint32_t mt = 0; mt < 2; ++mt) {
+                    const uint32_t index = (w * 2 + mt) * 2 + k2;
+                    o.kt_hi[mt][k2] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecKtHi, index, lane));
+                    o.kt_lo[mt][k2] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecKtLo, index, lane));
+                }
+            }
+            o.gam = *reinterpret_cast<const f32x4*>(rec + kRecGam + at * 4);
+            o.beta = *reinterpret_cast<const f32x4*>(rec + kRecBeta + at * 4);
+            o.gamma_c = *reinterpret_cast<const float*>(rec + kRecGamma);
+            return o;
         };
         // one chunk of the recurrence with the operands `cur`
-        const auto step = [&](const StateOperands<NT>& cur) {
-            // P1 = Wk S^T for token tile w: [16 x DV]
+        const auto step = [&](const StateOperands& cur) {
+            // P = K S^T for token tile w: [16 x DV], in two chains
+            f32x4 p_hi = {0.0f, 0.0f, 0.0f, 0.0f}, p_lo = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-                f32x4 p1 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (uint32_t kk = 0; kk < 4; ++kk) {
-                    const bf16x8 sh = operand(&s_hi[nt * 16 + m][kk * 32 + g * 8]);
-                    const bf16x8 sl = operand(&s_lo[nt * 16 + m][kk * 32 + g * 8]);
-                    p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.wk_lo[kk], sh, p1, 0, 0, 0);
-                    p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.wk_hi[kk], sl, p1, 0, 0, 0);
-                    p1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.wk_hi[kk], sh, p1, 0, 0, 0);
-                }
-                // U = Wv - P1; this lane holds tokens 16w+4g+i of value column 16nt+m
-                const f32x4 u = cur.wv[nt] - p1;
-                const f32x4 d = u * cur.ratio;
-                u32x2 uh, ul, dh, dl;
-                split4(u, uh, ul);
-                split4(d, dh, dl);
-                *reinterpret_cast<u32x2*>(&u_hi[nt * 16 + m][at]) = uh;
-                *reinterpret_cast<u32x2*>(&u_lo[nt * 16 + m][at]) = ul;
-                *reinterpret_cast<u32x2*>(&d_hi[nt * 16 + m][at]) = dh;
-                *reinterpret_cast<u32x2*>(&d_lo[nt * 16 + m][at]) = dl;
+            for (uint32_t kk = 0; kk < 4; ++kk) {
+                const bf16x8 sh = operand(&s_hi[m][kk * 32 + g * 8]);
+                const bf16x8 sl = operand(&s_lo[m][kk * 32 + g * 8]);
+                p_lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.k[kk], sl, p_lo, 0, 0, 0);
+                p_hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.k[kk], sh, p_hi, 0, 0, 0);
             }
-            __syncthreads();  // U^T complete; every read of the old state copy is done
-            // S^T = g_C S^T + K^T ((g_C/g) o U) for key rows 32w..32w+31
+            // R = beta o (V - g o P); this lane holds tokens 16w+4g+i of value column m
+            f32x4 r;
 #pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-                bf16x8 dlo[2], dhi[2];
+            for (uint32_t i = 0; i < 4; ++i) {
+                r[i] = cur.beta[i] * fmaf(-cur.gam[i], p_lo[i] + p_hi[i], widen_half(cur.v[i >> 1], i));
+            }
+            u32x2 hi, lo;
+            split4(r, hi, lo);
+            *reinterpret_cast<u32x2*>(&r_hi[m][at_slot]) = hi;
+            *reinterpret_cast<u32x2*>(&r_lo[m][at_slot]) = lo;
+            __syncthreads();  // R^T complete; every read of the old state copy is done
+            // S^T = g_C S^T + K^T ((g_C/g) o T) R for key rows 32w..32w+31
+            bf16x8 rh[2], rl[2];
 #pragma unroll
-                for (uint32_t k2 = 0; k2 < 2; ++k2) {
-                    dlo[k2] = operand(&d_lo[nt * 16 + m][k2 * 32 + g * 8]);
-                    dhi[k2] = operand(&d_hi[nt * 16 + m][k2 * 32 + g * 8]);
+            for (uint32_t k2 = 0; k2 < 2; ++k2) {
+                rh[k2] = operand(&r_hi[m][k2 * 32 + g * 8]);
+                rl[k2] = operand(&r_lo[m][k2 * 32 + g * 8]);
+            }
+            f32x4 low[2];
+#pragma unroll
+            for (uint32_t mt = 0; mt < 2; ++mt) {
+                sacc[mt] *= cur.gamma_c;
+                low[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt_lo[mt][0], rl[0], f32x4{0.0f, 0.0f, 0.0f, 0.0f},
+                                                                  0, 0, 0);
+                low[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt_lo[mt][1], rl[1], low[mt], 0, 0, 0);
+            }
+#pragma unroll
+            for (uint32_t k2 = 0; k2 < 2; ++k2) {
+#pragma unroll
+                for (uint32_t mt = 0; mt < 2; ++mt) {
+                    low[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt_lo[mt][k2], rh[k2], low[mt], 0, 0, 0);
+                    sacc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt_hi[mt][k2], rh[k2], sacc[mt], 0, 0, 0);
                 }
 #pragma unroll
                 for (uint32_t mt = 0; mt < 2; ++mt) {
-                    sacc[mt][nt] *= cur.gamma_c;
-#pragma unroll
-                    for (uint32_t k2 = 0; k2 < 2; ++k2) {
-                        sacc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt[mt][k2], dlo[k2],
-                                                                               sacc[mt][nt], 0, 0, 0);
-                        sacc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt[mt][k2], dhi[k2],
-                                                                               sacc[mt][nt], 0, 0, 0);
-                    }
-                    u32x2 hi, lo;
-                    split4(sacc[mt][nt], hi, lo);
-                    const uint32_t dk = w * 32 + mt * 16 + g * 4;
-                    *reinterpret_cast<u32x2*>(&s_hi[nt * 16 + m][dk]) = hi;
-                    *reinterpret_cast<u32x2*>(&s_lo[nt * 16 + m][dk]) = lo;
+                    low[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.kt_hi[mt][k2], rl[k2], low[mt], 0, 0, 0);
                 }
             }
-            __syncthreads();  // new state copy visible; U^T free for the next chunk
+#pragma unroll
+            for (uint32_t mt = 0; mt < 2; ++mt) {
+                sacc[mt] += low[mt];
+                u32x2 s_high, s_low;
+                split4(sacc[mt], s_high, s_low);
+                const uint32_t dk = w * 32 + mt * 16 + g * 4;
+                *reinterpret_cast<u32x2*>(&s_hi[m][dk]) = s_high;
+                *reinterpret_cast<u32x2*>(&s_lo[m][dk]) = s_low;
+            }
+            __syncthreads();  // new state copy visible; R^T free for the next chunk
         };
         // Operands are requested two chunks ahead of their use, in three register sets
         // that take turns (no copies: a copy would wait for the newest request).
-        StateOperands<NT> set_a = fetch(0);
-        StateOperands<NT> set_b = fetch(1);
+        StateOperands set_a = fetch(0);
+        StateOperands set_b = fetch(1);
         __syncthreads();
         for (uint32_t chunk = 0; chunk < chunks; chunk += 3) {
-            const StateOperands<NT> set_c = fetch(chunk + 2);
+            const StateOperands set_c = fetch(chunk + 2);
             step(set_a);
             if (chunk + 1 < chunks) {
                 set_a = fetch(chunk + 3);
@@ -1460,56 +1472,60 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {
         }
 #pragma unroll
         for (uint32_t mt = 0; mt < 2; ++mt) {
-#pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-                const uint32_t dk = w * 32 + mt * 16 + g * 4;
-                *reinterpret_cast<f32x4*>(a.state_out + (static_cast<uint64_t>(h) * kGD + slice * DV +
-                                                         nt * 16 + m) * kGD + dk) = sacc[mt][nt];
-            }
+            const uint32_t dk = w * 32 + mt * 16 + g * 4;
+            *reinterpret_cast<f32x4*>(a.state_out + (static_cast<uint64_t>(h) * kGD + slice * DV + m) * kGD +
+                                      dk) = sacc[mt];
         }
     } else {
-        const uint32_t last = chunks - 1;
-        const auto fetch = [&](uint32_t chunk) {
-            return load_output_operands(chunk_record(a, min(chunk, last), h), w, lane);
+        const auto fetch = [&](uint32_t ahead) {
+            const uint32_t chunk = min(ahead, last);
+            const uint8_t* records = records_of(chunk);
+            const uint8_t* rec = records + h * kRecordBytes;
+            const uint8_t* key_rec = records + kChunkKeys + kh * kKeyRecBytes;
+            OutputOperands o;
+#pragma unroll
+            for (uint32_t kk = 0; kk < 4; ++kk) {
+                o.q[kk] = __builtin_bit_cast(bf16x8, record_fragment(key_rec, kKeyRecQ, w * 4 + kk, lane));
+            }
+#pragma unroll
+            for (uint32_t k2 = 0; k2 < 2; ++k2) {
+                if (2 * k2 > w) continue;
+                o.at_hi[k2] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecAtHi, w * 2 + k2, lane));
+                o.at_lo[k2] = __builtin_bit_cast(bf16x8, record_fragment(rec, kRecAtLo, w * 2 + k2, lane));
+            }
+            o.gam = *reinterpret_cast<const f32x4*>(rec + kRecGam + at * 4);
+            return o;
         };
         const auto step = [&](const OutputOperands& cur, uint32_t chunk) {
             // P2 = Q S^T for token tile w against the state the chunk starts from
-            f32x4 y[NT];
+            f32x4 y = {0.0f, 0.0f, 0.0f, 0.0f}, low = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-                f32x4 p2 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (uint32_t kk = 0; kk < 4; ++kk) {
-                    const bf16x8 sh = operand(&s_hi[nt * 16 + m][kk * 32 + g * 8]);
-                    const bf16x8 sl = operand(&s_lo[nt * 16 + m][kk * 32 + g * 8]);
-                    p2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.q[kk], sl, p2, 0, 0, 0);
-                    p2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.q[kk], sh, p2, 0, 0, 0);
-                }
-                y[nt] = p2 * cur.gam;
+            for (uint32_t kk = 0; kk < 4; ++kk) {
+                const bf16x8 sh = operand(&s_hi[m][kk * 32 + g * 8]);
+                const bf16x8 sl = operand(&s_lo[m][kk * 32 + g * 8]);
+                low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.q[kk], sl, low, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.q[kk], sh, y, 0, 0, 0);
             }
-            __syncthreads();  // U^T complete; this wave is done with the old state copy
-            // Y = g o (Q S^T) + A U
+            y = (y + low) * cur.gam;
+            __syncthreads();  // R^T complete; this wave is done with the old state copy
+            // Y = g o (Q S^T) + (A T) R
+            low = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-#pragma unroll
-                for (uint32_t k2 = 0; k2 < 2; ++k2) {
-                    const bf16x8 bh = operand(&u_hi[nt * 16 + m][k2 * 32 + g * 8]);
-                    const bf16x8 bl = operand(&u_lo[nt * 16 + m][k2 * 32 + g * 8]);
-                    y[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.aq_lo[k2], bh, y[nt], 0, 0, 0);
-                    y[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.aq_hi[k2], bl, y[nt], 0, 0, 0);
-                    y[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.aq_hi[k2], bh, y[nt], 0, 0, 0);
-                }
+            for (uint32_t k2 = 0; k2 < 2; ++k2) {
+                if (2 * k2 > w) continue;
+                const bf16x8 rh = operand(&r_hi[m][k2 * 32 + g * 8]);
+                const bf16x8 rl = operand(&r_lo[m][k2 * 32 + g * 8]);
+                low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.at_lo[k2], rh, low, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.at_hi[k2], rh, y, 0, 0, 0);
+                low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(cur.at_hi[k2], rl, low, 0, 0, 0);
             }
-            __syncthreads();  // this wave is done with U^T
+            y += low;
+            __syncthreads();  // this wave is done with R^T
 #pragma unroll
-            for (uint32_t nt = 0; nt < NT; ++nt) {
-#pragma unroll
-                for (uint32_t i = 0; i < 4; ++i) {
-                    const uint32_t token = chunk * kChunk + at + i;
-                    if (token < a.rows) {
-                        a.y[static_cast<uint64_t>(token) * kGdnValueValues + h * kGD + slice * DV +
-                            nt * 16 + m] = narrow(y[nt][i]);
-                    }
+            for (uint32_t i = 0; i < 4; ++i) {
+                const uint32_t token = chunk * kChunk + at + i;
+                if (token < a.rows) {
+                    a.y[static_cast<uint64_t>(token) * kGdnValueValues + h * kGD + slice * DV + m] = narrow(y[i]);
                 }
             }
         };
@@ -1530,10 +1546,9 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {
         }
     }
 }
-
-// value tiles of 16 per scan workgroup: 1 -> 256 workgroups (0.47 ms for 16384 rows),
-// 2 -> 128 workgroups with half the L2 traffic (0.57 ms: the chunk chain gets longer)
-constexpr uint32_t kScanTiles = 1;
+// 16 wide: 256 workgroups; 32 wide, 128 of them with half the L2 traffic, the chunk chain got longer
+// (16384 rows, stage 2 alone 0.47 -> 0.57 ms)
+constexpr uint32_t kScanSlices = kGD / 16;   // of a head
 
 // ---------------------------------------------------------------- launchers --
 
@@ -1991,8 +2006,7 @@ int32_t op_gdn_chunk_prepare(const Bindings& b, const Grid& g, hipStream_t strea
     p.beta = a.buffer<const float>(3, rows * kGdnValueHeads * 4);
     p.scratch = a.buffer<uint8_t>(4, chunk_scratch_bytes(p.rows));
     if (a.status != TT_OK || validate_only) return a.status;
-    hipLaunchKernelGGL(gdn_chunk_prepare_kernel, dim3(chunks, kGdnValueHeads), dim3(256), 0, stream,
-                       p);
+    hipLaunchKernelGGL(gdn_chunk_prepare_kernel, dim3(chunks, kGdnValueHeads), dim3(256), 0, stream, p);
     return TT_OK;
 }
 
@@ -2012,16 +2026,18 @@ int32_t op_gdn_chunk_scan(const Bindings& b, const Grid& g, hipStream_t stream,
     p.y = a.buffer<uint16_t>(2, static_cast<uint64_t>(p.rows) * kGdnValueValues * 2);
     p.state_out = a.buffer<float>(3, kGdnStateFloats * 4ull);
     if (a.status != TT_OK || validate_only) return a.status;
-    hipLaunchKernelGGL(gdn_chunk_scan_kernel<kScanTiles>, dim3(8, kGdnValueHeads / kScanTiles), dim3(512), 0, stream, p);
+    hipLaunchKernelGGL(gdn_chunk_scan_kernel, dim3(8, kGdnValueHeads * kScanSlices / 8), dim3(512), 0, stream, p);
     return TT_OK;
 }
 
 // Rows one prepare + scan pair of gdn_chunk_recurrence_blk covers: the chunk records
-// of a group (118 MB) stay in the 256 MB last-level cache between the two stages.
+// of a group (85 MB) stay in the 256 MB last-level cache between the two stages, and stage 1 is one
+// round of four workgroups to a compute unit.
 constexpr uint32_t kChunkGroupRows = 2048;
 
-// Up to this many rows the token loop is the shorter chain (and the reference's own order): both
-// dispatches of a chunk take 21 us whatever it holds, the loop 8.3 us for 12 rows, 16.4 for 32,
+// Up to this many rows the token loop is used, which is the reference's own order: both
+// dispatches of a chunk take 15 us whatever it holds (21 once: from 33 rows on they would be the shorter
+// chain, but the loop's state is exact to fp32), the loop 8.3 us for 12 rows, 16.4 for 32,
 // 22.4 for 48.  (Requesting a step's operands a step ahead made the loop slower, 9.0 us for 12.)
 constexpr uint32_t kTokenLoopRows = 40;
 
@@ -2080,7 +2096,8 @@ int32_t op_gdn_chunk_recurrence(const Bindings& b, const Grid& g, hipStream_t st
         c.state_out = state_out;
         c.y = y + static_cast<uint64_t>(start) * kGdnValueValues;
         c.rows = count;
-        hipLaunchKernelGGL(gdn_chunk_scan_kernel<kScanTiles>, dim3(8, kGdnValueHeads / kScanTiles), dim3(512), 0, stream, c);
+        hipLaunchKernelGGL(gdn_chunk_scan_kernel, dim3(8, kGdnValueHeads * kScanSlices / 8), dim3(512), 0, stream,
+                           c);
     }
     return TT_OK;
 }
