@@ -43,13 +43,30 @@ __device__ __forceinline__ float rms_inverse(float total, uint32_t hidden) {
     return 1.0f / sqrtf(total / static_cast<float>(hidden) + kRmsNormEpsilon);
 }
 
+// a magnitude below the normal range to signed zero
+__device__ __forceinline__ float rms_flush(float v) {
+    return fabsf(v) < 0x1p-126f ? __uint_as_float(__float_as_uint(v) & 0x80000000u) : v;
+}
+// rms_store16 of two values, packed, by the hardware's conversion (round to nearest even; a value
+// that is not subnormal does not round to one; a NaN comes out quiet instead of with its upper bits)
+__device__ __forceinline__ uint32_t rms_store_pair(float a, float b) {
+    typedef __attribute__((ext_vector_type(2))) float Pair;
+    typedef __attribute__((ext_vector_type(2))) __bf16 Rounded;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(Pair{rms_flush(a), rms_flush(b)}, Rounded));
+}
+__device__ __forceinline__ float rms_low(uint32_t pair) { return __uint_as_float(pair << 16); }
+__device__ __forceinline__ float rms_high(uint32_t pair) { return __uint_as_float(pair & 0xFFFF0000u); }
+
 // two values of a row and their weights, packed: bf16(w * bf16(x * inverse)) of each
 __device__ __forceinline__ uint32_t rms_scale_pair(uint32_t x_pair, uint32_t w_pair, float inverse) {
-    const float x0 = __uint_as_float(x_pair << 16), x1 = __uint_as_float(x_pair & 0xFFFF0000u);
-    const uint16_t s0 = rms_store16(x0 * inverse), s1 = rms_store16(x1 * inverse);
-    const uint16_t r0 = rms_store16(rms_widen(rms_fz16(static_cast<uint16_t>(w_pair))) * rms_widen(s0));
-    const uint16_t r1 = rms_store16(rms_widen(rms_fz16(static_cast<uint16_t>(w_pair >> 16))) * rms_widen(s1));
-    return r0 | (static_cast<uint32_t>(r1) << 16);
+    const uint32_t scaled = rms_store_pair(rms_low(x_pair) * inverse, rms_high(x_pair) * inverse);
+    return rms_store_pair(rms_flush(rms_low(w_pair)) * rms_low(scaled),
+                          rms_flush(rms_high(w_pair)) * rms_high(scaled));
+}
+// the residual sum of two pairs: bf16(a + b) of each
+__device__ __forceinline__ uint32_t rms_add_pair(uint32_t a_pair, uint32_t b_pair) {
+    return rms_store_pair(rms_flush(rms_low(a_pair)) + rms_flush(rms_low(b_pair)),
+                          rms_flush(rms_high(a_pair)) + rms_flush(rms_high(b_pair)));
 }
 
 }  // namespace tt

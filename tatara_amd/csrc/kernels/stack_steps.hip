@@ -43,54 +43,69 @@ __device__ __forceinline__ uint16_t fz16(uint16_t h) {
 }
 
 // One row of `hidden` values (a multiple of 128, at most 4096) per workgroup of
-// hidden/4 threads: thread t squares values 4t..4t+3 in order, 32-lane groups sum
+// hidden / (4 kPieces) threads: a slice of four values is squared in order, 32 slices sum
 // in the adjacent-pairs tree (= xor butterfly), the group sums land in a 32-slot
 // stage that is summed by the same tree; out = bf16(w * bf16(x * inverse)).
 // With `addend`, the row normalised is residual = bf16(input + addend), which is also
 // written to `residual_out` (residual_rms): the norm consumes the rounded sums.
-__global__ __launch_bounds__(1024) void rms_only_kernel(const uint16_t* input, const uint16_t* weight,
-                                                        uint16_t* output, uint32_t hidden,
-                                                        uint32_t in_stride, uint32_t out_stride,
-                                                        const uint16_t* addend, uint16_t* residual_out,
-                                                        uint32_t residual_stride) {
+// kPieces: slices of a thread.  One, and one barrier, for the few rows of a wave, whose time is the
+// chain of a row; two, with 16-byte loads, for a block.  residual_rms_ms of 2048 values: 1 / 4 / 16 / 100
+// rows 3.3 / 3.4 / 3.5 / 3.6 -> 2.6 / 2.7 / 2.8 / 2.9 us (of which a dispatch is about 2) without the barriers that
+// cleared the stage and passed the sum on and with the hardware's rounding; 777 / 2048 / 16384 rows
+// 5.9 / 9.7 / 52 -> 4.4 / 6.7 / 39 us (one slice a thread 4.7 / 7.7 / 43), 16384 rows at 6.8 TB/s.
+template <uint32_t kPieces>
+__global__ __launch_bounds__(1024 / kPieces) void rms_only_kernel(const uint16_t* input, const uint16_t* weight,
+                                                                  uint16_t* output, uint32_t hidden,
+                                                                  uint32_t in_stride, uint32_t out_stride,
+                                                                  const uint16_t* addend, uint16_t* residual_out,
+                                                                  uint32_t residual_stride) {
+    typedef __attribute__((ext_vector_type(2 * kPieces))) uint32_t Piece;
     __shared__ float stage[32];
-    __shared__ float inverse_norm;
+    constexpr uint32_t kLanes = 32 / kPieces;   // of a group of 32 slices
     const uint32_t t = threadIdx.x;
     const uint16_t* in = input + static_cast<uint64_t>(blockIdx.y) * in_stride;
     uint16_t* out = output + static_cast<uint64_t>(blockIdx.y) * out_stride;
-    u32x2 raw = *reinterpret_cast<const u32x2*>(in + 4 * t);
+    Piece raw = *reinterpret_cast<const Piece*>(in + 4 * kPieces * t);
     // requested with the row, not after the reduction
-    const u32x2 wraw = *reinterpret_cast<const u32x2*>(weight + 4 * t);
+    const Piece wraw = *reinterpret_cast<const Piece*>(weight + 4 * kPieces * t);
     if (addend != nullptr) {
-        const u32x2 other = *reinterpret_cast<const u32x2*>(
-            addend + static_cast<uint64_t>(blockIdx.y) * residual_stride + 4 * t);
-        uint16_t sum[4];
+        const uint64_t at = static_cast<uint64_t>(blockIdx.y) * residual_stride + 4 * kPieces * t;
+        const Piece other = *reinterpret_cast<const Piece*>(addend + at);
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            const uint16_t xa = static_cast<uint16_t>(raw[i >> 1] >> ((i & 1) * 16));
-            const uint16_t xb = static_cast<uint16_t>(other[i >> 1] >> ((i & 1) * 16));
-            sum[i] = store16(widen(fz16(xa)) + widen(fz16(xb)));
-        }
-        raw = u32x2{sum[0] | (static_cast<uint32_t>(sum[1]) << 16),
-                    sum[2] | (static_cast<uint32_t>(sum[3]) << 16)};
-        *reinterpret_cast<u32x2*>(residual_out + static_cast<uint64_t>(blockIdx.y) * residual_stride +
-                                  4 * t) = raw;
+        for (uint32_t i = 0; i < 2 * kPieces; ++i) raw[i] = rms_add_pair(raw[i], other[i]);
+        *reinterpret_cast<Piece*>(residual_out + at) = raw;
     }
-    float sum = rms_slice_squares(raw.x, raw.y);
-    sum = half_wave_sum(sum);
-    if (t < 32) stage[t] = 0.0f;
+    float sum = rms_slice_squares(raw[0], raw[1]);
+    if constexpr (kPieces == 2) sum = row_sum(sum + rms_slice_squares(raw[2], raw[3]));
+    else sum = half_wave_sum(sum);
+    if (t % kLanes == 0) stage[t / kLanes] = sum;
     __syncthreads();
-    if ((t & 31) == 0) stage[t >> 5] = sum;
-    __syncthreads();
-    if (t < 32) {
-        float total = stage[t];
-        total = half_wave_sum(total);
-        if (t == 0) inverse_norm = rms_inverse(total, hidden);
+    // every wave sums the stage itself; slots without a group count as zeros
+    const uint32_t slot = t & 31;
+    const float inverse = rms_inverse(half_wave_sum(slot < hidden / 128 ? stage[slot] : 0.0f), hidden);
+    Piece result;
+#pragma unroll
+    for (uint32_t i = 0; i < 2 * kPieces; ++i) result[i] = rms_scale_pair(raw[i], wraw[i], inverse);
+    *reinterpret_cast<Piece*>(out + 4 * kPieces * t) = result;
+}
+
+// From this many rows on two slices a thread (fewer take as long either way).
+constexpr uint32_t kRmsBlockRows = 128;
+void launch_rms_rows(const uint16_t* input, const uint16_t* weight, uint16_t* output, uint32_t rows,
+                     uint32_t hidden, uint32_t in_stride, uint32_t out_stride, const uint16_t* addend,
+                     uint16_t* residual_out, uint32_t residual_stride, hipStream_t stream) {
+    const uintptr_t all = reinterpret_cast<uintptr_t>(input) | reinterpret_cast<uintptr_t>(weight) |
+                          reinterpret_cast<uintptr_t>(output) | reinterpret_cast<uintptr_t>(addend) |
+                          reinterpret_cast<uintptr_t>(residual_out) |
+                          (static_cast<uintptr_t>(in_stride | out_stride | residual_stride) * 2);
+    // (whole half waves of 32 lanes)
+    if (rows >= kRmsBlockRows && all % 16 == 0 && hidden % 256 == 0) {
+        hipLaunchKernelGGL(rms_only_kernel<2>, dim3(1, rows), dim3(hidden / 8), 0, stream, input, weight, output,
+                           hidden, in_stride, out_stride, addend, residual_out, residual_stride);
+    } else {
+        hipLaunchKernelGGL(rms_only_kernel<1>, dim3(1, rows), dim3(hidden / 4), 0, stream, input, weight, output,
+                           hidden, in_stride, out_stride, addend, residual_out, residual_stride);
     }
-    __syncthreads();
-    const float inverse = inverse_norm;
-    *reinterpret_cast<u32x2*>(out + 4 * t) =
-        u32x2{rms_scale_pair(raw.x, wraw.x, inverse), rms_scale_pair(raw.y, wraw.y, inverse)};
 }
 
 // out[r][n] = bf16(sum_k x[r][k] w[n][k]).  grid (ceil(N/64), ceil(rows/16)) x 256:
@@ -223,9 +238,7 @@ int32_t launch_rms(const Bindings& b, const Grid& g, hipStream_t stream, bool va
     uint16_t* output =
         a.buffer<uint16_t>(2, (static_cast<uint64_t>(rows - 1) * out_stride + hidden) * 2);
     if (a.status != TT_OK || validate_only) return a.status;
-    hipLaunchKernelGGL(rms_only_kernel, dim3(1, rows), dim3(hidden / 4), 0, stream, input, weight,
-                       output, hidden, in_stride, out_stride, static_cast<const uint16_t*>(nullptr),
-                       static_cast<uint16_t*>(nullptr), 0u);
+    launch_rms_rows(input, weight, output, rows, hidden, in_stride, out_stride, nullptr, nullptr, 0, stream);
     return TT_OK;
 }
 
@@ -257,8 +270,8 @@ int32_t launch_residual_rms(const Bindings& b, const Grid& g, hipStream_t stream
     const uint16_t* weight = a.buffer<const uint16_t>(3, static_cast<uint64_t>(hidden) * 2);
     uint16_t* normed = a.buffer<uint16_t>(4, extent(normed_stride));
     if (a.status != TT_OK || validate_only) return a.status;
-    hipLaunchKernelGGL(rms_only_kernel, dim3(1, rows), dim3(hidden / 4), 0, stream, first, weight,
-                       normed, hidden, a_stride, normed_stride, second, residual, lane_stride);
+    launch_rms_rows(first, weight, normed, rows, hidden, a_stride, normed_stride, second, residual, lane_stride,
+                    stream);
     return TT_OK;
 }
 int32_t op_residual_rms(const Bindings& b, const Grid& g, hipStream_t stream, bool validate_only) {

@@ -277,6 +277,44 @@ def test_norm_and_residual_sum_over_every_bf16_value():
                                   f"{want[differ[0]]:#06x}")
 
 
+@pytest.mark.parametrize("rows,hidden,gap", [(256, 256, 0), (128, 512, 0), (127, 512, 0), (130, 2048, 8),
+                                             (128, 4096, 0), (150, 384, 0), (140, 2048, 2)])
+def test_norm_and_residual_sum_of_a_block_bit_for_bit(rows, hidden, gap):
+    """rms_only_ms and residual_rms_ms of blocks: 128 rows and more take 16-byte pieces of a row
+    where every row has them (rows `gap` elements apart: 8 keeps the alignment, 2 does not; half
+    waves of 384 / 8 threads would not be whole), over every bf16 value and strided rows."""
+    print(f"[case] block norm rows={rows} hidden={hidden} gap={gap}", flush=True)
+    B, dev, queue, lib = gpu()
+    patterns = np.arange(65536, dtype=np.uint32).astype(np.uint16)
+    patterns[(patterns & 0x7F80) == 0x7F80] = 0
+    x = patterns[np.argsort(patterns & 0x7FFF, kind="stable")]
+    x = np.resize(x, rows * hidden).reshape(rows, hidden)
+    other = np.ascontiguousarray(np.roll(x.reshape(-1), 193) ^ np.uint16(0x8000)).reshape(rows, hidden)
+    w = ol.f32_to_bf16(1.0 + 0.1 * ol.gaussian_f32(0xE3, hidden))
+    x = np.ascontiguousarray(x)
+    want, sums, want_sum = (np.zeros((rows, hidden), np.uint16) for _ in range(3))
+    o.tto_rms_only(x.reshape(-1), w, rows, hidden, want.reshape(-1))
+    o.tto_add_bf16(x.reshape(-1), other.reshape(-1), rows * hidden, sums.reshape(-1))
+    o.tto_rms_only(sums.reshape(-1), w, rows, hidden, want_sum.reshape(-1))
+    stride = hidden + gap
+
+    def spread(a):
+        out = np.full((rows, stride), 0x7FC0, np.uint16)
+        out[:, :hidden] = a
+        return dev.buffer_from(out.reshape(-1))
+    b_x, b_y, b_w = spread(x), spread(other), dev.buffer_from(w)
+    b_norm, b_res, b_sum = (dev.create_buffer(rows * stride * 2) for _ in range(3))
+
+    def rec(cb):
+        cb.encode(lib.pipeline("rms_only_ms"), {0: b_x, 1: b_w, 2: b_norm}, {3: stride, 4: stride},
+                  (1, rows), (hidden // 4,))
+        cb.encode(lib.pipeline("residual_rms_ms"), {0: b_x, 1: b_y, 2: b_res, 3: b_w, 4: b_sum},
+                  {5: stride, 6: stride, 7: stride}, (1, rows), (hidden // 4,))
+    run(rec)
+    for what, got, expected in (("norm", b_norm, want), ("residual", b_res, sums), ("residual norm", b_sum, want_sum)):
+        assert np.array_equal(got.read(np.uint16).reshape(rows, stride)[:, :hidden], expected), what
+
+
 @pytest.mark.parametrize("rows,in_dim,out_dim", [(1, 2048, 9216), (4, 2048, 12352), (16, 4096, 2048),
                                                  (37, 2048, 4096), (3, 64, 70), (2, 2048, 70),
                                                  (13, 4096, 24)])
