@@ -1123,30 +1123,48 @@ __device__ __forceinline__ void request_parts(const float* base, uint32_t stride
         part_sum[d] = rec[kD + 1];
     }
 }
-// Merge of the first `nparts` (at most kParts) of the requested records.
+// the largest of a wave's values
+__device__ __forceinline__ float wave_max(float v) {
+    v = fmaxf(v, lane_dpp<0xB1>(v));    // the steps of row_sum
+    v = fmaxf(v, lane_dpp<0x4E>(v));
+    v = fmaxf(v, lane_dpp<0x141>(v));
+    v = fmaxf(v, lane_dpp<0x140>(v));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F)));   // lane ^ 16
+    return fmaxf(v, __shfl_xor(v, 32, 64));
+}
+// Merge of the first `nparts` (at most kParts, the same for all lanes) of the requested records.  A
+// wave's lanes take a record's maximum and weight each; the weights come back from their lanes one
+// by one as the numerators are added up.  (With every lane computing all weights the dispatch took
+// 4.6 / 6.8 / 9.5 us with 8 / 47 / 125 records, now 4.0 / 5.2 / 6.4.)
 template <uint32_t kParts>
 __device__ __forceinline__ MergedParts reduce_parts(const float (&numerator)[kParts], uint32_t nparts,
                                                     const float* part_max, const float* part_sum) {
+    constexpr uint32_t kEach = (kParts + 63) / 64;
+    const uint32_t lane = threadIdx.x & 63;
     MergedParts r{0.0f, 0.0f, -INFINITY};
+    float max_here[kEach], sum_here[kEach];
 #pragma unroll
-    for (uint32_t p = 0; p < kParts; p += 4) {
-        const f32x4 m4 = *reinterpret_cast<const f32x4*>(part_max + p);
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            if (p + u < nparts) r.gmax = fmaxf(r.gmax, m4[u]);
-        }
+    for (uint32_t j = 0; j < kEach; ++j) {
+        const uint32_t p = min(lane + 64 * j, kParts - 1);
+        max_here[j] = lane + 64 * j < nparts ? part_max[p] : -INFINITY;
+        sum_here[j] = part_sum[p];
+        r.gmax = fmaxf(r.gmax, max_here[j]);
     }
+    r.gmax = wave_max(r.gmax);
+    float weight[kEach], denom = 0.0f;
 #pragma unroll
-    for (uint32_t p = 0; p < kParts; p += 4) {
-        const f32x4 m4 = *reinterpret_cast<const f32x4*>(part_max + p);
-        const f32x4 s4 = *reinterpret_cast<const f32x4*>(part_sum + p);
+    for (uint32_t j = 0; j < kEach; ++j) {
+        weight[j] = max_here[j] == -INFINITY ? 0.0f : __expf(max_here[j] - r.gmax);
+        // (a slot without a record holds anything)
+        denom += lane + 64 * j < nparts ? weight[j] * sum_here[j] : 0.0f;
+    }
+    denom = half_wave_sum(denom);
+    r.denom = denom + __shfl_xor(denom, 32, 64);
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            if (p + u < nparts) {
-                const float w = m4[u] == -INFINITY ? 0.0f : __expf(m4[u] - r.gmax);
-                r.acc = fmaf(w, numerator[p + u], r.acc);
-                r.denom += w * s4[u];
-            }
+    for (uint32_t p = 0; p < kParts; ++p) {
+        if (p < nparts) {
+            const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight[p / 64]), p % 64));
+            r.acc = fmaf(w, numerator[p], r.acc);
         }
     }
     return r;
@@ -1202,7 +1220,7 @@ __device__ __forceinline__ void finish_row_head(const FinishArgs& a, uint32_t he
     const uint32_t context = entry[1];
     // a row the table places outside its cache has no records and no slot to append to
     if (context >= a.capacity) return;
-    const uint32_t nparts = (context + part - 1) / part;
+    const uint32_t nparts = __builtin_amdgcn_readfirstlane((context + part - 1) / part);   // the row's
     if (!kBalanced && nparts > a.record_splits) return;
     float c = 1.0f, sn = 0.0f;
     if (d < 2 * kAttnRopePairs) {
