@@ -34,7 +34,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
-typedef __attribute__((ext_vector_type(4))) short bf16x4_bits;
 
 constexpr uint32_t kQ4Block = 512;        // columns one pass of a 32-lane row group covers
 constexpr uint32_t kQ4Group = 64;         // columns per {scale, bias}
@@ -874,34 +873,34 @@ int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
 // The same mathematics as the block product for 2..16 input rows (a decode wave), sized for
 // latency: a workgroup owns 16 output rows and all input rows, its waves split K in slices
 // of 512 columns (eight groups each), every operand of a slice is requested before the
-// first is used, and the slices are summed through LDS in a fixed order.  Per group four
-// v_mfma_f32_16x16x16_bf16 multiply the x rows with the nibbles as bf16 16 + nibble (lane g
-// of a row owns the group's columns 16 g .. 16 g + 15) and four more, against a ones operand, give
+// first is used, and the slices are summed through LDS in a fixed order.  Per group two
+// v_mfma_f32_16x16x32_bf16 multiply the x rows with the nibbles as bf16 16 + nibble (lane g
+// of a row owns the group's columns 16 g .. 16 g + 15) and two more, against a ones operand, give
 // the group sums of x; then acc += scale[n] * products + bias[n] * sums in fp32.  The
 // result has n along its columns, so a lane needs one scale and one bias per group, and
 // reads all eight of a slice with two 16-byte loads.
 
 constexpr float kNibbleOffset = 16.0f;   // nibbles enter the matrix unit as 16 + nibble
 
-// nibbles 0..3 (upper = false) or 4..7 of `word` -> the four bf16 numbers 16 + nibble: a
-// nibble dropped into mantissa bits 3..6 of bf16 16.0 (0x4180), where it counts units.  The
-// offset leaves the products as 16 * (sum of x) too much, which the caller takes out of the
-// bias term; 16 is the smallest offset that keeps all sixteen values in one binade, and
-// keeps the fp32 partial sums about three times as large as the plain ones.
-template <bool upper>
-__device__ __forceinline__ bf16x4_bits offset_four(uint32_t word) {
-    constexpr uint32_t kBase = 0x41804180u, kLow = 0x00000078u, kHigh = 0x00780000u;
-    // nibble i sits at bits 4 i .. 4 i + 3; the even one of a pair goes to bits 3..6, the
-    // odd one to bits 19..22
-    u32x2 out;
-    if (!upper) {
-        out[0] = ((word << 15) & kHigh) | (((word << 3) & kLow) | kBase);   // nibbles 0, 1
-        out[1] = ((word << 7) & kHigh) | (((word >> 5) & kLow) | kBase);    // nibbles 2, 3
-    } else {
-        out[0] = ((word >> 1) & kHigh) | (((word >> 13) & kLow) | kBase);   // nibbles 4, 5
-        out[1] = ((word >> 9) & kHigh) | (((word >> 21) & kLow) | kBase);   // nibbles 6, 7
-    }
-    return __builtin_bit_cast(bf16x4_bits, out);
+// The eight nibbles of `word` as the bf16 numbers 16 + nibble, in pairs 0 and 4, 1 and 5, 2 and 6, 3
+// and 7: a nibble dropped into mantissa bits 3..6 of bf16 16.0 (0x4180), where it counts units, a
+// shift, a mask and an or for two.  The offset leaves the products as 16 * (sum of x) too much, which the
+// caller takes out of the bias term; 16 is the smallest offset that keeps all sixteen values in one
+// binade, and keeps the fp32 partial sums about three times as large as the plain ones.
+__device__ __forceinline__ bf16x8 offset_eight(uint32_t word) {
+    uint32_t sixteens = 0x41804180u;
+    asm("" : "+v"(sixteens));   // kept in a register: one v_and_or_b32 instead of two instructions
+    u32x4 out;
+    out[0] = ((word << 3) & 0x00780078u) | sixteens;
+    out[1] = ((word >> 1) & 0x00780078u) | sixteens;
+    out[2] = ((word >> 5) & 0x00780078u) | sixteens;
+    out[3] = ((word >> 9) & 0x00780078u) | sixteens;
+    return __builtin_bit_cast(bf16x8, out);
+}
+// eight values of x in that order
+__device__ __forceinline__ u32x4 paired_eight(u32x4 x) {
+    return u32x4{__builtin_amdgcn_perm(x[2], x[0], 0x05040100u), __builtin_amdgcn_perm(x[2], x[0], 0x07060302u),
+                 __builtin_amdgcn_perm(x[3], x[1], 0x05040100u), __builtin_amdgcn_perm(x[3], x[1], 0x07060302u)};
 }
 
 // The eight nibbles of `word` less 8, as bf16, for a block of 2..16 rows.  A block used to be
@@ -961,6 +960,8 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
         scale_bits = *reinterpret_cast<const u32x4*>(scales);
         bias_bits = *reinterpret_cast<const u32x4*>(biases);
     };
+    // as the nibbles of a word come apart
+    const auto in_order = [](u32x4 eight) { return kCentred ? eight : paired_eight(eight); };
     if constexpr (kNorm) {
         // The rows go through the RMS norm on their way into LDS, bit for bit as the norm
         // operator does it with one thread per four values: a thread here holds eight
@@ -1005,7 +1006,7 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
                 u32x4 normed;
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) normed[j] = rms_scale_pair(raw[r][j], weight[j], inverse[r]);
-                *reinterpret_cast<u32x4*>(wave_lds + r * kWaveRowBytes<kWaves> + threadIdx.x * 16) = normed;
+                *reinterpret_cast<u32x4*>(wave_lds + r * kWaveRowBytes<kWaves> + threadIdx.x * 16) = in_order(normed);
             }
         }
     } else {
@@ -1026,7 +1027,7 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
 #pragma unroll
             for (uint32_t r = 0; r < kRowsMax; ++r) {
                 *reinterpret_cast<u32x4*>(wave_lds + min(r, p.rows - 1) * kWaveRowBytes<kWaves> +
-                                          threadIdx.x * 16) = raw[r];
+                                          threadIdx.x * 16) = in_order(raw[r]);
             }
         } else {
             for (uint32_t first = 0; first < p.rows; first += 4) {
@@ -1040,7 +1041,7 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) {
                     *reinterpret_cast<u32x4*>(wave_lds + min(first + j, p.rows - 1) * kWaveRowBytes<kWaves> +
-                                              threadIdx.x * 16) = staged[j];
+                                              threadIdx.x * 16) = in_order(staged[j]);
                 }
             }
             request_weights();
@@ -1050,7 +1051,9 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
 
     const uint8_t* x_row = wave_lds + min(i16, p.rows - 1) * kWaveRowBytes<kWaves> +
                            first_group * (kQ4Group * 2) + 32 * g;
-    const bf16x4_bits ones = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+    bf16x8 eight_ones;
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) eight_ones[j] = static_cast<__bf16>(1.0f);
     const f32x4 zero = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     f32x4 acc = zero;
     [[maybe_unused]] double wide[4] = {0.0, 0.0, 0.0, 0.0};
@@ -1059,38 +1062,25 @@ __global__ __launch_bounds__(64 * kWaves) void q4_wave_kernel(Q4Projection p) {
         const u32x4 x_low = *reinterpret_cast<const u32x4*>(x_row + group * (kQ4Group * 2));
         const u32x4 x_high = *reinterpret_cast<const u32x4*>(x_row + group * (kQ4Group * 2) + 16);
         f32x4 products = zero, sums = zero;
-        if constexpr (kCentred) {
-            bf16x8 eight_ones;
 #pragma unroll
-            for (uint32_t j = 0; j < 8; ++j) eight_ones[j] = static_cast<__bf16>(1.0f);
-#pragma unroll
-            for (uint32_t j = 0; j < 2; ++j) {
-                const bf16x8 xf = __builtin_bit_cast(bf16x8, j == 0 ? x_low : x_high);
-                products = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, centred_eight(q[group][j]), products,
-                                                                   0, 0, 0);
-                sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, eight_ones, sums, 0, 0, 0);
-            }
-            const float scale = widen_half(scale_bits[group >> 1], group & 1);
-            const float bias = fmaf(8.0f, scale, widen_half(bias_bits[group >> 1], group & 1));
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) wide[i] += fmaf(scale, products[i], bias * sums[i]);
-            continue;
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const u32x4 half = j < 2 ? x_low : x_high;
-            const u32x2 x_bits = {half[2 * (j & 1)], half[2 * (j & 1) + 1]};
-            const bf16x4_bits xf = __builtin_bit_cast(bf16x4_bits, x_bits);
-            const uint32_t word = q[group][j >> 1];
-            const bf16x4_bits qf = (j & 1) ? offset_four<true>(word) : offset_four<false>(word);
-            products = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xf, qf, products, 0, 0, 0);
-            sums = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xf, ones, sums, 0, 0, 0);
+        for (uint32_t j = 0; j < 2; ++j) {
+            const bf16x8 xf = __builtin_bit_cast(bf16x8, j == 0 ? x_low : x_high);
+            const bf16x8 qf = kCentred ? centred_eight(q[group][j]) : offset_eight(q[group][j]);
+            products = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, qf, products, 0, 0, 0);
+            sums = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xf, eight_ones, sums, 0, 0, 0);
         }
         const float scale = widen_half(scale_bits[group >> 1], group & 1);
-        // scale * (products - 16 sums) + bias * sums
-        const float bias = fmaf(-kNibbleOffset, scale, widen_half(bias_bits[group >> 1], group & 1));
+        // scale * (products + kBack sums) + bias * sums
+        constexpr float kBack = kCentred ? 8.0f : -kNibbleOffset;
+        const float bias = fmaf(kBack, scale, widen_half(bias_bits[group >> 1], group & 1));
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) acc[i] = fmaf(bias, sums[i], fmaf(scale, products[i], acc[i]));
+        for (uint32_t i = 0; i < 4; ++i) {
+            if constexpr (kCentred) {
+                wide[i] += fmaf(scale, products[i], bias * sums[i]);
+            } else {
+                acc[i] = fmaf(bias, sums[i], fmaf(scale, products[i], acc[i]));
+            }
+        }
     }
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
