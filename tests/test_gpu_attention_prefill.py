@@ -268,7 +268,7 @@ def test_merged_walk_with_a_share_in_the_exact_loop():
 
 def test_shared_walk_of_a_2048_row_block_deep_in_a_cache():
     """The shape the operator is for: a 2048-row block behind 6144 cached tokens, as many shares
-    as fill the device (two on 256 compute units); sampled rows against the checker, every row
+    as fill the device (two on 256 compute units); sampled rows against the oracle, every row
     against the one-workgroup operator."""
     B, dev, queue, lib = gpu()
     splits = B.flash_prefill_splits(2048, 8192, dev.compute_units)

@@ -157,7 +157,7 @@ def test_element_wise_block_kernels_at_every_rows_per_group(rows):
 def test_conv_with_gates_and_gate_norm_from_the_projection(rows, in_place):
     """gdn_conv_gates_blk and gdn_gate_norm_proj_blk either side of the 8 rows a workgroup gates,
     of the 16 from which the gate-norm is vectorised and at 1, 2 and 6 rows a workgroup: the
-    checker's bit patterns, and gdn_gates_blk's decay and beta bit for bit."""
+    oracle's bit patterns, and gdn_gates_blk's decay and beta bit for bit."""
     print(f"[case] gdn conv with gates rows={rows} in place={in_place}", flush=True)
     B, dev, queue, lib = gpu()
     weights = _weights()

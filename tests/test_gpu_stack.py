@@ -380,7 +380,7 @@ def test_dense_bf16_block_kernel(rows, in_dim, out_dim):
 
 @pytest.mark.parametrize("tile,rows,in_dim,out_dim", DENSE_TILE_CASES, ids=lambda v: str(v))
 def test_dense_bf16_block_tiles(tile, rows, in_dim, out_dim):
-    """The tiles a block is launched with, at their edges: sampled rows against the checker,
+    """The tiles a block is launched with, at their edges: sampled rows against the oracle,
     every output stored."""
     print(f"[case] dense_bf16 tile {tile} rows={rows} in={in_dim} out={out_dim}", flush=True)
     B, dev, queue, lib = gpu()
@@ -393,7 +393,7 @@ def test_dense_bf16_block_tiles(tile, rows, in_dim, out_dim):
 
 @pytest.mark.parametrize("shape,rows,in_dim,out_dim", REFINED_TILE_CASES, ids=lambda v: str(v))
 def test_dense_bf16_refined_tiles(shape, rows, in_dim, out_dim):
-    """The tiles that fill the rounds better, at their edges: sampled rows against the checker,
+    """The tiles that fill the rounds better, at their edges: sampled rows against the oracle,
     every output stored."""
     print(f"[case] dense_bf16 tile {shape} rows={rows} in={in_dim} out={out_dim}", flush=True)
     B, dev, queue, lib = gpu()
