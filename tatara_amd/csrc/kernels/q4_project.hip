@@ -281,9 +281,9 @@ int32_t launch_rows(const Q4Projection& p, hipStream_t stream) {
 // A scale has 8 significant bits and nibble - 8 (-8 .. 7) three or a power of two, so their
 // product has at most 11: an f16 number, exactly.  So is x, of 8 bits.  Both are brought into
 // f16's range by a power of two per row (an output row's largest of 8 |scale| and |bias| below
-// 2^14, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): an x that
+// 2^15, an input row's largest |x| below 2^9, so that its group sums stay below 2^15): an x that
 // lies so far below the row's largest that f16 rounds it is off by 2^-33 of that one at most, a
-// weight by 2^-38.  The affine terms are four further columns a group, {bias, 8 scale, bias,
+// weight by 2^-39.  The affine terms are four further columns a group, {bias, 8 scale, bias,
 // 8 scale} against {hi, hi, lo, lo} of the group sum in two f16 parts, 2^-23 of the sum at most
 // from it: the largest of these roundings, about one of the fp32 sums' own.  One pass writes both
 // operands so into the queue's workspace; the product is then a plain one (block_product.h) and the
@@ -331,18 +331,19 @@ __device__ __forceinline__ uint32_t unfolded_piece(uint32_t piece) {
     const uint32_t within = piece % kSpan;
     return piece - within + within % 4 * (kSpan / 4) + within / 4;
 }
-// Nibbles i and i + 4 of `word`, less 8, times the steps, exactly: a nibble in bits 6 .. 9 of
-// f16 16.0 counts units, and both (16 + nibble) step and 24 step (of 10 bits) are what the fused
-// multiply-add says they are.  A shift, a mask and an add for two weights.
-__device__ __forceinline__ f16x2 unfold_offset(f16x2 steps) {
-    return steps * f16x2{static_cast<_Float16>(-24.0f), static_cast<_Float16>(-24.0f)};
-}
-__device__ __forceinline__ uint32_t unfold_pair(uint32_t word, uint32_t i, f16x2 steps, f16x2 offset) {
-    const uint32_t there = i == 0 ? word << 6 : i == 1 ? word << 2 : i == 2 ? word >> 2 : word >> 6;
-    uint32_t sixteens = 0x4C004C00u;
-    asm("" : "+v"(sixteens));   // kept in a register: one v_and_or_b32 instead of two instructions
-    const uint32_t pair = (there & 0x03C003C0u) | sixteens;
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, pair), steps, offset));
+// Nibbles i and i + 4 of `word`, less 8, times the steps: the nibbles in the lowest four bits of f16
+// 1024.0, or in the four above of 64.0, where they count units; less 1032 or 72 they are n - 8, exactly.
+// Eight weights are a shift, four and-ors, four sums and four products.  (16 + n from one position and a
+// fused multiply-add are 12 instructions instead of 13, gdn_project of 17 / 100 / 256 rows 12.65 / 20.2 / 36.4 us
+// instead of 12.8 / 20.4 / 36.6, but the 24 steps it takes off must fit f16: the row's largest below 2^14,
+// and a bit less of the small steps beside it.)
+__device__ __forceinline__ uint32_t unfold_pair(uint32_t word, uint32_t i, f16x2 steps) {
+    const bool lowest = i % 2 == 0;
+    uint32_t base = lowest ? 0x64006400u : 0x54005400u;
+    asm("" : "+v"(base));   // kept in a register: one v_and_or_b32 instead of two instructions
+    const uint32_t pair = ((i < 2 ? word : word >> 8) & (lowest ? 0x000F000Fu : 0x00F000F0u)) | base;
+    const _Float16 less = static_cast<_Float16>(lowest ? 1032.0f : 72.0f);
+    return __builtin_bit_cast(uint32_t, (__builtin_bit_cast(f16x2, pair) - f16x2{less, less}) * steps);
 }
 
 // the largest of four values, one to a row of 16 lanes
@@ -380,18 +381,17 @@ __global__ __launch_bounds__(256) void q4_unfold_kernel(Q4Projection p, Unfold u
         // over the lanes of other groups of eight
         largest = fmaxf(largest, lane_dpp<0x128>(largest));   // row_ror:8
         largest = wave_largest_of_rows(largest);
-        const int32_t shift = shift_below(largest, 14);
+        const int32_t shift = shift_below(largest, 15);
         if (lane == 0) u.weight_exponents[row] = -shift;
         _Float16* out = u.weights + static_cast<uint64_t>(row) * kColumns;
 #pragma unroll
         for (uint32_t b = 0; b < kBlocks; ++b) {
             const _Float16 step = static_cast<_Float16>(ldexpf(scale[b], shift));
             const f16x2 steps = f16x2{step, step};
-            const f16x2 offset = unfold_offset(steps);
             u32x4 eight;
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
-                eight[i] = unfold_pair(packed[b], i, steps, offset);
+                eight[i] = unfold_pair(packed[b], i, steps);
             }
             *reinterpret_cast<u32x4*>(out + b * kQ4Block + lane * 8) = eight;
             if ((lane & 7) == 0) {
@@ -599,14 +599,14 @@ __global__ __launch_bounds__(512, Product::kWavesPerSimd) void q4_short_kernel(Q
         }
         largest = fmaxf(largest, __shfl_xor(largest, 16));
         largest = fmaxf(largest, __shfl_xor(largest, 32));
-        shift[tn] = shift_below(largest, 14);
+        shift[tn] = shift_below(largest, 15);
         if (kh == 0 && g == 0) {
             *reinterpret_cast<int32_t*>(short_lds + kRing * Product::kUnitBytes +
                                         (nw * 32 + tn * 16 + i16) * 4) = -shift[tn];
         }
     }
     // the step of span s: of its groups the one of number 2 kh + (g >> 1), all held by lane group s
-    f16x2 steps[2][kSpans], offsets[2][kSpans];
+    f16x2 steps[2][kSpans];
 #pragma unroll
     for (uint32_t tn = 0; tn < 2; ++tn) {
         const u32x4 held = scale_bits[tn][kBlocks == 4 ? 0 : kh >> 2];
@@ -618,7 +618,6 @@ __global__ __launch_bounds__(512, Product::kWavesPerSimd) void q4_short_kernel(Q
                 static_cast<uint32_t>(__shfl(static_cast<int>(mine), span * 16 + i16));
             const _Float16 step = static_cast<_Float16>(ldexpf(widen_half(pair, g >> 1), shift[tn]));
             steps[tn][span] = f16x2{step, step};
-            offsets[tn][span] = unfold_offset(steps[tn][span]);
         }
     }
 
@@ -678,7 +677,7 @@ __global__ __launch_bounds__(512, Product::kWavesPerSimd) void q4_short_kernel(Q
             u32x4 eight;
 #pragma unroll
             for (uint32_t i = 0; i < 4; ++i) {
-                eight[i] = unfold_pair(words[tn][span][j], i, steps[tn][span], offsets[tn][span]);
+                eight[i] = unfold_pair(words[tn][span][j], i, steps[tn][span]);
             }
             w[tn] = __builtin_bit_cast(f16x8, eight);
         }

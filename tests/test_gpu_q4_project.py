@@ -276,6 +276,47 @@ def test_block_projection_with_the_weights_unpacked_in_the_product(family, name,
 
 @pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
                                          (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
+@pytest.mark.parametrize("rows", [17, 100, 600])
+def test_block_projection_keeps_scales_far_below_the_largest_of_their_row(family, name, rows):
+    """Every output row has a group of scale 1 whose inputs are zero, and scales of 129 to 255 times 2^-35
+    beside it: with the largest of 8 |scale| brought below 2^15 each of those is a whole number of f16's
+    smallest subnormals, with one bit less room the odd ones are not.  Inputs are small whole numbers
+    and the biases take the nibbles' offset of 8 out, so that every sum is exact and the result correctly
+    rounded, by either route of a block (17 and 100 rows unpack the weights in the product, 600 do not)."""
+    print(f"[case] {name} rows={rows} scales far below their row's largest", flush=True)
+    B, dev, queue, lib = gpu()
+    rng = np.random.default_rng(0xB0 + rows)
+    k, total = family["k"], sum(family["segments"])
+    x = rng.integers(-2, 3, (rows, k)) * (rng.random((rows, k)) < 0.05)
+    x[:, :64] = 0
+    bindings, want = {0: dev.buffer_from(ol.f32_to_bf16(x.astype(np.float32).reshape(-1)))}, []
+    for index, n in enumerate(family["segments"]):
+        words = rng.integers(0, 2 ** 32, n * k // 8, dtype=np.uint64).astype(np.uint32)
+        units = rng.integers(64, 128, n) * 2 + 1
+        scale = np.repeat(units[:, None] * 2.0 ** -35, k // 64, axis=1)
+        scale[:, 0] = 1.0
+        slot = 1 + 3 * index
+        bindings.update({slot: dev.buffer_from(words),
+                         slot + 1: dev.buffer_from(ol.f32_to_bf16(scale.astype(np.float32).reshape(-1))),
+                         slot + 2: dev.buffer_from(ol.f32_to_bf16((-8.0 * scale).astype(np.float32).reshape(-1)))})
+        nibbles = ((words[:, None] >> (4 * np.arange(8, dtype=np.uint32))[None, :]) & 15).reshape(n, k)
+        sums = x.astype(np.float64) @ (nibbles.astype(np.float64) - 8.0).T * units
+        assert np.abs(sums).max() < 2 ** 24
+        want.append((sums * 2.0 ** -35).astype(np.float32))
+    out = dev.buffer_from(np.full(rows * total, 0x7FC0, np.uint16))      # NaN until written
+    bindings[family["out"]] = out
+    slot = family["out"] + 1
+    constants = {slot: rows, slot + 1: k} if family is OUT else {slot: rows}
+    run(lambda cb: cb.encode(lib.pipeline(name), bindings, constants, (_groups(family), 1, 1),
+                             (family["threads"], 1, 1)))
+    got = ol.bf16_to_f32(out.read(np.uint16))
+    want = ol.bf16_to_f32(ol.f32_to_bf16(np.concatenate(want, axis=1).reshape(-1)))
+    assert np.count_nonzero(want) > want.size // 2
+    assert np.array_equal(got, want), f"{np.mean(got != want):.4f} of the outputs differ"
+
+
+@pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
+                                         (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
 @pytest.mark.parametrize("rows", [17, 300, 1500])
 def test_block_projection_in_queues_of_less_workspace(family, name, rows):
     """A queue that could not have its whole workspace takes the operands through in slices of output
