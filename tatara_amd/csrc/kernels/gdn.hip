@@ -865,10 +865,11 @@ constexpr uint32_t kKeyRecK = 0;
 constexpr uint32_t kKeyRecQ = 16384;
 constexpr uint32_t kKeyRecBytes = 32768;
 constexpr uint32_t kChunkKeys = kGdnValueHeads * kRecordBytes;
-constexpr uint32_t kChunkRecords = kChunkKeys + kGdnKeyHeads * kKeyRecBytes;
-// what a caller binds, per chunk and head
+// What a caller binds, per chunk and head, and where the next chunk's records begin: a caller that
+// prepares or scans a block in parts finds each part's records at its first chunk's place.
 constexpr uint32_t kRecBytes = 115712;
-static_assert(kRecordBytes % 256 == 0 && kChunkRecords <= kGdnValueHeads * kRecBytes);
+constexpr uint32_t kChunkStride = kGdnValueHeads * kRecBytes;
+static_assert(kRecordBytes % 256 == 0 && kChunkKeys + kGdnKeyHeads * kKeyRecBytes <= kChunkStride);
 
 struct ChunkPrepareArgs {
     const uint16_t* qk;      // [rows][4096]
@@ -958,7 +959,7 @@ __global__ __launch_bounds__(256, 4) void gdn_chunk_prepare_kernel(ChunkPrepareA
     const uint32_t g = lane >> 4;
     const uint32_t t0 = chunk * kChunk;
     const uint32_t valid = min(kChunk, a.rows - t0);
-    uint8_t* records = a.scratch + static_cast<uint64_t>(chunk) * kChunkRecords;
+    uint8_t* records = a.scratch + static_cast<uint64_t>(chunk) * kChunkStride;
     uint8_t* rec = records + h * kRecordBytes;
     uint8_t* key_rec = records + kChunkKeys + kh * kKeyRecBytes;
 
@@ -1352,7 +1353,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {
     const uint32_t at = w * 16 + g * 4;  // this lane's token rows of a chunk
     const uint32_t at_slot = 32 * (w >> 1) + 8 * g + 4 * (w & 1);   // where they stand in r_hi, r_lo
     const auto records_of = [&](uint32_t chunk) {
-        return a.scratch + static_cast<uint64_t>(chunk) * kChunkRecords;
+        return a.scratch + static_cast<uint64_t>(chunk) * kChunkStride;
     };
 
     if (state_wave) {

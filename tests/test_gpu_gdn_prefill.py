@@ -421,6 +421,47 @@ def test_chunked_recurrence_in_place_and_chained_blocks():
     assert np.array_equal(conv_in, ref["conv"])
 
 
+@pytest.mark.parametrize("first", [64, 192])
+@pytest.mark.parametrize("parted", ["prepare", "scan"])
+def test_either_stage_of_the_chunked_recurrence_in_parts(parted, first):
+    """A block of 300 rows prepared in two parts and scanned at once, or prepared at once and scanned in
+    two parts (to take the state between them): a part's records begin at its first chunk's place,
+    32 records of 115,712 bytes a chunk, and results are those of whole stages, bit for bit."""
+    rows = 300
+    print(f"[case] gdn chunked recurrence, {parted} in parts of {first} and {rows - first} rows", flush=True)
+    B, dev, queue, lib = gpu()
+    weights = _weights()
+    proj, conv_state, state = _block(rows, 0x5500)
+    bufs = _buffers(dev, proj, conv_state, state, weights, rows)
+
+    def rec(cb):
+        _encode_front(cb, lib, bufs, rows)
+        _encode_chunked(cb, lib, bufs, rows)
+    run(rec)
+    y, state_out = bufs["y"].read(np.uint16), bufs["state_out"].read(np.float32)
+    chunk_bytes = 32 * 115712
+    records = dev.create_buffer((rows + 63) // 64 * chunk_bytes)
+    y2, state2 = dev.create_buffer(rows * 8192), dev.create_buffer(STATE * 4)
+    parts = ((0, first), (first, rows - first))
+
+    def in_parts(cb):
+        for start, count in parts if parted == "prepare" else ((0, rows),):
+            cb.encode(lib.pipeline("gdn_chunk_prepare_blk"),
+                      {0: (bufs["qk"], start * 8192), 1: (bufs["value"], start * 8192),
+                       2: (bufs["decay"], start * 128), 3: (bufs["beta"], start * 128),
+                       4: (records, start // 64 * chunk_bytes)}, {5: count}, ((count + 63) // 64, 32, 1),
+                      (256, 1, 1))
+        cb.barrier()
+        for start, count in parts if parted == "scan" else ((0, rows),):
+            cb.encode(lib.pipeline("gdn_chunk_scan_blk"),
+                      {0: (records, start // 64 * chunk_bytes), 1: bufs["state_in"] if start == 0 else state2,
+                       2: (y2, start * 8192), 3: state2}, {4: count}, (8, 32, 1), (256, 1, 1))
+            cb.barrier()
+    run(in_parts)
+    assert np.array_equal(y2.read(np.uint16), y)
+    assert np.array_equal(state2.read(np.float32), state_out)
+
+
 def test_chunked_recurrence_validation():
     B, dev, queue, lib = gpu()
     rows = 100
