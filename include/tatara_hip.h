@@ -355,6 +355,10 @@ uint32_t tt_block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                uint32_t compute_units);
 uint32_t tt_block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                 uint32_t compute_units);
+/* Which rounds of its tiles the workgroups of an XCD take in runs of consecutive ones: 1 the whole
+ * rounds, 2 the last one, 3 both, 0 none.  For tests and measurements as well. */
+uint32_t tt_block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
+                               uint32_t compute_units);
 
 #ifdef __cplusplus
 }

@@ -34,7 +34,7 @@ EXPORTED_SYMBOLS = [
     "tt_event_create", "tt_event_destroy", "tt_encode_signal_event", "tt_encode_wait_for_event",
     "tt_split_workgroups", "tt_choose_split_keys",
     "tt_flash_prefill_splits", "tt_flash_prefill_scratch_bytes", "tt_block_product_tile",
-    "tt_block_product_shape",
+    "tt_block_product_shape", "tt_block_product_runs",
 ]
 
 
@@ -114,6 +114,7 @@ def lib():
         "tt_flash_prefill_splits": (u32, [u32, u32, u32]),
         "tt_block_product_tile": (u32, [u32] * 4),
         "tt_block_product_shape": (u32, [u32] * 4),
+        "tt_block_product_runs": (u32, [u32] * 4),
         "tt_flash_prefill_scratch_bytes": (u64, [u32, u32]),
         "tt_event_create": (i32, [vp, pvp]), "tt_event_destroy": (None, [vp]),
         "tt_encode_signal_event": (i32, [vp, vp, u64]),
@@ -514,6 +515,13 @@ def block_product_shape(rows, in_dim, out_dim, compute_units=256):
     """(rows, outputs) of the tile that is launched (tt_block_product_shape)."""
     shape = lib().tt_block_product_shape(int(rows), int(in_dim), int(out_dim), int(compute_units))
     return shape >> 16, shape & 0xFFFF
+
+
+def block_product_runs(rows, in_dim, out_dim, compute_units=256):
+    """(whole rounds, the last round): whether a block product deals them in runs per XCD
+    (tt_block_product_runs)."""
+    runs = lib().tt_block_product_runs(int(rows), int(in_dim), int(out_dim), int(compute_units))
+    return bool(runs & 1), bool(runs & 2)
 
 
 def flash_prefill_splits(rows, visible_keys, compute_units=256):

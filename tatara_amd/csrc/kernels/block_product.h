@@ -34,6 +34,9 @@ __device__ __forceinline__ void block_transfer(const uint8_t* base, uint32_t off
                  : "memory");
 }
 
+// the rounds of tiles dealt in runs (block_launch); of the first, the workgroups mod 8 and by 8
+constexpr uint32_t kWholeRounds = 1, kLastRound = 2, kRunsMore = 2, kRunsShare = 5;
+
 // s_waitcnt until at most `left` (< 64) transfers are in flight
 constexpr uint32_t block_vmcnt(uint32_t left) { return 0x0F70u | (left & 15u) | ((left >> 4) << 14); }
 
@@ -109,11 +112,15 @@ struct BlockProduct {
     }
 
     // x [rows][in_dim], weights [out_dim][in_dim], in_dim a multiple of 64; 16-byte aligned and
-    // each smaller than 4 GiB.  store(m, n, sums) gets the sums of row m, columns n .. n + 3.
+    // each smaller than 4 GiB.  runs: the rounds dealt in runs, block_launch's.  store(m, n, sums) gets the
+    // sums of row m, columns n .. n + 3.
     template <typename Store>
     static __device__ __forceinline__ void run(const void* x, const void* weights, uint32_t rows,
-                                               uint32_t in_dim, uint32_t out_dim, Store store) {
+                                               uint32_t in_dim, uint32_t out_dim, uint32_t runs, Store store) {
         extern __shared__ __align__(16) uint8_t block_lds[];
+        // one wait for all arguments: fetched where each is used, a short product waits three times
+        const uint32_t workgroups = gridDim.x;
+        asm volatile("" ::"s"(x), "s"(weights), "s"(workgroups));
         const uint32_t lane = threadIdx.x & 63;
         const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         const uint32_t i16 = lane & 15, g = lane >> 4;
@@ -258,19 +265,26 @@ struct BlockProduct {
             multiply(second, bool_constant<true>{}, unit + 1, 0, first_of_next, with_request, unit + kRing);
         };
 
-        // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own: of
-        // a round's tiles, filled or not, the workgroups of an XCD (b / 8 = 0, 1, ...) take a run of
-        // consecutive ones - the operand panels a patch shares are then fetched into one L2 once
-        // instead of into several.  (Only for whole rounds of a multiple of eight workgroups, and
-        // otherwise in dispatch order: 777 x 2048 x 12352, one round of 245 tiles, 49 us instead of 39.5, and
-        // 1000 x 2048 x 9216 53 instead of 40; 300 x 2048 x 12352, 256 and 35 tiles, 33 instead of 26.)
-        const uint32_t xcd = blockIdx.x & 7;
-        auto of_round = [&](uint32_t first) {
-            const uint32_t count = min(gridDim.x, tiles - min(first, tiles));
-            const uint32_t share = count / 8, more = count % 8, at = blockIdx.x >> 3;
-            return at < share + (xcd < more ? 1 : 0) ? first + xcd * share + min(xcd, more) + at : tiles;
+        // Workgroup b of the dispatch order runs on XCD b mod 8, each XCD with an L2 of its own.  Dealt
+        // in runs, the workgroups of an XCD (b / 8 = 0, 1, ...) take consecutive tiles of a round - the
+        // operand panels a patch shares are then fetched into one L2 once instead of into several;
+        // otherwise a workgroup takes the tile of its number (see block_launch).
+        const auto in_runs = [&](uint32_t share, uint32_t more) {   // of a round of 8 share + more tiles
+            const uint32_t xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+            return at < share + (xcd < more ? 1 : 0) ? xcd * share + min(xcd, more) + at : tiles;
         };
-        uint32_t round = 0, tile = of_round(0);
+        const auto of_round = [&](uint32_t first) {
+            const uint32_t left = tiles - min(first, tiles);
+            if ((runs & (left >= workgroups ? kWholeRounds : kLastRound)) == 0) return first + blockIdx.x;
+            const uint32_t count = min(workgroups, left);
+            return first + in_runs(count / 8, count % 8);
+        };
+        // (the first round without of_round's work, of which a short product would wait for every instruction)
+        uint32_t round = 0, tile = blockIdx.x;
+        if (runs & kWholeRounds) {
+            asm volatile("");   // a branch
+            tile = in_runs(runs >> kRunsShare, runs >> kRunsMore & 7);
+        }
         if (tile >= tiles) return;
         aim(tile);
         const uint32_t ahead = min(kRing, units);
@@ -304,7 +318,7 @@ struct BlockProduct {
 
             uint32_t m0, n0;
             place(tile, m0, n0);
-            round += gridDim.x;
+            round += workgroups;
             const uint32_t next_tile = of_round(round);
             __syncthreads();   // nobody reads the stages any more
             if (next_tile < tiles) {
@@ -456,14 +470,30 @@ struct BlockTiles {
     }
 };
 
-// workgroups of a launch: a persistent one per place on the device, or one per tile
+// A launch: its workgroups, a persistent one per place on the device or one per tile, and the rounds of
+// tiles that an XCD's workgroups take in runs.  Tiles are numbered down bands of eight tile rows (place):
+// in a whole band the tile of a workgroup's own number gives an XCD one row of tiles, a good share by
+// itself, in a lower band the rows shift from column to column.  So every round goes in runs where there is
+// one lower band of many tiles, or a wide product over a long K; otherwise whole rounds of a multiple of
+// eight workgroups do.  In runs and without, bf16:
+//   777 x 2048 x 12352, one round of 5 x 49 tiles, 39.5 and 49.5 us; 1000 x 2048 x 9216 (7 x 36) 39.5 and 53;
+//   300 x 2048 x 12352 (5 x 193) 25 and 32.5; 2500 x 2048 x 9216 (20 x 72) 108 and 111
+//   776 x 256 x 1119 (13 x 18) 5.5 and 5.1; 3380 x 960 x 1083 (27 x 9) 18.7 and 17.3; 11448 x 640 x 533 (90 x 5)
+//   22.7 and 21.6; 4431 x 3776 x 104 (70 x 2) 13.8 and 13.2; 74 x 256 x 1023 (3 x 16) 3.85 and 3.70
+struct BlockLaunch {
+    uint32_t workgroups, runs;
+};
 template <typename Product>
-uint32_t block_workgroups(uint32_t rows, uint32_t out_dim, uint32_t compute_units) {
+BlockLaunch block_launch(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
     const uint32_t per_unit = 160 * 1024 / Product::kLdsBytes;
-    const uint32_t tiles = ((rows + Product::kTileM - 1) / Product::kTileM) *
-                           ((out_dim + Product::kTileN - 1) / Product::kTileN);
+    const uint32_t m_tiles = (rows + Product::kTileM - 1) / Product::kTileM;
+    const uint32_t n_tiles = (out_dim + Product::kTileN - 1) / Product::kTileN;
     const uint32_t places = compute_units * (per_unit < 2 ? per_unit : 2);
-    return tiles < places ? tiles : places;
+    const uint32_t workgroups = std::min(m_tiles * n_tiles, places);
+    const bool low = m_tiles < 8 && m_tiles * n_tiles >= 128 && in_dim >= 256;
+    const bool wide = m_tiles >= 8 && n_tiles >= 16 && in_dim >= 1024;
+    const uint32_t rounds = low || wide ? kWholeRounds | kLastRound : workgroups % 8 == 0 ? kWholeRounds : 0;
+    return {workgroups, rounds | workgroups % 8 << kRunsMore | workgroups / 8 << kRunsShare};
 }
 
 }  // namespace

@@ -459,9 +459,9 @@ template <typename Product>
 __global__ __launch_bounds__(Product::kThreads) void q4_product_kernel(Unfold u, uint16_t* output,
                                                                       uint64_t output_stride,
                                                                       uint32_t columns,
-                                                                      uint32_t out_rows) {
+                                                                      uint32_t out_rows, uint32_t runs) {
     const bool wide = ((reinterpret_cast<uintptr_t>(output) | (output_stride * 2)) & 7) == 0;
-    Product::run(u.rows, u.weights, u.x_rows, columns, out_rows,
+    Product::run(u.rows, u.weights, u.x_rows, columns, out_rows, runs,
                  [&](uint32_t m, uint32_t n, typename Product::Sums sums) {
                      typedef __attribute__((ext_vector_type(4))) int32_t Exponents;
                      const int32_t row_exponent = u.row_exponents[m];
@@ -868,11 +868,11 @@ int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
             u.weight_rows = 0;
             Q4Tiles::choose(u.x_rows, columns, columns_out, workspace.compute_units, [&](auto product) {
                 typedef decltype(product) Product;
-                hipLaunchKernelGGL(
-                    q4_product_kernel<Product>,
-                    dim3(block_workgroups<Product>(u.x_rows, columns_out, workspace.compute_units)),
-                    dim3(Product::kThreads), Product::kLdsBytes, stream, u, p.output + u.first_weight,
-                    p.output_stride, columns, columns_out);
+                const BlockLaunch launch =
+                    block_launch<Product>(u.x_rows, columns, columns_out, workspace.compute_units);
+                hipLaunchKernelGGL(q4_product_kernel<Product>, dim3(launch.workgroups), dim3(Product::kThreads),
+                                   Product::kLdsBytes, stream, u, p.output + u.first_weight, p.output_stride,
+                                   columns, columns_out, launch.runs);
             });
         }
     }

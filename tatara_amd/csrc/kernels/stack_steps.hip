@@ -149,9 +149,9 @@ __global__ __launch_bounds__(256) void dense_bf16_kernel(const uint16_t* input,
 template <typename Product>
 __global__ __launch_bounds__(Product::kThreads) void dense_block_kernel(
     const uint16_t* input, const uint16_t* weights, uint16_t* output, uint32_t rows, uint32_t in_dim,
-    uint32_t out_dim) {
+    uint32_t out_dim, uint32_t runs) {
     const bool wide = ((reinterpret_cast<uintptr_t>(output) | (out_dim * 2)) & 7) == 0;
-    Product::run(input, weights, rows, in_dim, out_dim,
+    Product::run(input, weights, rows, in_dim, out_dim, runs,
                  [&](uint32_t m, uint32_t n, typename Product::Sums sums) {
                      block_store(output + static_cast<uint64_t>(m) * out_dim, n, out_dim, wide, sums);
                  });
@@ -319,9 +319,9 @@ void launch_dense_block(const uint16_t* input, const uint16_t* weights, uint16_t
     const uint32_t units = current_device_compute_units();
     DenseTiles::choose(rows, in_dim, out_dim, units, [&](auto product) {
         typedef decltype(product) Product;
-        hipLaunchKernelGGL(dense_block_kernel<Product>, dim3(block_workgroups<Product>(rows, out_dim, units)),
-                           dim3(Product::kThreads), Product::kLdsBytes, stream, input, weights, output, rows,
-                           in_dim, out_dim);
+        const BlockLaunch launch = block_launch<Product>(rows, in_dim, out_dim, units);
+        hipLaunchKernelGGL(dense_block_kernel<Product>, dim3(launch.workgroups), dim3(Product::kThreads),
+                           Product::kLdsBytes, stream, input, weights, output, rows, in_dim, out_dim, launch.runs);
     });
 }
 
@@ -382,6 +382,12 @@ uint32_t block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, ui
 uint32_t block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
     const BlockChoice choice = block_tile(rows, in_dim, out_dim, std::max(compute_units, 1u));
     return choice.m << 16 | choice.n;
+}
+uint32_t block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
+    const uint32_t units = std::max(compute_units, 1u);
+    return DenseTiles::choose(rows, in_dim, out_dim, units, [&](auto product) {
+        return block_launch<decltype(product)>(rows, in_dim, out_dim, units).runs & (kWholeRounds | kLastRound);
+    });
 }
 
 #if !defined(__HIP_DEVICE_COMPILE__)  // host-side table of launchers

@@ -248,6 +248,9 @@ uint32_t tt_block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
 uint32_t tt_block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
     return tt::block_product_shape(rows, in_dim, out_dim, compute_units);
 }
+uint32_t tt_block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
+    return tt::block_product_runs(rows, in_dim, out_dim, compute_units);
+}
 
 uint32_t tt_flash_prefill_splits(uint32_t rows, uint32_t visible_keys, uint32_t compute_units) {
     return tt::flash_prefill_splits(rows, visible_keys, compute_units);

@@ -110,6 +110,7 @@ uint64_t stream_workspace_bytes(uint32_t compute_units);
 // the BlockTile (block_product.h) of a block product, compute_units >= 1
 uint32_t block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
 uint32_t block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
+uint32_t block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
 // what a block of the 4-bit projections needs of it
 uint64_t q4_workspace_bytes();
 

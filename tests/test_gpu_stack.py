@@ -13,7 +13,7 @@ import pytest
 
 import oracle_lib as ol
 from gpu_util import gpu, run
-from test_host_rules import DENSE_TILE_CASES, REFINED_TILE_CASES
+from test_host_rules import DEALT_CASES, DENSE_TILE_CASES, REFINED_TILE_CASES
 
 pytestmark = pytest.mark.gpu
 o = ol.oracle
@@ -402,6 +402,18 @@ def test_dense_bf16_refined_tiles(shape, rows, in_dim, out_dim):
     sample = sorted({0, 15, 16, rows // 2, rows - 2, rows - 1} | set(range(height - 1, rows, 2 * height)) |
                     set(range(height, rows, 2 * height)))
     got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB222 + rows)
+    assert not np.any((got & 0x7F80) == 0x7F80), "an output was not stored"
+
+
+@pytest.mark.parametrize("runs,rows,in_dim,out_dim", DEALT_CASES, ids=lambda v: str(v))
+def test_dense_bf16_tiles_dealt_either_way(runs, rows, in_dim, out_dim):
+    """Rounds whose tiles go to the workgroups in runs per XCD and by number, whole ones and the last:
+    every output stored, sampled rows of every band against the oracle."""
+    print(f"[case] dense_bf16 dealt {runs} rows={rows} in={in_dim} out={out_dim}", flush=True)
+    B, dev, queue, lib = gpu()
+    assert B.block_product_runs(rows, in_dim, out_dim, dev.compute_units) == runs
+    sample = sorted({0, rows // 2, rows - 2, rows - 1} | set(range(31, rows, max(32, rows // 40))))
+    got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB333 + rows)
     assert not np.any((got & 0x7F80) == 0x7F80), "an output was not stored"
 
 

@@ -134,3 +134,23 @@ def test_refined_shape_of_the_cases(shape, rows, in_dim, out_dim):
 def test_shape_is_the_basic_tile_where_no_other_fills_better(rows, in_dim, out_dim, shape):
     from tatara_amd import backend as B
     assert B.block_product_shape(rows, in_dim, out_dim, 256) == shape
+
+
+# ((whole rounds, last round) in runs, rows, in_dim, out_dim): one round of a lower band, one of tiles in order of
+# the workgroups, of whole bands, rounds of which the last one goes by number and in runs.
+DEALT_CASES = [
+    ((True, True), 777, 1088, 12350), ((False, False), 776, 256, 1119), ((True, False), 1000, 64, 4096),
+    ((True, False), 20000, 64, 900), ((True, True), 300, 256, 12349)]
+
+
+@pytest.mark.parametrize("runs,rows,in_dim,out_dim", DEALT_CASES + [
+    # measured either way: narrow and short products were up to 9 % slower in runs, wide and low ones up to 25 % without
+    ((True, True), 777, 2048, 12352), ((True, True), 1000, 2048, 9216), ((True, True), 300, 2048, 12352),
+    ((True, True), 2500, 2048, 9216), ((False, False), 3380, 960, 1083), ((False, False), 11448, 640, 533),
+    ((False, False), 7210, 3392, 756), ((False, False), 4431, 3776, 104), ((False, False), 17, 3648, 17)],
+    ids=lambda v: str(v))
+def test_rounds_dealt_in_runs(runs, rows, in_dim, out_dim):
+    from tatara_amd import backend as B
+    assert B.block_product_runs(rows, in_dim, out_dim, 256) == runs
+    for units in (0, 1, 64, 304):
+        assert isinstance(B.block_product_runs(rows, in_dim, out_dim, units), tuple)
