@@ -18,6 +18,7 @@
 // m and n past the end are clamped on the way in; the caller does not store them.
 #pragma once
 
+#include <algorithm>
 #include <type_traits>
 
 #include "../tt_internal.h"
@@ -394,17 +395,25 @@ inline BlockChoice choose_block_tile(uint32_t rows, uint32_t in_dim, uint32_t ou
 }
 // Where 256 x 256 leaves a round short (or 128 x 128 takes its place for that) another height or a
 // wider tile may fill the rounds better.  Taken where its estimate is 3 % shorter, which is what
-// the estimates are good for, and from 1024 columns on: they were fitted to 2048 and more.
+// the estimates are good for, down to 1024 columns: they were fitted to 2048 and more, and below that
+// are 5 % beside the pairs of 128 x 128 (1647 x 1152 x 7237, 3.3 % shorter as 224 x 256, took 50.6 us instead of
+// 48.9).  One round of 224 x 256 over
+// a long K is none: more compute units at once run at a lower clock, bf16 6000 x 4096 x 2048 96 us instead of
+// 93, 2401 x 5120 x 4294 135 instead of 130.5, 11294 x 3520 x 1049 98.5 instead of 95.5, 2550 x 3648 x 4203 97.5
+// instead of 99.5 (f16 operands of unfolded 4-bit weights, 5450 x 4352 x 2048 with their unfolding, 107
+// instead of 111: not for these).
 inline BlockChoice refine_block_tile(BlockChoice choice, uint32_t rows, uint32_t in_dim, uint32_t out_dim,
-                                     uint32_t compute_units) {
+                                     uint32_t compute_units, bool bf16) {
     static constexpr BlockCost kCosts[] = {
         {BlockTile::Wide, 256, 288, 1800, 10500, 3600, 21000},
         {BlockTile::Seven, 224, 256, 1370, 8000, 2740, 16000},
         {BlockTile::Five, 160, 256, 1130, 5000, 2260, 10000},
     };
     if (in_dim < 1024) return choice;
-    uint64_t bar = choice.ns - choice.ns * 3 / 100;
+    uint64_t bar = choice.ns - choice.ns * (in_dim < 2048 && choice.tile == BlockTile::Even ? 5 : 3) / 100;
     for (const BlockCost& c : kCosts) {
+        const uint64_t tiles = static_cast<uint64_t>((rows + c.m - 1) / c.m) * ((out_dim + c.n - 1) / c.n);
+        if (bf16 && c.tile == BlockTile::Seven && in_dim >= 3072 && tiles <= compute_units) continue;
         const uint64_t ns = block_ns(c, rows, in_dim, out_dim, compute_units);
         if (ns < bar) {
             choice = BlockChoice{c.tile, c.m, c.n, ns};
@@ -413,9 +422,10 @@ inline BlockChoice refine_block_tile(BlockChoice choice, uint32_t rows, uint32_t
     }
     return choice;
 }
-inline BlockChoice block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
+template <typename Element>
+BlockChoice block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
     return refine_block_tile(choose_block_tile(rows, in_dim, out_dim, compute_units), rows, in_dim, out_dim,
-                             compute_units);
+                             compute_units, std::is_same<Element, __bf16>::value);
 }
 // The tiles a block product is launched with.  What bounds one is how the products of the two
 // to four waves of a SIMD fill each other's waits, and the power (Large, 8192 x 4352 x 2048: matrix unit
@@ -450,7 +460,7 @@ struct BlockTiles {
     // the tile a call takes, as use(product) of a value of its type
     template <typename Use>
     static auto choose(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units, Use use) {
-        switch (block_tile(rows, in_dim, out_dim, compute_units).tile) {
+        switch (block_tile<Element>(rows, in_dim, out_dim, compute_units).tile) {
         case BlockTile::Even: return use(Even{});
         case BlockTile::Deep: return use(Deep{});
         case BlockTile::Tall: return use(Tall{});

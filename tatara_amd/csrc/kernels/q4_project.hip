@@ -841,7 +841,7 @@ int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
         reinterpret_cast<uint8_t*>(u.weight_exponents) + kWeightExponentBytes);
     // what writing the weights out takes, 5 bytes a ns, is spared where each row tile unpacks its own
     const ShortChoice brief = choose_short_tile(p.rows, p.k_size, out_rows, workspace.compute_units);
-    if (brief.ns < block_tile(p.rows, columns, out_rows, workspace.compute_units).ns +
+    if (brief.ns < block_tile<_Float16>(p.rows, columns, out_rows, workspace.compute_units).ns +
                        static_cast<uint64_t>(out_rows) * columns * 2 / 5000) {
         u.short_rows = true;
         for (; u.first_row < p.rows; u.first_row += u.x_rows) {

@@ -380,7 +380,7 @@ uint32_t block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, ui
     return static_cast<uint32_t>(choose_block_tile(rows, in_dim, out_dim, std::max(compute_units, 1u)).tile);
 }
 uint32_t block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
-    const BlockChoice choice = block_tile(rows, in_dim, out_dim, std::max(compute_units, 1u));
+    const BlockChoice choice = block_tile<__bf16>(rows, in_dim, out_dim, std::max(compute_units, 1u));
     return choice.m << 16 | choice.n;
 }
 uint32_t block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {

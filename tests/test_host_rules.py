@@ -130,6 +130,9 @@ def test_refined_shape_of_the_cases(shape, rows, in_dim, out_dim):
 @pytest.mark.parametrize("rows,in_dim,out_dim,shape", [
     (16384, 2048, 12352, (256, 256)), (100, 2048, 12352, (128, 64)), (2048, 4096, 2048, (128, 128)),
     (640, 960, 12352, (128, 128)),       # under 1024 columns the six tiles only
+    # a shorter estimate of 224 x 256 that did not hold: one round over a long K, few columns
+    (5150, 4096, 2048, (256, 256)), (2401, 5120, 4294, (256, 256)), (6000, 4096, 2048, (256, 256)),
+    (1647, 1152, 7237, (128, 128)), (2095, 1088, 5501, (128, 128)),
 ])
 def test_shape_is_the_basic_tile_where_no_other_fills_better(rows, in_dim, out_dim, shape):
     from tatara_amd import backend as B
