@@ -343,14 +343,11 @@ uint32_t tt_choose_split_keys(const uint32_t* visible_keys, uint32_t rows, uint3
 uint32_t tt_flash_prefill_splits(uint32_t rows, uint32_t visible_keys, uint32_t compute_units);
 uint64_t tt_flash_prefill_scratch_bytes(uint32_t rows, uint32_t splits);
 
-/* The tile, of six, with which dense_bf16 (and the 4-bit blocks, in_dim then being the columns of
- * their unfolded operands, 17/16 of the input width) multiplies a block of more than 16 rows on that
- * many compute units: 0 256 x 256, 1 128 x 128 (two workgroups a compute unit), 2 128 x 128
- * (one), 3 128 x 64, 4 64 x 64, 5 32 x 64 rows x outputs.  From 1024 columns on another shape takes
- * its place where it fills the rounds of the compute units better: tt_block_product_shape gives the
- * one that is launched, its rows in the upper 16 bits and its outputs in the lower.  (4-bit blocks of
- * up to about 400 rows are not multiplied by these tiles at all.)  For tests and measurements; the
- * results do not depend on it. */
+/* The tile, of six, with which dense_bf16 multiplies a block of more than 16 rows on that many compute
+ * units: 0 256 x 256, 1 128 x 128 (two workgroups a compute unit), 2 128 x 128 (one), 3 128 x 64, 4 64 x 64, 5
+ * 32 x 64 rows x outputs.  From 1024 columns on another shape takes its place where it fills the rounds of
+ * the compute units better: tt_block_product_shape gives the one that is launched, its rows in the upper
+ * 16 bits and its outputs in the lower.  For tests and measurements; the results do not depend on it. */
 uint32_t tt_block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                uint32_t compute_units);
 uint32_t tt_block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
@@ -359,6 +356,12 @@ uint32_t tt_block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim
  * rounds, 2 the last one, 3 both, 0 none.  For tests and measurements as well. */
 uint32_t tt_block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
                                uint32_t compute_units);
+/* The tile of a 4-bit block (gdn_project_blk, attn_project_blk, outproj_blk) of more than 16 rows over
+ * in_dim columns, on a queue with its whole workspace: 16 + n where the weights are unpacked in the product, 16 n
+ * rows a tile; otherwise they are written out and multiplied over 17/16 of in_dim, and the tile (of the first
+ * 16384 rows, or 8192 of 4096 columns, which go together) is one of the six above or 6 256 x 288, 7 224 x 256, 8
+ * 160 x 256.  For tests and measurements. */
+uint32_t tt_q4_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
 
 #ifdef __cplusplus
 }

@@ -34,7 +34,7 @@ EXPORTED_SYMBOLS = [
     "tt_event_create", "tt_event_destroy", "tt_encode_signal_event", "tt_encode_wait_for_event",
     "tt_split_workgroups", "tt_choose_split_keys",
     "tt_flash_prefill_splits", "tt_flash_prefill_scratch_bytes", "tt_block_product_tile",
-    "tt_block_product_shape", "tt_block_product_runs",
+    "tt_block_product_shape", "tt_block_product_runs", "tt_q4_block_tile",
 ]
 
 
@@ -115,6 +115,7 @@ def lib():
         "tt_block_product_tile": (u32, [u32] * 4),
         "tt_block_product_shape": (u32, [u32] * 4),
         "tt_block_product_runs": (u32, [u32] * 4),
+        "tt_q4_block_tile": (u32, [u32] * 4),
         "tt_flash_prefill_scratch_bytes": (u64, [u32, u32]),
         "tt_event_create": (i32, [vp, pvp]), "tt_event_destroy": (None, [vp]),
         "tt_encode_signal_event": (i32, [vp, vp, u64]),
@@ -503,6 +504,7 @@ def choose_split_keys(visible_keys, compute_units=256):
 
 
 BLOCK_TILES = ("256x256", "128x128", "128x128-deep", "128x64", "64x64", "32x64")
+REFINED_TILES = ("256x288", "224x256", "160x256")
 
 
 def block_product_tile(rows, in_dim, out_dim, compute_units=256):
@@ -522,6 +524,13 @@ def block_product_runs(rows, in_dim, out_dim, compute_units=256):
     (tt_block_product_runs)."""
     runs = lib().tt_block_product_runs(int(rows), int(in_dim), int(out_dim), int(compute_units))
     return bool(runs & 1), bool(runs & 2)
+
+
+def q4_block_tile(rows, in_dim, out_dim, compute_units=256):
+    """The tile of a 4-bit block of that size: "short-<rows>" where the weights are unpacked in the product,
+    otherwise one of BLOCK_TILES or of REFINED_TILES, rows x outputs (tt_q4_block_tile)."""
+    tile = lib().tt_q4_block_tile(int(rows), int(in_dim), int(out_dim), int(compute_units))
+    return f"short-{(tile - 16) * 16}" if tile >= 16 else (BLOCK_TILES + REFINED_TILES)[tile]
 
 
 def flash_prefill_splits(rows, visible_keys, compute_units=256):

@@ -486,7 +486,7 @@ __global__ __launch_bounds__(Product::kThreads) void q4_product_kernel(Unfold u,
 // four units are 16 bytes of a weight row (unfolded_piece): everything a workgroup needs of the
 // weights is requested at its start.  x comes through LDS as in block_product.h, a ring of units.
 // Over 2048 columns two waves share the columns' work (as many workgroups as compute units, nearly);
-// the 2048 outputs over 4096 columns are cut finer, and take half as many units.
+// the 2048 outputs over 4096 columns are cut finer, in as many units of twice the columns.
 template <uint32_t kTm_, uint32_t kBlocks_>   // kBlocks: k_size / 512
 struct ShortProduct {
     static constexpr uint32_t kTm = kTm_, kBlocks = kBlocks_;
@@ -502,7 +502,9 @@ struct ShortProduct {
     static_assert(kTm % 2 == 0 && kLdsBytes <= 160 * 1024);
     // the partial sums of all eight waves take the ring's place
     static_assert(8 * kTm * 2 * 1024 <= kRing * kUnitBytes);
-    // waves to a SIMD: 128 registers each, for a second workgroup, where that costs no spills
+    // Waves to a SIMD: 128 registers each where that costs no spills, for a second workgroup where two fit the LDS
+    // (64 rows over 4096 columns fill it alone, and are faster so all the same: outproj_blk of 129 / 256 rows 18.0 /
+    // 19.8 us, with 256 registers 18.5 / 20.4).
     static constexpr uint32_t kWavesPerSimd = kTm <= 4 ? 4 : 2;
 };
 
@@ -761,13 +763,15 @@ static_assert(static_cast<uint64_t>(kHidden) * unfolded_columns(kGdnValueValues)
               "the output projection's weights fit as well");
 
 // The row tile of a short block with the shortest estimate, and that estimate: ns of a launch, a
-// fixed part and one per workgroup of a compute unit, fitted to 17 .. 777 rows.  gdn_project_blk /
-// attn_project_blk / outproj_blk with unfolding, before (weights written out, block product) and now:
-// 17 rows 24.4 / 26.4 / 25.3 -> 12.7 / 12.6 / 14.7 us, 100 rows 28.1 / 30.6 / 26.7 -> 20 / 19.5 / 15.4,
-// 256 rows 36.4 / 35.3 / 26.6 -> 35.8 / 29.3 / 20.3, 300 rows 51.8 / 37.1 / 28.6 -> 37 / 29.6 / 25.2; from
-// about 400 rows on (outproj 350) the weights written out once are as fast or faster.  What bounds it: at 100
-// rows of gdn_project the x rows' unfolding and two launches 5.5 us, the weights' arrival 3, the products
-// and the barrier of each unit 7 (4 of them on the matrix unit), the partial sums 2.
+// fixed part and one per workgroup of a compute unit, fitted to 17 .. 777 rows (128 rows over 4096 columns, 23 us
+// a workgroup, are never the shortest).  gdn_project_blk / attn_project_blk / outproj_blk with unfolding,
+// weights written out and unpacked in the product:
+//   17 rows   29.5 / 26.4 / 25.0 and 12.8 / 12.7 / 14.7 us     384 rows  48.0 / 37.0 / 27.4 and 44.3 / 36.5 / 25.4
+//   100 rows  32.3 / 30.6 / 25.9 and 20.5 / 20.0 / 15.4        400 rows  47.8 / 41.9 / 27.2 and 50.0 / 36.3 / 30.4
+//   256 rows  38.1 / 35.1 / 25.9 and 36.2 / 28.9 / 20.1        448 rows  47.8 / 42.2 / 27.1 and 50.5 / 36.8 / 30.9
+//   320 rows  44.3 / 36.6 / 27.8 and 37.2 / 29.4 / 24.7        512 rows  48.9 / 45.6 / 27.1 and 57.1 / 43.7 / 31.3
+// What bounds it: at 100 rows of gdn_project the x rows' unfolding and two launches 5.5 us, the weights'
+// arrival 3, the products and the barrier of each unit 7 (4 of them on the matrix unit), the partial sums 2.
 struct ShortChoice {
     uint32_t tm;
     uint64_t ns;
@@ -780,25 +784,39 @@ inline ShortChoice choose_short_tile(uint32_t rows, uint32_t k_size, uint32_t ou
         {2, {3200, 1500}, {5200, 8500}},
         {4, {3500, 0}, {7000, 13500}},
         {6, {500, 0}, {12600, 18000}},
-        {8, {1800, 0}, {14200, 23000}},
+        {8, {1800, 0}, {14200, 0}},
     };
     const uint32_t deep = k_size > kHidden ? 1 : 0;
     ShortChoice best{0, ~0ull};
     for (const Cost& c : kCosts) {
+        if (c.each[deep] == 0) continue;
         const uint64_t groups = static_cast<uint64_t>((rows + 16 * c.tm - 1) / (16 * c.tm)) * (out_rows / (deep ? 32 : 64));
         const uint64_t ns = c.fixed[deep] + (groups + compute_units - 1) / compute_units * c.each[deep];
         if (ns < best.ns) best = ShortChoice{c.tm, ns};
     }
     return best;
 }
+// The tile of a short block if its weights are unpacked in the product, 0 if they are written out first: what that
+// takes, 5 bytes a ns, is spared where each row tile unpacks its own.  Estimates of products that do not
+// fill their rounds are too long, those of one round too short (30.4 us with the writing measured as 38 with
+// x's unfolding, 46.0 as 48): hence a line through both against the sum.
+inline uint32_t short_tile(uint32_t rows, uint32_t k_size, uint32_t out_rows, uint32_t compute_units) {
+    const uint32_t columns = unfolded_columns(k_size);
+    const uint64_t unfolded = block_tile<_Float16>(rows, columns, out_rows, compute_units).ns +
+                              static_cast<uint64_t>(out_rows) * columns * 2 / 5000;
+    const ShortChoice brief = choose_short_tile(rows, k_size, out_rows, compute_units);
+    return brief.ns < (unfolded + 6000) * 6 / 7 ? brief.tm : 0;
+}
 // use(product) of a short block's tile
 template <uint32_t kBlocks, typename Use>
 void short_product(uint32_t tm, Use use) {
+    if constexpr (kBlocks == 4) {
+        if (tm == 8) return use(ShortProduct<8, kBlocks>{});
+    }
     switch (tm) {
-    case 2: use(ShortProduct<2, kBlocks>{}); break;
-    case 4: use(ShortProduct<4, kBlocks>{}); break;
-    case 6: use(ShortProduct<6, kBlocks>{}); break;
-    default: use(ShortProduct<8, kBlocks>{}); break;
+    case 2: return use(ShortProduct<2, kBlocks>{});
+    case 4: return use(ShortProduct<4, kBlocks>{});
+    default: return use(ShortProduct<6, kBlocks>{});
     }
 }
 template <uint32_t kBlocks>
@@ -839,17 +857,15 @@ int32_t launch_block(const Q4Projection& p, hipStream_t stream) {
     u.weight_exponents = reinterpret_cast<int32_t*>(workspace.base + unfolded_bytes);
     u.row_exponents = reinterpret_cast<int32_t*>(
         reinterpret_cast<uint8_t*>(u.weight_exponents) + kWeightExponentBytes);
-    // what writing the weights out takes, 5 bytes a ns, is spared where each row tile unpacks its own
-    const ShortChoice brief = choose_short_tile(p.rows, p.k_size, out_rows, workspace.compute_units);
-    if (brief.ns < block_tile<_Float16>(p.rows, columns, out_rows, workspace.compute_units).ns +
-                       static_cast<uint64_t>(out_rows) * columns * 2 / 5000) {
+    const uint32_t tm = short_tile(p.rows, p.k_size, out_rows, workspace.compute_units);
+    if (tm != 0) {
         u.short_rows = true;
         for (; u.first_row < p.rows; u.first_row += u.x_rows) {
             u.x_rows = std::min(slice, p.rows - u.first_row);
             if (p.k_size == 4 * kQ4Block) {
-                launch_short<4>(p, u, brief.tm, stream);
+                launch_short<4>(p, u, tm, stream);
             } else {
-                launch_short<8>(p, u, brief.tm, stream);
+                launch_short<8>(p, u, tm, stream);
             }
         }
         return TT_OK;
@@ -1383,6 +1399,14 @@ int32_t op_outproj_mfma_blk(const Bindings& b, const Grid& g, hipStream_t s, boo
 uint64_t q4_workspace_bytes() { return kUnfoldWorkspaceBytes; }
 
 #if !defined(__HIP_DEVICE_COMPILE__)  // host-side table of launchers
+uint32_t q4_block_tile(uint32_t rows, uint32_t k_size, uint32_t out_rows, uint32_t compute_units) {
+    const uint32_t tm = short_tile(rows, k_size, out_rows, compute_units);
+    if (tm != 0) return kShortBlockTiles + tm;
+    const uint32_t columns = unfolded_columns(k_size);
+    const uint32_t slice = std::min<uint64_t>(kUnfoldedRowBytes / 2 / columns / 256 * 256, 16384);
+    return static_cast<uint32_t>(block_tile<_Float16>(std::min(rows, slice), columns, out_rows, compute_units).tile);
+}
+
 bool prepare_q4_kernels() {
     const auto allow = [](auto product) {
         typedef decltype(product) Product;
@@ -1406,10 +1430,8 @@ bool prepare_q4_kernels() {
                                             hipFuncAttributeMaxDynamicSharedMemorySize,
                                             Product::kLdsBytes) == hipSuccess;
     };
-    for (const uint32_t tm : {2u, 4u, 6u, 8u}) {
-        short_product<4>(tm, allow_short);
-        short_product<8>(tm, allow_short);
-    }
+    for (const uint32_t tm : {2u, 4u, 6u, 8u}) short_product<4>(tm, allow_short);
+    for (const uint32_t tm : {2u, 4u, 6u}) short_product<8>(tm, allow_short);
     return short_allowed && Q4Tiles::each(allow) &&
            allow_wave(q4_rows_kernel<4, true, false>, kRowsStagedBytes) &&
            allow_wave(q4_rows_kernel<8, true>, kRowsStagedBytes) &&

@@ -252,6 +252,10 @@ uint32_t tt_block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim,
     return tt::block_product_runs(rows, in_dim, out_dim, compute_units);
 }
 
+uint32_t tt_q4_block_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units) {
+    return tt::q4_block_tile(rows, in_dim, out_dim, compute_units == 0 ? 1 : compute_units);
+}
+
 uint32_t tt_flash_prefill_splits(uint32_t rows, uint32_t visible_keys, uint32_t compute_units) {
     return tt::flash_prefill_splits(rows, visible_keys, compute_units);
 }

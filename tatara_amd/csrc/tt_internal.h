@@ -111,6 +111,9 @@ uint64_t stream_workspace_bytes(uint32_t compute_units);
 uint32_t block_product_tile(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
 uint32_t block_product_shape(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
 uint32_t block_product_runs(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint32_t compute_units);
+// the BlockTile of a 4-bit block whose weights are written out, or kShortBlockTiles and the row tile's sixteens
+constexpr uint32_t kShortBlockTiles = 16;
+uint32_t q4_block_tile(uint32_t rows, uint32_t k_size, uint32_t out_rows, uint32_t compute_units);
 // what a block of the 4-bit projections needs of it
 uint64_t q4_workspace_bytes();
 

@@ -157,3 +157,22 @@ def test_rounds_dealt_in_runs(runs, rows, in_dim, out_dim):
     assert B.block_product_runs(rows, in_dim, out_dim, 256) == runs
     for units in (0, 1, 64, 304):
         assert isinstance(B.block_product_runs(rows, in_dim, out_dim, units), tuple)
+
+
+Q4_SHAPES = {"gdn": (2048, 12352), "attn": (2048, 9216), "out": (4096, 2048)}
+
+
+@pytest.mark.parametrize("family,rows,tile", [
+    ("gdn", 17, "short-32"), ("gdn", 64, "short-64"), ("gdn", 96, "short-96"), ("gdn", 256, "short-128"),
+    ("gdn", 384, "short-64"), ("gdn", 385, "128x128"), ("gdn", 448, "128x128"), ("gdn", 777, "160x256"),
+    ("attn", 320, "short-64"), ("attn", 400, "short-64"), ("attn", 480, "short-96"), ("attn", 512, "short-64"),
+    ("attn", 513, "128x128"), ("attn", 2048, "256x288"), ("out", 128, "short-32"), ("out", 256, "short-64"),
+    ("out", 384, "short-96"), ("out", 385, "64x64"), ("out", 8193, "256x256"), ("out", 5450, "224x256")])
+def test_q4_block_route_where_it_was_measured(family, rows, tile):
+    """4-bit blocks: weights unpacked in the product where that was faster on 256 compute units (GDN
+    projections up to 384 rows, attention projections up to 512, where 321 to 384 take as long either way,
+    output projections up to 384), and a tile for any number of compute units."""
+    from tatara_amd import backend as B
+    assert B.q4_block_tile(rows, *Q4_SHAPES[family], 256) == tile
+    for units in (0, 1, 64, 304):
+        assert isinstance(B.q4_block_tile(rows, *Q4_SHAPES[family], units), str)
