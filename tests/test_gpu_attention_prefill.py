@@ -329,25 +329,25 @@ def test_config4_prefill_16384_rows():
     print(f"[time] rope + flash prefill 16384 rows (first run): {ms:.3f} ms", flush=True)
 
 
-@pytest.mark.parametrize("rows", [1, 15, 17, 31, 33, 100])
-def test_output_gate_at_its_limits(rows):
-    """The gate's sigmoid of the finished rows, at row counts around the 16 a wave and the 32 a
-    workgroup finishes: gates far to either side, infinite and NaN ones, against the rows the same
+def _gate_limits(rows, base, cap, splits=None):
+    """The output with gates far to either side, infinite and NaN ones, against the rows the same
     queries give with a gate of zero (a half)."""
-    print(f"[case] flash prefill gate limits rows={rows}", flush=True)
     B, dev, queue, lib = gpu()
-    cap = 160
     q, k, v = (ol.gaussian_bf16(0x9A00 + i, n) for i, n in ((rows, rows * 4096), (1, 2 * cap * 256), (2, 2 * cap * 256)))
     cases = {0.0: 0.5, -200.0: 0.0, 200.0: 1.0, -np.inf: 0.0, np.inf: 1.0, np.nan: np.nan, 1.0: 1 / (1 + np.exp(-1.0))}
+    scratch = dev.create_buffer(max(256, B.flash_prefill_scratch_bytes(rows, splits or 1)))
     got = {}
     for gate in cases:
         out = dev.buffer_from(np.full(rows * 4096 + 64, 0x4242, np.uint16))
         gates = ol.f32_to_bf16(np.full(rows * 4096, gate, np.float32)) if not np.isnan(gate) else \
             np.full(rows * 4096, 0x7FC0, np.uint16)
-        run(lambda cb: cb.encode(lib.pipeline("attention_flash_v2_blk"),
-                                 {0: dev.buffer_from(q), 1: dev.buffer_from(k), 2: dev.buffer_from(v),
-                                  3: dev.buffer_from(gates), 4: out}, {5: rows + 7, 6: cap, 7: rows, 8: 7},
-                                 (16, (rows + 15) // 16), (256,)))
+        bindings = {0: dev.buffer_from(q), 1: dev.buffer_from(k), 2: dev.buffer_from(v), 3: dev.buffer_from(gates),
+                    4: out}
+        constants = {5: rows + base, 6: cap, 7: rows, 8: base}
+        name = "attention_flash_v2_blk"
+        if splits is not None:
+            name, bindings[9], constants[10] = "attention_flash_split_blk", scratch, splits
+        run(lambda cb: cb.encode(lib.pipeline(name), bindings, constants, (16, (rows + 15) // 16), (256,)))
         words = out.read(np.uint16)
         assert (words[rows * 4096:] == 0x4242).all()
         got[gate] = ol.bf16_to_f32(words[:rows * 4096]).astype(np.float64)
@@ -359,3 +359,19 @@ def test_output_gate_at_its_limits(rows):
         want = 2 * factor * got[0.0]
         bar = 2.0 ** -8 * (np.abs(got[gate]) + np.abs(want)) * (1 + 2.0 ** -8) + 1e-38
         assert (np.abs(got[gate] - want) <= bar).all(), gate
+
+
+@pytest.mark.parametrize("rows", [1, 15, 17, 31, 33, 100])
+def test_output_gate_at_its_limits(rows):
+    """The gate's sigmoid of the finished rows, at row counts around the 16 a wave and the 32 a
+    workgroup finishes, of walks that are not shared."""
+    print(f"[case] flash prefill gate limits rows={rows}", flush=True)
+    _gate_limits(rows, 7, 160)
+
+
+@pytest.mark.parametrize("rows,base,splits", [(12, 600, 2), (33, 600, 2), (12, 600, 3), (33, 600, 5), (12, 1500, None)])
+def test_output_gate_at_its_limits_behind_shared_walks(rows, base, splits):
+    """The same where the last of two sharers finishes the rows, and where a dispatch of its own does: of
+    the shares asked for, and of as many as fill the device."""
+    print(f"[case] flash prefill gate limits rows={rows} base={base} splits={splits}", flush=True)
+    _gate_limits(rows, base, 2048, splits)
