@@ -187,6 +187,46 @@ def test_conv_with_gates_and_gate_norm_from_the_projection(rows, in_place):
     assert np.array_equal(bufs["beta"].read(np.float32), beta)
 
 
+def test_conv_with_gates_and_gate_norm_from_the_projection_validation():
+    """What either operator refuses: other grids, no rows, buffers a row short - the projection's z
+    columns of the last row among them."""
+    B, dev, queue, lib = gpu()
+    rows = 5
+    buf = dev.create_buffer
+    conv = {0: buf(rows * 24704), 1: buf(49152), 2: buf(65536), 3: buf(rows * 8192), 4: buf(rows * 8192), 5: buf(64),
+            6: buf(64), 7: buf(rows * 128), 8: buf(rows * 128), 9: buf(49152)}
+    norm = {0: buf(rows * 8192), 1: buf(rows * 24704), 2: buf(256), 3: buf(rows * 8192)}
+    cb = queue.create_command_buffer()
+    cb.begin_compute_pass()
+
+    def refused(status, name, bindings, constants, grid, threads=(128, 1, 1)):
+        with pytest.raises(B.BackendError) as e:
+            cb.encode(lib.pipeline(name), bindings, constants, grid, threads)
+        assert e.value.status == status, (name, grid, e.value.status)
+    for grid, threads in (((96, rows, 1), (128, 1, 1)), ((64, rows + 1, 1), (128, 1, 1)), ((64, rows, 2), (128, 1, 1)),
+                          ((64, rows, 1), (256, 1, 1)), ((64, rows, 1), (64, 2, 1))):
+        refused(15, "gdn_conv_gates_blk", conv, {10: rows}, grid, threads)
+    with pytest.raises(B.BackendError):
+        cb.encode(lib.pipeline("gdn_conv_gates_blk"), conv, {10: 0}, (64, 0, 1), (128, 1, 1))
+    for slot, size in ((0, rows * 24704), (1, 49152), (2, 65536), (3, rows * 8192), (4, rows * 8192), (5, 64),
+                       (6, 64), (7, rows * 128), (8, rows * 128), (9, 49152)):
+        refused(10, "gdn_conv_gates_blk", {**conv, slot: buf(size - 2)}, {10: rows}, (64, rows, 1))
+    for grid, threads in (((64, rows, 1), (128, 1, 1)), ((32, rows, 2), (128, 1, 1)), ((32, rows, 1), (64, 1, 1)),
+                          ((32, rows, 1), (128, 2, 1))):
+        refused(15, "gdn_gate_norm_proj_blk", norm, {}, grid, threads)
+    with pytest.raises(B.BackendError):
+        cb.encode(lib.pipeline("gdn_gate_norm_proj_blk"), norm, {}, (32, 0, 1), (128, 1, 1))
+    z_end = (rows - 1) * 24704 + (8192 + 4096) * 2
+    for slot, size in ((0, rows * 8192), (1, z_end), (2, 256), (3, rows * 8192)):
+        refused(10, "gdn_gate_norm_proj_blk", {**norm, slot: buf(size - 2)}, {}, (32, rows, 1))
+    assert cb.command_count == 0
+    # as far as the last row's z and no further
+    cb.encode(lib.pipeline("gdn_gate_norm_proj_blk"), {**norm, 1: buf(z_end)}, {}, (32, rows, 1), (128, 1, 1))
+    assert cb.command_count == 1
+    cb.end_compute_pass()
+    cb.commit().wait()
+
+
 @pytest.mark.parametrize("shift", [0, 8192, -2048], ids=["same", "a-row-on", "overlapping"])
 @pytest.mark.parametrize("rows", [1, 2, 3, 12, 16, 17, 100, 600])
 def test_conv_window_written_in_place(rows, shift):
