@@ -12,6 +12,7 @@ import pytest
 
 import oracle_lib as ol
 from gpu_util import check_bf16, gpu, run
+from test_host_rules import Q4_SHORT_ROWS, Q4_UNFOLDED_ROWS, Q4_WIDE_RANGE_ROWS
 
 pytestmark = pytest.mark.gpu
 o = ol.oracle
@@ -212,7 +213,7 @@ def test_block_projection_over_several_row_tiles(family, name, rows):
 
 @pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
                                          (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
-@pytest.mark.parametrize("rows", [17, 63, 65, 129, 511, 8193])
+@pytest.mark.parametrize("rows", Q4_WIDE_RANGE_ROWS)
 def test_block_projection_against_64_bit_sums_over_the_whole_range(family, name, rows):
     """Rows either side of the tile heights a block is launched with, and of the 8192 rows the
     out-projection takes at a time, over inputs and weights of all magnitudes: rows of 2^-100 to
@@ -267,10 +268,23 @@ def test_block_projection_against_64_bit_sums_over_the_whole_range(family, name,
 
 @pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
                                          (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
-@pytest.mark.parametrize("rows", [32, 33, 64, 66, 96, 97, 128, 130, 200, 385, 420])
+@pytest.mark.parametrize("rows", Q4_SHORT_ROWS)
 def test_block_projection_with_the_weights_unpacked_in_the_product(family, name, rows):
-    """Either side of the row tiles of 32, 64, 96 and 128 that short blocks are multiplied in, one
-    and several of them, against the 64-bit sums and with the bound above."""
+    """Either side of the row tiles of 32, 64, 96 and (but for the output projection) 128 that short blocks
+    are multiplied in, one and several of them, and past the last rows that the GDN and the output projection
+    take so, against the 64-bit sums and with the bound above."""
+    B = gpu()[0]
+    tile = B.q4_block_tile(rows, family["k"], sum(family["segments"]), gpu()[1].compute_units)
+    assert tile.startswith("short") == (rows <= 384 or family is ATTN), tile
+    test_block_projection_against_64_bit_sums_over_the_whole_range(family, name, rows)
+
+
+@pytest.mark.parametrize("family,name", [(ATTN, "attn_project_blk"), (GDN, "gdn_project_blk"),
+                                         (OUT, "outproj_blk")], ids=["attn", "gdn", "out"])
+@pytest.mark.parametrize("rows", Q4_UNFOLDED_ROWS)
+def test_block_projection_on_the_tiles_that_fill_the_rounds(family, name, rows):
+    """Rows that take 256 x 288, 224 x 256, 160 x 256 and the tiles beside them over unfolded weights (see
+    tests/test_host_rules.py), with remainders, against the 64-bit sums and with the bound above."""
     test_block_projection_against_64_bit_sums_over_the_whole_range(family, name, rows)
 
 
@@ -324,6 +338,9 @@ def test_block_projection_in_queues_of_less_workspace(family, name, rows):
     the attention width): the same sums, bit for bit.  One without workspace evaluates the rows in
     the reference's order: the oracle's bits."""
     B, dev, _, lib = gpu()
+    # the output projection's slices of 256 rows and outputs: where unfolded weights take the 32 x 64 tile
+    assert B.block_product_tile(256, 4352, 256, dev.compute_units) == "32x64"
+    assert B.block_product_shape(256, 4352, 256, dev.compute_units) == (32, 64)
     host, bindings = _family(dev, family, 0xA800)
     k, total = family["k"], sum(family["segments"])
     x = ol.gaussian_bf16(0xA900 + rows, rows * k, 0.0, 1.0)

@@ -13,7 +13,7 @@ import pytest
 
 import oracle_lib as ol
 from gpu_util import gpu, run
-from test_host_rules import DEALT_CASES, DENSE_TILE_CASES, REFINED_TILE_CASES
+from test_host_rules import DEALT_CASES, DENSE_TILE_CASES, REFINED_TILE_CASES, tile_shape
 
 pytestmark = pytest.mark.gpu
 o = ol.oracle
@@ -385,6 +385,7 @@ def test_dense_bf16_block_tiles(tile, rows, in_dim, out_dim):
     print(f"[case] dense_bf16 tile {tile} rows={rows} in={in_dim} out={out_dim}", flush=True)
     B, dev, queue, lib = gpu()
     assert B.block_product_tile(rows, in_dim, out_dim, dev.compute_units) == tile
+    assert B.block_product_shape(rows, in_dim, out_dim, dev.compute_units) == tile_shape(tile)
     sample = sorted({r for r in (0, 15, 16, 31, 32, 63, 64, 65, rows // 2, rows - 2, rows - 1) if r < rows} |
                     {r for r in range(127, rows, 640)} | {r for r in range(128, rows, 640)})
     got = _dense_block_case(rows, in_dim, out_dim, sample, 0xB111 + rows)

@@ -63,34 +63,52 @@ def test_flash_prefill_sharing_plan(rows, units, splits, scratch):
 
 # (tile, rows, in_dim, out_dim) of the dense_bf16 blocks that tests/test_gpu_stack.py runs: every tile
 # with fewer units of 64 columns than its ring holds, as many and more (256 x 256 is not taken for two
-# units or less), at remainders of rows and outputs and at output rows that are not 8-byte aligned.
+# units or less), at remainders of rows and outputs and at output rows that are not 8-byte aligned.  None of
+# them is launched as another shape that fills the rounds better; those have cases of their own below.
 DENSE_TILE_CASES = [(tile, rows, in_dim, out_dim) for tile, rows, out_dim in [
     ("256x256", 3073, 4095), ("128x128", 641, 6141), ("128x128-deep", 129, 12350), ("128x64", 65, 12350),
     ("64x64", 33, 9213), ("32x64", 17, 61)]
     for in_dim in (64, 128, 192, 256) if tile != "256x256" or in_dim > 128] + [
-    ("256x256", 1025, 2048, 12349), ("128x128", 2049, 192, 12352), ("256x256", 5000, 4096, 2046),
+    ("256x256", 1021, 2048, 12349), ("128x128", 2049, 192, 12352), ("256x256", 7937, 4096, 2046),
     ("128x128", 500, 2048, 9213), ("128x128", 500, 2048, 9216), ("128x128-deep", 2047, 4096, 2045),
     ("128x64", 777, 4096, 2046), ("128x64", 100, 2048, 12352), ("64x64", 129, 256, 9216),
     ("64x64", 129, 2048, 9213), ("32x64", 66, 2048, 515), ("32x64", 100, 64, 4096)]
 
 
+def tile_shape(tile):
+    return tuple(int(side) for side in tile.removesuffix("-deep").split("x"))
+
+
 @pytest.mark.parametrize("tile,rows,in_dim,out_dim", DENSE_TILE_CASES, ids=lambda v: str(v))
 def test_block_tile_of_the_cases(tile, rows, in_dim, out_dim):
-    """The rule still gives the cases the tiles they are there for: a change of its figures that
-    left a tile without a case fails here."""
+    """The rule still gives the cases the tiles they are there for, and launches them: a change of
+    its figures that left a tile without a case fails here."""
     from tatara_amd import backend as B
     assert B.block_product_tile(rows, in_dim, out_dim, 256) == tile
+    assert B.block_product_shape(rows, in_dim, out_dim, 256) == tile_shape(tile)
+
+
+# Rows of the 4-bit blocks that tests/test_gpu_q4_project.py holds to 64-bit sums, and the way each goes by family.
+Q4_SHAPES = {"gdn": (2048, 12352), "attn": (2048, 9216), "out": (4096, 2048)}
+Q4_WIDE_RANGE_ROWS = [17, 63, 65, 129, 511, 8193]
+Q4_SHORT_ROWS = [32, 33, 64, 66, 96, 97, 128, 130, 200, 385, 420]
+Q4_UNFOLDED_ROWS = [350, 777, 1057, 2047, 4500, 5450]
 
 
 def test_every_block_tile_has_cases():
+    """What is launched, of bf16 and of f16 operands: every tile and every height of the rows that are multiplied
+    with weights unpacked in the product.  (The f16 32 x 64 is launched for slices of a queue with little
+    workspace only, and tested there.)"""
     from tatara_amd import backend as B
     assert {case[0] for case in DENSE_TILE_CASES} == set(B.BLOCK_TILES)
-    # the 4-bit blocks of tests/test_gpu_q4_project.py: their operands are 17/16 of the input wide, and
-    # the out-projection takes 8192 rows at a time
-    taken = {B.block_product_tile(min(rows, limit), k * 17 // 16, n, 256)
-             for k, n, limit in ((2048, 9216, 16384), (2048, 12352, 16384), (4096, 2048, 8192))
-             for rows in (17, 37, 63, 65, 129, 130, 511, 8193)}
-    assert taken == set(B.BLOCK_TILES)
+    assert {case[0] for case in REFINED_TILE_CASES} == {tile_shape(tile) for tile in B.REFINED_TILES}
+    taken = {name: {B.q4_block_tile(rows, *shape, 256)
+                    for rows in Q4_WIDE_RANGE_ROWS + Q4_SHORT_ROWS + Q4_UNFOLDED_ROWS}
+             for name, shape in Q4_SHAPES.items()}
+    short = {"short-32", "short-64", "short-96"}
+    assert taken["gdn"] >= short | {"short-128"} and taken["attn"] >= short | {"short-128"}
+    assert {tile for tile in taken["out"] if tile.startswith("short")} == short
+    assert set.union(*taken.values()) - short - {"short-128"} == set(B.BLOCK_TILES + B.REFINED_TILES) - {"32x64"}
 
 
 @pytest.mark.parametrize("rows,in_dim,out_dim,tile", [
@@ -102,8 +120,9 @@ def test_every_block_tile_has_cases():
     (4096, 2048, 9216, "128x128"), (2048, 2048, 9216, "128x128"), (2048, 4096, 2048, "128x128-deep"),
     (100, 2048, 12352, "128x64"), (300, 4096, 2048, "64x64"), (100, 4096, 2048, "32x64")])
 def test_block_tile_where_it_was_measured(rows, in_dim, out_dim, tile):
-    """The fastest tile at sizes where all of them were timed on 256 compute units; and a tile for
-    any number of compute units."""
+    """The fastest of the six tiles at sizes where all of them were timed on 256 compute units (some of
+    which are launched as a shape that fills the rounds better still); and a tile for any number of
+    compute units."""
     from tatara_amd import backend as B
     assert B.block_product_tile(rows, in_dim, out_dim, 256) == tile
     for units in (0, 1, 64, 304):
@@ -157,9 +176,6 @@ def test_rounds_dealt_in_runs(runs, rows, in_dim, out_dim):
     assert B.block_product_runs(rows, in_dim, out_dim, 256) == runs
     for units in (0, 1, 64, 304):
         assert isinstance(B.block_product_runs(rows, in_dim, out_dim, units), tuple)
-
-
-Q4_SHAPES = {"gdn": (2048, 12352), "attn": (2048, 9216), "out": (4096, 2048)}
 
 
 @pytest.mark.parametrize("family,rows,tile", [
