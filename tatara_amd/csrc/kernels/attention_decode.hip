@@ -1134,8 +1134,9 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 // Merge of the first `nparts` (at most kParts, the same for all lanes) of the requested records.  A
 // wave's lanes take a record's maximum and weight each; the weights come back from their lanes one
-// by one as the numerators are added up.  (With every lane computing all weights the dispatch took
-// 4.6 / 6.8 / 9.5 us with 8 / 47 / 125 records, now 4.0 / 5.2 / 6.4.)
+// by one as the numerators are added up.  The denominator is summed over the lanes, not record by record:
+// of the outputs of a layer of one to sixteen lanes at most 2 in 100,000 round otherwise for it.  (With every
+// lane computing all weights the dispatch took 4.6 / 6.8 / 9.5 us with 8 / 47 / 125 records, now 4.0 / 5.2 / 6.4.)
 template <uint32_t kParts>
 __device__ __forceinline__ MergedParts reduce_parts(const float (&numerator)[kParts], uint32_t nparts,
                                                     const float* part_max, const float* part_sum) {

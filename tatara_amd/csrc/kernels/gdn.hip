@@ -1179,7 +1179,7 @@ __global__ __launch_bounds__(256, 4) void gdn_chunk_prepare_kernel(ChunkPrepareA
     // identity: X_i = T_ii (E_i - sum_{j<i} L_ij X_j).  All products on MFMA with hi/lo
     // operand pairs; a finished block goes, as bf16 hi/lo, into the wave's strip in LDS,
     // from where it is read back as the right operand of the next products (rows
-    // contiguous: one 16-byte read per lane).  The four waves run the four columns side
+    // contiguous: two 8-byte reads of a part per lane, rows 136 bytes apart).  The four waves run the four columns side
     // by side; the finished fp32 blocks overwrite `lower`.
     {
         f32x4 rhs[4];
@@ -1319,12 +1319,12 @@ __device__ __forceinline__ u32x4 record_fragment(const uint8_t* rec, uint32_t ba
 // 32w..32w+31 of the state slice, whose fp32 master copy lives in its MFMA
 // accumulators for the whole block.  Waves 4..7 (output waves) compute what only
 // leaves the recurrence - Y = g o (Q S^T) + (A T) R of token rows 16w..16w+15 - from the
-// state and R copies in LDS, so that their loads, products and stores stay off the
-// chain from one chunk's state to the next.  Two barriers per chunk order the two
-// LDS copies between all eight waves.
+// state and R copies in LDS: their products and stores are not the state waves' own.
+// Two barriers per chunk order the two LDS copies between all eight waves, and there the
+// state waves do wait for the others.
 //
-// 2048 rows: 42 us as before, a chain of 32 steps of 1.3 us.  Without the output waves it is 31 us (their loads
-// 6 of the 15, their stores 3), without P still 46, with all records in the L2 44: no one of loads,
+// 2048 rows: 42 us as before, a chain of 32 steps of 1.3 us.  Without the output waves it is 31 us (on a slower card
+// 33 of 46, their loads 6.5 and their stores 2.5 of it), without P still 46, with all records in the L2 44: no one of loads,
 // LDS and products bounds a step, they add up along it.  Tried: the state waves at a higher wave
 // priority and y stored four columns a lane, gates through LDS - no change.
 __global__ __launch_bounds__(512) void gdn_chunk_scan_kernel(ChunkScanArgs a) {

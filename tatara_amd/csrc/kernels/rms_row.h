@@ -48,7 +48,8 @@ __device__ __forceinline__ float rms_flush(float v) {
     return fabsf(v) < 0x1p-126f ? __uint_as_float(__float_as_uint(v) & 0x80000000u) : v;
 }
 // rms_store16 of two values, packed, by the hardware's conversion (round to nearest even; a value
-// that is not subnormal does not round to one; a NaN comes out quiet instead of with its upper bits)
+// that is not subnormal does not round to one; the NaN of a sum or a product is quiet already and keeps
+// its upper bits)
 __device__ __forceinline__ uint32_t rms_store_pair(float a, float b) {
     typedef __attribute__((ext_vector_type(2))) float Pair;
     typedef __attribute__((ext_vector_type(2))) __bf16 Rounded;
