@@ -74,7 +74,7 @@ def test_single_row_projection_bit_for_bit(family):
     print(f"[time] {family['name']}: {ms * 1e3:.1f} us", flush=True)
 
 
-@pytest.mark.parametrize("rows,tile", [(1, 16), (3, 2), (16, 16), (13, 5)])
+@pytest.mark.parametrize("rows,tile", [(1, 16), (3, 1), (3, 2), (16, 16), (13, 5)])
 @pytest.mark.parametrize("family,suffix", [(ATTN, "_ms"), (ATTN, "_ms_v2"), (GDN, "_ms"),
                                            (GDN, "_ms_v2"), (OUT, "_ms"), (OUT, "_ms_v2")],
                          ids=["attn", "attn_v2", "gdn", "gdn_v2", "out", "out_v2"])
