@@ -484,13 +484,14 @@ struct BlockTiles {
 // tiles that an XCD's workgroups take in runs.  Tiles are numbered down bands of eight tile rows (place):
 // in a whole band the tile of a workgroup's own number gives an XCD one row of tiles, a good share by
 // itself, in a lower band the rows shift from column to column.  So every round goes in runs where there is
-// one lower band of many tiles, or a wide product over a long K; otherwise whole rounds of a multiple of
-// eight workgroups do.  In runs and without, bf16:
-//   777 x 2048 x 12352, one round of 5 x 49 tiles, 39.5 and 49.5 us; 1000 x 2048 x 9216 (7 x 36) 39.5 and 53;
-//   300 x 2048 x 12352 (5 x 193) 25 and 32.5; 2500 x 2048 x 9216 (20 x 72) 108 and 111
-//   331 x 64 x 8988 (3 x 71) 5.0 and 5.4; 956 x 2304 x 572 (15 x 9) 10.3 and 10.8
-//   776 x 256 x 1119 (13 x 18) 5.5 and 5.1; 3380 x 960 x 1083 (27 x 9) 18.7 and 17.3; 11448 x 640 x 533 (90 x 5)
-//   22.7 and 21.6; 4431 x 3776 x 104 (70 x 2) 13.8 and 13.2; 74 x 256 x 1023 (3 x 16) 3.85 and 3.70
+// one lower band of many tiles, or a wide product over a long K (less wide below three whole bands);
+// otherwise whole rounds of a multiple of eight workgroups do.  In runs and without, bf16, us:
+//   777 x 2048 x 12352, one round of 5 x 49 tiles, 39.5 and 49.5     776 x 256 x 1119 (13 x 18) 5.5 and 5.1
+//   1000 x 2048 x 9216 (7 x 36) 39.5 and 53                          3380 x 960 x 1083 (27 x 9) 18.7 and 17.3
+//   300 x 2048 x 12352 (5 x 193) 25 and 32.5                         3144 x 1408 x 1189 (25 x 10) 21.5 and 21.0
+//   2500 x 2048 x 9216 (20 x 72) 108 and 111                         11448 x 640 x 533 (90 x 5) 22.7 and 21.6
+//   956 x 2304 x 572 (15 x 9) 10.3 and 10.8                          4431 x 3776 x 104 (70 x 2) 13.8 and 13.2
+//   331 x 64 x 8988 (3 x 71) 5.0 and 5.4                             74 x 256 x 1023 (3 x 16) 3.85 and 3.70
 struct BlockLaunch {
     uint32_t workgroups, runs;
 };
@@ -502,7 +503,7 @@ BlockLaunch block_launch(uint32_t rows, uint32_t in_dim, uint32_t out_dim, uint3
     const uint32_t places = compute_units * (per_unit < 2 ? per_unit : 2);
     const uint32_t workgroups = std::min(m_tiles * n_tiles, places);
     const bool low = m_tiles < 8 && m_tiles * n_tiles >= 128 && (in_dim >= 256 || Product::kTileN >= 128);
-    const bool wide = m_tiles >= 8 && n_tiles >= 9 && in_dim >= 1024;
+    const bool wide = m_tiles >= 8 && n_tiles >= (m_tiles < 24 ? 9 : 16) && in_dim >= 1024;
     const uint32_t rounds = low || wide ? kWholeRounds | kLastRound : workgroups % 8 == 0 ? kWholeRounds : 0;
     return {workgroups, rounds | workgroups % 8 << kRunsMore | workgroups / 8 << kRunsShare};
 }

@@ -169,7 +169,8 @@ DEALT_CASES = [
     # measured either way: narrow and short products were up to 9 % slower in runs, wide and low ones up to 25 % without
     ((True, True), 777, 2048, 12352), ((True, True), 1000, 2048, 9216), ((True, True), 300, 2048, 12352),
     ((True, True), 2500, 2048, 9216), ((False, False), 3380, 960, 1083), ((False, False), 11448, 640, 533),
-    ((False, False), 7210, 3392, 756), ((False, False), 4431, 3776, 104), ((False, False), 17, 3648, 17)],
+    ((False, False), 7210, 3392, 756), ((False, False), 4431, 3776, 104), ((False, False), 17, 3648, 17),
+    ((True, True), 956, 2304, 572), ((True, True), 331, 64, 8988), ((False, False), 3144, 1408, 1189)],
     ids=lambda v: str(v))
 def test_rounds_dealt_in_runs(runs, rows, in_dim, out_dim):
     from tatara_amd import backend as B
